@@ -189,12 +189,23 @@ void select_work_bind(SelectWork* w, void* base, int segs, int N);
 // selection as a bitmap, ceil(N/32) words per segment, every word written.  map (optional,
 // unordered mode only): the keys are in that storage order; indices (ties, output) are the
 // natural ones
-// digits (optional, unordered mode only): the keys' first digits (as the FFT's `digits`
+// digits (optional; unordered mode, or select_in_block): the keys' first digits (as the FFT's `digits`
 // output), read instead of the keys wherever the first digit is all a pass needs
+// mark (optional, only where select_in_block): the selected indices are also marked in the
+// approved-residue bitmaps, as hash_bitmap_launch does from the output lists
+struct SelMark {
+  int loops = 0;               // location loops (0: nothing is marked)
+  const int* ai = nullptr;     // per loop
+  unsigned* bitmap = nullptr;  // loops x bm_words
+  int bm_words = 0;
+  unsigned wmask = 0;          // W - 1
+  int* maxfirst = nullptr;     // loops
+};
+bool select_in_block(int N);   // whether one workgroup does a segment
 hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int N, int K,
                        int segs, int* out, int ordered, const SelectWork& w, hipStream_t st,
                        unsigned* bits = nullptr, const KeyMap* map = nullptr,
-                       const uint16_t* digits = nullptr);
+                       const uint16_t* digits = nullptr, const SelMark* mark = nullptr);
 
 // ---- reverse hash (bitmap of approved residues, deterministic hit list) -----------------
 struct HashArgs {

@@ -295,6 +295,8 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   items.push_back({&P->bins_scr, (size_t)L * B * e});
   items.push_back({&P->bins_f, (size_t)L * B * e});
   items.push_back({&P->bkeys, (size_t)Ll * B * ke});
+  if (select_in_block((int)B))
+    items.push_back({(void**)&P->bucket_digits, (size_t)Ll * B * 2});
   items.push_back({(void**)&P->J, (size_t)Ll * K * 4});
   items.push_back({(void**)&P->J2, (size_t)Rl * K * 4});
   void* selW_base = nullptr;
@@ -512,9 +514,17 @@ static sfft_status run_cut(sfft_plan* P, const HashArgs& h, hipStream_t st, bool
   const sfft_params& p = P->p;
   const long long W = p.W_RLFC;
   const KeyMap km = fft_keys_map(comb_fft(P, nullptr));
+  SelMark mk;
+  mk.loops = h.loops_loc;
+  mk.ai = h.ai_dev;
+  mk.bitmap = h.bitmap;
+  mk.bm_words = h.bm_words;
+  mk.wmask = (unsigned)h.W - 1u;
+  mk.maxfirst = h.maxfirst;
+  const bool marks_too = select_in_block((int)W);
   HIPCK(select_topk(P->fp32, P->comb_keys, W, (int)W, p.B_thresh, p.RLFC_loops, P->J2, 0,
-                    P->selW, st, nullptr, &km, P->comb_digits));
-  HIPCK(hash_bitmap_launch(h, st));
+                    P->selW, st, nullptr, &km, P->comb_digits, marks_too ? &mk : nullptr));
+  if (!marks_too) HIPCK(hash_bitmap_launch(h, st));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[3], st));
   return SFFT_OK;
 }
@@ -562,6 +572,7 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
   f.batch = L;
   f.store = kStoreBoth;
   f.qmax = P->qmax_B;
+  f.digits = P->bucket_digits;
   if (P->bins_perm) {   // bucket r of loop l at column r * ai_l mod B
     f.load = kLoadPerm;
     f.perm = P->d_ai;
@@ -569,7 +580,8 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
   }
   HIPCK(fft_run(f, st));
   // ascending bucket lists: the hit list is ordered by (loop, bucket, walk)
-  HIPCK(select_topk(P->fp32, P->bkeys, B, (int)B, K, Ll, P->J, 1, P->selB, st, P->jsel));
+  HIPCK(select_topk(P->fp32, P->bkeys, B, (int)B, K, Ll, P->J, 1, P->selB, st, P->jsel, nullptr,
+                    P->bucket_digits));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[5], st));
   return SFFT_OK;
 }

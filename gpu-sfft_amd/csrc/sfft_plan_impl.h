@@ -34,6 +34,7 @@ struct sfft_plan {
   void* bins_scr = nullptr;
   void* bins_f = nullptr;
   void* bkeys = nullptr;
+  uint16_t* bucket_digits = nullptr; // first select digit of each bucket key (one-workgroup select)
   int* J = nullptr;
   int* J2 = nullptr;
   SelectWork selW, selB;

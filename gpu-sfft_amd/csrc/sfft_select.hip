@@ -16,6 +16,7 @@
 //                the ascending index list the reverse hash walks in order.  The selected
 //                count of each block (its digit > d0 count from the split plus its candidates
 //                >= T) and their exclusive prefix come out of the refine.
+// Short segments (select_in_block) take one launch instead: sel_block_kernel.
 #include "sfft_internal.h"
 
 namespace sfft {
@@ -666,10 +667,322 @@ __global__ __launch_bounds__(SEL_NT) void sel_write_kernel(const K* __restrict__
   }
 }
 
+// ---- one workgroup per segment -------------------------------------------------------------
+// The whole select of a short segment in one launch.  Thread t owns the PER elements from
+// t*PER on (storage order), their first digits packed in registers: histogram, the digit d0
+// holding the K-th largest, a mask of the digit > d0 elements per thread, the digit == d0
+// candidates in an LDS list narrowed by the 12 bits below the first digit (of the value
+// rounded to FP32, as the first digit) and then by rank, and the selected indices written at
+// the scan of the masks' counts (storage order, so ascending where that is the natural one).
+// For the comb cutoff the same loop marks the approved-residue bitmaps.
+// One CU does the work, so what bounds it is instructions per element: no ballots or index
+// maps per element, only for the selected ones.
+constexpr int SB_CAP = 2048;   // candidates kept in LDS
+constexpr int SB_RANK = 64;    // survivors ranked against each other
+
+// composite key: FP32 keys and their index fit 64 bits
+template <typename K>
+struct CompOf {
+  using type = u128;
+};
+template <>
+struct CompOf<unsigned int> {
+  using type = unsigned long long;
+};
+template <typename K>
+__device__ __forceinline__ typename CompOf<K>::type composite_n(K key, unsigned idx, int N,
+                                                                int IB) {
+  using CT = typename CompOf<K>::type;
+  const K km = key & (K)(~((K)1 << KeyBits<K>::KB));
+  return ((CT)km << IB) | (CT)(unsigned)((unsigned)(N - 1) - idx);
+}
+
+// the 12 bits below the first digit, of the same (rounded) value: non-decreasing in the key
+// among keys of one first digit
+__device__ __forceinline__ unsigned second_digit(unsigned key) { return (key >> 7) & 0xFFFu; }
+__device__ __forceinline__ unsigned second_digit(unsigned long long key) {
+  const float f = __double2float_rn(__longlong_as_double((long long)key));
+  return (__float_as_uint(f) >> 7) & 0xFFFu;
+}
+
+// The bin of h[0, nb) holding the r-th largest element, the count above it and the bin's own
+// count, to s_pick[0..2] (every thread calls; nb <= SEL_BINS, 1024 threads).
+__device__ __forceinline__ void sb_pick(const unsigned* h, int nb, int r, int* sh, int* s_pick) {
+  const int tid = threadIdx.x;
+  unsigned v[4];
+  int S = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int rank = 4 * tid + j;
+    v[j] = rank < nb ? h[nb - 1 - rank] : 0u;
+    S += (int)v[j];
+  }
+  const int E = block_excl_scan_s(S, sh);
+  if (E < r && r <= E + S) {
+    int cum = E;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (cum + (int)v[j] >= r) {
+        s_pick[0] = nb - 1 - (4 * tid + j);
+        s_pick[1] = cum;
+        s_pick[2] = (int)v[j];
+        break;
+      }
+      cum += (int)v[j];
+    }
+  }
+  __syncthreads();
+}
+
+template <typename K, int PER>
+__global__ __launch_bounds__(SEL_NT) void sel_block_kernel(const K* __restrict__ keys,
+                                                           long long seg_stride, int N, int Ksel,
+                                                           int* __restrict__ out,
+                                                           unsigned* __restrict__ bits,
+                                                           KeyMap km,
+                                                           const uint16_t* __restrict__ digits,
+                                                           int vec, SelMark mark) {
+  using CT = typename CompOf<K>::type;
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ unsigned h[SEL_BINS];
+  __shared__ K lkey[SB_CAP];
+  __shared__ int lpos[SB_CAP];
+  __shared__ unsigned picked[SEL_NT];   // candidates selected, as their owners' bits
+  __shared__ CT rkey[SB_RANK];
+  __shared__ int rpos[SB_RANK];
+  __shared__ int sh[16];
+  __shared__ int s_pick[3];
+  __shared__ int s_nc;
+  const int tid = threadIdx.x, seg = blockIdx.x;
+  const int IB = index_bits(N), TB = KeyBits<K>::KB + IB;
+  const K* kp = keys + (long long)seg * seg_stride;
+  const int i0 = tid * PER;
+  auto comp_at = [&](K key, int i) __attribute__((always_inline)) {
+    return composite_n<K>(key, (unsigned)key_natural(km, i), N, IB);
+  };
+  auto pick_one = [&](int i) __attribute__((always_inline)) {
+    atomicOr(&picked[i / PER], 1u << (i % PER));
+  };
+
+  // 1. the first digits of the thread's elements, two per register; past N: 0xFFFF (no digit)
+  unsigned pd[PER / 2];
+  if (digits) {
+    const uint16_t* dp = digits + (long long)seg * seg_stride;
+#pragma unroll
+    for (int j = 0; j < PER; j += 8) {
+      if (vec && i0 + j + 8 <= N) {
+        const u32x4 v = *(const u32x4*)(dp + i0 + j);
+        pd[j / 2] = v.x;
+        pd[j / 2 + 1] = v.y;
+        pd[j / 2 + 2] = v.z;
+        pd[j / 2 + 3] = v.w;
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; u += 2) {
+          const int i = i0 + j + u;
+          const unsigned a = i < N ? dp[i] : 0xFFFFu, b = i + 1 < N ? dp[i + 1] : 0xFFFFu;
+          pd[(j + u) / 2] = a | (b << 16);
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < PER; j += 8) {
+      K k[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) k[u] = kp[min(i0 + j + u, N - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) {
+        const int i = i0 + j + u;
+        const unsigned a = i < N ? top_digit<K>(k[u]) : 0xFFFFu;
+        const unsigned b = i + 1 < N ? top_digit<K>(k[u + 1]) : 0xFFFFu;
+        pd[(j + u) / 2] = a | (b << 16);
+      }
+    }
+  }
+  auto digit = [&](int j) __attribute__((always_inline)) {
+    return (pd[j / 2] >> ((j & 1) * 16)) & 0xFFFFu;
+  };
+  for (int i = tid; i < SEL_BINS; i += SEL_NT) h[i] = 0u;
+  picked[tid] = 0u;
+  if (tid == 0) s_nc = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const unsigned d = digit(j);
+    if (d < (unsigned)SEL_BINS) atomicAdd(&h[d], 1u);
+  }
+  __syncthreads();
+  sb_pick(h, SEL_BINS, Ksel, sh, s_pick);
+  const unsigned d0 = (unsigned)s_pick[0];
+  int r = Ksel - s_pick[1];      // still to select among the candidates
+  int nc = s_pick[2];
+  unsigned sel = 0u, cand = 0u;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const unsigned d = digit(j);
+    sel |= (unsigned)(d > d0 && d < (unsigned)SEL_BINS) << j;
+    cand |= (unsigned)(d == d0) << j;
+  }
+
+  // 2. the r largest of the nc candidates
+  if (nc == r) {
+    sel |= cand;
+  } else {
+    bool small = nc <= SB_CAP;
+    if (small) {
+      for (unsigned m = cand; m; m &= m - 1) {
+        const int i = i0 + __ffs(m) - 1;
+        const int q = atomicAdd(&s_nc, 1);
+        lkey[q] = kp[i];
+        lpos[q] = i;
+      }
+      __syncthreads();   // (also: every thread has read s_pick and h)
+      for (int i = tid; i < SEL_BINS; i += SEL_NT) h[i] = 0u;
+      __syncthreads();
+      for (int j = tid; j < nc; j += SEL_NT) atomicAdd(&h[second_digit(lkey[j])], 1u);
+      __syncthreads();
+      const int nc1 = nc;
+      sb_pick(h, SEL_BINS, r, sh, s_pick);
+      const int alive = s_pick[2], r1 = r - s_pick[1];
+      if (alive == r1 || alive <= SB_RANK) {
+        const unsigned d1 = (unsigned)s_pick[0];
+        if (tid == 0) s_nc = 0;
+        __syncthreads();
+        for (int j = tid; j < nc1; j += SEL_NT) {
+          const K key = lkey[j];
+          const unsigned d = second_digit(key);
+          if (d > d1 || (d == d1 && alive == r1)) {
+            pick_one(lpos[j]);
+          } else if (d == d1) {
+            const int q = atomicAdd(&s_nc, 1);
+            rkey[q] = comp_at(key, lpos[j]);
+            rpos[q] = lpos[j];
+          }
+        }
+        r = r1;
+        nc = alive;
+      } else {
+        small = false;
+      }
+    }
+    if (!small) {
+      // many candidates share what was looked at (flat or tied data): narrow them by the
+      // digits of the composite, whose index bits all differ, reading the keys again
+      CT prefix = 0;
+      int consumed = 0;
+      do {
+        const int width = min(SEL_DIG, TB - consumed), shift = TB - consumed - width;
+        __syncthreads();
+        for (int i = tid; i < SEL_BINS; i += SEL_NT) h[i] = 0u;
+        __syncthreads();
+        for (unsigned m = cand; m; m &= m - 1) {
+          const int i = i0 + __ffs(m) - 1;
+          const CT c = comp_at(kp[i], i);
+          if (consumed == 0 || (c >> (shift + width)) == prefix)
+            atomicAdd(&h[(unsigned)(c >> shift) & ((1u << width) - 1u)], 1u);
+        }
+        __syncthreads();
+        sb_pick(h, 1 << width, r, sh, s_pick);
+        prefix = (prefix << width) | (CT)(unsigned)s_pick[0];
+        r -= s_pick[1];
+        nc = s_pick[2];
+        consumed += width;
+      } while (nc > SB_RANK && nc != r);
+      if (tid == 0) s_nc = 0;
+      __syncthreads();
+      for (unsigned m = cand; m; m &= m - 1) {
+        const int i = i0 + __ffs(m) - 1;
+        const CT c = comp_at(kp[i], i), pre = c >> (TB - consumed);
+        if (pre > prefix || (pre == prefix && nc == r)) {
+          pick_one(i);
+        } else if (pre == prefix) {
+          const int q = atomicAdd(&s_nc, 1);
+          rkey[q] = c;
+          rpos[q] = i;
+        }
+      }
+    }
+    __syncthreads();
+    if (nc != r && tid < nc) {   // by rank: the composites are distinct
+      const CT c = rkey[tid];
+      int above = 0;
+      for (int j = 0; j < nc; ++j) above += rkey[j] > c ? 1 : 0;
+      if (above < r) pick_one(rpos[tid]);
+    }
+    __syncthreads();
+    sel |= picked[tid];
+  }
+
+  // 3. the selection: as a bitmap, and as the index list in storage order
+  if (bits) {
+    unsigned* bw = bits + (long long)seg * ((N + 31) / 32);
+    const int nb = (N + 31) / 32 * 32;   // every bit of every word is written
+    if (i0 < nb) {
+      if (PER == 8) ((uint8_t*)bw)[tid] = (uint8_t)sel;
+      if (PER == 16) ((uint16_t*)bw)[tid] = (uint16_t)sel;
+      if (PER == 32) bw[tid] = sel;
+    }
+  }
+  int pos = block_excl_scan_s(__popc(sel), sh);
+  int* o = out + (long long)seg * Ksel;
+  for (unsigned m = sel; m; m &= m - 1) {
+    const unsigned nat = (unsigned)key_natural(km, i0 + __ffs(m) - 1);
+    o[pos++] = (int)nat;
+    for (int l = 0; l < mark.loops; ++l) {
+      const unsigned f = (nat * (unsigned)mark.ai[l]) & mark.wmask;
+      atomicOr(&mark.bitmap[(size_t)l * mark.bm_words + (f >> 5)], 1u << (f & 31));
+    }
+  }
+  // the largest approved residue of each location loop
+  for (int l = 0; l < mark.loops; ++l) {
+    const unsigned a = (unsigned)mark.ai[l];
+    int v = -1;
+    for (unsigned m = sel; m; m &= m - 1)
+      v = max(v, (int)(((unsigned)key_natural(km, i0 + __ffs(m) - 1) * a) &
+                       mark.wmask));
+#pragma unroll
+    for (int q = 32; q > 0; q >>= 1) v = max(v, __shfl_xor(v, q, 64));
+    __syncthreads();
+    if ((tid & 63) == 0) sh[tid >> 6] = v;
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < SEL_NT / 64; ++w) v = max(v, sh[w]);
+      if (v >= 0) atomicMax(&mark.maxfirst[l], v);
+    }
+  }
+}
+
+template <typename K>
+static void sel_block_go(const K* keys, long long seg_stride, int N, int Ksel, int segs, int* out,
+                         unsigned* bits, const KeyMap& km, const uint16_t* digits,
+                         const SelMark& mark, hipStream_t st) {
+  const int vec = ((uintptr_t)digits & 15) == 0 && (seg_stride & 7) == 0;   // 16-byte loads
+  const dim3 grid(segs), nt(SEL_NT);
+#define SFFT_SB(PER)                                                                            \
+  if (N <= PER * SEL_NT) {                                                                      \
+    hipLaunchKernelGGL((sel_block_kernel<K, PER>), grid, nt, 0, st, keys, seg_stride, N, Ksel,  \
+                       out, bits, km, digits, vec, mark);                                       \
+    return;                                                                                     \
+  }
+  SFFT_SB(8)
+  SFFT_SB(16)
+  SFFT_SB(32)
+#undef SFFT_SB
+}
+
+// Up to 32768 keys one workgroup beats the chain of launches, in both precisions; at 65536 its
+// one CU takes as long as the launches it saves (whole graph transforms, chain -> one workgroup:
+// comb of 8192 keys FP64 128 -> 95 us, FP32 128 -> 96; 16384: 151 -> 117, 150 -> 115; 32768:
+// 143 -> 112, 139 -> 113; 65536: 153.4 -> 158.5, 141 -> 153).
+constexpr int SB_MAX_N = 32768;
+bool select_in_block(int N) { return N <= SB_MAX_N; }
+
 template <typename K>
 static hipError_t select_impl(const K* keys, long long seg_stride, int N, int Ksel, int segs,
                               int* out, int ordered, const SelectWork& w, hipStream_t st,
-                              unsigned* bits, const KeyMap* map, const uint16_t* digits) {
+                              unsigned* bits, const KeyMap* map, const uint16_t* digits,
+                              const SelMark* mark) {
   const int chunk = sel_chunk(N);
   const int nchunks = (N + chunk - 1) / chunk;
   if (nchunks > SEL_MAX_CHUNKS || nchunks > w.max_chunks || segs > w.max_segs)
@@ -680,6 +993,12 @@ static hipError_t select_impl(const K* keys, long long seg_stride, int N, int Ks
     if (ordered || (1LL << map->log2n) != (long long)N) return hipErrorInvalidValue;
     km = *map;
   }
+  if (select_in_block(N)) {
+    sel_block_go<K>(keys, seg_stride, N, Ksel, segs, out, bits, km, digits,
+                    mark ? *mark : SelMark(), st);
+    return hipGetLastError();
+  }
+  if (mark) return hipErrorInvalidValue;   // only the one-workgroup select marks
   dim3 grid(nchunks, segs);
   SelState* S = (SelState*)w.state;
   // work layout: column sums, then the per-block histogram rows
@@ -716,14 +1035,16 @@ static hipError_t select_impl(const K* keys, long long seg_stride, int N, int Ks
 
 hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int N, int K,
                        int segs, int* out, int ordered, const SelectWork& w, hipStream_t st,
-                       unsigned* bits, const KeyMap* map, const uint16_t* digits) {
-  if (ordered && digits) return hipErrorInvalidValue;   // the write pass reads the keys
+                       unsigned* bits, const KeyMap* map, const uint16_t* digits,
+                       const SelMark* mark) {
+  // the write pass reads the keys
+  if (ordered && digits && !select_in_block(N)) return hipErrorInvalidValue;
   if (N < 2 || K < 1 || K > N || segs < 1) return hipErrorInvalidValue;
   if (is_fp32)
     return select_impl<unsigned int>((const unsigned int*)keys, seg_stride, N, K, segs, out,
-                                     ordered, w, st, bits, map, digits);
+                                     ordered, w, st, bits, map, digits, mark);
   return select_impl<unsigned long long>((const unsigned long long*)keys, seg_stride, N, K, segs,
-                                         out, ordered, w, st, bits, map, digits);
+                                         out, ordered, w, st, bits, map, digits, mark);
 }
 
 }  // namespace sfft
