@@ -55,11 +55,10 @@ static sfft_status dft_any_device(double2* d_data, int N, int inverse, hipStream
   void *scr = nullptr, *A = nullptr, *Bv = nullptr, *c = nullptr, *tmp = nullptr;
   if (N <= 1) return SFFT_OK;
   if (l2 >= 0) {
-    HCK(hipMalloc(&scr, (size_t)N * 16));
-    HCK(hipMalloc(&tmp, (size_t)N * 16));
+    HCK(work_alloc(&scr, (size_t)N * 16, st));
+    HCK(work_alloc(&tmp, (size_t)N * 16, st));
     HCK(hipMemcpyAsync(tmp, d_data, (size_t)N * 16, hipMemcpyDeviceToDevice, st));
     HCK(fft_plain(tmp, d_data, scr, l2, 1, inverse, 0, st));
-    HCK(hipStreamSynchronize(st));
     goto done;
   }
   {
@@ -68,11 +67,11 @@ static sfft_status dft_any_device(double2* d_data, int N, int inverse, hipStream
     const long long M = 1LL << lm;
     std::vector<double2> hc, hb;
     const double sgn = inverse ? 1.0 : -1.0;
-    HCK(hipMalloc(&c, (size_t)N * 16));
-    HCK(hipMalloc(&A, (size_t)M * 16));
-    HCK(hipMalloc(&Bv, (size_t)M * 16));
-    HCK(hipMalloc(&tmp, (size_t)M * 16));
-    HCK(hipMalloc(&scr, (size_t)M * 16));
+    HCK(work_alloc(&c, (size_t)N * 16, st));
+    HCK(work_alloc(&A, (size_t)M * 16, st));
+    HCK(work_alloc(&Bv, (size_t)M * 16, st));
+    HCK(work_alloc(&tmp, (size_t)M * 16, st));
+    HCK(work_alloc(&scr, (size_t)M * 16, st));
     if (device_chirp) {
       HCK(aux_chirp((double2*)c, (double2*)tmp, N, M, inverse, st));
       goto chirp_ready;
@@ -93,8 +92,10 @@ static sfft_status dft_any_device(double2* d_data, int N, int inverse, hipStream
       hb[m] = make_double2(hc[m].x, -hc[m].y);
       hb[M - m] = hb[m];
     }
-    HCK(hipMemcpy(c, hc.data(), (size_t)N * 16, hipMemcpyHostToDevice));
-    HCK(hipMemcpy(tmp, hb.data(), (size_t)M * 16, hipMemcpyHostToDevice));
+    // in stream order (the scratch may still be another call's before it on the stream)
+    HCK(hipMemcpyAsync(c, hc.data(), (size_t)N * 16, hipMemcpyHostToDevice, st));
+    HCK(hipMemcpyAsync(tmp, hb.data(), (size_t)M * 16, hipMemcpyHostToDevice, st));
+    HCK(hipStreamSynchronize(st));
   chirp_ready:
     HCK(fft_plain(tmp, Bv, scr, lm, 1, 0, 0, st));
     HCK(aux_bluestein_pre(d_data, (const double2*)c, (double2*)tmp, N, M, st));
@@ -102,20 +103,21 @@ static sfft_status dft_any_device(double2* d_data, int N, int inverse, hipStream
     HCK(aux_cmul_pointwise((double2*)A, (const double2*)Bv, M, st));
     HCK(fft_plain(A, tmp, scr, lm, 1, 1, 0, st));
     HCK(aux_bluestein_post((const double2*)tmp, (const double2*)c, d_data, N, (double)M, st));
-    HCK(hipStreamSynchronize(st));
   }
 done:
-  if (scr) (void)hipFree(scr);
-  if (A) (void)hipFree(A);
-  if (Bv) (void)hipFree(Bv);
-  if (c) (void)hipFree(c);
-  if (tmp) (void)hipFree(tmp);
+  work_free(scr, st);
+  work_free(A, st);
+  work_free(Bv, st);
+  work_free(c, st);
+  work_free(tmp, st);
   return status;
 }
 
 extern "C" sfft_status sfft_dft_any_device(complex_t* d_data, int N, int inverse, void* stream) {
   if (!d_data || N < 1) return SFFT_ERR_INVALID;
-  return dft_any_device((double2*)d_data, N, inverse, (hipStream_t)stream);
+  const sfft_status s = dft_any_device((double2*)d_data, N, inverse, (hipStream_t)stream);
+  if (s != SFFT_OK) return s;
+  return hipStreamSynchronize((hipStream_t)stream) == hipSuccess ? SFFT_OK : SFFT_ERR_HIP;
 }
 
 // The parallel design: the same filter with every n-length step on the device and no
@@ -130,34 +132,40 @@ static sfft_status make_filter_parallel(double tolerance, int n, int ln, int b_f
   void *dv = nullptr, *g = nullptr, *G = nullptr, *scr = nullptr, *pan = nullptr, *mx = nullptr;
   const long long nb = aux_boxcar_blocks(n);
   double2* F = nullptr;
-  HCK(hipMalloc(&dv, (size_t)w * 16));
+  FftLaunch fold, head;
+  HCK(work_alloc(&dv, (size_t)w * 16, st));
   HCK(aux_cheb_samples((double2*)dv, w, tolerance, st));
   status = dft_any_device((double2*)dv, w, 0, st, true);
   if (status != SFFT_OK) goto done;
   HCK(aux_shift_real((const double2*)dv, (double2*)d_filter_time, w, st));
-  HCK(hipMalloc(&g, (size_t)n * 16));
-  HCK(hipMalloc(&G, (size_t)n * 16));
-  HCK(hipMalloc(&scr, (size_t)n * 16));
-  HCK(hipMalloc(&pan, (size_t)(n / 64 + n / 4096) * 16));
-  HCK(hipMalloc(&mx, (size_t)(nb + 1) * 8));
-  HCK(aux_fold((const double2*)d_filter_time, (double2*)g, w, n, st));
-  HCK(fft_plain(g, G, scr, ln, 1, 0, 0, st));
+  HCK(work_alloc(&g, (size_t)n * 16, st));
+  HCK(work_alloc(&G, (size_t)n * 16, st));
+  HCK(work_alloc(&scr, (size_t)n * 16, st));
+  HCK(work_alloc(&pan, (size_t)(n / 64 + n / 4096) * 16, st));
+  HCK(work_alloc(&mx, (size_t)(nb + 1) * 8, st));
+  // the FFT loads the folded taps straight from the window (no n-length array of them)
+  fold.load = kLoadTaps;
+  fold.taps = w;
+  HCK(fft_special(fold, d_filter_time, G, scr, ln, 1, 0, 0, st));
   HCK(aux_boxcar((const double2*)G, (double2*)g, n, b_f, (double2*)pan, (double*)mx + 1,
                  (double*)mx, st));
   F = d_filter_freq ? (double2*)d_filter_freq : (double2*)g;
   HCK(aux_ramp((const double2*)g, F, n, w / 2, (const double*)mx, st));
   if (h_filter_freq)
     HCK(hipMemcpyAsync(h_filter_freq, F, (size_t)n * 16, hipMemcpyDeviceToHost, st));
-  HCK(fft_plain(F, G, scr, ln, 1, 1, 0, st));
-  HCK(aux_scale_head((const double2*)G, (double2*)d_filter_time, w, (double)n, st));
+  head.store = kStoreHead;   // of the inverse FFT only the w taps are wanted
+  head.mid = G;
+  head.head = w;
+  head.scale = 1.0 / (double)n;
+  HCK(fft_special(head, F, d_filter_time, scr, ln, 1, 1, 0, st));
   HCK(hipStreamSynchronize(st));
 done:
-  if (dv) (void)hipFree(dv);
-  if (g) (void)hipFree(g);
-  if (G) (void)hipFree(G);
-  if (scr) (void)hipFree(scr);
-  if (pan) (void)hipFree(pan);
-  if (mx) (void)hipFree(mx);
+  work_free(dv, st);
+  work_free(g, st);
+  work_free(G, st);
+  work_free(scr, st);
+  work_free(pan, st);
+  work_free(mx, st);
   return status;
 }
 
@@ -180,7 +188,9 @@ extern "C" sfft_status sfft_make_filter_ex(double lobefrac, double tolerance, in
                                 d_filter_freq, st);
   }
   sfft_status status = SFFT_OK;
-  void *dv = nullptr, *g = nullptr, *G = nullptr, *scr = nullptr;
+  void *dv = nullptr, *G = nullptr, *scr = nullptr, *mid = nullptr;
+  int passes[8];
+  FftLaunch fold, head;
   std::vector<double2> hv((size_t)w);
   std::vector<double2> hG;
   complex_t* ff = h_filter_freq;
@@ -192,16 +202,16 @@ extern "C" sfft_status sfft_make_filter_ex(double lobefrac, double tolerance, in
     hv[i].x = std::isnan(val) ? 0.0 : val;
     hv[i].y = 0.0;
   }
-  HCK(hipMalloc(&dv, (size_t)w * 16));
-  HCK(hipMemcpy(dv, hv.data(), (size_t)w * 16, hipMemcpyHostToDevice));
+  HCK(work_alloc(&dv, (size_t)w * 16, st));
+  HCK(hipMemcpyAsync(dv, hv.data(), (size_t)w * 16, hipMemcpyHostToDevice, st));
   status = dft_any_device((double2*)dv, w, 0, st);   // FFT_w, cuExperiment.cu:305-308
   if (status != SFFT_OK) goto done;
   HCK(aux_shift_real((const double2*)dv, (double2*)d_filter_time, w, st));   // cuShift + Kernel2
-  HCK(hipMalloc(&g, (size_t)n * 16));
-  HCK(hipMalloc(&G, (size_t)n * 16));
-  HCK(hipMalloc(&scr, (size_t)n * 16));
-  HCK(aux_fold((const double2*)d_filter_time, (double2*)g, w, n, st));       // :336-352 (drops f[w-1])
-  HCK(fft_plain(g, G, scr, ln, 1, 0, 0, st));                               // FFT_n, :362-365
+  HCK(work_alloc(&G, (size_t)n * 16, st));
+  HCK(work_alloc(&scr, (size_t)n * 16, st));
+  fold.load = kLoadTaps;                                                    // :336-352 (drops f[w-1])
+  fold.taps = w;
+  HCK(fft_special(fold, d_filter_time, G, scr, ln, 1, 0, 0, st));           // FFT_n, :362-365
   hG.resize((size_t)n);
   HCK(hipMemcpyAsync(hG.data(), G, (size_t)n * 16, hipMemcpyDeviceToHost, st));
   HCK(hipStreamSynchronize(st));
@@ -244,17 +254,21 @@ extern "C" sfft_status sfft_make_filter_ex(double lobefrac, double tolerance, in
       oy = ny;
     }
   }
-  HCK(hipMemcpy(G, ff, (size_t)n * 16, hipMemcpyHostToDevice));
+  HCK(hipMemcpyAsync(G, ff, (size_t)n * 16, hipMemcpyHostToDevice, st));
   if (d_filter_freq)
     HCK(hipMemcpyAsync(d_filter_freq, G, (size_t)n * 16, hipMemcpyDeviceToDevice, st));
-  HCK(fft_plain(G, g, scr, ln, 1, 1, 0, st));                               // IFFT_n, :424-426
-  HCK(aux_scale_head((const double2*)g, (double2*)d_filter_time, w, (double)n, st));  // Kernel2
+  if (fft_plan_passes(ln, passes) > 2) HCK(work_alloc(&mid, (size_t)n * 16, st));
+  head.mid = mid;
+  head.store = kStoreHead;                                                  // IFFT_n, :424-426, and
+  head.head = w;                                                            // Kernel2 (w taps, / n)
+  head.scale = 1.0 / (double)n;
+  HCK(fft_special(head, G, d_filter_time, scr, ln, 1, 1, 0, st));
   HCK(hipStreamSynchronize(st));
 done:
-  if (dv) (void)hipFree(dv);
-  if (g) (void)hipFree(g);
-  if (G) (void)hipFree(G);
-  if (scr) (void)hipFree(scr);
+  work_free(dv, st);
+  work_free(mid, st);
+  work_free(G, st);
+  work_free(scr, st);
   return status;
 }
 
@@ -384,16 +398,16 @@ extern "C" sfft_status sfft_signal_synthesize(int n, int k, const int* h_locs,
   hipStream_t st = (hipStream_t)stream;
   sfft_status status = SFFT_OK;
   void *X = nullptr, *y = nullptr, *scr = nullptr, *dl = nullptr, *dv = nullptr;
-  HCK(hipMalloc(&X, (size_t)n * 16));
-  HCK(hipMalloc(&scr, (size_t)n * 16));
-  HCK(hipMalloc(&dl, (size_t)k * 4));
-  HCK(hipMalloc(&dv, (size_t)k * 16));
+  HCK(work_alloc(&X, (size_t)n * 16, st));
+  HCK(work_alloc(&scr, (size_t)n * 16, st));
+  HCK(work_alloc(&dl, (size_t)k * 4, st));
+  HCK(work_alloc(&dv, (size_t)k * 16, st));
   HCK(hipMemsetAsync(X, 0, (size_t)n * 16, st));
   HCK(hipMemcpyAsync(dl, h_locs, (size_t)k * 4, hipMemcpyHostToDevice, st));
   HCK(hipMemcpyAsync(dv, h_vals, (size_t)k * 16, hipMemcpyHostToDevice, st));
   HCK(aux_scatter_c128((double2*)X, (const int*)dl, (const double2*)dv, k, st));
   if (x_fp32) {
-    HCK(hipMalloc(&y, (size_t)n * 16));
+    HCK(work_alloc(&y, (size_t)n * 16, st));
   } else {
     y = d_x;
   }
@@ -405,15 +419,18 @@ extern "C" sfft_status sfft_signal_synthesize(int n, int k, const int* h_locs,
   if (x_fp32) HCK(aux_c128_to_c64((const double2*)y, (float2*)d_x, n, st));
   HCK(hipStreamSynchronize(st));
 done:
-  if (X) (void)hipFree(X);
-  if (scr) (void)hipFree(scr);
-  if (dl) (void)hipFree(dl);
-  if (dv) (void)hipFree(dv);
-  if (x_fp32 && y) (void)hipFree(y);
+  work_free(X, st);
+  work_free(scr, st);
+  work_free(dl, st);
+  work_free(dv, st);
+  if (x_fp32) work_free(y, st);
   return status;
 }
 
-// truth spectrum X = FFT_n(x) / n in FP64 (cuExperiment.cu:103-111), device complex128[n]
+// truth spectrum X = FFT_n(x) / n in FP64 (cuExperiment.cu:103-111), device complex128[n].  The
+// first pass widens a complex64 signal as it loads it and the last one scales as it stores, so
+// the passes of the FFT are all the traffic there is (n = 2^22, complex64: 76 us of kernels, where
+// the conversion, the copy and the scaling of their own made 131).
 extern "C" sfft_status sfft_truth_spectrum(const void* d_x, int n, int x_fp32, complex_t* d_X,
                                            void* stream) {
   const int ln = ilog2_pow2(n);
@@ -421,31 +438,36 @@ extern "C" sfft_status sfft_truth_spectrum(const void* d_x, int n, int x_fp32, c
   hipStream_t st = (hipStream_t)stream;
   sfft_status status = SFFT_OK;
   void *in = nullptr, *scr = nullptr;
-  HCK(hipMalloc(&scr, (size_t)n * 16));
-  HCK(hipMalloc(&in, (size_t)n * 16));
-  if (x_fp32)
-    HCK(aux_c64_to_c128((const float2*)d_x, (double2*)in, n, st));
-  else
-    HCK(hipMemcpyAsync(in, d_x, (size_t)n * 16, hipMemcpyDeviceToDevice, st));
-  HCK(fft_plain(in, d_X, scr, ln, 1, 0, 0, st));
-  HCK(aux_scale_c128((double2*)d_X, n, (double)n, st));
+  const size_t xb = (size_t)n * (x_fp32 ? 8 : 16), Xb = (size_t)n * 16;
+  FftLaunch L;
+  HCK(work_alloc(&scr, Xb, st));
+  if ((const char*)d_x < (const char*)d_X + Xb && (const char*)d_X < (const char*)d_x + xb) {
+    // the signal and its spectrum share memory: transform a copy of the signal
+    HCK(work_alloc(&in, xb, st));
+    HCK(hipMemcpyAsync(in, d_x, xb, hipMemcpyDeviceToDevice, st));
+  }
+  L.load = x_fp32 ? kLoadWiden : kLoadPlain;
+  L.store = kStoreHead;
+  L.head = n;
+  L.scale = 1.0 / (double)n;
+  HCK(fft_special(L, in ? in : d_x, d_X, scr, ln, 1, 0, 0, st));
   HCK(hipStreamSynchronize(st));
 done:
-  if (in) (void)hipFree(in);
-  if (scr) (void)hipFree(scr);
+  work_free(in, st);
+  work_free(scr, st);
   return status;
 }
 
 static double device_energy(const double2* a, long long n, hipStream_t st, hipError_t* err) {
   const int nb = 2048;
   double* part = nullptr;
-  *err = hipMalloc(&part, nb * sizeof(double));
+  *err = work_alloc((void**)&part, nb * sizeof(double), st);
   if (*err != hipSuccess) return 0.0;
   std::vector<double> h(nb);
   *err = aux_energy_partials(a, n, part, nb, st);
   if (*err == hipSuccess) *err = hipMemcpyAsync(h.data(), part, nb * 8, hipMemcpyDeviceToHost, st);
   if (*err == hipSuccess) *err = hipStreamSynchronize(st);
-  (void)hipFree(part);
+  work_free(part, st);
   double s = 0.0;
   for (double v : h) s += v;
   return s;
@@ -496,17 +518,18 @@ extern "C" sfft_status sfft_metric(const Node* nodes, int I_F, int k, const int*
   void *di = nullptr, *dt = nullptr, *dz = nullptr;
   double e_out = 0.0, e_sup = 0.0, e_miss = 0.0, mabs = 0.0;
   hipError_t herr = hipSuccess;
-  HCK(hipMalloc(&di, (size_t)ni * 4));
-  HCK(hipMalloc(&dt, (size_t)ni * 16));
-  HCK(hipMemcpy(di, idx.data(), (size_t)ni * 4, hipMemcpyHostToDevice));
+  HCK(work_alloc(&di, (size_t)ni * 4, st));
+  HCK(work_alloc(&dt, (size_t)ni * 16, st));
+  HCK(hipMemcpyAsync(di, idx.data(), (size_t)ni * 4, hipMemcpyHostToDevice, st));
   HCK(aux_gather_c128((const double2*)d_X, (const int*)di, (double2*)dt, ni, st));
   HCK(hipMemcpyAsync(tv.data(), dt, (size_t)ni * 16, hipMemcpyDeviceToHost, st));
   HCK(hipStreamSynchronize(st));
   // energy outside the support: zero the support entries, sum, restore
   if (top > 0) {
     std::vector<double2> zeros(top, make_double2(0.0, 0.0));
-    HCK(hipMalloc(&dz, (size_t)top * 16));
-    HCK(hipMemcpy(dz, zeros.data(), (size_t)top * 16, hipMemcpyHostToDevice));
+    HCK(work_alloc(&dz, (size_t)top * 16, st));
+    HCK(hipMemcpyAsync(dz, zeros.data(), (size_t)top * 16, hipMemcpyHostToDevice, st));
+    HCK(hipStreamSynchronize(st));   // zeros goes out of scope
     HCK(aux_scatter_c128((double2*)d_X, (const int*)di, (const double2*)dz, top, st));
   }
   e_out = device_energy((const double2*)d_X, n, st, &herr);
@@ -531,8 +554,8 @@ extern "C" sfft_status sfft_metric(const Node* nodes, int I_F, int k, const int*
   if (err_support) *err_support = e_sup + e_miss;
   if (max_abs) *max_abs = mabs;
 done:
-  if (di) (void)hipFree(di);
-  if (dt) (void)hipFree(dt);
-  if (dz) (void)hipFree(dz);
+  work_free(di, st);
+  work_free(dt, st);
+  work_free(dz, st);
   return status;
 }

@@ -145,6 +145,9 @@ struct PassArgs {
   int log2nlo, log2m;   // kLoadCombRows: g at in[(g mod 2^log2nlo) << log2m | g >> log2nlo]
   const int* perm;      // kLoadPerm: g of batch b at in[g * perm[b] mod 2^log2N]
   const int* perm_inv;  // kLoadPerm: the inverse of perm[b] mod 2^log2N
+  int taps;             // kLoadTaps
+  long long head;       // kStoreHead
+  double scale;         // kStoreHead
 };
 
 template <typename T2>
@@ -503,7 +506,19 @@ __global__ __launch_bounds__((Tile<Real, LOAD>::nt),
         src = in + ((uint32_t)q0 + (uint32_t)c + ((uint32_t)v << log2nq));
       else
         src = in + g;
-      vv[k] = *(const V2*)src;
+      if constexpr (LOAD == kLoadWiden) {
+        const NV<float>::type s = ((const NV<float>::type*)A.in)[b * A.in_bstride + g];
+        vv[k].x = (Real)s.x;
+        vv[k].y = (Real)s.y;
+      } else if constexpr (LOAD == kLoadTaps) {
+        // (a point outside the taps reads the first one and becomes zero: no branch)
+        const long long h = A.taps / 2, tail = (1LL << A.log2N) - h;
+        const bool lo = g < h, hi = g >= tail;
+        vv[k] = *(const V2*)(in + (lo ? h + g : (hi ? g - tail : 0)));
+        if (!lo && !hi) vv[k] = (V2)(Real)0;
+      } else {
+        vv[k] = *(const V2*)src;
+      }
     }
 #pragma unroll
     for (int k = 0; k < LB; ++k) {
@@ -563,7 +578,8 @@ __global__ __launch_bounds__((Tile<Real, LOAD>::nt),
   // loaded values in registers and writes only its outputs to LDS: the same operations on the
   // same values as storing the loads and running the stage, with one LDS round trip fewer.
   constexpr int FR = sizeof(Real) == 4 ? 16 : 4;
-  constexpr bool can_fuse = (LOAD == kLoadPlain || rows) && EPT == FR;
+  constexpr bool can_fuse = (LOAD == kLoadPlain || LOAD == kLoadWiden || LOAD == kLoadTaps ||
+                             rows) && EPT == FR;
   int log2ns0 = 0;
   bool fused = false;
   if constexpr (can_fuse) {
@@ -650,7 +666,7 @@ __global__ __launch_bounds__((Tile<Real, LOAD>::nt),
   // ---- store: out[q*Lcur + t + Lprev*k]
   T2* __restrict__ out = (T2*)A.out + b * A.out_bstride;
   KT* __restrict__ keys = (KT*)A.keys + b * A.keys_bstride;
-  const bool wkeys = (STORE != kStoreCplx) && (b < A.key_batches);
+  const bool wkeys = (STORE == kStoreKeys || STORE == kStoreBoth) && (b < A.key_batches);
 #pragma unroll
   for (int k = 0; k < EPT; ++k) {
     const int e = tid + k * NT;
@@ -672,7 +688,14 @@ __global__ __launch_bounds__((Tile<Real, LOAD>::nt),
         g = (q << log2Lcur) + t0 + c + Lprev * kk;
       }
       const T2 val = lds[c * RP + LPAD(kk)];
-      if (STORE != kStoreKeys) out[g] = val;
+      if constexpr (STORE == kStoreHead) {
+        T2 sv;
+        sv.x = val.x * (Real)A.scale;
+        sv.y = val.y * (Real)A.scale;
+        if (g < A.head) out[g] = sv;
+      } else if (STORE != kStoreKeys) {
+        out[g] = val;
+      }
       if (wkeys) {
         const long long kpos = A.keys_tiled ? (long long)tile * TE + e : g;
         const KT key = sample_key(val);
@@ -698,6 +721,28 @@ static hipError_t dispatch_store(const PassArgs& A, int store, int tiles, int ba
   if (store == kStoreCplx) return launch_pass<Real, LOAD, kStoreCplx, TW>(A, tiles, batch, st);
   if (store == kStoreKeys) return launch_pass<Real, LOAD, kStoreKeys, TW>(A, tiles, batch, st);
   return launch_pass<Real, LOAD, kStoreBoth, TW>(A, tiles, batch, st);
+}
+
+// the FP64-only loads and stores (truth spectra, filter design)
+static hipError_t dispatch_fp64(const PassArgs& A, int load, int store, int tw, int tiles,
+                                int batch, hipStream_t st) {
+  if (load == kLoadTaps)
+    return store == kStoreCplx
+               ? launch_pass<double, kLoadTaps, kStoreCplx, kTwNone>(A, tiles, batch, st)
+               : hipErrorInvalidValue;
+  if (load == kLoadWiden) {
+    if (store == kStoreCplx)
+      return launch_pass<double, kLoadWiden, kStoreCplx, kTwNone>(A, tiles, batch, st);
+    return store == kStoreHead
+               ? launch_pass<double, kLoadWiden, kStoreHead, kTwNone>(A, tiles, batch, st)
+               : hipErrorInvalidValue;
+  }
+  if (load != kLoadPlain) return hipErrorInvalidValue;
+  if (tw == kTwSplit)
+    return launch_pass<double, kLoadPlain, kStoreHead, kTwSplit>(A, tiles, batch, st);
+  if (tw == kTwDirect)
+    return launch_pass<double, kLoadPlain, kStoreHead, kTwDirect>(A, tiles, batch, st);
+  return launch_pass<double, kLoadPlain, kStoreHead, kTwNone>(A, tiles, batch, st);
 }
 
 // the special loads only occur in first passes (no outer twiddles)
@@ -758,8 +803,9 @@ hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
     const int r = T.logs[p];
     const int log2Lcur = log2Lprev + r;
     const bool last = (p == np - 1);
-    // pass p writes to out when (np - 1 - p) is even, else to scratch
-    void* dst = (((np - 1 - p) & 1) == 0) ? L.out : L.scratch;
+    // pass p writes to out (or mid, before the last) when (np - 1 - p) is even, else to scratch
+    void* even = (last || !L.mid) ? L.out : L.mid;
+    void* dst = (((np - 1 - p) & 1) == 0) ? even : L.scratch;
     const long long dst_stride = (dst == L.out) ? L.out_bstride : N;
     PassArgs A;
     A.in = cur_in;
@@ -802,13 +848,21 @@ hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
     A.perm_inv = L.perm_inv;
     if (load == kLoadPerm && (!L.perm || !L.perm_inv)) return hipErrorInvalidValue;
     A.nbatch = L.batch;
+    A.taps = L.taps;
+    A.head = L.head;
+    A.scale = L.scale;
     A.keys_tiled = (last && p > 0 && L.keys_tiled) ? 1 : 0;
     A.digits = last ? L.digits : nullptr;
     const int store = last ? L.store : kStoreCplx;
     const int tw = (p == 0) ? kTwNone : (log2Lcur > kMaxPassLog ? kTwSplit : kTwDirect);
     if (load != kLoadPlain && tw != kTwNone) return hipErrorInvalidValue;
-    hipError_t e = T.is_fp32 ? dispatch_pass<float>(A, load, store, tw, tiles, L.batch, st)
-                             : dispatch_pass<double>(A, load, store, tw, tiles, L.batch, st);
+    hipError_t e;
+    if (load == kLoadWiden || load == kLoadTaps || store == kStoreHead)
+      e = T.is_fp32 ? hipErrorInvalidValue
+                    : dispatch_fp64(A, load, store, tw, tiles, L.batch, st);
+    else
+      e = T.is_fp32 ? dispatch_pass<float>(A, load, store, tw, tiles, L.batch, st)
+                    : dispatch_pass<double>(A, load, store, tw, tiles, L.batch, st);
     if (e != hipSuccess) return e;
     cur_in = dst;
     cur_in_stride = dst_stride;

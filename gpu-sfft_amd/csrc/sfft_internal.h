@@ -53,8 +53,13 @@ __device__ __forceinline__ unsigned sel_first_digit(unsigned long long key) {
 
 // kLoadCombRowsG: kLoadCombRows with sibling sub-FFTs grouped per tile (chosen per pass by
 // fft_run; callers set kLoadCombRows)
-enum FftLoad { kLoadPlain = 0, kLoadComb = 1, kLoadCombRows = 2, kLoadPerm = 3, kLoadCombRowsG = 4 };
-enum FftStore { kStoreCplx = 0, kStoreKeys = 1, kStoreBoth = 2 };
+// kLoadWiden: FP64 transforms of a complex64 input, widened as it is loaded.
+// kLoadTaps: FP64 transforms of `taps` window taps t (h = taps / 2) laid out on N points:
+// element g is t[h + g] for g < h, t[g - (N - h)] for g >= N - h, else 0.
+// kStoreHead: FP64 values, the first `head` of the output, times `scale`.
+enum FftLoad { kLoadPlain = 0, kLoadComb = 1, kLoadCombRows = 2, kLoadPerm = 3, kLoadCombRowsG = 4,
+               kLoadWiden = 5, kLoadTaps = 6 };
+enum FftStore { kStoreCplx = 0, kStoreKeys = 1, kStoreBoth = 2, kStoreHead = 3 };
 
 // One canonical FFT of `batch` transforms.  Passes ping-pong between out and scratch so that
 // the last pass lands in `out` (keys for kStoreKeys/kStoreBoth).  in may equal out only for
@@ -86,6 +91,11 @@ struct FftLaunch {
   int keys_tiled = 0;            // keys in the last pass's tile order (see KeyMap)
   uint16_t* digits = nullptr;    // optional: each key's top 12 bits below the sign bit (the
                                  // select's first digit), same positions and stride as keys
+  void* mid = nullptr;           // batch * N elements for the passes before the last instead of
+                                 // out (out may then hold less than N: kStoreHead)
+  int taps = 0;                  // kLoadTaps
+  long long head = 0;            // kStoreHead
+  double scale = 1.0;            // kStoreHead
 };
 hipError_t fft_run(const FftLaunch& L, hipStream_t st);
 
@@ -258,6 +268,11 @@ hipError_t adjoint_taps_launch(const double2* f, const double2* gb, const int* a
                                int B, int w, int loops, int tiled, double2* gx, hipStream_t st);
 
 // ---- small utilities ---------------------------------------------------------------------
+// scratch memory kept between calls (sfft_pool.hip): allocated and freed in stream order, from
+// a pool of the library's own that keeps a bounded amount; work_trim gives the idle rest back
+hipError_t work_alloc(void** p, size_t bytes, hipStream_t st);
+void work_free(void* p, hipStream_t st);
+void work_trim();
 hipError_t fill_u32(void* p, uint32_t v, size_t words, hipStream_t st);
 
 }  // namespace sfft

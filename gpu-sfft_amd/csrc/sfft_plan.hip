@@ -319,8 +319,12 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   size_t total = 0;
   for (auto& it : items) total = align_up(total, 256) + align_up(it.bytes, 256);
   if (hipMalloc(&P->ws, total) != hipSuccess) {
-    delete P;
-    return SFFT_ERR_ALLOC;
+    (void)hipGetLastError();
+    work_trim();   // the scratch kept between calls may be what is missing
+    if (hipMalloc(&P->ws, total) != hipSuccess) {
+      delete P;
+      return SFFT_ERR_ALLOC;
+    }
   }
   P->ws_bytes = total;
   size_t off = 0;
@@ -969,11 +973,20 @@ extern "C" sfft_status sfft_fft_device(const void* d_in, void* d_out, int log2n,
   const void* in = d_in;
   void* tmp_in = nullptr;
   if (T->npass > 1) {
-    if (hipMallocAsync(&scratch, N * count * esz, st) != hipSuccess) return SFFT_ERR_ALLOC;
-    if (d_in == d_out) {
-      // multi-pass needs in != out: stage the input
-      if (hipMallocAsync(&tmp_in, N * count * esz, st) != hipSuccess) return SFFT_ERR_ALLOC;
-      HIPCK(hipMemcpyAsync(tmp_in, d_in, N * count * esz, hipMemcpyDeviceToDevice, st));
+    if (work_alloc(&scratch, N * count * esz, st) != hipSuccess) return SFFT_ERR_ALLOC;
+    if (d_in == d_out && (T->npass & 1)) {
+      // an odd number of passes writes the first one's output to d_out: stage the input (with
+      // an even number the first pass writes the scratch, and the input is not read again)
+      if (work_alloc(&tmp_in, N * count * esz, st) != hipSuccess) {
+        work_free(scratch, st);
+        return SFFT_ERR_ALLOC;
+      }
+      if (hipMemcpyAsync(tmp_in, d_in, N * count * esz, hipMemcpyDeviceToDevice, st) !=
+          hipSuccess) {
+        work_free(scratch, st);
+        work_free(tmp_in, st);
+        return SFFT_ERR_HIP;
+      }
       in = tmp_in;
     }
   }
@@ -988,8 +1001,8 @@ extern "C" sfft_status sfft_fft_device(const void* d_in, void* d_out, int log2n,
   L.load = kLoadPlain;
   L.store = kStoreCplx;
   err = fft_run(L, st);
-  if (scratch) (void)hipFreeAsync(scratch, st);
-  if (tmp_in) (void)hipFreeAsync(tmp_in, st);
+  work_free(scratch, st);
+  work_free(tmp_in, st);
   return err == hipSuccess ? SFFT_OK : SFFT_ERR_HIP;
 }
 
@@ -1010,13 +1023,12 @@ extern "C" int sfft_device_count(void) {
 }
 
 namespace sfft {
-hipError_t fft_plain(const void* in, void* out, void* scratch, int log2n, int count, int inverse,
-                     int is_fp32, hipStream_t st) {
+hipError_t fft_special(FftLaunch L, const void* in, void* out, void* scratch, int log2n, int count,
+                       int inverse, int is_fp32, hipStream_t st) {
   hipError_t err = hipSuccess;
   const FftTables* T = cached_tables(log2n, inverse ? 1 : 0, is_fp32, &err);
   if (!T) return err == hipSuccess ? hipErrorOutOfMemory : err;
   const long long N = 1LL << log2n;
-  FftLaunch L;
   L.tab = T;
   L.in = in;
   L.in_bstride = N;
@@ -1025,5 +1037,10 @@ hipError_t fft_plain(const void* in, void* out, void* scratch, int log2n, int co
   L.scratch = scratch;
   L.batch = count;
   return fft_run(L, st);
+}
+
+hipError_t fft_plain(const void* in, void* out, void* scratch, int log2n, int count, int inverse,
+                     int is_fp32, hipStream_t st) {
+  return fft_special(FftLaunch(), in, out, scratch, log2n, count, inverse, is_fp32, st);
 }
 }  // namespace sfft
