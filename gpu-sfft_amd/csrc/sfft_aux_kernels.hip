@@ -116,13 +116,17 @@ __global__ void chirp_kernel(double2* __restrict__ c, double2* __restrict__ b, i
   }
 }
 
+// complex128 as a native vector (arrays of HIP's double2 end up in scratch)
+typedef double d2v __attribute__((ext_vector_type(2)));
+
 // acc += a[(p0 + j) & mask] for j < cnt, added in that order, eight loads in flight at a time
 __device__ __forceinline__ void run_sum(const double2* __restrict__ a, long long p0, long long cnt,
                                         long long mask, double& sx, double& sy) {
   for (long long j = 0; j < cnt; j += 8) {
-    double2 v[8];
+    d2v v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = a[(p0 + (j + u < cnt ? j + u : cnt - 1)) & mask];
+    for (int u = 0; u < 8; ++u)
+      v[u] = ((const d2v*)a)[(p0 + (j + u < cnt ? j + u : cnt - 1)) & mask];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (j + u < cnt) {
@@ -133,40 +137,91 @@ __device__ __forceinline__ void run_sum(const double2* __restrict__ a, long long
   }
 }
 
-// ps[p] = sum of in[P p .. P p + P), one thread per panel
-__global__ void panel_sum_kernel(const double2* __restrict__ in, double2* __restrict__ ps,
-                                 long long npan, int P) {
-  for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < npan;
-       p += (long long)gridDim.x * blockDim.x) {
-    double sx = 0.0, sy = 0.0;
-    run_sum(in, p * P, P, -1LL, sx, sy);
-    ps[p] = make_double2(sx, sy);
-  }
-}
-
 constexpr int kPan1 = 64;     // level-1 panel (entries of G)
 constexpr int kPan2 = 4096;   // level-2 panel (64 level-1 panels)
 
+// One wave works on 64 rows of 64 entries (a level-2 panel): lane c walks row c in order, eight
+// entries at a time.  Read by the lanes themselves, an instruction would touch 64 lines for 16
+// bytes each; the wave instead moves 64 x 8 blocks as whole 128-byte lines (lane e of load k:
+// row k*8 + e/8, entry e%8) through LDS, the next block's lines in flight meanwhile.
+constexpr int kStep = 8;
+constexpr int kPitch = kStep + 1;   // LDS row pitch (banks)
+struct RowBlock {
+  d2v v[kStep];
+  // the 64 x 8 block whose row 0 starts at entry p0 (rows kPan1 apart, indices mod mask + 1)
+  __device__ __forceinline__ void load(const double2* __restrict__ a, long long p0,
+                                       long long mask) {
+    const int e = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kStep; ++k)
+      v[k] = ((const d2v*)a)[(p0 + (k * 8 + (e >> 3)) * (long long)kPan1 + (e & 7)) & mask];
+  }
+  __device__ __forceinline__ void put(d2v* lds) const {
+    const int e = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kStep; ++k) lds[(k * 8 + (e >> 3)) * kPitch + (e & 7)] = v[k];
+  }
+};
+
+// p1[c] = sum of in[64 c .. 64 c + 64), p2[b] = sum of p1[64 b .. 64 b + 64), both added in
+// order (block b: 64 level-1 panels)
+__global__ __launch_bounds__(64) void panel_sums_kernel(const double2* __restrict__ in,
+                                                        double2* __restrict__ p1,
+                                                        double2* __restrict__ p2) {
+  __shared__ d2v t[64 * kPitch];
+  const int c = threadIdx.x;
+  const long long i0 = blockIdx.x * (long long)kPan2;
+  double sx = 0.0, sy = 0.0;
+  RowBlock r;
+  r.load(in, i0, -1LL);
+  for (int t0 = 0; t0 < kPan1; t0 += kStep) {
+    r.put(t);
+    __syncthreads();
+    if (t0 + kStep < kPan1) r.load(in, i0 + t0 + kStep, -1LL);
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const d2v g = t[c * kPitch + u];
+      sx += g.x;
+      sy += g.y;
+    }
+    __syncthreads();
+  }
+  p1[blockIdx.x * 64LL + c] = make_double2(sx, sy);
+  t[c] = d2v{sx, sy};
+  __syncthreads();
+  if (c == 0) {
+    double ax = 0.0, ay = 0.0;
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      ax += t[j].x;
+      ay += t[j].y;
+    }
+    p2[blockIdx.x] = make_double2(ax, ay);
+  }
+}
+
 // boxcar s_i = sum of G[i .. i + b_f) (indices mod n) stored at (i + b_f/2) mod n, i.e. the
-// faithful running sum without its n-step rounding drift: each thread owns kPan1 consecutive
+// faithful running sum without its n-step rounding drift: each lane owns kPan1 consecutive
 // outputs, starts from a window sum over panel sums (at most 3*63 + b_f/4096 terms: level-1
 // panels up to a level-2 boundary, level-2 panels, level-1 panels, single entries) and slides
 // kPan1 - 1 steps.  blkmax[block] = max |s|^2 over the block's outputs.  n >= 4096.
-// A serial chain of n / 64 threads: its loads go out eight steps at a time, whole lines per
-// thread (n = 2^22: 75 -> 62 us).
-constexpr int BX_NT = 64;     // threads per block (few threads in all: spread over the CUs)
-__global__ __launch_bounds__(BX_NT) void boxcar_kernel(const double2* __restrict__ G,
-                                                       const double2* __restrict__ p1,
-                                                       const double2* __restrict__ p2,
-                                                       double2* __restrict__ out, long long n,
-                                                       long long b_f,
-                                                       double* __restrict__ blkmax) {
+// Only n / 64 lanes, each a serial chain: bound by the line requests of its loads and stores
+// until they went through LDS as whole lines (n = 2^22, with the panel sums: 102 us, then 65).
+__global__ __launch_bounds__(64) void boxcar_kernel(const double2* __restrict__ G,
+                                                    const double2* __restrict__ p1,
+                                                    const double2* __restrict__ p2,
+                                                    double2* __restrict__ out, long long n,
+                                                    long long b_f, double* __restrict__ blkmax) {
+  __shared__ d2v ta[64 * kPitch], tb[64 * kPitch];
   const long long mask = n - 1, np1 = n / kPan1, np2 = n / kPan2;
-  const long long c = blockIdx.x * (long long)BX_NT + threadIdx.x;
-  double mx2 = 0.0;
-  if (c < np1) {
-    const long long i0 = c * kPan1;
-    double sx = 0.0, sy = 0.0;
+  const long long b0 = blockIdx.x * (long long)kPan2;   // the block's first output
+  const int lane = threadIdx.x;
+  const long long c = blockIdx.x * 64LL + lane;
+  RowBlock ahead, behind;
+  ahead.load(G, b0 + b_f, mask);
+  behind.load(G, b0, mask);
+  double mx2 = 0.0, sx = 0.0, sy = 0.0;
+  {
     const long long all1 = b_f / kPan1, align = (64 - (c & 63)) & 63;
     const long long a1 = all1 < align ? all1 : align;
     run_sum(p1, c, a1, np1 - 1, sx, sy);
@@ -182,27 +237,36 @@ __global__ __launch_bounds__(BX_NT) void boxcar_kernel(const double2* __restrict
       left -= n1 * kPan1;
     }
     run_sum(G, pos * kPan1, left, mask, sx, sy);
-  const long long offset = b_f / 2;
-    for (int t0 = 0; t0 < kPan1; t0 += 8) {
-      double2 ahead[8], behind[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        ahead[u] = G[(i0 + t0 + u + b_f) & mask];
-        behind[u] = G[i0 + t0 + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        out[(i0 + t0 + u + offset) & mask] = make_double2(sx, sy);
-        const double a2 = sx * sx + sy * sy;
-        mx2 = mx2 > a2 ? mx2 : a2;
-        sx += ahead[u].x - behind[u].x;
-        sy += ahead[u].y - behind[u].y;
-      }
+  }
+  const long long o0 = b0 + b_f / 2;
+  for (int t0 = 0; t0 < kPan1; t0 += kStep) {
+    ahead.put(ta);
+    behind.put(tb);
+    __syncthreads();
+    if (t0 + kStep < kPan1) {
+      ahead.load(G, b0 + t0 + kStep + b_f, mask);
+      behind.load(G, b0 + t0 + kStep, mask);
     }
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const d2v ga = ta[lane * kPitch + u], gb = tb[lane * kPitch + u];
+      tb[lane * kPitch + u] = d2v{sx, sy};   // the output takes the read slot
+      const double a2 = sx * sx + sy * sy;
+      mx2 = mx2 > a2 ? mx2 : a2;
+      sx += ga.x - gb.x;
+      sy += ga.y - gb.y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kStep; ++k) {
+      const int row = k * 8 + (lane >> 3), u = lane & 7;
+      ((d2v*)out)[(o0 + row * (long long)kPan1 + t0 + u) & mask] = tb[row * kPitch + u];
+    }
+    __syncthreads();
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx2 = fmax(mx2, __shfl_xor(mx2, o, 64));
-  if (threadIdx.x == 0) blkmax[blockIdx.x] = mx2;
+  if (lane == 0) blkmax[blockIdx.x] = mx2;
 }
 
 // out[0] = max of part[0..np) (one block)
@@ -387,18 +451,15 @@ hipError_t aux_chirp(double2* c, double2* b, int N, long long M, int inverse, hi
                      inverse ? 1.0 : -1.0);
   return hipGetLastError();
 }
-long long aux_boxcar_blocks(long long n) { return (n / kPan1 + BX_NT - 1) / BX_NT; }
+long long aux_boxcar_blocks(long long n) { return n / kPan2; }
 hipError_t aux_boxcar(const double2* G, double2* out, long long n, long long b_f,
                       double2* panels, double* blkmax, double* mx2, hipStream_t st) {
   if (n < kPan2 || b_f < 1 || b_f > n) return hipErrorInvalidValue;
-  const long long np1 = n / kPan1, np2 = n / kPan2;
-  double2* p1 = panels;
-  double2* p2 = panels + np1;
-  hipLaunchKernelGGL(panel_sum_kernel, grid_for(np1), dim3(256), 0, st, G, p1, np1, kPan1);
-  hipLaunchKernelGGL(panel_sum_kernel, grid_for(np2), dim3(256), 0, st, (const double2*)p1, p2,
-                     np2, kPan2 / kPan1);
   const long long nb = aux_boxcar_blocks(n);
-  hipLaunchKernelGGL(boxcar_kernel, dim3((unsigned)nb), dim3(BX_NT), 0, st, G,
+  double2* p1 = panels;
+  double2* p2 = panels + n / kPan1;
+  hipLaunchKernelGGL(panel_sums_kernel, dim3((unsigned)nb), dim3(64), 0, st, G, p1, p2);
+  hipLaunchKernelGGL(boxcar_kernel, dim3((unsigned)nb), dim3(64), 0, st, G,
                      (const double2*)p1, (const double2*)p2, out, n, b_f, blkmax);
   hipLaunchKernelGGL(max_reduce_kernel, dim3(1), dim3(256), 0, st, (const double*)blkmax,
                      (int)nb, mx2);
