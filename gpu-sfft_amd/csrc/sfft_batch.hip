@@ -1,19 +1,17 @@
 // sfft_batch.hip -- many signals of uneven n and k transformed as one batch.
 //
-// Each signal keeps its own plan (parameters, workspace, draws).  One batch execution is:
-//   * the permute+filter of ALL signals as one persistent launch (perm_filter_batch_kernel:
-//     a work table of (signal, loop group, bucket block) items walked with a grid stride, so
-//     small and large signals share the chip evenly);
-//   * every signal's other stage groups (clear + comb restriction, then bucket FFT + cutoff,
-//     reverse hash, estimation) on one of several worker streams, joined back to the batch
-//     stream;
-// either enqueued eagerly or replayed from hipGraphs: each worker stream's front groups and
-// its back groups are captured once as two linear chains (on that stream), and a replay
-// launches them around the directly launched permute+filter (one graph over all streams
-// replayed slower than the eager launches: its cross-stream dependencies serialise the
-// ~1,600 nodes).  The draws are uploaded before the replay, outside the graphs; the graphs
-// hold no memset nodes (buffers are cleared by kernels).  The graphs are re-captured when
-// the signal pointers or the tuned shapes change.
+// Each signal keeps its own plan (parameters, workspace).  One batch execution runs every stage
+// of ALL its signals as one launch (sfft_jobs.h: a table of the signals' arguments, and each
+// workgroup's signal; the permute+filter is a persistent launch over its own work table), so
+// small and large signals share the chip and a batch of any size takes about thirty launches.
+// (One launch per signal and stage took 16-25 launches of a few us per signal: 64 complex64
+// signals of 2^18..2^24, 6.3 ms on four streams, now 2.6 ms.)  Two chains run beside each other, as in a single transform: the comb
+// chain (clear, comb FFT, comb cutoff, approved bitmaps) on a second stream, and permute+filter,
+// bucket FFT and bucket cutoff on the batch stream; joined there, the reverse hash and the
+// estimation follow.  The draws of all signals go up in one copy.  With graphs the two chains
+// are captured once as one graph and replayed (buffers are cleared by kernels, so it holds no
+// memset nodes); the tables and the graph are rebuilt when the signal or node pointers, the
+// filters or the tuned shapes change.
 //
 // Autotuner: times, on the batch itself, only launch shapes that compute the same bits --
 // the permute+filter loops per thread, block size and persistent grid (every shape runs the
@@ -24,62 +22,66 @@
 #include <vector>
 
 #include "sfft_plan_impl.h"
-
-namespace {
-constexpr int kWorkers = 4;
-}
+#include "sfft_jobs.h"
 
 struct sfft_batch {
   int count = 0;
   int fp32 = 0;
   hipStream_t st = nullptr;
   int own_st = 0;                    // st created here (a graph cannot capture stream 0)
+  hipStream_t st2 = nullptr;         // the comb chain
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::vector<sfft_plan*> plans;
-  std::vector<hipStream_t> workers;
-  hipEvent_t ev_fork = nullptr, ev_pf = nullptr;
-  std::vector<hipEvent_t> ev_join;
-  // batched permute+filter
+  // job tables of every stage, in one device buffer
   std::vector<PfJob> jobs;
-  PfJob* d_jobs = nullptr;
   int total_items = 0;
   int lpt = 3, nt = 256, grid = 2048;
-  std::vector<const void*> jobs_x;   // signal pointers the device job table holds
-  // per-signal hit counts, contiguous
+  std::vector<FftGroup> comb, bucket;
+  SelGroup sel_comb, sel_bucket;
+  JobTable<HashJob> clear, bitmap, hits;
+  std::vector<EstGroup> est;
+  char* d_tab = nullptr;
+  size_t tab_bytes = 0;
+  const PfJob* d_jobs = nullptr;
+  std::vector<const void*> tab_x;    // the pointers the tables hold: signals, nodes
+  std::vector<Node*> tab_nodes;
+  // the draws of all signals: signal i's (a, ai, offsets) at draw_at[i]
+  int* d_draws = nullptr;
+  int* h_draws = nullptr;            // pinned
+  std::vector<size_t> draw_at;
+  size_t draw_ints = 0;
+  hipEvent_t up_ev = nullptr;        // last upload out of h_draws
+  int up_pending = 0;
+  // per-signal hit counts, contiguous; the estimation also stores them into h_counts (pinned)
   int* d_counts = nullptr;
   int* h_counts = nullptr;
-  // graphs: per worker stream, one of its signals' front groups and one of their back groups
-  // (linear chains, each captured on its own worker stream); the persistent permute+filter
-  // between them is launched directly
+  int* h_counts_dev = nullptr;
   int use_graph = 0;
-  std::vector<hipGraph_t> graphs;
-  std::vector<hipGraphExec_t> execs;   // [2*s] front, [2*s+1] back of worker s (may be null)
-  bool captured = false;
-  std::vector<const void*> graph_x;
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
 };
 
 static void drop_graph(sfft_batch* b) {
-  for (auto e : b->execs)
-    if (e) (void)hipGraphExecDestroy(e);
-  for (auto g : b->graphs)
-    if (g) (void)hipGraphDestroy(g);
-  b->execs.clear();
-  b->graphs.clear();
-  b->captured = false;
-  b->graph_x.clear();
+  if (b->exec) (void)hipGraphExecDestroy(b->exec);
+  if (b->graph) (void)hipGraphDestroy(b->graph);
+  b->exec = nullptr;
+  b->graph = nullptr;
 }
 
 extern "C" void sfft_batch_destroy(sfft_batch* b) {
   if (!b) return;
   (void)hipStreamSynchronize(b->st);
-  for (auto w : b->workers) (void)hipStreamSynchronize(w);
+  if (b->st2) (void)hipStreamSynchronize(b->st2);
   drop_graph(b);
   for (auto p : b->plans) sfft_plan_destroy(p);
-  for (auto w : b->workers) (void)hipStreamDestroy(w);
-  for (auto e : b->ev_join) (void)hipEventDestroy(e);
+  if (b->st2) (void)hipStreamDestroy(b->st2);
   if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
-  if (b->ev_pf) (void)hipEventDestroy(b->ev_pf);
+  if (b->ev_join) (void)hipEventDestroy(b->ev_join);
+  if (b->up_ev) (void)hipEventDestroy(b->up_ev);
   if (b->own_st && b->st) (void)hipStreamDestroy(b->st);
-  if (b->d_jobs) (void)hipFree(b->d_jobs);
+  if (b->d_tab) (void)hipFree(b->d_tab);
+  if (b->d_draws) (void)hipFree(b->d_draws);
+  if (b->h_draws) (void)hipHostFree(b->h_draws);
   if (b->d_counts) (void)hipFree(b->d_counts);
   if (b->h_counts) (void)hipHostFree(b->h_counts);
   delete b;
@@ -118,20 +120,33 @@ extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
     }
     b->plans.push_back(p);
   }
-  b->workers.resize(kWorkers, nullptr);
-  b->ev_join.resize(kWorkers, nullptr);
-  bool ok = hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) == hipSuccess &&
-            hipEventCreateWithFlags(&b->ev_pf, hipEventDisableTiming) == hipSuccess &&
-            hipMalloc((void**)&b->d_jobs, sizeof(PfJob) * (size_t)count) == hipSuccess &&
-            hipMalloc((void**)&b->d_counts, sizeof(int) * (size_t)count) == hipSuccess &&
-            hipHostMalloc((void**)&b->h_counts, sizeof(int) * (size_t)count,
-                          hipHostMallocDefault) == hipSuccess;
-  for (int s = 0; ok && s < kWorkers; ++s)   // default priority, non-blocking
-    ok = hipStreamCreateWithFlags(&b->workers[s], hipStreamNonBlocking) == hipSuccess &&
-         hipEventCreateWithFlags(&b->ev_join[s], hipEventDisableTiming) == hipSuccess;
+  for (int i = 0; i < count; ++i) {
+    b->draw_at.push_back(b->draw_ints);
+    const size_t ints = (size_t)(2 * params[i].loops + params[i].RLFC_loops);
+    b->draw_ints += (ints + 15) / 16 * 16;
+  }
+  const bool ok =
+      hipStreamCreateWithFlags(&b->st2, hipStreamNonBlocking) == hipSuccess &&   // default priority
+      hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) == hipSuccess &&
+      hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming) == hipSuccess &&
+      hipEventCreateWithFlags(&b->up_ev, hipEventDisableTiming) == hipSuccess &&
+      hipMalloc((void**)&b->d_draws, sizeof(int) * b->draw_ints) == hipSuccess &&
+      hipHostMalloc((void**)&b->h_draws, sizeof(int) * b->draw_ints, hipHostMallocDefault) ==
+          hipSuccess &&
+      hipMalloc((void**)&b->d_counts, sizeof(int) * (size_t)count) == hipSuccess &&
+      hipHostMalloc((void**)&b->h_counts, sizeof(int) * (size_t)count, hipHostMallocDefault) ==
+          hipSuccess &&
+      hipHostGetDevicePointer((void**)&b->h_counts_dev, b->h_counts, 0) == hipSuccess;
   if (!ok) {
     sfft_batch_destroy(b);
     return SFFT_ERR_ALLOC;
+  }
+  memset(b->h_draws, 0, sizeof(int) * b->draw_ints);
+  for (int i = 0; i < count; ++i) {   // the plans read their draws from the batch's block
+    sfft_plan* P = b->plans[i];
+    P->d_a = b->d_draws + b->draw_at[i];
+    P->d_ai = P->d_a + P->p.loops;
+    P->d_offs = P->d_a + 2 * P->p.loops;
   }
   *out = b;
   return SFFT_OK;
@@ -145,164 +160,218 @@ extern "C" sfft_status sfft_batch_set_filter(sfft_batch* b, int i, const void* d
                                              const complex_t* h_filter_win) {
   if (!b || i < 0 || i >= b->count) return SFFT_ERR_INVALID;
   drop_graph(b);
-  b->jobs_x.clear();   // the job table holds the taps pointer
+  b->tab_x.clear();   // the tables hold the taps pointer
   return sfft_plan_set_filter(b->plans[i], d_filter_time, h_filter_win);
 }
 
-// (re)builds the permute+filter work table for the current shape and signal pointers
-static sfft_status build_jobs(sfft_batch* b, const void* const* d_x) {
-  b->jobs.resize(b->count);
+// (re)builds every stage's job table for the current shapes and pointers: signal i reads d_x[i]
+// and its nodes go to nodes[i] (the device view of pinned host memory, with a copy in the plan's
+// buffer; nullptr: the plan's buffer alone)
+static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes) {
+  drop_graph(b);
+  b->tab_x.clear();
+  b->jobs.assign(b->count, PfJob());
+  b->comb.clear();
+  b->bucket.clear();
+  b->est.clear();
+  b->sel_comb = SelGroup();
+  b->sel_bucket = SelGroup();
+  b->clear = b->bitmap = b->hits = JobTable<HashJob>();
   int item = 0;
   for (int i = 0; i < b->count; ++i) {
     const sfft_plan* P = b->plans[i];
+    const sfft_params& p = P->p;
     PfJob& J = b->jobs[i];
     J.x = d_x[i];
     J.f = P->d_ft;
     J.bins = P->bins_t;
     J.ai = P->d_ai;
-    J.mask = (uint32_t)P->p.n - 1u;
-    J.B = P->p.B;
-    J.w = P->p.w;
-    J.loops = P->p.loops;
-    J.tiled = (P->p.fold_mode == SFFT_FOLD_REFERENCE) && (P->p.n < (1 << 27));
+    J.mask = (uint32_t)p.n - 1u;
+    J.B = p.B;
+    J.w = p.w;
+    J.loops = p.loops;
+    J.tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
     J.item0 = item;
     item += pf_batch_items(J.B, J.loops, b->lpt, b->nt, &J.nbx);
+    const HashArgs h = hash_args(P, b->d_counts + i);
+    const FftLaunch comb = comb_fft(P, d_x[i]);
+    HIPCK(fft_jobs_add(b->comb, comb));
+    HIPCK(fft_jobs_add(b->bucket, bucket_fft(P)));
+    const KeyMap km = fft_keys_map(comb);
+    const SelMark mk = comb_mark(h);
+    const bool marks = select_in_block(p.W_RLFC);
+    HIPCK(select_jobs_add(b->sel_comb, b->fp32, P->comb_keys, p.W_RLFC, p.W_RLFC, p.B_thresh,
+                          p.RLFC_loops, P->J2, 0, P->selW, nullptr, &km, P->comb_digits,
+                          marks ? &mk : nullptr));
+    HIPCK(select_jobs_add(b->sel_bucket, b->fp32, P->bkeys, p.B, p.B, p.B_thresh, p.loops_loc,
+                          P->J, 1, P->selB, P->jsel, nullptr, P->bucket_digits, nullptr));
+    hash_jobs_clear(b->clear, h);
+    if (!marks) hash_jobs_bitmap(b->bitmap, h);
+    hash_jobs_hits(b->hits, h);
+    EstJob e = {};
+    e.hits = P->hits;
+    e.count = b->d_counts + i;
+    e.capacity = P->cap;
+    e.bins = P->bins_f;
+    e.loops = p.loops;
+    e.n = p.n;
+    e.ai = P->d_ai;
+    e.B = p.B;
+    e.win = P->win;
+    e.out = nodes[i] ? nodes[i] : P->nodes;
+    e.copy = nodes[i] ? P->nodes : nullptr;
+    e.sel = P->sel;
+    e.count_copy = b->h_counts_dev + i;
+    estimate_jobs_add(b->est, b->fp32, e);
   }
   b->total_items = item;
-  HIPCK(hipMemcpyAsync(b->d_jobs, b->jobs.data(), sizeof(PfJob) * (size_t)b->count,
-                       hipMemcpyHostToDevice, b->st));
-  b->jobs_x.assign(d_x, d_x + b->count);
-  return SFFT_OK;
-}
-
-// the stage groups of worker s's signals (i = s, s + kWorkers, ...): the front groups (clear,
-// comb FFT, comb cutoff, bitmaps) or the back groups (bucket FFT, cutoff, reverse hash,
-// estimation; after the fold)
-static sfft_status enqueue_worker(sfft_batch* b, const void* const* d_x, int s, bool back) {
-  for (int i = s; i < b->count; i += kWorkers) {
-    sfft_plan* P = b->plans[i];
-    const HashArgs h = hash_args(P, b->d_counts + i);
-    const sfft_status v = back ? run_back(P, h, nullptr, b->workers[s], false)
-                               : run_front(P, d_x[i], h, b->workers[s], false);
-    if (v != SFFT_OK) return v;
+  JobPack pack;
+  const size_t at_jobs = pack.put(b->jobs.data(), sizeof(PfJob) * b->jobs.size());
+  for (auto& g : b->comb) g.t.pack(pack);
+  for (auto& g : b->bucket) g.t.pack(pack);
+  for (auto& g : b->est) g.t.pack(pack);
+  b->sel_comb.pack(pack);
+  b->sel_bucket.pack(pack);
+  b->clear.pack(pack);
+  b->bitmap.pack(pack);
+  b->hits.pack(pack);
+  if (pack.bytes.size() > b->tab_bytes) {
+    HIPCK(hipStreamSynchronize(b->st));   // an earlier batch may still read the old tables
+    if (b->d_tab) (void)hipFree(b->d_tab);
+    b->d_tab = nullptr;
+    b->tab_bytes = 0;
+    if (hipMalloc((void**)&b->d_tab, pack.bytes.size()) != hipSuccess) return SFFT_ERR_ALLOC;
+    b->tab_bytes = pack.bytes.size();
   }
+  HIPCK(hipMemcpyAsync(b->d_tab, pack.bytes.data(), pack.bytes.size(), hipMemcpyHostToDevice,
+                       b->st));
+  HIPCK(hipStreamSynchronize(b->st));   // the packed bytes go out of scope
+  b->d_jobs = (const PfJob*)(b->d_tab + at_jobs);
+  for (auto& g : b->comb) g.t.bind(b->d_tab);
+  for (auto& g : b->bucket) g.t.bind(b->d_tab);
+  for (auto& g : b->est) g.t.bind(b->d_tab);
+  b->sel_comb.bind(b->d_tab);
+  b->sel_bucket.bind(b->d_tab);
+  b->clear.bind(b->d_tab);
+  b->bitmap.bind(b->d_tab);
+  b->hits.bind(b->d_tab);
+  b->tab_x.assign(d_x, d_x + b->count);
+  b->tab_nodes.assign(nodes, nodes + b->count);
   return SFFT_OK;
 }
 
-// one batch execution from the batch stream (fork/join): the persistent permute+filter of
-// all signals and the workers' front groups run concurrently, then the back groups.  Eager
-// launches go round-robin over the signals (so every worker starts at once); with graphs,
-// each worker's groups are replayed from its two captured chains.
-static sfft_status enqueue(sfft_batch* b, const void* const* d_x, bool graphs) {
+// one batch execution from the batch stream (the draws are up, the tables built)
+static sfft_status enqueue(sfft_batch* b) {
   HIPCK(hipEventRecord(b->ev_fork, b->st));
+  HIPCK(hipStreamWaitEvent(b->st2, b->ev_fork, 0));
   HIPCK(perm_filter_batch_launch(b->fp32, b->d_jobs, b->count, b->total_items, b->lpt, b->nt,
                                  b->grid, b->st));
-  HIPCK(hipEventRecord(b->ev_pf, b->st));
-  for (int s = 0; s < kWorkers; ++s) HIPCK(hipStreamWaitEvent(b->workers[s], b->ev_fork, 0));
-  for (int back = 0; back < 2; ++back) {
-    if (back)
-      for (int s = 0; s < kWorkers; ++s) HIPCK(hipStreamWaitEvent(b->workers[s], b->ev_pf, 0));
-    if (graphs) {
-      for (int s = 0; s < kWorkers; ++s)
-        if (b->execs[2 * s + back]) HIPCK(hipGraphLaunch(b->execs[2 * s + back], b->workers[s]));
-      continue;
-    }
-    for (int i = 0; i < b->count; ++i) {
-      sfft_plan* P = b->plans[i];
-      const HashArgs h = hash_args(P, b->d_counts + i);
-      hipStream_t w = b->workers[i % kWorkers];
-      const sfft_status v = back ? run_back(P, h, nullptr, w, false)
-                                 : run_front(P, d_x[i], h, w, false);
-      if (v != SFFT_OK) return v;
-    }
+  HIPCK(hash_clear_jobs(b->clear, b->st2));
+  HIPCK(fft_jobs_launch(b->comb, b->st2));
+  HIPCK(select_jobs_launch(b->sel_comb, b->st2));
+  HIPCK(hash_bitmap_jobs(b->bitmap, b->st2));
+  HIPCK(hipEventRecord(b->ev_join, b->st2));
+  HIPCK(fft_jobs_launch(b->bucket, b->st));
+  HIPCK(select_jobs_launch(b->sel_bucket, b->st));
+  HIPCK(hipStreamWaitEvent(b->st, b->ev_join, 0));
+  HIPCK(hash_hits_jobs(b->hits, b->st));
+  HIPCK(estimate_jobs_launch(b->est, b->st));
+  return SFFT_OK;
+}
+
+static sfft_status capture(sfft_batch* b) {
+  HIPCK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
+  const sfft_status v = enqueue(b);
+  hipGraph_t g = nullptr;
+  const hipError_t e = hipStreamEndCapture(b->st, &g);
+  if (v != SFFT_OK || e != hipSuccess) {
+    if (g) (void)hipGraphDestroy(g);
+    return v != SFFT_OK ? v : SFFT_ERR_HIP;
   }
-  for (int s = 0; s < kWorkers; ++s) {
-    HIPCK(hipEventRecord(b->ev_join[s], b->workers[s]));
-    HIPCK(hipStreamWaitEvent(b->st, b->ev_join[s], 0));
+  b->graph = g;
+  if (hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0) != hipSuccess) {
+    drop_graph(b);
+    return SFFT_ERR_HIP;
   }
   return SFFT_OK;
 }
 
-// capture every worker's front and back chains (each on its own worker stream)
-static sfft_status capture(sfft_batch* b, const void* const* d_x) {
-  b->graphs.assign(2 * kWorkers, nullptr);
-  b->execs.assign(2 * kWorkers, nullptr);
-  for (int s = 0; s < kWorkers && s < b->count; ++s) {
-    for (int part = 0; part < 2; ++part) {
-      HIPCK(hipStreamBeginCapture(b->workers[s], hipStreamCaptureModeThreadLocal));
-      const sfft_status v = enqueue_worker(b, d_x, s, part == 1);
-      hipGraph_t g = nullptr;
-      const hipError_t e = hipStreamEndCapture(b->workers[s], &g);
-      if (v != SFFT_OK || e != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        drop_graph(b);
-        return v != SFFT_OK ? v : SFFT_ERR_HIP;
-      }
-      b->graphs[2 * s + part] = g;
-      if (hipGraphInstantiate(&b->execs[2 * s + part], g, nullptr, nullptr, 0) != hipSuccess) {
-        drop_graph(b);
-        return SFFT_ERR_HIP;
-      }
-    }
-  }
-  b->captured = true;
-  b->graph_x.assign(d_x, d_x + b->count);
-  return SFFT_OK;
-}
-
-static sfft_status prepare(sfft_batch* b, const void* const* d_x, const sfft_draws* draws) {
+// checks, the draws of every signal up in one copy, the tables for these pointers
+static sfft_status prepare(sfft_batch* b, const void* const* d_x, const sfft_draws* draws,
+                           Node* const* nodes) {
   for (int i = 0; i < b->count; ++i) {
     if (!d_x[i]) return SFFT_ERR_INVALID;
     if (!b->plans[i]->has_filter) return SFFT_ERR_NO_FILTER;
   }
   for (int i = 0; i < b->count; ++i) {
-    const sfft_status v = upload_draws(b->plans[i], &draws[i]);
+    const sfft_status v = draws_check(b->plans[i], &draws[i]);
     if (v != SFFT_OK) return v;
   }
-  if (b->jobs_x.size() != (size_t)b->count ||
-      !std::equal(b->jobs_x.begin(), b->jobs_x.end(), d_x)) {
-    drop_graph(b);
-    return build_jobs(b, d_x);
+  if (b->up_pending) HIPCK(hipEventSynchronize(b->up_ev));
+  for (int i = 0; i < b->count; ++i) {
+    const sfft_params& p = b->plans[i]->p;
+    int* h = b->h_draws + b->draw_at[i];
+    memcpy(h, draws[i].a, (size_t)p.loops * 4);
+    memcpy(h + p.loops, draws[i].ai, (size_t)p.loops * 4);
+    memcpy(h + 2 * p.loops, draws[i].offsets, (size_t)p.RLFC_loops * 4);
   }
+  HIPCK(hipMemcpyAsync(b->d_draws, b->h_draws, sizeof(int) * b->draw_ints, hipMemcpyHostToDevice,
+                       b->st));
+  HIPCK(hipEventRecord(b->up_ev, b->st));
+  b->up_pending = 1;
+  if (b->tab_x.size() != (size_t)b->count ||
+      !std::equal(b->tab_x.begin(), b->tab_x.end(), d_x) ||
+      !std::equal(b->tab_nodes.begin(), b->tab_nodes.end(), nodes))
+    return build_tables(b, d_x, nodes);
+  return SFFT_OK;
+}
+
+static sfft_status execute(sfft_batch* b, const void* const* d_x, const sfft_draws* draws,
+                           Node* const* nodes) {
+  sfft_status v = prepare(b, d_x, draws, nodes);
+  if (v != SFFT_OK) return v;
+  if (!b->use_graph) return enqueue(b);
+  if (!b->exec && (v = capture(b)) != SFFT_OK) return v;
+  HIPCK(hipGraphLaunch(b->exec, b->st));
   return SFFT_OK;
 }
 
 extern "C" sfft_status sfft_batch_execute_async(sfft_batch* b, const void* const* d_x,
                                                 const sfft_draws* draws) {
   if (!b || !d_x || !draws) return SFFT_ERR_INVALID;
-  sfft_status v = prepare(b, d_x, draws);
-  if (v != SFFT_OK) return v;
-  if (!b->use_graph) return enqueue(b, d_x, false);
-  if (!b->captured) {
-    // nothing in flight may still use the worker streams' captured work
-    for (int s = 0; s < kWorkers; ++s) HIPCK(hipStreamSynchronize(b->workers[s]));
-    v = capture(b, d_x);
-    if (v != SFFT_OK) return v;
-  }
-  return enqueue(b, d_x, true);
+  const std::vector<Node*> none(b->count, nullptr);
+  return execute(b, d_x, draws, none.data());
 }
 
 extern "C" sfft_status sfft_batch_execute(sfft_batch* b, const void* const* d_x,
                                           const sfft_draws* draws, Node* const* h_nodes,
                                           int* h_counts) {
-  sfft_status v = sfft_batch_execute_async(b, d_x, draws);
+  if (!b || !d_x || !draws) return SFFT_ERR_INVALID;
+  // pinned node memory: the estimation stores the nodes straight into it
+  std::vector<Node*> view(b->count, nullptr);
+  PinnedRange pinned;
+  for (int i = 0; h_nodes && i < b->count; ++i)
+    if (h_nodes[i])
+      view[i] = (Node*)pinned.view(h_nodes[i], (size_t)b->plans[i]->cap * sizeof(Node));
+  sfft_status v = execute(b, d_x, draws, view.data());
   if (v != SFFT_OK) return v;
-  HIPCK(hipMemcpyAsync(b->h_counts, b->d_counts, sizeof(int) * (size_t)b->count,
-                       hipMemcpyDeviceToHost, b->st));
-  HIPCK(hipStreamSynchronize(b->st));
+  HIPCK(hipStreamSynchronize(b->st));   // (the estimation stored the counts too)
   sfft_status res = SFFT_OK;
+  bool copies = false;
   for (int i = 0; i < b->count; ++i) {
     sfft_plan* P = b->plans[i];
-    const int cnt = b->h_counts[i];
+    const int cnt = ((volatile int*)b->h_counts)[i];
     P->last_count = cnt;
     if (h_counts) h_counts[i] = cnt;
     if (cnt > P->cap) res = SFFT_ERR_HIT_OVERFLOW;
     const int ncopy = std::min(cnt, P->cap);
-    if (h_nodes && h_nodes[i] && ncopy > 0)
+    if (h_nodes && h_nodes[i] && !view[i] && ncopy > 0) {
       HIPCK(hipMemcpyAsync(h_nodes[i], P->nodes, sizeof(Node) * (size_t)ncopy,
                            hipMemcpyDeviceToHost, b->st));
+      copies = true;
+    }
   }
-  HIPCK(hipStreamSynchronize(b->st));
+  if (copies) HIPCK(hipStreamSynchronize(b->st));
   return res;
 }
 
@@ -339,8 +408,8 @@ static sfft_status time_ms(sfft_batch* b, int reps, F fn, float* ms) {
 extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
                                        const sfft_draws* draws, int reps, int* choice4) {
   if (!b || !d_x || !draws || reps < 1) return SFFT_ERR_INVALID;
-  drop_graph(b);
-  sfft_status v = prepare(b, d_x, draws);
+  const std::vector<Node*> none(b->count, nullptr);
+  sfft_status v = prepare(b, d_x, draws, none.data());
   if (v != SFFT_OK) return v;
   // 1. permute+filter: loops per thread x block size x persistent grid
   const int lpts[] = {1, 2, 3, 4, 5, 6, 7, 8, 9}, nts[] = {128, 256},
@@ -348,16 +417,15 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
   float best = 1e30f;
   int bl = b->lpt, bn = b->nt, bg = b->grid;
   for (int lpt : lpts)
-    for (int nt : nts)
+    for (int nt : nts) {
+      b->lpt = lpt;
+      b->nt = nt;
+      if ((v = build_tables(b, d_x, none.data())) != SFFT_OK) return v;
       for (int grid : grids) {
-        b->lpt = lpt;
-        b->nt = nt;
-        b->grid = grid;
-        if ((v = build_jobs(b, d_x)) != SFFT_OK) return v;
         float ms = 0;
         v = time_ms(b, reps, [&]() -> sfft_status {
           HIPCK(perm_filter_batch_launch(b->fp32, b->d_jobs, b->count, b->total_items, b->lpt,
-                                         b->nt, b->grid, b->st));
+                                         b->nt, grid, b->st));
           return SFFT_OK;
         }, &ms);
         if (v != SFFT_OK) return v;
@@ -368,53 +436,21 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
           bg = grid;
         }
       }
+    }
   b->lpt = bl;
   b->nt = bn;
   b->grid = bg;
-  if ((v = build_jobs(b, d_x)) != SFFT_OK) return v;
   // 2. FFT columns per tile, bucket FFTs then comb FFTs, one choice for the whole batch
   const int qs[] = {1, 2, 4, 8, 16, 32};
   int best_q[2] = {0, 0};
   for (int which = 0; which < 2; ++which) {
     float bq = 1e30f;
     for (int q : qs) {
+      for (auto P : b->plans) (which == 0 ? P->qmax_B : P->qmax_W) = q;
+      if ((v = build_tables(b, d_x, none.data())) != SFFT_OK) return v;
       float ms = 0;
       v = time_ms(b, reps, [&]() -> sfft_status {
-        for (int i = 0; i < b->count; ++i) {
-          sfft_plan* P = b->plans[i];
-          FftLaunch f;
-          if (which == 0) {
-            f.tab = &P->tabB;
-            f.in = P->bins_t;
-            f.in_bstride = P->p.B;
-            f.out = P->bins_f;
-            f.out_bstride = P->p.B;
-            f.scratch = P->bins_scr;
-            f.keys = P->bkeys;
-            f.keys_bstride = P->p.B;
-            f.key_batches = P->p.loops_loc;
-            f.batch = P->p.loops;
-            f.store = kStoreBoth;
-          } else {
-            f.tab = &P->tabW;
-            f.out = P->comb0;
-            f.out_bstride = P->p.W_RLFC;
-            f.scratch = P->comb1;
-            f.keys = P->comb_keys;
-            f.keys_bstride = P->p.W_RLFC;
-            f.key_batches = P->p.RLFC_loops;
-            f.batch = P->p.RLFC_loops;
-            f.store = kStoreKeys;
-            f.keys_tiled = 1;
-            f.digits = P->comb_digits;
-            f.load = kLoadComb;
-            f.comb_x = d_x[i];
-            f.comb_offs = P->d_offs;
-            f.comb_sigma = P->p.n / P->p.W_RLFC;
-          }
-          f.qmax = q;
-          HIPCK(fft_run(f, b->st));
-        }
+        HIPCK(fft_jobs_launch(which == 0 ? b->bucket : b->comb, b->st));
         return SFFT_OK;
       }, &ms);
       if (v != SFFT_OK) return v;
@@ -428,6 +464,8 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
     P->qmax_B = best_q[0];
     P->qmax_W = best_q[1];
   }
+  b->tab_x.clear();   // built again for the chosen shapes
+  drop_graph(b);
   if (choice4) {
     choice4[0] = b->lpt;
     choice4[1] = b->nt;
@@ -445,7 +483,7 @@ extern "C" sfft_status sfft_batch_set_shape(sfft_batch* b, int lpt, int nt, int 
       qmax_bucket > 32 || qmax_comb < 0 || qmax_comb > 32)
     return SFFT_ERR_INVALID;
   drop_graph(b);
-  b->jobs_x.clear();
+  b->tab_x.clear();
   b->lpt = lpt;
   b->nt = nt;
   b->grid = grid;

@@ -13,7 +13,7 @@
 #include <mutex>
 #include <utility>
 
-#include "sfft_internal.h"
+#include "sfft_jobs.h"
 
 namespace sfft {
 
@@ -119,36 +119,6 @@ static int tile_cap(int is_fp32, int load) {
 __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return (nb & 7) ? b : (b & 7) * (nb >> 3) + (b >> 3);
 }
-
-struct PassArgs {
-  const void* in;
-  long long in_bstride;
-  void* out;
-  long long out_bstride;
-  void* keys;
-  long long keys_bstride;
-  int key_batches;
-  int log2N, r, log2Lprev, log2Q;
-  int inverse;
-  const void* twR;
-  const void* tw4;      // radix-4 stage twiddle quads (see fft_tables_create)
-  const void* tdir;
-  const void* thi;
-  const void* tlo;
-  int s;
-  const void* comb_x;
-  const int* comb_offs;
-  int comb_sigma;
-  int nbatch;
-  int keys_tiled;   // store keys at tile * TE + e (the tile's own contiguous range)
-  uint16_t* digits; // optional first digits of the keys (same positions)
-  int log2nlo, log2m;   // kLoadCombRows: g at in[(g mod 2^log2nlo) << log2m | g >> log2nlo]
-  const int* perm;      // kLoadPerm: g of batch b at in[g * perm[b] mod 2^log2N]
-  const int* perm_inv;  // kLoadPerm: the inverse of perm[b] mod 2^log2N
-  int taps;             // kLoadTaps
-  long long head;       // kStoreHead
-  double scale;         // kStoreHead
-};
 
 template <typename T2>
 __device__ __forceinline__ T2 outer_tw(const PassArgs& A, uint32_t e, int log2Lcur) {
@@ -396,11 +366,9 @@ __device__ __forceinline__ void fft_stage2(T2* lds, int RP, int r, int log2ncol,
 // code: 0 none (the first pass), 1 direct table entries, 2 products of a high and a low entry
 enum PassTw { kTwNone = 0, kTwDirect = 1, kTwSplit = 2 };
 
+// (bx, by) of nbx: the workgroup's tile and batch (comb gathers: tile and batch in bx alone)
 template <typename Real, int LOAD, int STORE, int TW>
-// two workgroups per CU for the plain tiles: 8 waves per SIMD at 1024 threads, 4 at 512
-__global__ __launch_bounds__((Tile<Real, LOAD>::nt),
-                             (LOAD == 1 ? 1 : Tile<Real, LOAD>::nt / 128)) void fft_pass_kernel(
-    PassArgs A) {
+__device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx, int by) {
   using T2 = typename CT<Real>::T2;
   using KT = typename CT<Real>::K;
   constexpr int CAP = Tile<Real, LOAD>::cap, EPT = Tile<Real, LOAD>::ept;
@@ -413,12 +381,12 @@ __global__ __launch_bounds__((Tile<Real, LOAD>::nt),
   int tile;
   long long b;
   if (LOAD == kLoadComb) {
-    const int s = xcd_tile(blockIdx.x, gridDim.x);
+    const int s = xcd_tile(bx, nbx);
     b = s % A.nbatch;
     tile = s / A.nbatch;
   } else {
-    tile = xcd_tile(blockIdx.x, gridDim.x);
-    b = blockIdx.y;
+    tile = xcd_tile(bx, nbx);
+    b = by;
   }
   const int r = A.r;
   const int R = 1 << r;
@@ -708,6 +676,31 @@ __global__ __launch_bounds__((Tile<Real, LOAD>::nt),
 }
 
 template <typename Real, int LOAD, int STORE, int TW>
+// two workgroups per CU for the plain tiles: 8 waves per SIMD at 1024 threads, 4 at 512
+__global__ __launch_bounds__((Tile<Real, LOAD>::nt),
+                             (LOAD == 1 ? 1 : Tile<Real, LOAD>::nt / 128)) void fft_pass_kernel(
+    PassArgs A) {
+  fft_pass_body<Real, LOAD, STORE, TW>(A, blockIdx.x, gridDim.x, blockIdx.y);
+}
+
+// the same pass of many signals (jobs of tiles x batch workgroups)
+template <typename Real, int LOAD, int STORE, int TW>
+__global__ __launch_bounds__((Tile<Real, LOAD>::nt),
+                             (LOAD == 1 ? 1
+                                        : Tile<Real, LOAD>::nt / 128)) void fft_jobs_kernel(
+    JobsDev t) {
+  const FftJob* j = job_here<FftJob>(t);
+  if (!j) return;
+  const PassArgs A = j->a;
+  const int i = (int)blockIdx.x - j->block0;
+  if constexpr (LOAD == kLoadComb) {
+    fft_pass_body<Real, LOAD, STORE, TW>(A, i, j->tiles * A.nbatch, 0);
+  } else {
+    fft_pass_body<Real, LOAD, STORE, TW>(A, i % j->tiles, j->tiles, i / j->tiles);
+  }
+}
+
+template <typename Real, int LOAD, int STORE, int TW>
 static hipError_t launch_pass(const PassArgs& A, int tiles, int batch, hipStream_t st) {
   const dim3 grid = (LOAD == kLoadComb) ? dim3(tiles * batch, 1) : dim3(tiles, batch);
   hipLaunchKernelGGL((fft_pass_kernel<Real, LOAD, STORE, TW>), grid, dim3(Tile<Real, LOAD>::nt),
@@ -787,7 +780,9 @@ KeyMap fft_keys_map(const FftLaunch& L) {
   return m;
 }
 
-hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
+// calls fn(p, args, load, store, tw, tiles) for each pass of L in order
+template <typename F>
+static hipError_t each_pass(const FftLaunch& L, F&& fn) {
   const FftTables& T = *L.tab;
   const int log2N = T.log2n;
   const long long N = 1LL << log2N;
@@ -856,17 +851,80 @@ hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
     const int store = last ? L.store : kStoreCplx;
     const int tw = (p == 0) ? kTwNone : (log2Lcur > kMaxPassLog ? kTwSplit : kTwDirect);
     if (load != kLoadPlain && tw != kTwNone) return hipErrorInvalidValue;
-    hipError_t e;
-    if (load == kLoadWiden || load == kLoadTaps || store == kStoreHead)
-      e = T.is_fp32 ? hipErrorInvalidValue
-                    : dispatch_fp64(A, load, store, tw, tiles, L.batch, st);
-    else
-      e = T.is_fp32 ? dispatch_pass<float>(A, load, store, tw, tiles, L.batch, st)
-                    : dispatch_pass<double>(A, load, store, tw, tiles, L.batch, st);
+    const hipError_t e = fn(p, A, load, store, tw, tiles);
     if (e != hipSuccess) return e;
     cur_in = dst;
     cur_in_stride = dst_stride;
     log2Lprev = log2Lcur;
+  }
+  return hipSuccess;
+}
+
+hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
+  const int fp32 = L.tab->is_fp32;
+  return each_pass(L, [&](int, const PassArgs& A, int load, int store, int tw, int tiles) {
+    if (load == kLoadWiden || load == kLoadTaps || store == kStoreHead)
+      return fp32 ? hipErrorInvalidValue : dispatch_fp64(A, load, store, tw, tiles, L.batch, st);
+    return fp32 ? dispatch_pass<float>(A, load, store, tw, tiles, L.batch, st)
+                : dispatch_pass<double>(A, load, store, tw, tiles, L.batch, st);
+  });
+}
+
+hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L) {
+  const int fp32 = L.tab->is_fp32;
+  return each_pass(L, [&](int p, const PassArgs& A, int load, int store, int tw, int tiles) {
+    if (load == kLoadWiden || load == kLoadTaps || store == kStoreHead)
+      return hipErrorInvalidValue;
+    auto it = std::find_if(g.begin(), g.end(), [&](const FftGroup& x) {
+      return x.pass == p && x.load == load && x.store == store && x.tw == tw && x.fp32 == fp32;
+    });
+    if (it == g.end()) {
+      FftGroup n;
+      n.pass = p;
+      n.load = load;
+      n.store = store;
+      n.tw = tw;
+      n.fp32 = fp32;
+      // in the order of the passes
+      it = g.insert(std::find_if(g.begin(), g.end(),
+                                 [&](const FftGroup& x) { return x.pass > p; }), n);
+    }
+    FftJob j;
+    j.a = A;
+    j.tiles = tiles;
+    j.block0 = 0;
+    it->t.add(j, tiles * L.batch);
+    return hipSuccess;
+  });
+}
+
+template <typename Real, int LOAD, int STORE, int TW>
+static hipError_t launch_jobs(const JobsDev& d, hipStream_t st) {
+  hipLaunchKernelGGL((fft_jobs_kernel<Real, LOAD, STORE, TW>), dim3(d.blocks),
+                     dim3(Tile<Real, LOAD>::nt), 0, st, d);
+  return hipGetLastError();
+}
+
+template <typename Real, int LOAD, int TW>
+static hipError_t jobs_store(const FftGroup& g, hipStream_t st) {
+  if (g.store == kStoreCplx) return launch_jobs<Real, LOAD, kStoreCplx, TW>(g.t.dev, st);
+  if (g.store == kStoreKeys) return launch_jobs<Real, LOAD, kStoreKeys, TW>(g.t.dev, st);
+  return launch_jobs<Real, LOAD, kStoreBoth, TW>(g.t.dev, st);
+}
+
+template <typename Real>
+static hipError_t jobs_pass(const FftGroup& g, hipStream_t st) {
+  if (g.load == kLoadComb) return jobs_store<Real, kLoadComb, kTwNone>(g, st);
+  if (g.load != kLoadPlain) return hipErrorInvalidValue;
+  if (g.tw == kTwSplit) return jobs_store<Real, kLoadPlain, kTwSplit>(g, st);
+  if (g.tw == kTwDirect) return jobs_store<Real, kLoadPlain, kTwDirect>(g, st);
+  return jobs_store<Real, kLoadPlain, kTwNone>(g, st);
+}
+
+hipError_t fft_jobs_launch(std::vector<FftGroup>& groups, hipStream_t st) {
+  for (const FftGroup& g : groups) {
+    const hipError_t e = g.fp32 ? jobs_pass<float>(g, st) : jobs_pass<double>(g, st);
+    if (e != hipSuccess) return e;
   }
   return hipSuccess;
 }

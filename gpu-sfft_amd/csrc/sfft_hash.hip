@@ -7,7 +7,9 @@
 //
 // Floating-point operations that must match the CPU oracle bit for bit are written out
 // explicitly (fma where fused); the library is built with -ffp-contract=off.
-#include "sfft_internal.h"
+#include <algorithm>
+
+#include "sfft_jobs.h"
 
 namespace sfft {
 
@@ -87,12 +89,34 @@ __global__ void hash_clear_kernel(uint32_t* __restrict__ bm, size_t nbm,
   if (i0 < (size_t)nmax) maxfirst[i0] = 0xFFFFFFFFu;
 }
 
+static int clear_blocks(const HashArgs& h) {
+  const size_t blocks = ((size_t)h.loops_loc * h.bm_words + 255) / 256;
+  return (int)(blocks > 4096 ? 4096 : blocks < 1 ? 1 : blocks);
+}
+
+// the same for the signals of a batch
+__global__ void hash_clear_jobs_kernel(JobsDev t) {
+  const HashJob* j = job_here<HashJob>(t);
+  if (!j) return;
+  const HashArgs& h = j->h;
+  const size_t nbm = (size_t)h.loops_loc * h.bm_words, s = (size_t)j->blocks * 256;
+  const size_t i0 = (size_t)((int)blockIdx.x - j->block0) * 256 + threadIdx.x;
+  for (size_t i = i0; i < nbm; i += s) h.bitmap[i] = 0u;
+  if (i0 < (size_t)h.loops_loc) h.maxfirst[i0] = -1;
+}
+void hash_jobs_clear(JobTable<HashJob>& t, const HashArgs& h) {
+  HashJob j{h, clear_blocks(h), 0};
+  t.add(j, j.blocks);
+}
+hipError_t hash_clear_jobs(const JobTable<HashJob>& t, hipStream_t st) {
+  if (!t.dev.blocks) return hipSuccess;
+  hipLaunchKernelGGL(hash_clear_jobs_kernel, dim3(t.dev.blocks), dim3(256), 0, st, t.dev);
+  return hipGetLastError();
+}
+
 hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st) {
   const size_t bm_words = (size_t)h.loops_loc * h.bm_words;
-  size_t blocks = (bm_words + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(hash_clear_kernel, dim3((unsigned)blocks), dim3(256), 0, st,
+  hipLaunchKernelGGL(hash_clear_kernel, dim3(clear_blocks(h)), dim3(256), 0, st,
                      (uint32_t*)h.bitmap, bm_words, (uint32_t*)h.maxfirst, h.loops_loc);
   return hipGetLastError();
 }
@@ -101,10 +125,9 @@ hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st) {
 // loop, and the largest one (reduced across the block first: one atomic per block on the
 // loop's single max word -- same-address atomics serialise)
 constexpr int BM_NT = 1024;
-__global__ __launch_bounds__(BM_NT) void hash_bitmap_kernel(HashArgs h) {
+__device__ __forceinline__ void hash_bitmap_body(const HashArgs& h, int bx, int l) {
   __shared__ int wmax[BM_NT / 64];
-  const int i = blockIdx.x * BM_NT + threadIdx.x;
-  const int l = blockIdx.y;
+  const int i = bx * BM_NT + threadIdx.x;
   int v = -1;
   if (i < h.nJ2) {
     const uint64_t j2 = (uint64_t)h.J2[i];
@@ -122,6 +145,25 @@ __global__ __launch_bounds__(BM_NT) void hash_bitmap_kernel(HashArgs h) {
     for (int w = 0; w < BM_NT / 64; ++w) m = max(m, wmax[w]);
     if (m >= 0) atomicMax(&h.maxfirst[l], m);
   }
+}
+
+__global__ __launch_bounds__(BM_NT) void hash_bitmap_kernel(HashArgs h) {
+  hash_bitmap_body(h, blockIdx.x, blockIdx.y);
+}
+__global__ __launch_bounds__(BM_NT) void hash_bitmap_jobs_kernel(JobsDev t) {
+  const HashJob* j = job_here<HashJob>(t);
+  if (!j) return;
+  const int i = (int)blockIdx.x - j->block0, nx = (j->h.nJ2 + BM_NT - 1) / BM_NT;
+  hash_bitmap_body(j->h, i % nx, i / nx);
+}
+void hash_jobs_bitmap(JobTable<HashJob>& t, const HashArgs& h) {
+  HashJob j{h, (h.nJ2 + BM_NT - 1) / BM_NT * h.loops_loc, 0};
+  t.add(j, j.blocks);
+}
+hipError_t hash_bitmap_jobs(const JobTable<HashJob>& t, hipStream_t st) {
+  if (!t.dev.blocks) return hipSuccess;
+  hipLaunchKernelGGL(hash_bitmap_jobs_kernel, dim3(t.dev.blocks), dim3(BM_NT), 0, st, t.dev);
+  return hipGetLastError();
 }
 
 hipError_t hash_bitmap_launch(const HashArgs& h, hipStream_t st) {
@@ -215,11 +257,11 @@ __device__ __forceinline__ int hash_hit_count_d(const HashArgs& h) {
 }
 
 // threads cover loops [l_first, l_first + nloops)
-__device__ __forceinline__ HashSlot hash_slot(const HashArgs& h, int l_first, int nloops) {
+__device__ __forceinline__ HashSlot hash_slot(const HashArgs& h, int l_first, int nloops, int bx) {
   HashSlot s;
   const long long m = (long long)h.n / h.B;
   s.lpj = hash_lpj(m);
-  const long long gid = (long long)blockIdx.x * HASH_NT + threadIdx.x;
+  const long long gid = (long long)bx * HASH_NT + threadIdx.x;
   const long long local = gid / s.lpj;
   s.sub = (int)(gid % s.lpj);
   s.valid = local < (long long)nloops * h.K;
@@ -282,32 +324,33 @@ __device__ __forceinline__ int hash_count_slice(const HashArgs& h, const HashSlo
   return c;
 }
 
-__global__ __launch_bounds__(HASH_NT) void hash_count_kernel(HashArgs h) {
+// (block bx of the nb blocks of one signal's walk)
+__device__ __forceinline__ void hash_count_body(const HashArgs& h, int bx) {
   __shared__ int sh[16];
-  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h));
+  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
   const int words = hash_slice_words((long long)h.n / h.B);
-  const long long gid = (long long)blockIdx.x * HASH_NT + threadIdx.x;
+  const long long gid = (long long)bx * HASH_NT + threadIdx.x;
   const int c = hash_count_slice(h, s, h.hmask + gid * words, words);
   int tot = c;   // total of the bucket's lanes (aligned groups of lpj lanes)
   for (int o = 1; o < s.lpj; o <<= 1) tot += __shfl_xor(tot, o, 64);
   const int v = (s.valid && s.sub == 0) ? tot : 0;
   const int ex = block_excl_scan(v, sh);
   if (s.valid && s.sub == 0) h.hitoff[s.jidx] = ex;
-  if (threadIdx.x == HASH_NT - 1) h.blocksum[blockIdx.x] = ex + v;
+  if (threadIdx.x == HASH_NT - 1) h.blocksum[bx] = ex + v;
 }
 
 // the hits of each slice, from the count pass's hit mask (no second walk).  Each block first
 // sums the hit totals of the blocks before it (a few KB, read by every block in parallel: no
 // separate scan launch); the last block stores the total hit count.
-__global__ __launch_bounds__(HASH_NT) void hash_write_kernel(HashArgs h) {
+__device__ __forceinline__ void hash_write_body(const HashArgs& h, int bx, int nb) {
   __shared__ int sh[16];
   int pre = 0;
-  for (int b = threadIdx.x; b < (int)blockIdx.x; b += HASH_NT) pre += h.blocksum[b];
+  for (int b = threadIdx.x; b < bx; b += HASH_NT) pre += h.blocksum[b];
   const int boff = block_sum(pre, sh);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *h.count = boff + h.blocksum[blockIdx.x];
-  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h));
+  if (bx == nb - 1 && threadIdx.x == 0) *h.count = boff + h.blocksum[bx];
+  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
   const int words = hash_slice_words((long long)h.n / h.B);
-  const long long gid = (long long)blockIdx.x * HASH_NT + threadIdx.x;
+  const long long gid = (long long)bx * HASH_NT + threadIdx.x;
   const unsigned* __restrict__ mk = h.hmask + gid * words;
   int c = 0;
   if (s.valid)
@@ -338,6 +381,31 @@ __global__ __launch_bounds__(HASH_NT) void hash_write_kernel(HashArgs h) {
   }
 }
 
+__global__ __launch_bounds__(HASH_NT) void hash_count_kernel(HashArgs h) {
+  hash_count_body(h, blockIdx.x);
+}
+__global__ __launch_bounds__(HASH_NT) void hash_write_kernel(HashArgs h) {
+  hash_write_body(h, blockIdx.x, gridDim.x);
+}
+__global__ __launch_bounds__(HASH_NT) void hash_count_jobs_kernel(JobsDev t) {
+  const HashJob* j = job_here<HashJob>(t);
+  if (j) hash_count_body(j->h, (int)blockIdx.x - j->block0);
+}
+__global__ __launch_bounds__(HASH_NT) void hash_write_jobs_kernel(JobsDev t) {
+  const HashJob* j = job_here<HashJob>(t);
+  if (j) hash_write_body(j->h, (int)blockIdx.x - j->block0, j->blocks);
+}
+void hash_jobs_hits(JobTable<HashJob>& t, const HashArgs& h) {
+  HashJob j{h, hash_blocks(hash_hit_count(h), h.K, (long long)h.n / h.B), 0};
+  t.add(j, j.blocks);
+}
+hipError_t hash_hits_jobs(const JobTable<HashJob>& t, hipStream_t st) {
+  if (!t.dev.blocks) return hipSuccess;
+  hipLaunchKernelGGL(hash_count_jobs_kernel, dim3(t.dev.blocks), dim3(HASH_NT), 0, st, t.dev);
+  hipLaunchKernelGGL(hash_write_jobs_kernel, dim3(t.dev.blocks), dim3(HASH_NT), 0, st, t.dev);
+  return hipGetLastError();
+}
+
 hipError_t hash_hits_launch(const HashArgs& h, hipStream_t st) {
   const int nb = hash_blocks(hash_hit_count(h), h.K, (long long)h.n / h.B);
   hipLaunchKernelGGL(hash_count_kernel, dim3(nb), dim3(HASH_NT), 0, st, h);
@@ -361,22 +429,23 @@ __device__ __forceinline__ double2 to_d2(float2 v) {
 constexpr int EST_NT = 256;
 constexpr int EST_GRID = 512;   // blocks of the estimation launch (grid-stride over the hits)
 template <typename Real, int MAXL, bool EXACT>
-__global__ __launch_bounds__(EST_NT) void estimate_kernel(
+__device__ __forceinline__ void estimate_body(
     const int* __restrict__ hits, const int* __restrict__ count, int capacity,
     const typename CT<Real>::T2* __restrict__ bins, int loops_rt, uint32_t n,
     const int* __restrict__ ai_dev, int B, const double2* __restrict__ win,
-    Node* __restrict__ out, uint8_t* __restrict__ sel, int* __restrict__ count_copy) {
+    Node* __restrict__ out, Node* __restrict__ copy, uint8_t* __restrict__ sel,
+    int* __restrict__ count_copy, int bx, int nb) {
   static_assert(sizeof(Node) == 24, "Node: key, 4 bytes of padding, two doubles");
   __shared__ unsigned long long stage[EST_NT * 3];
   const int loops = EXACT ? MAXL : loops_rt;
   const int cnt_all = *count;
   const int total = min(cnt_all, capacity);
-  if (count_copy && blockIdx.x == 0 && threadIdx.x == 0) *count_copy = cnt_all;
+  if (count_copy && bx == 0 && threadIdx.x == 0) *count_copy = cnt_all;
   const long long m = (long long)(n / (uint32_t)B);
   const int lm = 63 - __clzll(m);   // m = n / B, both powers of two
   const long long nn = n;
   const int med = (loops - 1) / 2;
-  for (int h0 = blockIdx.x * EST_NT; h0 < total; h0 += gridDim.x * EST_NT) {
+  for (int h0 = bx * EST_NT; h0 < total; h0 += nb * EST_NT) {
     const int h = h0 + (int)threadIdx.x;
     const bool valid = h < total;
     const uint32_t I = (uint32_t)hits[valid ? h : h0];
@@ -446,52 +515,87 @@ __global__ __launch_bounds__(EST_NT) void estimate_kernel(
     const int words = 3 * min(EST_NT, total - h0);
     unsigned long long* o = reinterpret_cast<unsigned long long*>(out + h0);
     for (int j = threadIdx.x; j < words; j += EST_NT) o[j] = stage[j];
+    if (copy) {
+      unsigned long long* c = reinterpret_cast<unsigned long long*>(copy + h0);
+      for (int j = threadIdx.x; j < words; j += EST_NT) c[j] = stage[j];
+    }
     __syncthreads();
   }
 }
 
-template <typename Real, int L, bool EXACT>
-static void estimate_go(const int* hits, const int* count, int capacity, const void* bins,
-                        int loops, int n, const int* ai_dev, int B, const double2* win,
-                        Node* out, uint8_t* sel, int* count_copy, hipStream_t st) {
-  using T2 = typename CT<Real>::T2;
-  hipLaunchKernelGGL((estimate_kernel<Real, L, EXACT>), dim3(EST_GRID), dim3(EST_NT), 0, st,
-                     hits,
-                     count, capacity, (const T2*)bins, loops, (uint32_t)n, ai_dev, B, win, out,
-                     sel, count_copy);
+template <typename Real, int MAXL, bool EXACT>
+__global__ __launch_bounds__(EST_NT) void estimate_kernel(EstJob j) {
+  estimate_body<Real, MAXL, EXACT>(j.hits, j.count, j.capacity,
+                                   (const typename CT<Real>::T2*)j.bins, j.loops, (uint32_t)j.n,
+                                   j.ai, j.B, j.win, j.out, j.copy, j.sel, j.count_copy, blockIdx.x,
+                                   gridDim.x);
+}
+template <typename Real, int MAXL, bool EXACT>
+__global__ __launch_bounds__(EST_NT) void estimate_jobs_kernel(JobsDev t) {
+  const EstJob* p = job_here<EstJob>(t);
+  if (!p) return;
+  const EstJob j = *p;
+  estimate_body<Real, MAXL, EXACT>(j.hits, j.count, j.capacity,
+                                   (const typename CT<Real>::T2*)j.bins, j.loops, (uint32_t)j.n,
+                                   j.ai, j.B, j.win, j.out, j.copy, j.sel, j.count_copy,
+                                   (int)blockIdx.x - j.block0, j.blocks);
 }
 
-template <typename Real>
-static hipError_t estimate_dispatch(const int* hits, const int* count, int capacity,
-                                    const void* bins, int loops, int n, const int* ai_dev, int B,
-                                    const double2* win, Node* out, uint8_t* sel,
-                                    int* count_copy, hipStream_t st) {
-#define SFFT_EST(L)                                                                         \
-  case L:                                                                                   \
-    estimate_go<Real, L, true>(hits, count, capacity, bins, loops, n, ai_dev, B, win, out, \
-                               sel, count_copy, st);                                        \
-    break;
+// f(kernel of one estimation, kernel of many) for the loop count
+template <typename Real, typename F>
+static hipError_t with_loops(int loops, F&& f) {
+#define SFFT_EST(L) \
+  case L:           \
+    return f(estimate_kernel<Real, L, true>, estimate_jobs_kernel<Real, L, true>);
   switch (loops) {
     SFFT_EST(1) SFFT_EST(2) SFFT_EST(3) SFFT_EST(4) SFFT_EST(5) SFFT_EST(6) SFFT_EST(7)
     SFFT_EST(8) SFFT_EST(9) SFFT_EST(10) SFFT_EST(11) SFFT_EST(12) SFFT_EST(13) SFFT_EST(14)
     SFFT_EST(15) SFFT_EST(16)
     default:
-      estimate_go<Real, 32, false>(hits, count, capacity, bins, loops, n, ai_dev, B, win, out,
-                                   sel, count_copy, st);
+      return f(estimate_kernel<Real, 32, false>, estimate_jobs_kernel<Real, 32, false>);
   }
 #undef SFFT_EST
-  return hipGetLastError();
 }
 
 hipError_t estimate_launch(int is_fp32, const int* hits, const int* count, int capacity,
                            const void* bins_f, int loops, int n, const int* ai_dev, int B,
                            const double2* filter_win, Node* out, uint8_t* sel,
                            hipStream_t st, int* count_copy) {
-  if (is_fp32)
-    return estimate_dispatch<float>(hits, count, capacity, bins_f, loops, n, ai_dev, B,
-                                    filter_win, out, sel, count_copy, st);
-  return estimate_dispatch<double>(hits, count, capacity, bins_f, loops, n, ai_dev, B,
-                                   filter_win, out, sel, count_copy, st);
+  EstJob j{hits,       count, capacity, bins_f, loops,      n, ai_dev, B,
+           filter_win, out,   nullptr,  sel,    count_copy, 0, 0};
+  auto go = [&](auto one, auto) {
+    hipLaunchKernelGGL(one, dim3(EST_GRID), dim3(EST_NT), 0, st, j);
+    return hipGetLastError();
+  };
+  return is_fp32 ? with_loops<float>(loops, go) : with_loops<double>(loops, go);
+}
+
+void estimate_jobs_add(std::vector<EstGroup>& g, int is_fp32, EstJob j) {
+  const int key = j.loops <= 16 ? j.loops : 32;   // one kernel takes every count above 16
+  auto it = std::find_if(g.begin(), g.end(), [&](const EstGroup& x) { return x.loops == key; });
+  if (it == g.end()) {
+    g.emplace_back();
+    it = g.end() - 1;
+    it->loops = key;
+    it->fp32 = is_fp32;
+  }
+  // the hits are known on the device only: a few blocks per signal, each taking every
+  // blocks-th group of EST_NT hits
+  j.blocks = std::min(EST_GRID / 16, (j.capacity + EST_NT - 1) / EST_NT);
+  it->t.add(j, j.blocks);
+}
+
+hipError_t estimate_jobs_launch(const std::vector<EstGroup>& groups, hipStream_t st) {
+  for (const EstGroup& g : groups) {
+    auto go = [&](auto, auto many) {
+      hipLaunchKernelGGL(many, dim3(g.t.dev.blocks), dim3(EST_NT), 0, st, g.t.dev);
+      return hipGetLastError();
+    };
+    const hipError_t e =
+        g.fp32 ? with_loops<float>(g.loops, go) : with_loops<double>(g.loops, go);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace sfft

@@ -452,7 +452,6 @@ HashArgs hash_args(const sfft_plan* P, int* d_count) {
 // mode are recorded by the front and back groups when `marks` is set.
 // front: bitmap clear, streaming pass (option), comb FFT (run_comb), then the comb
 // cutoff and the approved bitmaps (run_cut)
-static FftLaunch comb_fft(const sfft_plan* P, const void* d_x);
 static sfft_status run_comb(sfft_plan* P, const void* d_x, const HashArgs& h, hipStream_t st,
                             bool marks) {
   const sfft_params& p = P->p;
@@ -475,7 +474,7 @@ static sfft_status run_comb(sfft_plan* P, const void* d_x, const HashArgs& h, hi
 // RLFC: comb samples (gathered in pass 0, or from the streaming pass) + W-point FFT, keys of
 // |Y|^2 out of the last pass in its tile order (whole-line stores; the comb cutoff maps the
 // storage positions back to the bins)
-static FftLaunch comb_fft(const sfft_plan* P, const void* d_x) {
+FftLaunch comb_fft(const sfft_plan* P, const void* d_x) {
   const sfft_params& p = P->p;
   const int Rl = p.RLFC_loops;
   const long long W = p.W_RLFC;
@@ -513,18 +512,24 @@ static FftLaunch comb_fft(const sfft_plan* P, const void* d_x) {
   return c;
 }
 
+// what a one-workgroup comb cutoff marks of its selection
+SelMark comb_mark(const HashArgs& h) {
+  SelMark m;
+  m.loops = h.loops_loc;
+  m.ai = h.ai_dev;
+  m.bitmap = h.bitmap;
+  m.bm_words = h.bm_words;
+  m.wmask = (unsigned)h.W - 1u;
+  m.maxfirst = h.maxfirst;
+  return m;
+}
+
 // comb cutoff: the comb lists only feed the order-free bitmap build (unordered output)
 static sfft_status run_cut(sfft_plan* P, const HashArgs& h, hipStream_t st, bool marks) {
   const sfft_params& p = P->p;
   const long long W = p.W_RLFC;
   const KeyMap km = fft_keys_map(comb_fft(P, nullptr));
-  SelMark mk;
-  mk.loops = h.loops_loc;
-  mk.ai = h.ai_dev;
-  mk.bitmap = h.bitmap;
-  mk.bm_words = h.bm_words;
-  mk.wmask = (unsigned)h.W - 1u;
-  mk.maxfirst = h.maxfirst;
+  const SelMark mk = comb_mark(h);
   const bool marks_too = select_in_block((int)W);
   HIPCK(select_topk(P->fp32, P->comb_keys, W, (int)W, p.B_thresh, p.RLFC_loops, P->J2, 0,
                     P->selW, st, nullptr, &km, P->comb_digits, marks_too ? &mk : nullptr));
@@ -557,12 +562,10 @@ sfft_status run_fold(sfft_plan* P, const void* d_x, hipStream_t st, const FoldCl
   return SFFT_OK;
 }
 
-// bucket: bucket FFT + cutoff (after the fold)
-sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
+// the bucket FFTs of every loop: spectra, and the keys of the location loops
+FftLaunch bucket_fft(const sfft_plan* P) {
   const sfft_params& p = P->p;
-  const int L = p.loops, Ll = p.loops_loc, K = p.B_thresh;
   const long long B = p.B;
-  if (marks && P->profile) HIPCK(hipEventRecord(P->ev[4], st));
   FftLaunch f;
   f.tab = &P->tabB;
   f.in = P->bins_t;
@@ -572,8 +575,8 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
   f.scratch = P->bins_scr;
   f.keys = P->bkeys;
   f.keys_bstride = B;
-  f.key_batches = Ll;
-  f.batch = L;
+  f.key_batches = p.loops_loc;
+  f.batch = p.loops;
   f.store = kStoreBoth;
   f.qmax = P->qmax_B;
   f.digits = P->bucket_digits;
@@ -582,10 +585,17 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
     f.perm = P->d_ai;
     f.perm_inv = P->d_a;
   }
-  HIPCK(fft_run(f, st));
+  return f;
+}
+
+// bucket: bucket FFT + cutoff (after the fold)
+sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
+  const sfft_params& p = P->p;
+  if (marks && P->profile) HIPCK(hipEventRecord(P->ev[4], st));
+  HIPCK(fft_run(bucket_fft(P), st));
   // ascending bucket lists: the hit list is ordered by (loop, bucket, walk)
-  HIPCK(select_topk(P->fp32, P->bkeys, B, (int)B, K, Ll, P->J, 1, P->selB, st, P->jsel, nullptr,
-                    P->bucket_digits));
+  HIPCK(select_topk(P->fp32, P->bkeys, p.B, p.B, p.B_thresh, p.loops_loc, P->J, 1, P->selB, st,
+                    P->jsel, nullptr, P->bucket_digits));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[5], st));
   return SFFT_OK;
 }
@@ -729,22 +739,32 @@ extern "C" sfft_status sfft_execute_async(sfft_plan* P, const void* d_x, const s
 
 // The device view of h when h is pinned host memory with room for `bytes` from h on, else
 // nullptr (pageable memory, or too short an allocation).  Asked on every call: an address
-// freed and reused for pageable memory must never be written through a stale view.
-static void* pinned_view(void* h, size_t bytes) {
-  hipPointerAttribute_t at;
-  if (hipPointerGetAttributes(&at, h) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
+// freed and reused for pageable memory must never be written through a stale view.  A range
+// lives for one call only, which asks once for all its pointers into one allocation.
+void* PinnedRange::view(void* h, size_t bytes) {
+  char* p = (char*)h;
+  if (!host || p < host || p >= host + size) {
+    host = nullptr;
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, h) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    if (at.type != hipMemoryTypeHost || !at.devicePointer) return nullptr;
+    hipDeviceptr_t base = nullptr;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)at.devicePointer) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    dev = (char*)base;
+    host = p - ((char*)at.devicePointer - dev);
+    if (p < host || p >= host + size) {
+      host = nullptr;
+      return nullptr;
+    }
   }
-  if (at.type != hipMemoryTypeHost || !at.devicePointer) return nullptr;
-  hipDeviceptr_t base = nullptr;
-  size_t size = 0;
-  if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)at.devicePointer) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  const size_t off = (size_t)((char*)at.devicePointer - (char*)base);
-  return (off <= size && size - off >= bytes) ? at.devicePointer : nullptr;
+  const size_t off = (size_t)(p - host);
+  return size - off >= bytes ? dev + off : nullptr;
 }
 
 // Graph mode: the transform's launch sequence is captured once and replayed (the draws are
@@ -890,7 +910,8 @@ extern "C" sfft_status sfft_execute(sfft_plan* P, const void* d_x, const sfft_dr
   if (!P) return SFFT_ERR_INVALID;
   // pinned h_nodes: the estimation kernel stores the nodes and the count straight into host
   // memory (no copies after the transform)
-  Node* zc = h_nodes ? (Node*)pinned_view(h_nodes, (size_t)P->cap * sizeof(Node)) : nullptr;
+  Node* zc =
+      h_nodes ? (Node*)PinnedRange().view(h_nodes, (size_t)P->cap * sizeof(Node)) : nullptr;
   if (zc) {
     sfft_status s = enqueue(P, d_x, dr, zc, P->count, P->h_count_dev);
     if (s != SFFT_OK) return s;

@@ -95,6 +95,17 @@ sfft_status draws_check(const sfft_plan* P, const sfft_draws* d);
 // packs the draws into the plan's pinned staging and copies them to the device on its stream
 sfft_status upload_draws(sfft_plan* P, const sfft_draws* dr);
 HashArgs hash_args(const sfft_plan* P, int* d_count);
+// the stages' launches, for a single transform or as jobs of a batch
+FftLaunch comb_fft(const sfft_plan* P, const void* d_x);
+FftLaunch bucket_fft(const sfft_plan* P);
+SelMark comb_mark(const HashArgs& h);
+// the device view of pinned host memory (one allocation at a time, for one call)
+struct PinnedRange {
+  char* host = nullptr;
+  char* dev = nullptr;
+  size_t size = 0;
+  void* view(void* h, size_t bytes);
+};
 // the transform in three stage groups on an explicit stream (marks: record the plan's
 // profiling events)
 sfft_status run_front(sfft_plan* P, const void* d_x, const HashArgs& h, hipStream_t st,

@@ -17,7 +17,7 @@
 //                count of each block (its digit > d0 count from the split plus its candidates
 //                >= T) and their exclusive prefix come out of the refine.
 // Short segments (select_in_block) take one launch instead: sel_block_kernel.
-#include "sfft_internal.h"
+#include "sfft_jobs.h"
 
 namespace sfft {
 
@@ -148,18 +148,19 @@ __device__ __forceinline__ u128 composite(K key, unsigned idx, int N, int IB) {
 }
 
 // ---- 1. top-digit histogram: one row of SEL_BINS counts per block (plain stores) ---------
+// (each stage's body takes its block bx and segment seg: a launch of one select, or of many)
 template <typename K>
-__global__ __launch_bounds__(SEL_NT) void sel_hist0_kernel(const K* __restrict__ keys,
-                                                           long long seg_stride, int N, int chunk,
-                                                           int nchunks,
-                                                           unsigned* __restrict__ rows,
-                                                           const uint16_t* __restrict__ digits) {
+__device__ __forceinline__ void sel_hist0_body(const K* __restrict__ keys, long long seg_stride,
+                                               int N, int chunk, int nchunks,
+                                               unsigned* __restrict__ rows,
+                                               const uint16_t* __restrict__ digits, int bx,
+                                               int seg) {
   __shared__ unsigned h[SEL_BINS];
-  const int tid = threadIdx.x, seg = blockIdx.y;
+  const int tid = threadIdx.x;
   for (int i = tid; i < SEL_BINS; i += SEL_NT) h[i] = 0u;
   __syncthreads();
   const K* kp = keys + (long long)seg * seg_stride;
-  const int begin = blockIdx.x * chunk, end = min(N, begin + chunk);
+  const int begin = bx * chunk, end = min(N, begin + chunk);
   constexpr int U = 8;   // independent loads in flight per thread
   if (digits) {          // the first digits only (2 bytes per key instead of 4 or 8)
     const uint16_t* dp = digits + (long long)seg * seg_stride;
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(SEL_NT) void sel_hist0_kernel(const K* __restrict__
     }
   }
   __syncthreads();
-  unsigned* row = rows + ((size_t)seg * nchunks + blockIdx.x) * SEL_BINS;
+  unsigned* row = rows + ((size_t)seg * nchunks + bx) * SEL_BINS;
   for (int i = tid; i < SEL_BINS; i += SEL_NT) row[i] = h[i];
 }
 
@@ -200,14 +201,13 @@ __global__ __launch_bounds__(SEL_NT) void sel_hist0_kernel(const K* __restrict__
 // a block sums 16 bins, 16 threads per bin each over every 16th row, then reduces in LDS
 constexpr int PICK_NT = 256;
 constexpr int PICK_BINS = 16;
-__global__ __launch_bounds__(PICK_NT) void sel_colsum_kernel(int nchunks,
-                                                             const unsigned* __restrict__ rows,
-                                                             unsigned* __restrict__ ghist) {
+__device__ __forceinline__ void sel_colsum_body(int nchunks, const unsigned* __restrict__ rows,
+                                                unsigned* __restrict__ ghist, int bx, int seg) {
   __shared__ unsigned part[PICK_NT / PICK_BINS][PICK_BINS];
-  const int tid = threadIdx.x, seg = blockIdx.y;
+  const int tid = threadIdx.x;
   const int bl = tid % PICK_BINS, g = tid / PICK_BINS;
   constexpr int G = PICK_NT / PICK_BINS;
-  const int bin0 = blockIdx.x * PICK_BINS;
+  const int bin0 = bx * PICK_BINS;
   const unsigned* r = rows + (size_t)seg * nchunks * SEL_BINS + bin0 + bl;
   unsigned a = 0u;
 #pragma unroll 4
@@ -229,22 +229,18 @@ __global__ __launch_bounds__(PICK_NT) void sel_colsum_kernel(int nchunks,
 // ccnt/ecnt[seg][b]: no global atomics (the refine pass compacts).  Keys stored in a KeyMap
 // order are recorded with their natural indices (the tie rule and the output use those).
 template <typename K>
-__global__ __launch_bounds__(SEL_NT) void sel_split_kernel(const K* __restrict__ keys,
-                                                           long long seg_stride, int N, int chunk,
-                                                           int nchunks, int emit, int Ksel,
-                                                           const unsigned* __restrict__ ghist,
-                                                           SelState* __restrict__ st,
-                                                           K* __restrict__ ckey,
-                                                           int* __restrict__ cidx,
-                                                           int* __restrict__ eidx,
-                                                           int* __restrict__ ccnt,
-                                                           int* __restrict__ ecnt,
-                                                           KeyMap km,
-                                                           const uint16_t* __restrict__ digits) {
+__device__ __forceinline__ void sel_split_body(const K* __restrict__ keys, long long seg_stride,
+                                               int N, int chunk, int nchunks, int emit, int Ksel,
+                                               const unsigned* __restrict__ ghist,
+                                               SelState* __restrict__ st, K* __restrict__ ckey,
+                                               int* __restrict__ cidx, int* __restrict__ eidx,
+                                               int* __restrict__ ccnt, int* __restrict__ ecnt,
+                                               KeyMap km, const uint16_t* __restrict__ digits,
+                                               int bx, int seg) {
   static_assert(SEL_NT * 4 == SEL_BINS, "the pick gives each thread four bins");
   __shared__ int s_nc, s_ne, s_d0;
   __shared__ int sh[16];
-  const int tid = threadIdx.x, seg = blockIdx.y;
+  const int tid = threadIdx.x;
   if (tid == 0) {
     s_nc = 0;
     s_ne = 0;
@@ -270,7 +266,7 @@ __global__ __launch_bounds__(SEL_NT) void sel_split_kernel(const K* __restrict__
         if (cum + (int)v[j] >= Ksel) {
           const int dd = SEL_BINS - 1 - (4 * tid + j);
           s_d0 = dd;
-          if (blockIdx.x == 0) {
+          if (bx == 0) {
             st[seg].d0 = dd;
             st[seg].need0 = Ksel - cum;
           }
@@ -283,11 +279,11 @@ __global__ __launch_bounds__(SEL_NT) void sel_split_kernel(const K* __restrict__
   __syncthreads();
   const unsigned d0 = (unsigned)s_d0;
   const K* kp = keys + (long long)seg * seg_stride;
-  const long long rb = (long long)seg * N + (long long)blockIdx.x * chunk;
+  const long long rb = (long long)seg * N + (long long)bx * chunk;
   K* ck = ckey + rb;
   int* ci = cidx + rb;
   int* ce = eidx + rb;
-  const int begin = blockIdx.x * chunk, end = min(N, begin + chunk);
+  const int begin = bx * chunk, end = min(N, begin + chunk);
   const uint16_t* dp = digits ? digits + (long long)seg * seg_stride : nullptr;
   // SU elements per thread at a time: their digit (or key) loads are in flight together, then
   // the candidates' key loads, so that the loop waits twice per SU elements, not twice per
@@ -333,8 +329,8 @@ __global__ __launch_bounds__(SEL_NT) void sel_split_kernel(const K* __restrict__
   }
   __syncthreads();
   if (tid == 0) {
-    ccnt[(long long)seg * nchunks + blockIdx.x] = s_nc;
-    ecnt[(long long)seg * nchunks + blockIdx.x] = s_ne;
+    ccnt[(long long)seg * nchunks + bx] = s_nc;
+    ecnt[(long long)seg * nchunks + bx] = s_ne;
   }
 }
 
@@ -344,19 +340,17 @@ constexpr int CMP_NT = 256;
 // ---- 2b. compaction: block b of the split moves its candidates to the contiguous list at
 // the sum of the counts of blocks < b, and (unordered mode) its emitted indices to out --------
 template <typename K>
-__global__ __launch_bounds__(CMP_NT) void sel_compact_kernel(int N, int Ksel, int chunk,
-                                                             int nchunks, int emit,
-                                                             SelState* __restrict__ st,
-                                                             const K* __restrict__ bkey,
-                                                             const int* __restrict__ bidx,
-                                                             const int* __restrict__ eidx,
-                                                             const int* __restrict__ ccnt,
-                                                             const int* __restrict__ ecnt,
-                                                             K* __restrict__ ckey,
-                                                             int* __restrict__ cidx,
-                                                             int* __restrict__ out) {
+__device__ __forceinline__ void sel_compact_body(int N, int Ksel, int chunk, int nchunks, int emit,
+                                                 SelState* __restrict__ st,
+                                                 const K* __restrict__ bkey,
+                                                 const int* __restrict__ bidx,
+                                                 const int* __restrict__ eidx,
+                                                 const int* __restrict__ ccnt,
+                                                 const int* __restrict__ ecnt,
+                                                 K* __restrict__ ckey, int* __restrict__ cidx,
+                                                 int* __restrict__ out, int bx, int seg) {
   __shared__ int sh[16];
-  const int tid = threadIdx.x, seg = blockIdx.y, b = blockIdx.x;
+  const int tid = threadIdx.x, b = bx;
   const int* cc = ccnt + (long long)seg * nchunks;
   const int* ec = ecnt + (long long)seg * nchunks;
   int pc = 0, pe = 0;
@@ -423,15 +417,14 @@ __device__ __forceinline__ u128 block_min_u128(u128 v, u128* s) {
 // ecnt and the candidates >= T of each block: the write pass needs no count pass.
 constexpr int RF_CAP = 2048;
 template <typename K>
-__global__ __launch_bounds__(1024) void sel_refine_kernel(int N, int Ksel, int emit,
-                                                          SelState* __restrict__ st,
-                                                          const K* __restrict__ ckey,
-                                                          const int* __restrict__ cidx,
-                                                          int* __restrict__ out,
-                                                          const int* __restrict__ ccnt,
-                                                          int nchunks, int chunk,
-                                                          const int* __restrict__ ecnt,
-                                                          int* __restrict__ base) {
+__device__ __forceinline__ void sel_refine_body(int N, int Ksel, int emit,
+                                                SelState* __restrict__ st,
+                                                const K* __restrict__ ckey,
+                                                const int* __restrict__ cidx,
+                                                int* __restrict__ out,
+                                                const int* __restrict__ ccnt, int nchunks,
+                                                int chunk, const int* __restrict__ ecnt,
+                                                int* __restrict__ base, int seg) {
   __shared__ unsigned h[SEL_BINS];
   __shared__ u128 lst[2][RF_CAP];
   __shared__ int s_len[2];
@@ -441,7 +434,7 @@ __global__ __launch_bounds__(1024) void sel_refine_kernel(int N, int Ksel, int e
   __shared__ int s_out;
   __shared__ int s_pre[SEL_MAX_CHUNKS + 1];
   __shared__ int s_bc[SEL_MAX_CHUNKS];
-  const int tid = threadIdx.x, seg = blockIdx.x;
+  const int tid = threadIdx.x;
   const int IB = index_bits(N);
   const int TB = KeyBits<K>::KB + IB;
   int nc;
@@ -629,22 +622,21 @@ __device__ __forceinline__ bool sel_pred(K k, int i, int N, int IB, u128 T) {
 }
 
 template <typename K>
-__global__ __launch_bounds__(SEL_NT) void sel_write_kernel(const K* __restrict__ keys,
-                                                           long long seg_stride, int N, int chunk,
-                                                           int nchunks, int Ksel,
-                                                           const SelState* __restrict__ st,
-                                                           const int* __restrict__ base0,
-                                                           int* __restrict__ out,
-                                                           unsigned* __restrict__ bits) {
+__device__ __forceinline__ void sel_write_body(const K* __restrict__ keys, long long seg_stride,
+                                               int N, int chunk, int nchunks, int Ksel,
+                                               const SelState* __restrict__ st,
+                                               const int* __restrict__ base0,
+                                               int* __restrict__ out,
+                                               unsigned* __restrict__ bits, int bx, int seg) {
   __shared__ int sh[16];
   __shared__ int s_tot;
-  const int seg = blockIdx.y, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const int IB = index_bits(N);
   const u128 T = ((u128)st[seg].thr_hi << 64) | (u128)st[seg].thr_lo;
   const K* kp = keys + (long long)seg * seg_stride;
-  int base = base0[(long long)seg * nchunks + blockIdx.x];
+  int base = base0[(long long)seg * nchunks + bx];
   int* o = out + (long long)seg * Ksel;
-  const int begin = blockIdx.x * chunk, end = min(N, begin + chunk);
+  const int begin = bx * chunk, end = min(N, begin + chunk);
   for (int b0 = begin; b0 < end; b0 += SEL_NT) {
     const int i = b0 + tid;
     const bool p = i < end && sel_pred<K>(kp[i], i, N, IB, T);
@@ -735,13 +727,11 @@ __device__ __forceinline__ void sb_pick(const unsigned* h, int nb, int r, int* s
 }
 
 template <typename K, int PER>
-__global__ __launch_bounds__(SEL_NT) void sel_block_kernel(const K* __restrict__ keys,
-                                                           long long seg_stride, int N, int Ksel,
-                                                           int* __restrict__ out,
-                                                           unsigned* __restrict__ bits,
-                                                           KeyMap km,
-                                                           const uint16_t* __restrict__ digits,
-                                                           int vec, SelMark mark) {
+__device__ __forceinline__ void sel_block_body(const K* __restrict__ keys, long long seg_stride,
+                                               int N, int Ksel, int* __restrict__ out,
+                                               unsigned* __restrict__ bits, KeyMap km,
+                                               const uint16_t* __restrict__ digits, int vec,
+                                               const SelMark& mark, int seg) {
   using CT = typename CompOf<K>::type;
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __shared__ unsigned h[SEL_BINS];
@@ -753,7 +743,7 @@ __global__ __launch_bounds__(SEL_NT) void sel_block_kernel(const K* __restrict__
   __shared__ int sh[16];
   __shared__ int s_pick[3];
   __shared__ int s_nc;
-  const int tid = threadIdx.x, seg = blockIdx.x;
+  const int tid = threadIdx.x;
   const int IB = index_bits(N), TB = KeyBits<K>::KB + IB;
   const K* kp = keys + (long long)seg * seg_stride;
   const int i0 = tid * PER;
@@ -953,22 +943,91 @@ __global__ __launch_bounds__(SEL_NT) void sel_block_kernel(const K* __restrict__
   }
 }
 
-template <typename K>
-static void sel_block_go(const K* keys, long long seg_stride, int N, int Ksel, int segs, int* out,
-                         unsigned* bits, const KeyMap& km, const uint16_t* digits,
-                         const SelMark& mark, hipStream_t st) {
-  const int vec = ((uintptr_t)digits & 15) == 0 && (seg_stride & 7) == 0;   // 16-byte loads
-  const dim3 grid(segs), nt(SEL_NT);
-#define SFFT_SB(PER)                                                                            \
-  if (N <= PER * SEL_NT) {                                                                      \
-    hipLaunchKernelGGL((sel_block_kernel<K, PER>), grid, nt, 0, st, keys, seg_stride, N, Ksel,  \
-                       out, bits, km, digits, vec, mark);                                       \
-    return;                                                                                     \
+// ---- kernels: every workgroup of a launch belongs to a job (sfft_jobs.h); one select is a
+// launch of one job, its workgroups in the grid's (x, y) ---------------------------------------
+struct SelOne {   // one select: its job, by value
+  SelJob j;
+  __device__ __forceinline__ bool get(SelJob& out, int& bx, int& seg, int) const {
+    out = j;
+    bx = blockIdx.x;
+    seg = blockIdx.y;
+    return true;
   }
-  SFFT_SB(8)
-  SFFT_SB(16)
-  SFFT_SB(32)
-#undef SFFT_SB
+};
+struct SelMany {  // many selects: per x workgroups of a job (0: its chunks) and segment
+  JobsDev t;
+  __device__ __forceinline__ bool get(SelJob& out, int& bx, int& seg, int per) const {
+    const SelJob* j = job_here<SelJob>(t);
+    if (!j) return false;
+    out = *j;
+    const int i = (int)blockIdx.x - j->block0, nx = per ? per : j->nchunks;
+    bx = i % nx;
+    seg = i / nx;
+    return true;
+  }
+};
+
+template <typename K, typename From>
+__global__ __launch_bounds__(SEL_NT) void sel_hist0_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, 0)) return;
+  sel_hist0_body<K>((const K*)j.keys, j.seg_stride, j.N, j.chunk, j.nchunks, j.rows, j.digits, bx,
+                    seg);
+}
+template <typename From>
+__global__ __launch_bounds__(PICK_NT) void sel_colsum_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, SEL_BINS / PICK_BINS)) return;
+  sel_colsum_body(j.nchunks, j.rows, j.sums, bx, seg);
+}
+template <typename K, typename From>
+__global__ __launch_bounds__(SEL_NT) void sel_split_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, 0)) return;
+  sel_split_body<K>((const K*)j.keys, j.seg_stride, j.N, j.chunk, j.nchunks, j.ordered ? 0 : 1, j.K,
+                    j.sums, (SelState*)j.state, (K*)j.blk_key, j.blk_idx, j.emit_idx, j.ccnt,
+                    j.ecnt, j.map, j.digits, bx, seg);
+}
+// unordered: the candidates of the split's blocks side by side, its winners to the output
+template <typename K, typename From>
+__global__ __launch_bounds__(CMP_NT) void sel_compact_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, 0)) return;
+  sel_compact_body<K>(j.N, j.K, j.chunk, j.nchunks, 1, (SelState*)j.state, (const K*)j.blk_key,
+                      j.blk_idx, j.emit_idx, j.ccnt, j.ecnt, (K*)j.cand_key, j.cand_idx, j.out, bx,
+                      seg);
+}
+// ordered: the refine reads the candidates from the split's per-block regions
+template <typename K, typename From>
+__global__ __launch_bounds__(1024) void sel_refine_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, 1)) return;
+  const bool o = j.ordered != 0;
+  sel_refine_body<K>(j.N, j.K, o ? 0 : 1, (SelState*)j.state,
+                     (const K*)(o ? j.blk_key : j.cand_key), o ? j.blk_idx : j.cand_idx, j.out,
+                     o ? j.ccnt : nullptr, j.nchunks, j.chunk, o ? j.ecnt : nullptr,
+                     o ? j.cnt : nullptr, seg);
+}
+template <typename K, typename From>
+__global__ __launch_bounds__(SEL_NT) void sel_write_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, 0)) return;
+  sel_write_body<K>((const K*)j.keys, j.seg_stride, j.N, j.chunk, j.nchunks, j.K,
+                    (const SelState*)j.state, j.cnt, j.out, j.bits, bx, seg);
+}
+template <typename K, int PER, typename From>
+__global__ __launch_bounds__(SEL_NT) void sel_block_kernel(From f) {
+  SelJob j;
+  int bx, seg;
+  if (!f.get(j, bx, seg, 1)) return;
+  sel_block_body<K, PER>((const K*)j.keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits,
+                         j.vec, j.mark, seg);
 }
 
 // Up to 32768 keys one workgroup beats the chain of launches, in both precisions; at 65536 its
@@ -978,58 +1037,83 @@ static void sel_block_go(const K* keys, long long seg_stride, int N, int Ksel, i
 constexpr int SB_MAX_N = 32768;
 bool select_in_block(int N) { return N <= SB_MAX_N; }
 
-template <typename K>
-static hipError_t select_impl(const K* keys, long long seg_stride, int N, int Ksel, int segs,
-                              int* out, int ordered, const SelectWork& w, hipStream_t st,
-                              unsigned* bits, const KeyMap* map, const uint16_t* digits,
-                              const SelMark* mark) {
-  const int chunk = sel_chunk(N);
-  const int nchunks = (N + chunk - 1) / chunk;
-  if (nchunks > SEL_MAX_CHUNKS || nchunks > w.max_chunks || segs > w.max_segs)
+// the job of one select_topk call
+static hipError_t select_job(SelJob& j, int is_fp32, const void* keys, long long seg_stride, int N,
+                             int K, int segs, int* out, int ordered, const SelectWork& w,
+                             unsigned* bits, const KeyMap* map, const uint16_t* digits,
+                             const SelMark* mark) {
+  // the write pass reads the keys
+  if (ordered && digits && !select_in_block(N)) return hipErrorInvalidValue;
+  if (mark && !select_in_block(N)) return hipErrorInvalidValue;   // the one-workgroup select marks
+  if (N < 2 || K < 1 || K > N || segs < 1) return hipErrorInvalidValue;
+  j = SelJob();
+  j.chunk = sel_chunk(N);
+  j.nchunks = (N + j.chunk - 1) / j.chunk;
+  if (j.nchunks > SEL_MAX_CHUNKS || j.nchunks > w.max_chunks || segs > w.max_segs)
     return hipErrorInvalidValue;
-  KeyMap km;
   if (map && map->mid != 0) {
     // the ordered compaction walks storage order: natural order only
     if (ordered || (1LL << map->log2n) != (long long)N) return hipErrorInvalidValue;
-    km = *map;
+    j.map = *map;
   }
-  if (select_in_block(N)) {
-    sel_block_go<K>(keys, seg_stride, N, Ksel, segs, out, bits, km, digits,
-                    mark ? *mark : SelMark(), st);
+  j.keys = keys;
+  j.seg_stride = seg_stride;
+  j.N = N;
+  j.K = K;
+  j.ordered = ordered;
+  j.segs = segs;
+  j.vec = ((uintptr_t)digits & 15) == 0 && (seg_stride & 7) == 0;   // 16-byte loads of digits
+  // work layout: column sums, then the per-block histogram rows
+  j.sums = w.hist;
+  j.rows = w.hist + (size_t)segs * SEL_BINS;
+  j.state = w.state;
+  j.blk_key = w.blk_key;
+  j.blk_idx = w.blk_idx;
+  j.emit_idx = w.emit_idx;
+  j.ccnt = w.ccnt;
+  j.ecnt = w.ecnt;
+  j.cand_key = w.cand_key;
+  j.cand_idx = w.cand_idx;
+  j.cnt = w.cnt;
+  j.out = out;
+  j.bits = bits;
+  j.digits = digits;
+  if (mark) j.mark = *mark;
+  (void)is_fp32;
+  return hipSuccess;
+}
+
+// elements per thread of the one-workgroup select, as an index into 8, 16, 32
+static int block_variant(int N) { return N <= 8 * SEL_NT ? 0 : N <= 16 * SEL_NT ? 1 : 2; }
+
+template <typename K, typename From>
+static void block_go(int variant, const From& f, dim3 grid, hipStream_t st) {
+  if (variant == 0)
+    hipLaunchKernelGGL((sel_block_kernel<K, 8, From>), grid, dim3(SEL_NT), 0, st, f);
+  else if (variant == 1)
+    hipLaunchKernelGGL((sel_block_kernel<K, 16, From>), grid, dim3(SEL_NT), 0, st, f);
+  else
+    hipLaunchKernelGGL((sel_block_kernel<K, 32, From>), grid, dim3(SEL_NT), 0, st, f);
+}
+
+template <typename K>
+static hipError_t select_one(const SelJob& j, hipStream_t st) {
+  const SelOne f{j};
+  const dim3 wide(j.nchunks, j.segs);
+  if (select_in_block(j.N)) {
+    block_go<K>(block_variant(j.N), f, dim3(1, j.segs), st);
     return hipGetLastError();
   }
-  if (mark) return hipErrorInvalidValue;   // only the one-workgroup select marks
-  dim3 grid(nchunks, segs);
-  SelState* S = (SelState*)w.state;
-  // work layout: column sums, then the per-block histogram rows
-  unsigned* rows = w.hist + (size_t)segs * SEL_BINS;
-  hipLaunchKernelGGL((sel_hist0_kernel<K>), grid, dim3(SEL_NT), 0, st, keys, seg_stride, N,
-                     chunk, nchunks, rows, digits);
-  hipLaunchKernelGGL(sel_colsum_kernel, dim3(SEL_BINS / PICK_BINS, segs), dim3(PICK_NT), 0, st,
-                     nchunks, (const unsigned*)rows, w.hist);
+  hipLaunchKernelGGL((sel_hist0_kernel<K, SelOne>), wide, dim3(SEL_NT), 0, st, f);
+  hipLaunchKernelGGL((sel_colsum_kernel<SelOne>), dim3(SEL_BINS / PICK_BINS, j.segs),
+                     dim3(PICK_NT), 0, st, f);
   // (the split blocks pick d0 from the column sums themselves)
-  hipLaunchKernelGGL((sel_split_kernel<K>), grid, dim3(SEL_NT), 0, st, keys, seg_stride, N,
-                     chunk, nchunks, ordered ? 0 : 1, Ksel, (const unsigned*)w.hist, S,
-                     (K*)w.blk_key,
-                     w.blk_idx, w.emit_idx, w.ccnt, w.ecnt, km, digits);
-  if (ordered) {
-    // the refine reads the candidates from the split's per-block regions
-    hipLaunchKernelGGL((sel_refine_kernel<K>), dim3(segs), dim3(1024), 0, st, N, Ksel, 0, S,
-                       (const K*)w.blk_key, (const int*)w.blk_idx, out, (const int*)w.ccnt,
-                       nchunks, chunk, (const int*)w.ecnt, w.cnt);
-  } else {
-    hipLaunchKernelGGL((sel_compact_kernel<K>), grid, dim3(CMP_NT), 0, st, N, Ksel, chunk,
-                       nchunks, 1, S, (const K*)w.blk_key, (const int*)w.blk_idx,
-                       (const int*)w.emit_idx, (const int*)w.ccnt, (const int*)w.ecnt,
-                       (K*)w.cand_key, w.cand_idx, out);
-    hipLaunchKernelGGL((sel_refine_kernel<K>), dim3(segs), dim3(1024), 0, st, N, Ksel, 1, S,
-                       (const K*)w.cand_key, (const int*)w.cand_idx, out, (const int*)nullptr,
-                       nchunks, chunk, (const int*)nullptr, (int*)nullptr);
-  }
-  if (ordered) {
-    hipLaunchKernelGGL((sel_write_kernel<K>), grid, dim3(SEL_NT), 0, st, keys, seg_stride, N,
-                       chunk, nchunks, Ksel, (const SelState*)S, (const int*)w.cnt, out, bits);
-  }
+  hipLaunchKernelGGL((sel_split_kernel<K, SelOne>), wide, dim3(SEL_NT), 0, st, f);
+  if (!j.ordered)
+    hipLaunchKernelGGL((sel_compact_kernel<K, SelOne>), wide, dim3(CMP_NT), 0, st, f);
+  hipLaunchKernelGGL((sel_refine_kernel<K, SelOne>), dim3(1, j.segs), dim3(1024), 0, st, f);
+  if (j.ordered)
+    hipLaunchKernelGGL((sel_write_kernel<K, SelOne>), wide, dim3(SEL_NT), 0, st, f);
   return hipGetLastError();
 }
 
@@ -1037,14 +1121,58 @@ hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int 
                        int segs, int* out, int ordered, const SelectWork& w, hipStream_t st,
                        unsigned* bits, const KeyMap* map, const uint16_t* digits,
                        const SelMark* mark) {
-  // the write pass reads the keys
-  if (ordered && digits && !select_in_block(N)) return hipErrorInvalidValue;
-  if (N < 2 || K < 1 || K > N || segs < 1) return hipErrorInvalidValue;
-  if (is_fp32)
-    return select_impl<unsigned int>((const unsigned int*)keys, seg_stride, N, K, segs, out,
-                                     ordered, w, st, bits, map, digits, mark);
-  return select_impl<unsigned long long>((const unsigned long long*)keys, seg_stride, N, K, segs,
-                                         out, ordered, w, st, bits, map, digits, mark);
+  SelJob j;
+  const hipError_t e = select_job(j, is_fp32, keys, seg_stride, N, K, segs, out, ordered, w, bits,
+                                  map, digits, mark);
+  if (e != hipSuccess) return e;
+  return is_fp32 ? select_one<unsigned int>(j, st) : select_one<unsigned long long>(j, st);
+}
+
+hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long seg_stride, int N,
+                           int K, int segs, int* out, int ordered, const SelectWork& w,
+                           unsigned* bits, const KeyMap* map, const uint16_t* digits,
+                           const SelMark* mark) {
+  SelJob j;
+  const hipError_t e = select_job(j, is_fp32, keys, seg_stride, N, K, segs, out, ordered, w, bits,
+                                  map, digits, mark);
+  if (e != hipSuccess) return e;
+  g.fp32 = is_fp32;
+  if (select_in_block(N)) {
+    g.block[block_variant(N)].add(j, segs);
+  } else {
+    g.wide.add(j, j.nchunks * segs);
+    g.sums.add(j, SEL_BINS / PICK_BINS * segs);
+    g.refine.add(j, segs);
+  }
+  return hipSuccess;
+}
+
+// every select of the group is ordered, or none is (a batch's bucket cutoffs, or its combs')
+template <typename K>
+static hipError_t select_many(const SelGroup& g, hipStream_t st) {
+  for (int v = 0; v < 3; ++v)
+    if (g.block[v].dev.blocks)
+      block_go<K>(v, SelMany{g.block[v].dev}, dim3(g.block[v].dev.blocks), st);
+  if (g.wide.dev.blocks) {
+    const SelMany wide{g.wide.dev}, sums{g.sums.dev}, refine{g.refine.dev};
+    const dim3 nw(wide.t.blocks);
+    const bool ordered = g.wide.jobs[0].ordered != 0;
+    hipLaunchKernelGGL((sel_hist0_kernel<K, SelMany>), nw, dim3(SEL_NT), 0, st, wide);
+    hipLaunchKernelGGL((sel_colsum_kernel<SelMany>), dim3(sums.t.blocks), dim3(PICK_NT), 0, st,
+                       sums);
+    hipLaunchKernelGGL((sel_split_kernel<K, SelMany>), nw, dim3(SEL_NT), 0, st, wide);
+    if (!ordered)
+      hipLaunchKernelGGL((sel_compact_kernel<K, SelMany>), nw, dim3(CMP_NT), 0, st, wide);
+    hipLaunchKernelGGL((sel_refine_kernel<K, SelMany>), dim3(refine.t.blocks), dim3(1024), 0, st,
+                       refine);
+    if (ordered)
+      hipLaunchKernelGGL((sel_write_kernel<K, SelMany>), nw, dim3(SEL_NT), 0, st, wide);
+  }
+  return hipGetLastError();
+}
+
+hipError_t select_jobs_launch(const SelGroup& g, hipStream_t st) {
+  return g.fp32 ? select_many<unsigned int>(g, st) : select_many<unsigned long long>(g, st);
 }
 
 }  // namespace sfft
