@@ -390,7 +390,9 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
   }
   const int r = A.r;
   const int R = 1 << r;
-  const int RP = R + (R >> 4) + 1;   // padded column stride (see LPAD)
+  // padded column stride (see LPAD); rows of 16 points and more: no skew slot, so that any
+  // number of them fits the tile
+  const int RP = R + (R >> 4) + ((LOAD == kLoadRows && R >= 16) ? 0 : 1);
   const int log2Lprev = A.log2Lprev;
   const int log2Lcur = log2Lprev + r;
   const long long Lprev = 1LL << log2Lprev;
@@ -405,7 +407,10 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
   // grouped differently).
   constexpr bool rows = (LOAD == kLoadCombRows || LOAD == kLoadCombRowsG);
   int log2cpj = 0;
-  if (first) {
+  if (LOAD == kLoadRows) {
+    log2ncol = A.log2Q;   // tile column c is row (tile << log2Q) + c
+    log2cpj = log2ncol;
+  } else if (first) {
     log2ncol = min(A.log2Q, A.log2N - log2Lcur);
     log2cpj = log2ncol;
     if (LOAD == kLoadCombRowsG) log2cpj = log2ncol - ((A.log2N - log2Lcur) - A.log2nlo);
@@ -464,7 +469,9 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
       const int v = e >> log2ncol;
       const long long g = gbase + c + vstride * v;
       const T2* src;
-      if (LOAD == kLoadComb)
+      if (LOAD == kLoadRows)   // (a row past the last one reads the last one)
+        src = in + (min(((long long)tile << (log2ncol + r)) + e, ((long long)A.nbatch << r) - 1));
+      else if (LOAD == kLoadComb)
         src = cx + g * (long long)A.comb_sigma;
       else if (rows) {
         const long long gr = (LOAD == kLoadCombRowsG) ? gbase + qoff(c) + vstride * v : g;
@@ -587,8 +594,9 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
       for (int k = 0; k < LB; ++k) {
         // (a clamped element is stored again with its own value: no branch)
         const int e = min(tid + (kb + k) * NT, TE - 1);
-        const int c = e & (ncol - 1);
-        const int v = (LOAD == kLoadPerm) ? perm_v(e) : e >> log2ncol;
+        const int c = (LOAD == kLoadRows) ? e >> r : e & (ncol - 1);
+        const int v = (LOAD == kLoadPerm) ? perm_v(e)
+                                          : (LOAD == kLoadRows ? e & (R - 1) : e >> log2ncol);
         lds[c * RP + LPAD(v)] = val[k];
       }
     }
@@ -650,6 +658,10 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
                 ? (long long)(((uint32_t)(q0 + c) * pinv) & (((uint32_t)nq) - 1u))
                 : (LOAD == kLoadCombRowsG ? q0 + qoff(c) : q0 + c);
         g = qc * R + kk;
+        if (LOAD == kLoadRows) {
+          g = ((long long)tile << (log2ncol + r)) + e;
+          if (g >= ((long long)A.nbatch << r)) continue;
+        }
       } else {
         c = e & (ncol - 1);
         kk = e >> log2ncol;
@@ -750,6 +762,8 @@ static hipError_t dispatch_pass(const PassArgs& A, int load, int store, int tw, 
     return dispatch_store<Real, kLoadPerm, kTwNone>(A, store, tiles, batch, st);
   if (load == kLoadComb)
     return dispatch_store<Real, kLoadComb, kTwNone>(A, store, tiles, batch, st);
+  if (load == kLoadRows)
+    return launch_pass<Real, kLoadRows, kStoreCplx, kTwNone>(A, tiles, 1, st);
   if (tw == kTwSplit)
     return dispatch_store<Real, kLoadPlain, kTwSplit>(A, store, tiles, batch, st);
   if (tw == kTwDirect)
@@ -766,6 +780,25 @@ static int pass_log2q(const FftTables& T, const FftLaunch& L, int p, int r, int 
   while ((1 << (log2Q + 1)) <= qmax && ((1 << (log2Q + 1)) << r) <= cap) ++log2Q;
   if (p > 0 && log2Q > log2Lprev) log2Q = log2Lprev;
   return log2Q;
+}
+
+// Single-pass transforms of adjacent rows: rows per tile (log2), or -1 where the plain pass runs
+// them (one row per workgroup and batch index).  As many rows as fill a tile, while at least
+// 512 tiles are left (two workgroups per CU).  2^24 complex64 points in all, one row per workgroup,
+// then rows filling tiles: rows of 16 points 6158 -> 42 us, 128 points 904 -> 53 us, 512 points
+// 387 -> 60 us, 2048 points 94 -> 62 us.
+static int rows_log2q(const FftTables& T, const FftLaunch& L) {
+  const long long N = 1LL << T.log2n;
+  if (T.npass != 1 || L.load != kLoadPlain || L.store != kStoreCplx || L.batch < 2 ||
+      L.in_bstride != N || L.out_bstride != N)
+    return -1;
+  const int r = T.log2n, cap = tile_cap(T.is_fp32, kLoadRows);
+  const int R = 1 << r, RP = R + (R >> 4) + (R >= 16 ? 0 : 1);
+  int q = 0;
+  while ((2LL << q) * R <= cap && (2LL << q) * RP <= cap + cap / 16 &&
+         (L.batch >> (q + 1)) >= 512)
+    ++q;
+  return q;
 }
 
 KeyMap fft_keys_map(const FftLaunch& L) {
@@ -814,9 +847,14 @@ static hipError_t each_pass(const FftLaunch& L, F&& fn) {
     A.r = r;
     A.log2Lprev = log2Lprev;
     int load = (p == 0) ? L.load : kLoadPlain;
-    const int log2Q = pass_log2q(T, L, p, r, log2Lprev);
+    int log2Q = pass_log2q(T, L, p, r, log2Lprev);
+    const int rq = rows_log2q(T, L);
     int tiles;
-    if (p == 0) {
+    if (rq >= 0) {
+      load = kLoadRows;
+      log2Q = rq;
+      tiles = (int)(((long long)L.batch + (1LL << rq) - 1) >> rq);
+    } else if (p == 0) {
       const int lnq = log2N - log2Lcur;
       const int lq = log2Q < lnq ? log2Q : lnq;
       tiles = 1 << (lnq - lq);
@@ -873,7 +911,7 @@ hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
 hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L) {
   const int fp32 = L.tab->is_fp32;
   return each_pass(L, [&](int p, const PassArgs& A, int load, int store, int tw, int tiles) {
-    if (load == kLoadWiden || load == kLoadTaps || store == kStoreHead)
+    if (load == kLoadWiden || load == kLoadTaps || load == kLoadRows || store == kStoreHead)
       return hipErrorInvalidValue;
     auto it = std::find_if(g.begin(), g.end(), [&](const FftGroup& x) {
       return x.pass == p && x.load == load && x.store == store && x.tw == tw && x.fp32 == fp32;

@@ -56,9 +56,11 @@ __device__ __forceinline__ unsigned sel_first_digit(unsigned long long key) {
 // kLoadWiden: FP64 transforms of a complex64 input, widened as it is loaded.
 // kLoadTaps: FP64 transforms of `taps` window taps t (h = taps / 2) laid out on N points:
 // element g is t[h + g] for g < h, t[g - (N - h)] for g >= N - h, else 0.
+// kLoadRows: single-pass transforms of adjacent rows, a tile's columns being whole rows (chosen
+// per launch by fft_run; callers set kLoadPlain).
 // kStoreHead: FP64 values, the first `head` of the output, times `scale`.
 enum FftLoad { kLoadPlain = 0, kLoadComb = 1, kLoadCombRows = 2, kLoadPerm = 3, kLoadCombRowsG = 4,
-               kLoadWiden = 5, kLoadTaps = 6 };
+               kLoadWiden = 5, kLoadTaps = 6, kLoadRows = 7 };
 enum FftStore { kStoreCplx = 0, kStoreKeys = 1, kStoreBoth = 2, kStoreHead = 3 };
 
 // One canonical FFT of `batch` transforms.  Passes ping-pong between out and scratch so that
