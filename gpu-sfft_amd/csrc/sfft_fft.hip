@@ -98,17 +98,26 @@ constexpr int FFT_QMAX = 32;
 // column per tile (32 KB FP64 / 16 KB FP32) with 512 threads (FP64: four workgroups per CU)
 // or 256 (FP32: eight), so more gathers are in flight while other workgroups compute
 // (measured at n = 2^27: 256 threads cost FP64 10 us, 1024 cost it 65 us; FP32 gains 6 us).
-template <typename Real, int LOAD = 0>
-struct Tile {   // LOAD: kLoadComb (gathers from x); kLoadPlain, kLoadCombRows, kLoadPerm (plain)
-  static constexpr int cap = LOAD == 1 ? 2048 : (sizeof(Real) == 8 ? 4096 : 8192);
+// LOADX: an FftLoad, plus kSmallTile for a quarter of the elements and threads.  A thread's
+// loops cover its share of a full tile whatever the tile holds, so a pass whose columns cannot
+// fill one (few columns, short sub-FFTs) takes the quarter instead of idling three of four
+// threads (pass_shape).
+constexpr int kSmallTile = 16;
+template <typename Real, int LOADX = 0>
+struct Tile {   // kLoadComb (gathers from x), or any other load (plain)
+  static constexpr bool comb = LOADX == kLoadComb, small = (LOADX & kSmallTile) != 0;
+  static constexpr int cap = comb ? 2048 : (sizeof(Real) == 8 ? 4096 : 8192) / (small ? 4 : 1);
   // threads per workgroup; FP32 plain tiles: 512, so that a radix-16 step's 16 complex64
   // values and their twiddles fit the 128 registers of two 512-thread workgroups per CU
   // (FP64 keeps 1024 threads and single radix-4 stages: measured faster at 2^22)
-  static constexpr int nt = LOAD == 1 ? (sizeof(Real) == 8 ? 512 : 256) : (sizeof(Real) == 8 ? 1024 : 512);
+  static constexpr int nt = comb ? (sizeof(Real) == 8 ? 512 : 256)
+                                 : (sizeof(Real) == 8 ? 1024 : 512) / (small ? 4 : 1);
   static constexpr int ept = cap / nt;                 // elements per thread
+  // 8 (FP64) or 4 (FP32) waves per SIMD: two full plain tiles per CU
+  static constexpr int waves = comb ? 1 : sizeof(Real) == 8 ? 8 : 4;
 };
 static int tile_cap(int is_fp32, int load) {
-  if (load == 1) return Tile<float, 1>::cap;
+  if (load == kLoadComb) return Tile<float, kLoadComb>::cap;
   return is_fp32 ? Tile<float>::cap : Tile<double>::cap;
 }
 
@@ -367,12 +376,13 @@ __device__ __forceinline__ void fft_stage2(T2* lds, int RP, int r, int log2ncol,
 enum PassTw { kTwNone = 0, kTwDirect = 1, kTwSplit = 2 };
 
 // (bx, by) of nbx: the workgroup's tile and batch (comb gathers: tile and batch in bx alone)
-template <typename Real, int LOAD, int STORE, int TW>
+template <typename Real, int LOADX, int STORE, int TW>
 __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx, int by) {
+  constexpr int LOAD = LOADX & ~kSmallTile;
   using T2 = typename CT<Real>::T2;
   using KT = typename CT<Real>::K;
-  constexpr int CAP = Tile<Real, LOAD>::cap, EPT = Tile<Real, LOAD>::ept;
-  constexpr int NT = Tile<Real, LOAD>::nt;
+  constexpr int CAP = Tile<Real, LOADX>::cap, EPT = Tile<Real, LOADX>::ept;
+  constexpr int NT = Tile<Real, LOADX>::nt;
   __shared__ T2 lds[CAP + CAP / 16 + FFT_QMAX];
   const int tid = threadIdx.x;
   // The comb-gathering pass runs all comb loops in one grid dimension, loop index fastest,
@@ -687,37 +697,49 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
   }
 }
 
-template <typename Real, int LOAD, int STORE, int TW>
-// two workgroups per CU for the plain tiles: 8 waves per SIMD at 1024 threads, 4 at 512
-__global__ __launch_bounds__((Tile<Real, LOAD>::nt),
-                             (LOAD == 1 ? 1 : Tile<Real, LOAD>::nt / 128)) void fft_pass_kernel(
-    PassArgs A) {
-  fft_pass_body<Real, LOAD, STORE, TW>(A, blockIdx.x, gridDim.x, blockIdx.y);
+template <typename Real, int LOADX, int STORE, int TW>
+__global__ __launch_bounds__((Tile<Real, LOADX>::nt), (Tile<Real, LOADX>::waves)) void
+fft_pass_kernel(PassArgs A) {
+  fft_pass_body<Real, LOADX, STORE, TW>(A, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
 // the same pass of many signals (jobs of tiles x batch workgroups)
-template <typename Real, int LOAD, int STORE, int TW>
-__global__ __launch_bounds__((Tile<Real, LOAD>::nt),
-                             (LOAD == 1 ? 1
-                                        : Tile<Real, LOAD>::nt / 128)) void fft_jobs_kernel(
-    JobsDev t) {
+template <typename Real, int LOADX, int STORE, int TW>
+__global__ __launch_bounds__((Tile<Real, LOADX>::nt), (Tile<Real, LOADX>::waves)) void
+fft_jobs_kernel(JobsDev t) {
   const FftJob* j = job_here<FftJob>(t);
   if (!j) return;
   const PassArgs A = j->a;
   const int i = (int)blockIdx.x - j->block0;
-  if constexpr (LOAD == kLoadComb) {
-    fft_pass_body<Real, LOAD, STORE, TW>(A, i, j->tiles * A.nbatch, 0);
+  if constexpr (LOADX == kLoadComb) {
+    fft_pass_body<Real, LOADX, STORE, TW>(A, i, j->tiles * A.nbatch, 0);
   } else {
-    fft_pass_body<Real, LOAD, STORE, TW>(A, i % j->tiles, j->tiles, i / j->tiles);
+    fft_pass_body<Real, LOADX, STORE, TW>(A, i % j->tiles, j->tiles, i / j->tiles);
   }
+}
+
+template <typename Real, int LOADX, int STORE, int TW>
+static hipError_t launch_tile(const PassArgs& A, int tiles, int batch, hipStream_t st) {
+  const dim3 grid = (LOADX == kLoadComb) ? dim3(tiles * batch, 1) : dim3(tiles, batch);
+  hipLaunchKernelGGL((fft_pass_kernel<Real, LOADX, STORE, TW>), grid,
+                     dim3(Tile<Real, LOADX>::nt), 0, st, A);
+  return hipGetLastError();
+}
+
+// the loads that have a quarter tile
+static constexpr bool has_small(int load, int store) {
+  return store != kStoreHead && (load == kLoadPlain || load == kLoadPerm ||
+                                 load == kLoadCombRows || load == kLoadCombRowsG);
 }
 
 template <typename Real, int LOAD, int STORE, int TW>
 static hipError_t launch_pass(const PassArgs& A, int tiles, int batch, hipStream_t st) {
-  const dim3 grid = (LOAD == kLoadComb) ? dim3(tiles * batch, 1) : dim3(tiles, batch);
-  hipLaunchKernelGGL((fft_pass_kernel<Real, LOAD, STORE, TW>), grid, dim3(Tile<Real, LOAD>::nt),
-                     0, st, A);
-  return hipGetLastError();
+  if constexpr (has_small(LOAD, STORE)) {
+    if (A.small_tile)
+      return launch_tile<Real, LOAD | kSmallTile, STORE, TW>(A, tiles, batch, st);
+  }
+  if (A.small_tile) return hipErrorInvalidValue;
+  return launch_tile<Real, LOAD, STORE, TW>(A, tiles, batch, st);
 }
 
 template <typename Real, int LOAD, int TW>
@@ -771,15 +793,38 @@ static hipError_t dispatch_pass(const PassArgs& A, int load, int store, int tw, 
   return dispatch_store<Real, kLoadPlain, kTwNone>(A, store, tiles, batch, st);
 }
 
-static int pass_log2q(const FftTables& T, const FftLaunch& L, int p, int r, int log2Lprev) {
+// Columns per tile (log2) of pass p, and whether it takes quarter tiles: where a full tile's
+// columns would not fill more than a quarter anyway; where they would not fill all of it and a
+// quarter still holds whole lines of 128 bytes per row (complex64 sub-FFTs of up to 128 points,
+// complex128 of up to 64; 2^24 points as transforms of 2^12, complex64 256 -> 101 us,
+// complex128 274 -> 208; of 2^13 and 2^14, complex64 211 -> 111 and 145 -> 111; a complex128 tile
+// that 128-point sub-FFTs fill stays full: 215 against 223 at 2^14); and, with half lines, where
+// the launch would be fewer than 128 full tiles, half the CUs.
+struct PassShape {
+  int log2q, small_tile;
+};
+static PassShape pass_shape(const FftTables& T, const FftLaunch& L, int p, int r, int log2Lprev) {
   const int load = (p == 0) ? L.load : kLoadPlain;
   // a kLoadPerm pass takes as many columns as fit: whole lines of its input per tile
   const int qmax = (load != kLoadPerm && L.qmax > 0 && L.qmax <= FFT_QMAX) ? L.qmax : FFT_QMAX;
   const int cap = tile_cap(T.is_fp32, load);
-  int log2Q = 0;
-  while ((1 << (log2Q + 1)) <= qmax && ((1 << (log2Q + 1)) << r) <= cap) ++log2Q;
-  if (p > 0 && log2Q > log2Lprev) log2Q = log2Lprev;
-  return log2Q;
+  const int limit = p > 0 ? log2Lprev : T.log2n - r;   // columns there are
+  auto cols = [&](int elems) {
+    int q = 0;
+    while ((1 << (q + 1)) <= qmax && ((1 << (q + 1)) << r) <= elems) ++q;
+    return (p > 0 && q > log2Lprev) ? log2Lprev : q;
+  };
+  const int full = cols(cap), quarter = cols(cap / 4);
+  const int store = (p == T.npass - 1) ? L.store : kStoreCplx;
+  if (!has_small(load, store) || (1 << r) > cap / 4) return {full, 0};
+  const int nf = full < limit ? full : limit, nq = quarter < limit ? quarter : limit;
+  const int line = T.is_fp32 ? 4 : 3;
+  const long long tiles = ((long long)L.batch << T.log2n) >> (nf + r);
+  const bool fits = ((1 << nf) << r) <= cap / 4;
+  const bool lines = ((1 << nf) << r) < cap && nq >= (line < nf ? line : nf);
+  const bool idle = tiles < 128 && nq >= (line - 1 < nf ? line - 1 : nf);
+  if (fits || lines || idle) return {quarter, 1};
+  return {full, 0};
 }
 
 // Single-pass transforms of adjacent rows: rows per tile (log2), or -1 where the plain pass runs
@@ -809,7 +854,7 @@ KeyMap fft_keys_map(const FftLaunch& L) {
   const int last = T.npass - 1;
   const int r = T.logs[last];
   m.mid = r;
-  m.lo = pass_log2q(T, L, last, r, T.log2n - r);
+  m.lo = pass_shape(T, L, last, r, T.log2n - r).log2q;
   return m;
 }
 
@@ -847,11 +892,14 @@ static hipError_t each_pass(const FftLaunch& L, F&& fn) {
     A.r = r;
     A.log2Lprev = log2Lprev;
     int load = (p == 0) ? L.load : kLoadPlain;
-    int log2Q = pass_log2q(T, L, p, r, log2Lprev);
+    const PassShape shape = pass_shape(T, L, p, r, log2Lprev);
+    int log2Q = shape.log2q;
+    A.small_tile = shape.small_tile;
     const int rq = rows_log2q(T, L);
     int tiles;
     if (rq >= 0) {
       load = kLoadRows;
+      A.small_tile = 0;
       log2Q = rq;
       tiles = (int)(((long long)L.batch + (1LL << rq) - 1) >> rq);
     } else if (p == 0) {
@@ -914,7 +962,8 @@ hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L) {
     if (load == kLoadWiden || load == kLoadTaps || load == kLoadRows || store == kStoreHead)
       return hipErrorInvalidValue;
     auto it = std::find_if(g.begin(), g.end(), [&](const FftGroup& x) {
-      return x.pass == p && x.load == load && x.store == store && x.tw == tw && x.fp32 == fp32;
+      return x.pass == p && x.load == load && x.store == store && x.tw == tw &&
+             x.small_tile == A.small_tile && x.fp32 == fp32;
     });
     if (it == g.end()) {
       FftGroup n;
@@ -922,6 +971,7 @@ hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L) {
       n.load = load;
       n.store = store;
       n.tw = tw;
+      n.small_tile = A.small_tile;
       n.fp32 = fp32;
       // in the order of the passes
       it = g.insert(std::find_if(g.begin(), g.end(),
@@ -936,18 +986,27 @@ hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L) {
   });
 }
 
-template <typename Real, int LOAD, int STORE, int TW>
-static hipError_t launch_jobs(const JobsDev& d, hipStream_t st) {
-  hipLaunchKernelGGL((fft_jobs_kernel<Real, LOAD, STORE, TW>), dim3(d.blocks),
-                     dim3(Tile<Real, LOAD>::nt), 0, st, d);
+template <typename Real, int LOADX, int STORE, int TW>
+static hipError_t launch_jobs_tile(const JobsDev& d, hipStream_t st) {
+  hipLaunchKernelGGL((fft_jobs_kernel<Real, LOADX, STORE, TW>), dim3(d.blocks),
+                     dim3(Tile<Real, LOADX>::nt), 0, st, d);
   return hipGetLastError();
+}
+
+template <typename Real, int LOAD, int STORE, int TW>
+static hipError_t launch_jobs(const FftGroup& g, hipStream_t st) {
+  if constexpr (has_small(LOAD, STORE)) {
+    if (g.small_tile) return launch_jobs_tile<Real, LOAD | kSmallTile, STORE, TW>(g.t.dev, st);
+  }
+  if (g.small_tile) return hipErrorInvalidValue;
+  return launch_jobs_tile<Real, LOAD, STORE, TW>(g.t.dev, st);
 }
 
 template <typename Real, int LOAD, int TW>
 static hipError_t jobs_store(const FftGroup& g, hipStream_t st) {
-  if (g.store == kStoreCplx) return launch_jobs<Real, LOAD, kStoreCplx, TW>(g.t.dev, st);
-  if (g.store == kStoreKeys) return launch_jobs<Real, LOAD, kStoreKeys, TW>(g.t.dev, st);
-  return launch_jobs<Real, LOAD, kStoreBoth, TW>(g.t.dev, st);
+  if (g.store == kStoreCplx) return launch_jobs<Real, LOAD, kStoreCplx, TW>(g, st);
+  if (g.store == kStoreKeys) return launch_jobs<Real, LOAD, kStoreKeys, TW>(g, st);
+  return launch_jobs<Real, LOAD, kStoreBoth, TW>(g, st);
 }
 
 template <typename Real>

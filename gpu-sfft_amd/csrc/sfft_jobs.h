@@ -75,6 +75,7 @@ struct PassArgs {
   long long keys_bstride;
   int key_batches;
   int log2N, r, log2Lprev, log2Q;
+  int small_tile;   // a tile of a quarter of the elements and threads (pass_shape)
   int inverse;
   const void* twR;
   const void* tw4;      // radix-4 stage twiddle quads (see fft_tables_create)
@@ -101,7 +102,7 @@ struct FftJob {
 };
 // the jobs of one kernel variant, run in the order of their pass
 struct FftGroup {
-  int pass = 0, load = 0, store = 0, tw = 0, fp32 = 0;
+  int pass = 0, load = 0, store = 0, tw = 0, small_tile = 0, fp32 = 0;
   JobTable<FftJob> t;
 };
 // appends the passes of L to their groups (comb gathers, plain, comb rows and column-permuted
