@@ -242,7 +242,8 @@ struct HashArgs {
 hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st);
 hipError_t hash_bitmap_launch(const HashArgs& h, hipStream_t st);
 hipError_t hash_hits_launch(const HashArgs& h, hipStream_t st);
-int hash_blocks(int loops_loc, int K, long long m);   // m = n / B
+// blocks that walk `loops` of the location loops (m = n / B)
+int hash_blocks(int loops, int loops_loc, int K, long long m);
 size_t hash_mask_bytes(int loops_loc, int K, long long m);   // hit masks of the slices
 
 // ---- estimation ---------------------------------------------------------------------------

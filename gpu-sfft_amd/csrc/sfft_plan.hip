@@ -262,7 +262,7 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   const size_t W = prm->W_RLFC, B = prm->B;
   const size_t e = P->fp32 ? 8 : 16, ke = P->fp32 ? 4 : 8;
   P->bm_words = (int)((W + 31) / 32);
-  const int nhb = hash_blocks(Ll, K, (long long)prm->n / prm->B);
+  const int nhb = hash_blocks(Ll, Ll, K, (long long)prm->n / prm->B);
   // carve one workspace
   struct Item {
     void** dst;
