@@ -212,7 +212,7 @@ def run_precision(args, S, prm, prec, seeds_draws, snr, log):
 
 
 # the functions whose source text a kernel's counter figures belong to (sfft_fft.hip)
-KERNEL_SOURCE = {"fold_slab_kernel": ("fold_slab_kernel",),
+KERNEL_SOURCE = {"fold_slab_kernel": ("fold_slab_body", "fold_slab_kernel"),
                  "perm_filter_kernel": ("pf_body", "perm_filter_kernel"),
                  "stream_scatter_kernel": ("stream_scatter_kernel",)}
 

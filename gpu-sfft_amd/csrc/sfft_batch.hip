@@ -2,16 +2,21 @@
 //
 // Each signal keeps its own plan (parameters, workspace).  One batch execution runs every stage
 // of ALL its signals as one launch (sfft_jobs.h: a table of the signals' arguments, and each
-// workgroup's signal; the permute+filter is a persistent launch over its own work table), so
+// workgroup's signal), so
 // small and large signals share the chip and a batch of any size takes about thirty launches.
 // (One launch per signal and stage took 16-25 launches of a few us per signal: 64 complex64
-// signals of 2^18..2^24, 6.3 ms on four streams, now 2.6 ms.)  Two chains run beside each other, as in a single transform: the comb
-// chain (clear, comb FFT, comb cutoff, approved bitmaps) on a second stream, and permute+filter,
-// bucket FFT and bucket cutoff on the batch stream; joined there, the reverse hash and the
-// estimation follow.  The draws of all signals go up in one copy.  With graphs the two chains
-// are captured once as one graph and replayed (buffers are cleared by kernels, so it holds no
-// memset nodes); the tables and the graph are rebuilt when the signal or node pointers, the
-// filters or the tuned shapes change.
+// signals of 2^18..2^24, 6.3 ms on four streams, 2.6 ms as one launch per stage.)
+// Signals whose plan takes the column front end (AUTO, where the slab applies) are folded by one
+// slab launch, which also copies their comb samples; the others are gathered by one persistent
+// permute+filter launch (all 64 gathered: permute+filter 1074 us, comb gather 363 us; slab
+// 763 us and comb first passes 150 us, the whole batch 2.57 -> 2.04 ms).
+// Two chains run beside each other, as in a single transform: the comb chain (comb FFT, comb
+// cutoff, approved bitmaps) on a second stream, and bucket FFT and bucket cutoff (after the
+// permute+filter) on the batch stream; joined there, the reverse hash and the estimation follow.
+// The draws of all signals go up in one copy.  With graphs the two chains are captured once as
+// one graph and replayed (buffers are cleared by kernels, so it holds no memset nodes); the
+// tables and the graph are rebuilt when the signal or node pointers, the filters or the tuned
+// shapes change.
 //
 // Autotuner: times, on the batch itself, only launch shapes that compute the same bits --
 // the permute+filter loops per thread, block size and persistent grid (every shape runs the
@@ -33,10 +38,11 @@ struct sfft_batch {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::vector<sfft_plan*> plans;
   // job tables of every stage, in one device buffer
-  std::vector<PfJob> jobs;
+  std::vector<PfJob> jobs;           // gathering signals
+  std::vector<SlabGroup> slab;                    // signals with the column front end
   int total_items = 0;
   int lpt = 3, nt = 256, grid = 2048;
-  std::vector<FftGroup> comb, bucket;
+  std::vector<FftGroup> comb, comb_slab, bucket;   // combs gathered, combs the slab fold copied
   SelGroup sel_comb, sel_bucket;
   JobTable<HashJob> clear, bitmap, hits;
   std::vector<EstGroup> est;
@@ -94,7 +100,7 @@ extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
   for (int i = 0; i < count; ++i) {
     const sfft_status s = sfft_params_validate(&params[i]);
     if (s != SFFT_OK) return s;
-    // the batch folds every signal with the gathering permute+filter (one persistent launch)
+    // AUTO: the column slab fold where it applies, else gathers
     if (params[i].front_end != SFFT_FRONT_AUTO && params[i].front_end != SFFT_FRONT_GATHER)
       return SFFT_ERR_INVALID;
   }
@@ -111,9 +117,7 @@ extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
   }
   for (int i = 0; i < count; ++i) {
     sfft_plan* p = nullptr;
-    sfft_params pi = params[i];
-    pi.front_end = SFFT_FRONT_GATHER;   // AUTO: the batch's own front end
-    const sfft_status s = sfft_plan_create(&pi, prec, b->st, &p);
+    const sfft_status s = sfft_plan_create(&params[i], prec, b->st, &p);
     if (s != SFFT_OK) {
       sfft_batch_destroy(b);
       return s;
@@ -170,8 +174,10 @@ extern "C" sfft_status sfft_batch_set_filter(sfft_batch* b, int i, const void* d
 static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes) {
   drop_graph(b);
   b->tab_x.clear();
-  b->jobs.assign(b->count, PfJob());
+  b->jobs.clear();
+  b->slab.clear();
   b->comb.clear();
+  b->comb_slab.clear();
   b->bucket.clear();
   b->est.clear();
   b->sel_comb = SelGroup();
@@ -181,21 +187,35 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   for (int i = 0; i < b->count; ++i) {
     const sfft_plan* P = b->plans[i];
     const sfft_params& p = P->p;
-    PfJob& J = b->jobs[i];
-    J.x = d_x[i];
-    J.f = P->d_ft;
-    J.bins = P->bins_t;
-    J.ai = P->d_ai;
-    J.mask = (uint32_t)p.n - 1u;
-    J.B = p.B;
-    J.w = p.w;
-    J.loops = p.loops;
-    J.tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
-    J.item0 = item;
-    item += pf_batch_items(J.B, J.loops, b->lpt, b->nt, &J.nbx);
+    const int tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
     const HashArgs h = hash_args(P, b->d_counts + i);
+    if (P->columns) {
+      FoldClear clr;   // the slab fold clears for the transform, as a single one's does
+      clr.bm = h.bitmap;
+      clr.nbm = (size_t)h.loops_loc * (size_t)h.bm_words;
+      clr.maxf = (uint32_t*)h.maxfirst;
+      clr.nmax = h.loops_loc;
+      HIPCK(slab_jobs_add(b->slab, b->fp32, d_x[i], P->frows, P->bins_t, P->d_a, P->d_ai, p.n, p.B,
+                          p.w, p.loops, tiled, P->comb_y, P->d_offs, p.RLFC_loops, p.W_RLFC,
+                          clr));
+    } else {
+      PfJob J;
+      J.x = d_x[i];
+      J.f = P->d_ft;
+      J.bins = P->bins_t;
+      J.ai = P->d_ai;
+      J.mask = (uint32_t)p.n - 1u;
+      J.B = p.B;
+      J.w = p.w;
+      J.loops = p.loops;
+      J.tiled = tiled;
+      J.item0 = item;
+      item += pf_batch_items(J.B, J.loops, b->lpt, b->nt, &J.nbx);
+      b->jobs.push_back(J);
+      hash_jobs_clear(b->clear, h);
+    }
     const FftLaunch comb = comb_fft(P, d_x[i]);
-    HIPCK(fft_jobs_add(b->comb, comb));
+    HIPCK(fft_jobs_add(P->columns ? b->comb_slab : b->comb, comb));
     HIPCK(fft_jobs_add(b->bucket, bucket_fft(P)));
     const KeyMap km = fft_keys_map(comb);
     const SelMark mk = comb_mark(h);
@@ -205,7 +225,6 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
                           marks ? &mk : nullptr));
     HIPCK(select_jobs_add(b->sel_bucket, b->fp32, P->bkeys, p.B, p.B, p.B_thresh, p.loops_loc,
                           P->J, 1, P->selB, P->jsel, nullptr, P->bucket_digits, nullptr));
-    hash_jobs_clear(b->clear, h);
     if (!marks) hash_jobs_bitmap(b->bitmap, h);
     hash_jobs_hits(b->hits, h);
     EstJob e = {};
@@ -225,9 +244,12 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
     estimate_jobs_add(b->est, b->fp32, e);
   }
   b->total_items = item;
+  slab_jobs_share(b->slab);
   JobPack pack;
   const size_t at_jobs = pack.put(b->jobs.data(), sizeof(PfJob) * b->jobs.size());
+  for (auto& g : b->slab) g.t.pack(pack);
   for (auto& g : b->comb) g.t.pack(pack);
+  for (auto& g : b->comb_slab) g.t.pack(pack);
   for (auto& g : b->bucket) g.t.pack(pack);
   for (auto& g : b->est) g.t.pack(pack);
   b->sel_comb.pack(pack);
@@ -247,7 +269,9 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
                        b->st));
   HIPCK(hipStreamSynchronize(b->st));   // the packed bytes go out of scope
   b->d_jobs = (const PfJob*)(b->d_tab + at_jobs);
+  for (auto& g : b->slab) g.t.bind(b->d_tab);
   for (auto& g : b->comb) g.t.bind(b->d_tab);
+  for (auto& g : b->comb_slab) g.t.bind(b->d_tab);
   for (auto& g : b->bucket) g.t.bind(b->d_tab);
   for (auto& g : b->est) g.t.bind(b->d_tab);
   b->sel_comb.bind(b->d_tab);
@@ -260,17 +284,21 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   return SFFT_OK;
 }
 
-// one batch execution from the batch stream (the draws are up, the tables built)
+// one batch execution from the batch stream (the draws are up, the tables built).  The gathering
+// signals' comb chain starts beside their permute+filter, the others' after the slab fold, which
+// copies their comb samples (and clears for them).
 static sfft_status enqueue(sfft_batch* b) {
+  HIPCK(hash_clear_jobs(b->clear, b->st));
+  HIPCK(slab_jobs_launch(b->slab, b->st));
   HIPCK(hipEventRecord(b->ev_fork, b->st));
   HIPCK(hipStreamWaitEvent(b->st2, b->ev_fork, 0));
-  HIPCK(perm_filter_batch_launch(b->fp32, b->d_jobs, b->count, b->total_items, b->lpt, b->nt,
-                                 b->grid, b->st));
-  HIPCK(hash_clear_jobs(b->clear, b->st2));
   HIPCK(fft_jobs_launch(b->comb, b->st2));
+  HIPCK(fft_jobs_launch(b->comb_slab, b->st2));
   HIPCK(select_jobs_launch(b->sel_comb, b->st2));
   HIPCK(hash_bitmap_jobs(b->bitmap, b->st2));
   HIPCK(hipEventRecord(b->ev_join, b->st2));
+  HIPCK(perm_filter_batch_launch(b->fp32, b->d_jobs, (int)b->jobs.size(), b->total_items, b->lpt,
+                                 b->nt, b->grid, b->st));
   HIPCK(fft_jobs_launch(b->bucket, b->st));
   HIPCK(select_jobs_launch(b->sel_bucket, b->st));
   HIPCK(hipStreamWaitEvent(b->st, b->ev_join, 0));
@@ -420,6 +448,7 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
     for (int nt : nts) {
       b->lpt = lpt;
       b->nt = nt;
+      if (b->jobs.empty()) continue;   // every signal takes the column front end
       if ((v = build_tables(b, d_x, none.data())) != SFFT_OK) return v;
       for (int grid : grids) {
         float ms = 0;
@@ -451,6 +480,7 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
       float ms = 0;
       v = time_ms(b, reps, [&]() -> sfft_status {
         HIPCK(fft_jobs_launch(which == 0 ? b->bucket : b->comb, b->st));
+        if (which) HIPCK(fft_jobs_launch(b->comb_slab, b->st));
         return SFFT_OK;
       }, &ms);
       if (v != SFFT_OK) return v;

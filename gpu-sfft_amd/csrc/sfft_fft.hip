@@ -1012,6 +1012,9 @@ static hipError_t jobs_store(const FftGroup& g, hipStream_t st) {
 template <typename Real>
 static hipError_t jobs_pass(const FftGroup& g, hipStream_t st) {
   if (g.load == kLoadComb) return jobs_store<Real, kLoadComb, kTwNone>(g, st);
+  if (g.load == kLoadCombRows) return jobs_store<Real, kLoadCombRows, kTwNone>(g, st);
+  if (g.load == kLoadCombRowsG) return jobs_store<Real, kLoadCombRowsG, kTwNone>(g, st);
+  if (g.load == kLoadPerm) return jobs_store<Real, kLoadPerm, kTwNone>(g, st);
   if (g.load != kLoadPlain) return hipErrorInvalidValue;
   if (g.tw == kTwSplit) return jobs_store<Real, kLoadPlain, kTwSplit>(g, st);
   if (g.tw == kTwDirect) return jobs_store<Real, kLoadPlain, kTwDirect>(g, st);
@@ -1384,16 +1387,20 @@ struct SlabFetch {            // filter-row loads per thread per slab (all in fl
   static constexpr int fb = sizeof(Real) == 8 ? 8 : 16;
 };
 
+// (workgroup bx of the G that share the signal's slabs)
 template <typename Real, int PMAX, int NT>
-__global__ __launch_bounds__(NT, 4) void fold_slab_kernel(
-    const typename CT<Real>::T2* __restrict__ x, const typename CT<Real>::T2* __restrict__ fT,
-    typename CT<Real>::T2* __restrict__ bins, const int* __restrict__ a_dev,
-    const int* __restrict__ ai_dev, uint32_t mask, int log2B, int log2m, int w, int loops,
-    int tiled, int T, int P, int log2sc, typename CT<Real>::T2* __restrict__ yc,
-    const int* __restrict__ offs, int Rl, int log2sigma, FoldClear clr) {
+__device__ __forceinline__ void fold_slab_body(const SlabArgs& A, uint32_t bx, uint32_t G) {
   using T2 = typename CT<Real>::T2;
   using V2 = typename NV<Real>::type;
   using AC = typename AccOf<Real>::A;
+  const T2* __restrict__ x = (const T2*)A.x;
+  const T2* __restrict__ fT = (const T2*)A.fT;
+  T2* __restrict__ bins = (T2*)A.bins;
+  T2* __restrict__ yc = (T2*)A.yc;
+  const uint32_t mask = A.mask;
+  const int log2B = A.log2B, log2m = A.log2m, w = A.w, loops = A.loops, tiled = A.tiled, T = A.T,
+            P = A.P, log2sc = A.log2sc, Rl = A.Rl, log2sigma = A.log2sigma;
+  const FoldClear& clr = A.clr;
   constexpr int EPU = 16 / (int)sizeof(T2);             // elements per 16-byte unit
   constexpr int FB = SlabFetch<Real>::fb;
   extern __shared__ u32x4 dyn16[];
@@ -1424,18 +1431,17 @@ __global__ __launch_bounds__(NT, 4) void fold_slab_kernel(
   const V2* __restrict__ fTv = (const V2*)fT;
 
   // The chunks of the workgroup in order: chunk q is chunk (q mod nchunks) of its slab
-  // q / nchunks (slab blockIdx.x + (q / nchunks) * G).  The next chunk is in flight in
+  // q / nchunks (slab bx + (q / nchunks) * G).  The next chunk is in flight in
   // registers (xa) while one is used from LDS.  q past the last chunk is clamped to it.
   const int log2nch = log2m - log2rows;
-  const uint32_t G = gridDim.x;
-  const int nsl = (int)((nslabs - blockIdx.x + G - 1) / G);   // slabs of this workgroup
+  const int nsl = (int)((nslabs - bx + G - 1) / G);   // slabs of this workgroup
   const int Q = nsl << log2nch;
   u32x4 xa[SL_U];
   // the loads of a chunk in one basic block (clamped addresses): in flight together.  Unit
   // indices in 32 bits (n * e / 16 < 2^32).
   auto load = [&](u32x4* buf, int q) __attribute__((always_inline)) {
     const int qq = min(q, Q - 1);
-    const uint32_t c0 = (blockIdx.x + (uint32_t)(qq >> log2nch) * G) << log2sc;
+    const uint32_t c0 = (bx + (uint32_t)(qq >> log2nch) * G) << log2sc;
     const int ch = qq & (nchunks - 1);
     const uint32_t col16 = (uint32_t)(((size_t)c0 * sizeof(T2)) / 16);
 #pragma unroll
@@ -1502,15 +1508,15 @@ __global__ __launch_bounds__(NT, 4) void fold_slab_kernel(
   // (a, ai) of every loop and the comb offsets into LDS: their loads go out before the first
   // chunk's, so that waiting for them does not wait for the chunk
   // the caller's clear, spread over the grid (one 4-byte store per thread at n = 2^27)
-  for (size_t i = (size_t)blockIdx.x * NT + tid; i < clr.nbm; i += (size_t)gridDim.x * NT)
+  for (size_t i = (size_t)bx * NT + tid; i < clr.nbm; i += (size_t)G * NT)
     clr.bm[i] = 0u;
-  if (blockIdx.x == 0 && tid < clr.nmax) clr.maxf[tid] = 0xFFFFFFFFu;
+  if (bx == 0 && tid < clr.nmax) clr.maxf[tid] = 0xFFFFFFFFu;
   int av = 0, aiv = 0, ov = 0;
   if (tid < loops) {
-    av = a_dev[tid];
-    aiv = ai_dev[tid];
+    av = A.a_dev[tid];
+    aiv = A.ai_dev[tid];
   }
-  if (tid < Rl) ov = offs[tid];
+  if (tid < Rl) ov = A.offs[tid];
   load(xa, 0);
   if (tid < loops) {
     atab[tid] = av;
@@ -1518,9 +1524,9 @@ __global__ __launch_bounds__(NT, 4) void fold_slab_kernel(
   }
   if (tid < Rl) atab[64 + tid] = ov;
   __syncthreads();
-  fetch_rows(blockIdx.x << log2sc);
+  fetch_rows(bx << log2sc);
   put_rows();
-  pair_state(blockIdx.x << log2sc);
+  pair_state(bx << log2sc);
   store(xa);
   __syncthreads();
 
@@ -1530,8 +1536,8 @@ __global__ __launch_bounds__(NT, 4) void fold_slab_kernel(
   auto body = [&](int q) __attribute__((always_inline)) {
     const int ch = q & (nchunks - 1);
     const int sl = q >> log2nch;
-    const uint32_t c0 = (blockIdx.x + (uint32_t)sl * G) << log2sc;
-    const uint32_t cnext = (blockIdx.x + (uint32_t)min(sl + 1, nsl - 1) * G) << log2sc;
+    const uint32_t c0 = (bx + (uint32_t)sl * G) << log2sc;
+    const uint32_t cnext = (bx + (uint32_t)min(sl + 1, nsl - 1) * G) << log2sc;
     const uint32_t r0 = (uint32_t)(ch * rows);
     // comb columns of the slab: this chunk's rows
     for (int e = tid; e < ncopy; e += NT) {
@@ -1622,6 +1628,20 @@ __global__ __launch_bounds__(NT, 4) void fold_slab_kernel(
   for (int q = 0; q < Q; ++q) body(q);
 }
 
+template <typename Real, int PMAX, int NT>
+__global__ __launch_bounds__(NT, 4) void fold_slab_kernel(SlabArgs A) {
+  fold_slab_body<Real, PMAX, NT>(A, blockIdx.x, gridDim.x);
+}
+
+// the slabs of many signals: a signal's workgroups stream its slabs, as in a launch of their own
+template <typename Real, int PMAX, int NT>
+__global__ __launch_bounds__(NT, 4) void fold_slab_jobs_kernel(JobsDev t) {
+  const SlabJob* j = job_here<SlabJob>(t);
+  if (!j) return;
+  const SlabArgs A = j->a;
+  fold_slab_body<Real, PMAX, NT>(A, blockIdx.x - (uint32_t)j->block0, (uint32_t)j->groups);
+}
+
 int fold_rows_pitch(int B, int w) { return w / B + 1; }
 
 static size_t slab_lds_bytes(int is_fp32, int loops, int lsc, int P) {
@@ -1644,66 +1664,57 @@ static int slab_log2sc(int is_fp32, int log2B, int log2m, int loops, int P) {
   return lsc;
 }
 
-template <typename Real, int PMAX, int NT>
-static hipError_t slab_launch(const void* x, const void* fT, void* bins, const int* a_dev,
-                              const int* ai_dev, uint32_t mask, int log2B, int log2m, int w,
-                              int loops, int tiled, int T, int P, int lsc, void* yc,
-                              const int* offs, int Rl, int log2sigma, const FoldClear& clr,
-                              hipStream_t st) {
-  using T2 = typename CT<Real>::T2;
-  const unsigned nslabs = 1u << (log2B - lsc);
-  const size_t lds = slab_lds_bytes(sizeof(Real) == 4, loops, lsc, P);
-  // one workgroup per resident slot (each streams nslabs / grid slabs); any grid is correct.
-  // The resident count is asked of the runtime once per (device, LDS size) and kept.
+// resident workgroups of a slab kernel on the current device: asked of the runtime once per
+// (kernel, device, LDS size) and kept; 0 where it cannot be asked
+static int slab_resident(const void* kernel, int nt, size_t lds) {
   static std::mutex mu;
-  static std::map<std::pair<int, size_t>, int> resident;
+  static std::map<std::pair<const void*, std::pair<int, size_t>>, int> resident;
   int dev = 0;
-  unsigned blocks = nslabs;
-  if (hipGetDevice(&dev) == hipSuccess) {
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = resident.find({dev, lds});
-    if (it == resident.end()) {
-      int cus = 0, per_cu = 0;
-      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &per_cu, reinterpret_cast<const void*>(&fold_slab_kernel<Real, PMAX, NT>), NT,
-              lds) != hipSuccess)
-        cus = per_cu = 0;
-      it = resident.emplace(std::make_pair(dev, lds), cus * per_cu).first;
-    }
-    if (it->second > 0) blocks = std::min(nslabs, (unsigned)it->second);
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  std::lock_guard<std::mutex> lock(mu);
+  const std::pair<const void*, std::pair<int, size_t>> key(kernel, {dev, lds});
+  auto it = resident.find(key);
+  if (it == resident.end()) {
+    int cus = 0, per_cu = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, nt, lds) != hipSuccess)
+      cus = per_cu = 0;
+    it = resident.emplace(key, cus * per_cu).first;
   }
-  hipLaunchKernelGGL((fold_slab_kernel<Real, PMAX, NT>), dim3(blocks), dim3(NT), lds, st,
-                     (const T2*)x, (const T2*)fT, (T2*)bins, a_dev, ai_dev, mask, log2B, log2m,
-                     w, loops, tiled, T, P, lsc, (T2*)yc, offs, Rl, log2sigma, clr);
-  return hipGetLastError();
-}
-
-template <typename Real, int NT>
-static hipError_t slab_dispatch_nt(int P, const void* x, const void* fT, void* bins,
-                                   const int* a_dev, const int* ai_dev, uint32_t mask, int log2B,
-                                   int log2m, int w, int loops, int tiled, int T, int lsc,
-                                   void* yc, const int* offs, int Rl, int log2sigma,
-                                   const FoldClear& clr, hipStream_t st) {
-  if (P <= 16)
-    return slab_launch<Real, 16, NT>(x, fT, bins, a_dev, ai_dev, mask, log2B, log2m, w, loops,
-                                     tiled, T, P, lsc, yc, offs, Rl, log2sigma, clr, st);
-  if (P <= 24)
-    return slab_launch<Real, 24, NT>(x, fT, bins, a_dev, ai_dev, mask, log2B, log2m, w, loops,
-                                     tiled, T, P, lsc, yc, offs, Rl, log2sigma, clr, st);
-  return slab_launch<Real, 32, NT>(x, fT, bins, a_dev, ai_dev, mask, log2B, log2m, w, loops,
-                                   tiled, T, P, lsc, yc, offs, Rl, log2sigma, clr, st);
+  return it->second;
 }
 
 // 512 threads per workgroup: two chunks of loads in flight per workgroup at 4 loads per thread
+constexpr int SL_NT = 512;
+
+// taps per bucket of the kernel variant that takes P
+static int slab_pmax(int P) { return P <= 16 ? 16 : P <= 24 ? 24 : 32; }
+
+// f(kernel of one signal, kernel of many) for the taps per bucket
+template <typename Real, typename F>
+static hipError_t with_pmax(int pmax, F&& f) {
+  if (pmax == 16)
+    return f(fold_slab_kernel<Real, 16, SL_NT>, fold_slab_jobs_kernel<Real, 16, SL_NT>);
+  if (pmax == 24)
+    return f(fold_slab_kernel<Real, 24, SL_NT>, fold_slab_jobs_kernel<Real, 24, SL_NT>);
+  return f(fold_slab_kernel<Real, 32, SL_NT>, fold_slab_jobs_kernel<Real, 32, SL_NT>);
+}
+
+static size_t slab_lds(int is_fp32, const SlabArgs& A) {
+  return slab_lds_bytes(is_fp32, A.loops, A.log2sc, A.P);
+}
+
+// one workgroup per resident slot (each streams nslabs / grid slabs); any grid is correct
 template <typename Real>
-static hipError_t slab_dispatch(int P, const void* x, const void* fT, void* bins,
-                                const int* a_dev, const int* ai_dev, uint32_t mask, int log2B,
-                                int log2m, int w, int loops, int tiled, int T, int lsc, void* yc,
-                                const int* offs, int Rl, int log2sigma, const FoldClear& clr,
-                                hipStream_t st) {
-  return slab_dispatch_nt<Real, 512>(P, x, fT, bins, a_dev, ai_dev, mask, log2B, log2m, w,
-                                     loops, tiled, T, lsc, yc, offs, Rl, log2sigma, clr, st);
+static hipError_t slab_launch(const SlabArgs& A, hipStream_t st) {
+  const unsigned nslabs = 1u << (A.log2B - A.log2sc);
+  const size_t lds = slab_lds(sizeof(Real) == 4, A);
+  return with_pmax<Real>(slab_pmax(A.P), [&](auto one, auto) {
+    const int res = slab_resident(reinterpret_cast<const void*>(one), SL_NT, lds);
+    const unsigned blocks = res > 0 ? std::min(nslabs, (unsigned)res) : nslabs;
+    hipLaunchKernelGGL(one, dim3(blocks), dim3(SL_NT), lds, st, A);
+    return hipGetLastError();
+  });
 }
 
 int fold_slab_applies(int is_fp32, int n, int B, int w, int loops) {
@@ -1727,28 +1738,131 @@ hipError_t filter_rows_launch(int is_fp32, const void* f, void* fT, int B, int w
   return hipGetLastError();
 }
 
+// the slab fold's arguments; false where the slab does not apply
+static bool slab_args(SlabArgs& A, int is_fp32, const void* x, const void* fT, void* bins,
+                      const int* a_dev, const int* ai_dev, int n, int B, int w, int loops,
+                      int tiled, void* yc, const int* offs, int Rl, int W, const FoldClear& clr) {
+  int log2B = 0, log2n = 0, log2W = 0;
+  while ((1 << log2B) < B) ++log2B;
+  while ((1LL << log2n) < n) ++log2n;
+  while ((1 << log2W) < W) ++log2W;
+  A = SlabArgs();
+  A.x = x;
+  A.fT = fT;
+  A.bins = bins;
+  A.a_dev = a_dev;
+  A.ai_dev = ai_dev;
+  A.mask = (uint32_t)n - 1u;
+  A.log2B = log2B;
+  A.log2m = log2n - log2B;
+  A.w = w;
+  A.loops = loops;
+  A.tiled = tiled;
+  A.T = w / B;
+  A.P = fold_rows_pitch(B, w);
+  A.yc = yc;
+  A.offs = offs;
+  A.log2sigma = log2n - log2W;
+  A.Rl = (!yc || A.log2sigma > log2B) ? 0 : Rl;   // no comb columns to copy (sigma must divide B)
+  A.clr = clr;
+  const int lsc = A.Rl <= 64 ? slab_log2sc(is_fp32, log2B, A.log2m, loops, A.P) : -1;
+  A.log2sc = lsc;
+  return lsc >= 0;
+}
+
+hipError_t slab_jobs_add(std::vector<SlabGroup>& groups, int is_fp32, const void* x,
+                         const void* fT, void* bins, const int* a_dev, const int* ai_dev, int n, int B, int w, int loops,
+                         int tiled, void* yc, const int* offs, int Rl, int W,
+                         const FoldClear& clr) {
+  SlabArgs A;
+  if (!slab_args(A, is_fp32, x, fT, bins, a_dev, ai_dev, n, B, w, loops, tiled, yc, offs, Rl, W,
+                 clr))
+    return hipErrorInvalidValue;
+  // (signals whose slabs are over half a CU's LDS apart: they would leave every signal of the
+  // launch one workgroup per CU)
+  const size_t lds = slab_lds(is_fp32, A);
+  const int wide = lds > 80 * 1024;
+  auto it = std::find_if(groups.begin(), groups.end(),
+                         [&](const SlabGroup& g) { return g.wide == wide; });
+  if (it == groups.end()) {
+    groups.emplace_back();
+    it = groups.end() - 1;
+    it->wide = wide;
+    it->fp32 = is_fp32;
+  }
+  it->pmax = std::max(it->pmax, slab_pmax(A.P));
+  it->lds = std::max(it->lds, lds);
+  it->args.push_back(A);
+  return hipSuccess;
+}
+
+// Workgroups of a quarter of a resident slot's even share each (a slab at least), the longest
+// streams first: the card deals the rest to the slots that come free, so that slabs of 16 KB
+// (2^18 points) and of 4 MB (2^24) leave no slot with a long tail.  (As many workgroups as slots,
+// shared out by bytes: signals of 32 slabs on 28 workgroups stream two slabs on some, 64 complex64
+// signals of 2^18..2^24 1571 us, now 763.)
+static void share_group(SlabGroup& g) {
+  const int n = (int)g.args.size();
+  if (!n) return;
+  int res = 0;
+  auto ask = [&](auto, auto many) {
+    res = slab_resident(reinterpret_cast<const void*>(many), SL_NT, g.lds);
+    return hipSuccess;
+  };
+  (void)(g.fp32 ? with_pmax<float>(g.pmax, ask) : with_pmax<double>(g.pmax, ask));
+  auto slabs = [&](int i) { return 1LL << (g.args[i].log2B - g.args[i].log2sc); };
+  auto rows = [&](int i) { return 1LL << g.args[i].log2m; };   // of 256 bytes per slab
+  long long total = 0;
+  for (int i = 0; i < n; ++i) total += slabs(i) * rows(i);
+  const long long part = total / (4 * (res > 0 ? res : 512)) + 1;
+  std::vector<long long> per(n);   // slabs per workgroup
+  std::vector<int> order(n);
+  for (int i = 0; i < n; ++i) {
+    per[i] = std::max(1LL, part / rows(i));
+    order[i] = i;
+  }
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int i, int j) { return per[i] * rows(i) > per[j] * rows(j); });
+  for (int i : order) {
+    SlabJob j;
+    j.a = g.args[i];
+    j.groups = (int)((slabs(i) + per[i] - 1) / per[i]);
+    j.block0 = 0;
+    g.t.add(j, j.groups);
+  }
+}
+
+void slab_jobs_share(std::vector<SlabGroup>& groups) {
+  for (SlabGroup& g : groups) share_group(g);
+}
+
+hipError_t slab_jobs_launch(const std::vector<SlabGroup>& groups, hipStream_t st) {
+  for (const SlabGroup& g : groups) {
+    auto go = [&](auto, auto many) {
+      hipLaunchKernelGGL(many, dim3(g.t.dev.blocks), dim3(SL_NT), g.lds, st, g.t.dev);
+      return hipGetLastError();
+    };
+    const hipError_t e = g.fp32 ? with_pmax<float>(g.pmax, go) : with_pmax<double>(g.pmax, go);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t fold_columns_launch(int is_fp32, const void* x, const void* fT, void* bins,
                                const int* a_dev, const int* ai_dev, int n, int B, int w,
                                int loops, int tiled, int by_column, int remap, void* yc,
                                const int* offs, int Rl, int W, const FoldClear& clr,
                                hipStream_t st) {
-  int log2B = 0, log2n = 0, log2W = 0;
-  while ((1 << log2B) < B) ++log2B;
-  while ((1LL << log2n) < n) ++log2n;
-  while ((1 << log2W) < W) ++log2W;
-  const int log2m = log2n - log2B, log2sigma = log2n - log2W;
-  if (!yc || log2sigma > log2B) Rl = 0;   // no comb columns to copy (sigma must divide B)
-  const int T = w / B, P = fold_rows_pitch(B, w);
-  const uint32_t mask = (uint32_t)n - 1u;
+  SlabArgs A;
+  const bool slab = slab_args(A, is_fp32, x, fT, bins, a_dev, ai_dev, n, B, w, loops, tiled, yc,
+                              offs, Rl, W, clr);
   if (by_column) {
-    const int lsc = Rl <= 64 ? slab_log2sc(is_fp32, log2B, log2m, loops, P) : -1;
-    if (lsc < 0) return hipErrorInvalidValue;
-    return is_fp32 ? slab_dispatch<float>(P, x, fT, bins, a_dev, ai_dev, mask, log2B, log2m, w,
-                                          loops, tiled, T, lsc, yc, offs, Rl, log2sigma, clr, st)
-                   : slab_dispatch<double>(P, x, fT, bins, a_dev, ai_dev, mask, log2B, log2m, w,
-                                           loops, tiled, T, lsc, yc, offs, Rl, log2sigma, clr,
-                                           st);
+    if (!slab) return hipErrorInvalidValue;
+    return is_fp32 ? slab_launch<float>(A, st) : slab_launch<double>(A, st);
   }
+  const int log2B = A.log2B, log2m = A.log2m, log2sigma = A.log2sigma, T = A.T, P = A.P;
+  const uint32_t mask = A.mask;
+  Rl = A.Rl;
   if (clr.nbm || clr.nmax) return hipErrorInvalidValue;   // only the slab fold clears
   // columns per block: one 128-byte line of x (8 complex128 / 16 complex64), fewer if B is
   // smaller

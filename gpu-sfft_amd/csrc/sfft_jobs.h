@@ -110,6 +110,41 @@ struct FftGroup {
 hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L);
 hipError_t fft_jobs_launch(std::vector<FftGroup>& g, hipStream_t st);
 
+// ---- slab fold -----------------------------------------------------------------------------
+struct SlabArgs {
+  const void* x;
+  const void* fT;       // bucket-major filter rows
+  void* bins;
+  const int* a_dev;
+  const int* ai_dev;
+  uint32_t mask;
+  int log2B, log2m, w, loops, tiled, T, P, log2sc;
+  void* yc;             // comb samples
+  const int* offs;
+  int Rl, log2sigma;
+  FoldClear clr;
+};
+struct SlabJob {
+  SlabArgs a;
+  int groups, block0;   // workgroups that share the signal's slabs
+};
+// the signals of a batch whose slabs fit two workgroups per CU, or the others (one launch each):
+// the kernel variant of the most taps per bucket, with the LDS of the largest
+struct SlabGroup {
+  int pmax = 0, fp32 = 0, wide = 0;
+  size_t lds = 0;
+  std::vector<SlabArgs> args;
+  JobTable<SlabJob> t;
+};
+// the arguments of fold_columns_launch with by_column = 1
+hipError_t slab_jobs_add(std::vector<SlabGroup>& groups, int is_fp32, const void* x, const void* fT, void* bins,
+                         const int* a_dev, const int* ai_dev, int n, int B, int w, int loops,
+                         int tiled, void* yc, const int* offs, int Rl, int W,
+                         const FoldClear& clr);
+// shares the card's resident workgroups out among the signals (after the last add)
+void slab_jobs_share(std::vector<SlabGroup>& groups);
+hipError_t slab_jobs_launch(const std::vector<SlabGroup>& groups, hipStream_t st);
+
 // ---- top-K select --------------------------------------------------------------------------
 struct SelJob {
   const void* keys;

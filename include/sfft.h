@@ -275,8 +275,8 @@ sfft_status sfft_value_adjoint(sfft_plan *plan, const complex_t *d_grad, const s
 /* ---- batches of uneven signals -----------------------------------------------------------
  * No counterpart in the reference (which transforms one signal per outer_loop call): count
  * signals, each with its own parameters (n, k, B, ... may all differ), transformed together.
- * Every stage of all signals runs as one launch (the permute+filter is the gathering front end:
- * params[i].front_end must be SFFT_FRONT_AUTO or SFFT_FRONT_GATHER); with
+ * Every stage of all signals runs as one launch (params[i].front_end must be SFFT_FRONT_AUTO,
+ * which takes the columns where a single plan does, or SFFT_FRONT_GATHER); with
  * sfft_batch_set_graph(b, 1) the launch sequence is captured into a hipGraph once and replayed
  * (re-captured when the signal or node pointers, filters or shapes change).  Each signal's
  * results are bit-identical to sfft_execute of the same signal with the same plan parameters

@@ -26,23 +26,35 @@ def S():
     return sfft_amd
 
 
+# every signal gathered; every signal the plan's own choice (columns where the slab applies); an
+# oversized window beside them, which the slab does not take
+@pytest.mark.parametrize("front_end", ["gather", "auto"])
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
-def test_batch_mixed_variants_and_node_memory(S, precision):
+def test_batch_mixed_variants_and_node_memory(S, precision, front_end):
     import torch
     cdt = np.complex64 if precision == "fp32" else np.complex128
     prms = [params(c) for c in CONFIGS]
+    prms.append(dict(prms[0], B=64, w=64 * 40 + 7, B_thresh=20))   # 41 taps per bucket
     xs, fts, wins, dr, want = [], [], [], [], []
     for i, p in enumerate(prms):
         x, _, _ = sparse_signal(p["n"], p["k"], 50 + i, snr_db=30.0)
-        ft, ff = oracle_filter(p)
+        if i < len(CONFIGS):
+            ft, ff = oracle_filter(p)
+            win = O.filter_window_slice(ff, p["n"], p["B"])
+        else:
+            rng = np.random.default_rng(8)
+            ft = rng.standard_normal(p["w"]) + 1j * rng.standard_normal(p["w"])
+            win = 1.0 + rng.random(p["n"] // p["B"]) + 0j
         xs.append(torch.from_numpy(x.astype(cdt)).cuda())
         fts.append(torch.from_numpy(ft.astype(cdt)).cuda())
-        wins.append(O.filter_window_slice(ff, p["n"], p["B"]))
+        wins.append(win)
         dr.append(draws(p["n"], p["loops"], p["RLFC_loops"], p["W_RLFC"], 70 + i))
         plan = S.Plan(p, precision)
         plan.set_filter(fts[i], wins[i])
         want.append(plan.execute(xs[i], *dr[i]))
-    b = S.Batch(prms, precision)
+    b = S.Batch(prms, precision, front_end=front_end)
+    fronts = {S.lib.sfft_plan_front_end(S.lib.sfft_batch_plan(b._h, i)) for i in range(len(prms))}
+    assert fronts == ({1} if front_end == "gather" else {1, 3})
     for i in range(len(prms)):
         b.set_filter(i, fts[i], wins[i])
     cap = 524288
