@@ -192,7 +192,7 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
     if (P->columns) {
       FoldClear clr;   // the slab fold clears for the transform, as a single one's does
       clr.bm = h.bitmap;
-      clr.nbm = (size_t)h.loops_loc * (size_t)h.bm_words;
+      clr.nbm = h.clear_words;
       clr.maxf = (uint32_t*)h.maxfirst;
       clr.nmax = h.loops_loc;
       HIPCK(slab_jobs_add(b->slab, b->fp32, d_x[i], P->frows, P->bins_t, P->d_a, P->d_ai, p.n, p.B,
@@ -222,9 +222,10 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
     const bool marks = select_in_block(p.W_RLFC);
     HIPCK(select_jobs_add(b->sel_comb, b->fp32, P->comb_keys, p.W_RLFC, p.W_RLFC, p.B_thresh,
                           p.RLFC_loops, P->J2, 0, P->selW, nullptr, &km, P->comb_digits,
-                          marks ? &mk : nullptr));
+                          marks ? &mk : nullptr, P->hist_W));
     HIPCK(select_jobs_add(b->sel_bucket, b->fp32, P->bkeys, p.B, p.B, p.B_thresh, p.loops_loc,
-                          P->J, 1, P->selB, P->jsel, nullptr, P->bucket_digits, nullptr));
+                          P->J, 1, P->selB, P->jsel, nullptr, P->bucket_digits, nullptr,
+                          P->hist_B));
     if (!marks) hash_jobs_bitmap(b->bitmap, h);
     hash_jobs_hits(b->hits, h);
     EstJob e = {};

@@ -653,6 +653,7 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
   T2* __restrict__ out = (T2*)A.out + b * A.out_bstride;
   KT* __restrict__ keys = (KT*)A.keys + b * A.keys_bstride;
   const bool wkeys = (STORE == kStoreKeys || STORE == kStoreBoth) && (b < A.key_batches);
+  uint32_t dg[EPT];   // the first digits of the thread's keys
 #pragma unroll
   for (int k = 0; k < EPT; ++k) {
     const int e = tid + k * NT;
@@ -690,8 +691,31 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
         const long long kpos = A.keys_tiled ? (long long)tile * TE + e : g;
         const KT key = sample_key(val);
         keys[kpos] = key;
-        if (A.digits)
-          A.digits[b * A.keys_bstride + kpos] = (uint16_t)sel_first_digit(key);
+        dg[k] = sel_first_digit(key);
+        if (A.digits) A.digits[b * A.keys_bstride + kpos] = (uint16_t)dg[k];
+      }
+    }
+  }
+  // ---- the cutoff's histogram of the tile's first digits: counted in LDS (two 16-bit counts per
+  // word, over the tile's values once they are read), then the bins that are not empty added to
+  // one of the segment's global histograms: the cutoff needs no launch that reads every digit and
+  // none that sums a row of counts per block (n = 2^27, k = 16000: a transform 841 -> 829 us FP64,
+  // 487 -> 479 FP32; k = 40000 FP32 1106 -> 1093).
+  if constexpr (STORE == kStoreKeys || STORE == kStoreBoth) {
+    if (wkeys && A.hist) {
+      uint32_t* cnt = reinterpret_cast<uint32_t*>(lds);
+      __syncthreads();
+      for (int i = tid; i < kSelBins / 2; i += NT) cnt[i] = 0u;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < EPT; ++k)
+        if (tid + k * NT < TE) atomicAdd(&cnt[dg[k] >> 1], 1u << ((dg[k] & 1u) * 16u));
+      __syncthreads();
+      uint32_t* g = A.hist + ((size_t)b * kSelCopies + (size_t)(tile & (kSelCopies - 1))) * kSelBins;
+      for (int i = tid; i < kSelBins / 2; i += NT) {
+        const uint32_t w = cnt[i];
+        if (w & 0xFFFFu) atomicAdd(&g[2 * i], w & 0xFFFFu);
+        if (w >> 16) atomicAdd(&g[2 * i + 1], w >> 16);
       }
     }
   }
@@ -934,6 +958,7 @@ static hipError_t each_pass(const FftLaunch& L, F&& fn) {
     A.scale = L.scale;
     A.keys_tiled = (last && p > 0 && L.keys_tiled) ? 1 : 0;
     A.digits = last ? L.digits : nullptr;
+    A.hist = last ? L.hist : nullptr;
     const int store = last ? L.store : kStoreCplx;
     const int tw = (p == 0) ? kTwNone : (log2Lcur > kMaxPassLog ? kTwSplit : kTwDirect);
     if (load != kLoadPlain && tw != kTwNone) return hipErrorInvalidValue;

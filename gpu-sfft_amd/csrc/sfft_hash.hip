@@ -78,7 +78,8 @@ hipError_t fill_u32(void* p, uint32_t v, size_t words, hipStream_t st) {
   return hipGetLastError();
 }
 
-// the per-transform clear in one launch: approved-residue bitmaps to 0, the largest approved
+// the per-transform clear in one launch: approved-residue bitmaps (and what lies behind them:
+// the cutoffs' histograms) to 0, the largest approved
 // residue of each location loop to -1 (the bucket selection bitmaps are rewritten whole by the
 // cutoff)
 __global__ void hash_clear_kernel(uint32_t* __restrict__ bm, size_t nbm,
@@ -90,7 +91,7 @@ __global__ void hash_clear_kernel(uint32_t* __restrict__ bm, size_t nbm,
 }
 
 static int clear_blocks(const HashArgs& h) {
-  const size_t blocks = ((size_t)h.loops_loc * h.bm_words + 255) / 256;
+  const size_t blocks = (h.clear_words + 255) / 256;
   return (int)(blocks > 4096 ? 4096 : blocks < 1 ? 1 : blocks);
 }
 
@@ -99,7 +100,7 @@ __global__ void hash_clear_jobs_kernel(JobsDev t) {
   const HashJob* j = job_here<HashJob>(t);
   if (!j) return;
   const HashArgs& h = j->h;
-  const size_t nbm = (size_t)h.loops_loc * h.bm_words, s = (size_t)j->blocks * 256;
+  const size_t nbm = h.clear_words, s = (size_t)j->blocks * 256;
   const size_t i0 = (size_t)((int)blockIdx.x - j->block0) * 256 + threadIdx.x;
   for (size_t i = i0; i < nbm; i += s) h.bitmap[i] = 0u;
   if (i0 < (size_t)h.loops_loc) h.maxfirst[i0] = -1;
@@ -115,9 +116,8 @@ hipError_t hash_clear_jobs(const JobTable<HashJob>& t, hipStream_t st) {
 }
 
 hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st) {
-  const size_t bm_words = (size_t)h.loops_loc * h.bm_words;
   hipLaunchKernelGGL(hash_clear_kernel, dim3(clear_blocks(h)), dim3(256), 0, st,
-                     (uint32_t*)h.bitmap, bm_words, (uint32_t*)h.maxfirst, h.loops_loc);
+                     (uint32_t*)h.bitmap, h.clear_words, (uint32_t*)h.maxfirst, h.loops_loc);
   return hipGetLastError();
 }
 

@@ -51,6 +51,12 @@ __device__ __forceinline__ unsigned sel_first_digit(unsigned long long key) {
   return (__float_as_uint(f) >> 19) & 0xFFFu;
 }
 
+constexpr int kSelDigit = 12;            // bits of the first digit
+constexpr int kSelBins = 1 << kSelDigit;
+// Histograms of a segment's first digits that the last FFT pass adds to (FftLaunch::hist) and the
+// select sums: a few, so that tiles meet on a bin's counter less often.
+constexpr int kSelCopies = 4;
+
 // kLoadCombRowsG: kLoadCombRows with sibling sub-FFTs grouped per tile (chosen per pass by
 // fft_run; callers set kLoadCombRows)
 // kLoadWiden: FP64 transforms of a complex64 input, widened as it is loaded.
@@ -93,6 +99,9 @@ struct FftLaunch {
   int keys_tiled = 0;            // keys in the last pass's tile order (see KeyMap)
   uint16_t* digits = nullptr;    // optional: each key's top 12 bits below the sign bit (the
                                  // select's first digit), same positions and stride as keys
+  unsigned* hist = nullptr;      // optional: kSelCopies histograms of the keys' first digits per
+                                 // key batch (kSelBins counts each, zero before), each tile
+                                 // adding to one of them
   void* mid = nullptr;           // batch * N elements for the passes before the last instead of
                                  // out (out may then hold less than N: kStoreHead)
   int taps = 0;                  // kLoadTaps
@@ -214,10 +223,13 @@ struct SelMark {
   int* maxfirst = nullptr;     // loops
 };
 bool select_in_block(int N);   // whether one workgroup does a segment
+// hist (optional): the first digits' histograms as the FFT leaves them (FftLaunch::hist); a
+// chained select then reads no key for its histogram
 hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int N, int K,
                        int segs, int* out, int ordered, const SelectWork& w, hipStream_t st,
                        unsigned* bits = nullptr, const KeyMap* map = nullptr,
-                       const uint16_t* digits = nullptr, const SelMark* mark = nullptr);
+                       const uint16_t* digits = nullptr, const SelMark* mark = nullptr,
+                       const unsigned* hist = nullptr);
 
 // ---- reverse hash (bitmap of approved residues, deterministic hit list) -----------------
 struct HashArgs {
@@ -229,6 +241,8 @@ struct HashArgs {
   const int* ai_dev;
   unsigned* bitmap;      // loops_loc x words
   int bm_words;
+  size_t clear_words;    // from bitmap on: what a transform clears (the bitmaps, the cutoffs'
+                         // histograms behind them)
   int* maxfirst;         // loops_loc
   unsigned* jsel;        // loops_loc x jsel_words: the buckets each location loop selected
   int jsel_words;

@@ -89,6 +89,7 @@ struct PassArgs {
   int nbatch;
   int keys_tiled;   // store keys at tile * TE + e (the tile's own contiguous range)
   uint16_t* digits; // optional first digits of the keys (same positions)
+  unsigned* hist;   // optional histograms of the first digits (FftLaunch::hist)
   int log2nlo, log2m;   // kLoadCombRows: g at in[(g mod 2^log2nlo) << log2m | g >> log2nlo]
   const int* perm;      // kLoadPerm: g of batch b at in[g * perm[b] mod 2^log2N]
   const int* perm_inv;  // kLoadPerm: the inverse of perm[b] mod 2^log2N
@@ -151,7 +152,8 @@ struct SelJob {
   long long seg_stride;
   int N, K, chunk, nchunks, ordered, vec, segs;
   unsigned* rows;
-  unsigned* sums;
+  const unsigned* sums; // nsum histograms per segment, summed by the split
+  int nsum;
   void* state;
   void* blk_key;
   int* blk_idx;
@@ -171,27 +173,24 @@ struct SelJob {
 struct SelGroup {
   int fp32 = 0;
   JobTable<SelJob> block[3];   // one workgroup per segment: 8, 16, 32 elements per thread
-  JobTable<SelJob> wide;       // nchunks x segs workgroups: hist0, split, compact / write
-  JobTable<SelJob> sums;       // column sums
+  JobTable<SelJob> wide;       // nchunks x segs workgroups: split, compact / write
   JobTable<SelJob> refine;     // one workgroup per segment
   void pack(JobPack& p) {
     for (auto& b : block) b.pack(p);
     wide.pack(p);
-    sums.pack(p);
     refine.pack(p);
   }
   void bind(const char* base) {
     for (auto& b : block) b.bind(base);
     wide.bind(base);
-    sums.bind(base);
     refine.bind(base);
   }
 };
-// the arguments of select_topk
+// the arguments of select_topk (hist: where one workgroup does not do a segment)
 hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long seg_stride, int N,
                            int K, int segs, int* out, int ordered, const SelectWork& w,
                            unsigned* bits, const KeyMap* map, const uint16_t* digits,
-                           const SelMark* mark);
+                           const SelMark* mark, const unsigned* hist);
 hipError_t select_jobs_launch(const SelGroup& g, hipStream_t st);
 
 // ---- reverse hash, estimation --------------------------------------------------------------

@@ -303,7 +303,12 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   void* selB_base = nullptr;
   items.push_back({&selW_base, select_work_bytes(Rl, (int)W)});
   items.push_back({&selB_base, select_work_bytes(Ll, (int)B)});
-  items.push_back({(void**)&P->bitmap, (size_t)Ll * P->bm_words * 4});
+  // the bitmaps, and behind them the histograms of the chained cutoffs, cleared together
+  const size_t bmw = ((size_t)Ll * P->bm_words + 63) / 64 * 64;
+  const size_t histW = select_in_block((int)W) ? 0 : (size_t)Rl * kSelCopies * kSelBins;
+  const size_t histB = select_in_block((int)B) ? 0 : (size_t)Ll * kSelCopies * kSelBins;
+  P->clear_words = bmw + histW + histB;
+  items.push_back({(void**)&P->bitmap, P->clear_words * 4});
   items.push_back({(void**)&P->maxfirst, (size_t)Ll * 4});
   items.push_back({(void**)&P->jsel, (size_t)Ll * ((B + 31) / 32) * 4});
   items.push_back({(void**)&P->hitoff, (size_t)Ll * K * 4});
@@ -335,6 +340,8 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   }
   P->d_ai = P->d_a + L;
   P->d_offs = P->d_a + 2 * L;
+  P->hist_W = histW ? P->bitmap + bmw : nullptr;
+  P->hist_B = histB ? P->bitmap + bmw + histW : nullptr;
   select_work_bind(&P->selW, selW_base, Rl, (int)W);
   select_work_bind(&P->selB, selB_base, Ll, (int)B);
   // select state must start at zero (hist/done are reset by the kernels themselves)
@@ -434,6 +441,7 @@ HashArgs hash_args(const sfft_plan* P, int* d_count) {
   h.ai_dev = P->d_ai;
   h.bitmap = P->bitmap;
   h.bm_words = P->bm_words;
+  h.clear_words = P->clear_words;
   h.maxfirst = P->maxfirst;
   h.jsel = P->jsel;
   h.jsel_words = (p.B + 31) / 32;
@@ -491,6 +499,7 @@ FftLaunch comb_fft(const sfft_plan* P, const void* d_x) {
   c.qmax = P->qmax_W;
   c.keys_tiled = 1;
   c.digits = P->comb_digits;
+  c.hist = P->hist_W;
   if (P->stream) {
     c.in = P->comb_y;
     c.in_bstride = W;
@@ -532,7 +541,7 @@ static sfft_status run_cut(sfft_plan* P, const HashArgs& h, hipStream_t st, bool
   const SelMark mk = comb_mark(h);
   const bool marks_too = select_in_block((int)W);
   HIPCK(select_topk(P->fp32, P->comb_keys, W, (int)W, p.B_thresh, p.RLFC_loops, P->J2, 0,
-                    P->selW, st, nullptr, &km, P->comb_digits, marks_too ? &mk : nullptr));
+                    P->selW, st, nullptr, &km, P->comb_digits, marks_too ? &mk : nullptr, P->hist_W));
   if (!marks_too) HIPCK(hash_bitmap_launch(h, st));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[3], st));
   return SFFT_OK;
@@ -580,6 +589,7 @@ FftLaunch bucket_fft(const sfft_plan* P) {
   f.store = kStoreBoth;
   f.qmax = P->qmax_B;
   f.digits = P->bucket_digits;
+  f.hist = P->hist_B;
   if (P->bins_perm) {   // bucket r of loop l at column r * ai_l mod B
     f.load = kLoadPerm;
     f.perm = P->d_ai;
@@ -595,7 +605,7 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
   HIPCK(fft_run(bucket_fft(P), st));
   // ascending bucket lists: the hit list is ordered by (loop, bucket, walk)
   HIPCK(select_topk(P->fp32, P->bkeys, p.B, p.B, p.B_thresh, p.loops_loc, P->J, 1, P->selB, st,
-                    P->jsel, nullptr, P->bucket_digits));
+                    P->jsel, nullptr, P->bucket_digits, nullptr, P->hist_B));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[5], st));
   return SFFT_OK;
 }
@@ -636,7 +646,7 @@ static sfft_status run_all_columns(sfft_plan* P, const void* d_x, const HashArgs
   };
   FoldClear clr;
   clr.bm = h.bitmap;
-  clr.nbm = (size_t)h.loops_loc * (size_t)h.bm_words;
+  clr.nbm = h.clear_words;
   clr.maxf = (uint32_t*)h.maxfirst;
   clr.nmax = h.loops_loc;
   HIPCK(mark(0));

@@ -40,6 +40,9 @@ struct sfft_plan {
   SelectWork selW, selB;
   unsigned* bitmap = nullptr;
   int bm_words = 0;
+  size_t clear_words = 0;       // the bitmaps and the histograms behind them
+  unsigned* hist_W = nullptr;   // first-digit histograms of the chained cutoffs (the last FFT
+  unsigned* hist_B = nullptr;   // passes count them; nullptr: one workgroup per segment)
   int* maxfirst = nullptr;
   unsigned* jsel = nullptr;     // buckets selected per location loop (bitmaps)
   int* hitoff = nullptr;

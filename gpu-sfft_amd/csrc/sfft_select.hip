@@ -4,8 +4,9 @@
 // Every element gets a unique composite key  c = (key without sign bit) . (N-1-index)  so that
 // "larger c" means "larger |X|^2, or equal and lower index"; the top-K set is {c >= T}.
 //   1. hist0   : histogram of the top 12 bits of c, one row per block (wave-aggregated LDS
-//                atomics), then colsum: the column sums of the rows.
-//   2. split   : every block picks the digit d0 holding the K-th largest from the column
+//                atomics), then colsum: the column sums of the rows.  A transform's cutoffs skip
+//                both: the last FFT pass leaves the histogram (FftLaunch::hist).
+//   2. split   : every block picks the digit d0 holding the K-th largest from the
 //                sums, then one pass over N: digit > d0 -> selected (emitted at once in
 //                unordered mode), digit == d0 -> appended to a candidate list (typically ~1%
 //                of N).
@@ -33,8 +34,8 @@ struct SelState {
 
 constexpr int SEL_NT = 1024;   // threads of the streaming select kernels (512: +11 us comb
                                // cutoff, +3 us bucket cutoff at n = 2^27, k = 16000)
-constexpr int SEL_DIG = 12;
-constexpr int SEL_BINS = 1 << SEL_DIG;
+constexpr int SEL_DIG = kSelDigit;
+constexpr int SEL_BINS = kSelBins;
 
 template <typename K>
 struct KeyBits;
@@ -231,7 +232,7 @@ __device__ __forceinline__ void sel_colsum_body(int nchunks, const unsigned* __r
 template <typename K>
 __device__ __forceinline__ void sel_split_body(const K* __restrict__ keys, long long seg_stride,
                                                int N, int chunk, int nchunks, int emit, int Ksel,
-                                               const unsigned* __restrict__ ghist,
+                                               const unsigned* __restrict__ ghist, int nsum,
                                                SelState* __restrict__ st, K* __restrict__ ckey,
                                                int* __restrict__ cidx, int* __restrict__ eidx,
                                                int* __restrict__ ccnt, int* __restrict__ ecnt,
@@ -250,14 +251,19 @@ __device__ __forceinline__ void sel_split_body(const K* __restrict__ keys, long 
   // the same one (16 KB of sums, no separate pick launch); block 0 records it and the count
   // still needed inside it for the refine
   {
-    const unsigned* gh = ghist + (size_t)seg * SEL_BINS;
+    const unsigned* gh = ghist + (size_t)seg * nsum * SEL_BINS;
     unsigned v[4];
     int S = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[j] = gh[SEL_BINS - 1 - (4 * tid + j)];
-      S += (int)v[j];
+    for (int j = 0; j < 4; ++j) v[j] = gh[SEL_BINS - 1 - (4 * tid + j)];
+    if (nsum == kSelCopies) {   // the FFT's histograms (their loads in flight together)
+#pragma unroll
+      for (int c = 1; c < kSelCopies; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += gh[c * SEL_BINS + SEL_BINS - 1 - (4 * tid + j)];
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S += (int)v[j];
     const int E = block_excl_scan_s(S, sh);   // (its barriers also publish the defaults)
     if (E < Ksel && Ksel <= E + S) {
       int cum = E;
@@ -980,7 +986,7 @@ __global__ __launch_bounds__(PICK_NT) void sel_colsum_kernel(From f) {
   SelJob j;
   int bx, seg;
   if (!f.get(j, bx, seg, SEL_BINS / PICK_BINS)) return;
-  sel_colsum_body(j.nchunks, j.rows, j.sums, bx, seg);
+  sel_colsum_body(j.nchunks, j.rows, const_cast<unsigned*>(j.sums), bx, seg);
 }
 template <typename K, typename From>
 __global__ __launch_bounds__(SEL_NT) void sel_split_kernel(From f) {
@@ -988,7 +994,7 @@ __global__ __launch_bounds__(SEL_NT) void sel_split_kernel(From f) {
   int bx, seg;
   if (!f.get(j, bx, seg, 0)) return;
   sel_split_body<K>((const K*)j.keys, j.seg_stride, j.N, j.chunk, j.nchunks, j.ordered ? 0 : 1, j.K,
-                    j.sums, (SelState*)j.state, (K*)j.blk_key, j.blk_idx, j.emit_idx, j.ccnt,
+                    j.sums, j.nsum, (SelState*)j.state, (K*)j.blk_key, j.blk_idx, j.emit_idx, j.ccnt,
                     j.ecnt, j.map, j.digits, bx, seg);
 }
 // unordered: the candidates of the split's blocks side by side, its winners to the output
@@ -1038,10 +1044,10 @@ constexpr int SB_MAX_N = 32768;
 bool select_in_block(int N) { return N <= SB_MAX_N; }
 
 // the job of one select_topk call
-static hipError_t select_job(SelJob& j, int is_fp32, const void* keys, long long seg_stride, int N,
+static hipError_t select_job(SelJob& j, const void* keys, long long seg_stride, int N,
                              int K, int segs, int* out, int ordered, const SelectWork& w,
                              unsigned* bits, const KeyMap* map, const uint16_t* digits,
-                             const SelMark* mark) {
+                             const SelMark* mark, const unsigned* hist) {
   // the write pass reads the keys
   if (ordered && digits && !select_in_block(N)) return hipErrorInvalidValue;
   if (mark && !select_in_block(N)) return hipErrorInvalidValue;   // the one-workgroup select marks
@@ -1064,7 +1070,8 @@ static hipError_t select_job(SelJob& j, int is_fp32, const void* keys, long long
   j.segs = segs;
   j.vec = ((uintptr_t)digits & 15) == 0 && (seg_stride & 7) == 0;   // 16-byte loads of digits
   // work layout: column sums, then the per-block histogram rows
-  j.sums = w.hist;
+  j.sums = hist ? hist : w.hist;
+  j.nsum = hist ? kSelCopies : 1;
   j.rows = w.hist + (size_t)segs * SEL_BINS;
   j.state = w.state;
   j.blk_key = w.blk_key;
@@ -1079,7 +1086,6 @@ static hipError_t select_job(SelJob& j, int is_fp32, const void* keys, long long
   j.bits = bits;
   j.digits = digits;
   if (mark) j.mark = *mark;
-  (void)is_fp32;
   return hipSuccess;
 }
 
@@ -1104,10 +1110,12 @@ static hipError_t select_one(const SelJob& j, hipStream_t st) {
     block_go<K>(block_variant(j.N), f, dim3(1, j.segs), st);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((sel_hist0_kernel<K, SelOne>), wide, dim3(SEL_NT), 0, st, f);
-  hipLaunchKernelGGL((sel_colsum_kernel<SelOne>), dim3(SEL_BINS / PICK_BINS, j.segs),
-                     dim3(PICK_NT), 0, st, f);
-  // (the split blocks pick d0 from the column sums themselves)
+  if (j.nsum == 1) {   // no histograms at hand
+    hipLaunchKernelGGL((sel_hist0_kernel<K, SelOne>), wide, dim3(SEL_NT), 0, st, f);
+    hipLaunchKernelGGL((sel_colsum_kernel<SelOne>), dim3(SEL_BINS / PICK_BINS, j.segs),
+                       dim3(PICK_NT), 0, st, f);
+  }
+  // (the split blocks pick d0 from the sums themselves)
   hipLaunchKernelGGL((sel_split_kernel<K, SelOne>), wide, dim3(SEL_NT), 0, st, f);
   if (!j.ordered)
     hipLaunchKernelGGL((sel_compact_kernel<K, SelOne>), wide, dim3(CMP_NT), 0, st, f);
@@ -1120,10 +1128,10 @@ static hipError_t select_one(const SelJob& j, hipStream_t st) {
 hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int N, int K,
                        int segs, int* out, int ordered, const SelectWork& w, hipStream_t st,
                        unsigned* bits, const KeyMap* map, const uint16_t* digits,
-                       const SelMark* mark) {
+                       const SelMark* mark, const unsigned* hist) {
   SelJob j;
-  const hipError_t e = select_job(j, is_fp32, keys, seg_stride, N, K, segs, out, ordered, w, bits,
-                                  map, digits, mark);
+  const hipError_t e = select_job(j, keys, seg_stride, N, K, segs, out, ordered, w, bits,
+                                  map, digits, mark, hist);
   if (e != hipSuccess) return e;
   return is_fp32 ? select_one<unsigned int>(j, st) : select_one<unsigned long long>(j, st);
 }
@@ -1131,17 +1139,16 @@ hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int 
 hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long seg_stride, int N,
                            int K, int segs, int* out, int ordered, const SelectWork& w,
                            unsigned* bits, const KeyMap* map, const uint16_t* digits,
-                           const SelMark* mark) {
+                           const SelMark* mark, const unsigned* hist) {
   SelJob j;
-  const hipError_t e = select_job(j, is_fp32, keys, seg_stride, N, K, segs, out, ordered, w, bits,
-                                  map, digits, mark);
+  const hipError_t e = select_job(j, keys, seg_stride, N, K, segs, out, ordered, w, bits,
+                                  map, digits, mark, hist);
   if (e != hipSuccess) return e;
   g.fp32 = is_fp32;
   if (select_in_block(N)) {
     g.block[block_variant(N)].add(j, segs);
   } else {
     g.wide.add(j, j.nchunks * segs);
-    g.sums.add(j, SEL_BINS / PICK_BINS * segs);
     g.refine.add(j, segs);
   }
   return hipSuccess;
@@ -1154,12 +1161,9 @@ static hipError_t select_many(const SelGroup& g, hipStream_t st) {
     if (g.block[v].dev.blocks)
       block_go<K>(v, SelMany{g.block[v].dev}, dim3(g.block[v].dev.blocks), st);
   if (g.wide.dev.blocks) {
-    const SelMany wide{g.wide.dev}, sums{g.sums.dev}, refine{g.refine.dev};
+    const SelMany wide{g.wide.dev}, refine{g.refine.dev};
     const dim3 nw(wide.t.blocks);
     const bool ordered = g.wide.jobs[0].ordered != 0;
-    hipLaunchKernelGGL((sel_hist0_kernel<K, SelMany>), nw, dim3(SEL_NT), 0, st, wide);
-    hipLaunchKernelGGL((sel_colsum_kernel<SelMany>), dim3(sums.t.blocks), dim3(PICK_NT), 0, st,
-                       sums);
     hipLaunchKernelGGL((sel_split_kernel<K, SelMany>), nw, dim3(SEL_NT), 0, st, wide);
     if (!ordered)
       hipLaunchKernelGGL((sel_compact_kernel<K, SelMany>), nw, dim3(CMP_NT), 0, st, wide);
