@@ -45,7 +45,7 @@ struct sfft_batch {
   std::vector<FftGroup> comb, comb_slab, bucket;   // combs gathered, combs the slab fold copied
   SelGroup sel_comb, sel_bucket;
   JobTable<HashJob> clear, bitmap, hits;
-  std::vector<EstGroup> est;
+  std::vector<NodeGroup> est;
   char* d_tab = nullptr;
   size_t tab_bytes = 0;
   const PfJob* d_jobs = nullptr;
@@ -227,22 +227,17 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
                           P->J, 1, P->selB, P->jsel, nullptr, P->bucket_digits, nullptr,
                           P->hist_B));
     if (!marks) hash_jobs_bitmap(b->bitmap, h);
-    hash_jobs_hits(b->hits, h);
-    EstJob e = {};
-    e.hits = P->hits;
-    e.count = b->d_counts + i;
-    e.capacity = P->cap;
+    hash_jobs_count(b->hits, h);
+    NodeJob e = {};
+    e.h = h;
     e.bins = P->bins_f;
     e.loops = p.loops;
-    e.n = p.n;
-    e.ai = P->d_ai;
-    e.B = p.B;
     e.win = P->win;
     e.out = nodes[i] ? nodes[i] : P->nodes;
     e.copy = nodes[i] ? P->nodes : nullptr;
     e.sel = P->sel;
     e.count_copy = b->h_counts_dev + i;
-    estimate_jobs_add(b->est, b->fp32, e);
+    nodes_jobs_add(b->est, b->fp32, e);
   }
   b->total_items = item;
   slab_jobs_share(b->slab);
@@ -303,8 +298,8 @@ static sfft_status enqueue(sfft_batch* b) {
   HIPCK(fft_jobs_launch(b->bucket, b->st));
   HIPCK(select_jobs_launch(b->sel_bucket, b->st));
   HIPCK(hipStreamWaitEvent(b->st, b->ev_join, 0));
-  HIPCK(hash_hits_jobs(b->hits, b->st));
-  HIPCK(estimate_jobs_launch(b->est, b->st));
+  HIPCK(hash_count_jobs(b->hits, b->st));
+  HIPCK(nodes_jobs_launch(b->est, b->st));
   return SFFT_OK;
 }
 

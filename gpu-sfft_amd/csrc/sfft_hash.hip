@@ -248,7 +248,9 @@ size_t hash_mask_bytes(int loops_loc, int K, long long m) {
 // walk's early exit), and p's residue p mod W is approved: three table reads instead of a
 // vote pass over every window and a vote table.  The count and write passes cover the loops
 // [thresh-1, loops_loc) (loops_thresh >= 1 is checked when the plan is made).
-static int hash_hit_count(const HashArgs& h) { return h.loops_loc - (h.loops_thresh - 1); }
+static int hash_hit_blocks(const HashArgs& h) {
+  return hash_blocks(h.loops_loc - (h.loops_thresh - 1), h.loops_loc, h.K, (long long)h.n / h.B);
+}
 
 // thread -> (location loop l, bucket index i, slice sub of lpj)
 struct HashSlot {
@@ -345,77 +347,25 @@ __device__ __forceinline__ void hash_count_body(const HashArgs& h, int bx) {
   if (threadIdx.x == HASH_NT - 1) h.blocksum[bx] = ex + v;
 }
 
-// the hits of each slice, from the count pass's hit mask (no second walk).  Each block first
-// sums the hit totals of the blocks before it (a few KB, read by every block in parallel: no
-// separate scan launch); the last block stores the total hit count.
-__device__ __forceinline__ void hash_write_body(const HashArgs& h, int bx, int nb) {
-  __shared__ int sh[16];
-  int pre = 0;
-  for (int b = threadIdx.x; b < bx; b += HASH_NT) pre += h.blocksum[b];
-  const int boff = block_sum(pre, sh);
-  if (bx == nb - 1 && threadIdx.x == 0) *h.count = boff + h.blocksum[bx];
-  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
-  const int words = hash_slice_words(h.loops_loc, h.K, (long long)h.n / h.B);
-  const long long gid = (long long)bx * HASH_NT + threadIdx.x;
-  const unsigned* __restrict__ mk = h.hmask + gid * words;
-  int c = 0;
-  if (s.valid)
-    for (int w = 0; w < words; ++w) c += __popc(mk[w]);
-  // exclusive scan over the bucket's lanes (in window order)
-  const int lane = threadIdx.x & 63;
-  int x = c;
-  for (int o = 1; o < s.lpj; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if ((lane & (s.lpj - 1)) >= o) x += y;
-  }
-  if (!s.valid || c == 0) return;
-  int pos = boff + h.hitoff[s.jidx] + (x - c);
-  const long long n = h.n;
-  const long long m = n / h.B;
-  const long long J = h.J[(long long)s.l * h.K + s.i];
-  const long long start = ((J * m - (m >> 1)) + n + s.d0) & (n - 1);   // low + d0
-  const uint64_t a = (uint64_t)(uint32_t)h.a_dev[s.l];
-  for (int w = 0; w < words; ++w) {
-    unsigned word = mk[w];
-    while (word) {
-      const int rel = w * 32 + __ffs(word) - 1;
-      word &= word - 1u;
-      const uint64_t p = (uint64_t)((start + rel) & (n - 1));
-      if (pos < h.capacity) h.hits[pos] = (int)((p * a) & ((uint64_t)n - 1));
-      ++pos;
-    }
-  }
-}
-
 __global__ __launch_bounds__(HASH_NT) void hash_count_kernel(HashArgs h) {
   hash_count_body(h, blockIdx.x);
-}
-__global__ __launch_bounds__(HASH_NT) void hash_write_kernel(HashArgs h) {
-  hash_write_body(h, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(HASH_NT) void hash_count_jobs_kernel(JobsDev t) {
   const HashJob* j = job_here<HashJob>(t);
   if (j) hash_count_body(j->h, (int)blockIdx.x - j->block0);
 }
-__global__ __launch_bounds__(HASH_NT) void hash_write_jobs_kernel(JobsDev t) {
-  const HashJob* j = job_here<HashJob>(t);
-  if (j) hash_write_body(j->h, (int)blockIdx.x - j->block0, j->blocks);
-}
-void hash_jobs_hits(JobTable<HashJob>& t, const HashArgs& h) {
-  HashJob j{h, hash_blocks(hash_hit_count(h), h.loops_loc, h.K, (long long)h.n / h.B), 0};
+void hash_jobs_count(JobTable<HashJob>& t, const HashArgs& h) {
+  HashJob j{h, hash_hit_blocks(h), 0};
   t.add(j, j.blocks);
 }
-hipError_t hash_hits_jobs(const JobTable<HashJob>& t, hipStream_t st) {
+hipError_t hash_count_jobs(const JobTable<HashJob>& t, hipStream_t st) {
   if (!t.dev.blocks) return hipSuccess;
   hipLaunchKernelGGL(hash_count_jobs_kernel, dim3(t.dev.blocks), dim3(HASH_NT), 0, st, t.dev);
-  hipLaunchKernelGGL(hash_write_jobs_kernel, dim3(t.dev.blocks), dim3(HASH_NT), 0, st, t.dev);
   return hipGetLastError();
 }
 
-hipError_t hash_hits_launch(const HashArgs& h, hipStream_t st) {
-  const int nb = hash_blocks(hash_hit_count(h), h.loops_loc, h.K, (long long)h.n / h.B);
-  hipLaunchKernelGGL(hash_count_kernel, dim3(nb), dim3(HASH_NT), 0, st, h);
-  hipLaunchKernelGGL(hash_write_kernel, dim3(nb), dim3(HASH_NT), 0, st, h);
+hipError_t hash_count_launch(const HashArgs& h, hipStream_t st) {
+  hipLaunchKernelGGL(hash_count_kernel, dim3(hash_hit_blocks(h)), dim3(HASH_NT), 0, st, h);
   return hipGetLastError();
 }
 
@@ -427,179 +377,289 @@ __device__ __forceinline__ double2 to_d2(float2 v) {
   return make_double2((double)v.x, (double)v.y);
 }
 
-// One thread per hit.  EXACT: the loop count is the template constant MAXL (every address
-// first, then every load, so the 2*MAXL reads of a hit are in flight together); otherwise
-// loops <= MAXL at run time.  The arithmetic per loop is the same either way.  A block's
-// nodes are staged in LDS and stored as consecutive 8-byte words (coalesced, also when `out`
-// is pinned host memory written over the bus); count_copy (optional) receives the count.
-constexpr int EST_NT = 256;
-constexpr int EST_GRID = 512;   // blocks of the estimation launch (grid-stride over the hits)
+// The value of location I: the lower medians over the loops of the real and the imaginary parts
+// (rr, ri) and the loops they came from (sr, si).  EXACT: the loop count is the template constant
+// MAXL (every address first, then every load, so the 2*MAXL reads of a hit are in flight
+// together); otherwise loops <= MAXL at run time.  The arithmetic per loop is the same either way.
 template <typename Real, int MAXL, bool EXACT>
-__device__ __forceinline__ void estimate_body(
-    const int* __restrict__ hits, const int* __restrict__ count, int capacity,
-    const typename CT<Real>::T2* __restrict__ bins, int loops_rt, uint32_t n,
-    const int* __restrict__ ai_dev, int B, const double2* __restrict__ win,
-    Node* __restrict__ out, Node* __restrict__ copy, uint8_t* __restrict__ sel,
-    int* __restrict__ count_copy, int bx, int nb) {
-  static_assert(sizeof(Node) == 24, "Node: key, 4 bytes of padding, two doubles");
-  __shared__ unsigned long long stage[EST_NT * 3];
+__device__ __forceinline__ void estimate_one(uint32_t I,
+                                             const typename CT<Real>::T2* __restrict__ bins,
+                                             int loops_rt, uint32_t n,
+                                             const int* __restrict__ ai_dev, int B,
+                                             const double2* __restrict__ win, double& rr,
+                                             double& ri, int& sr, int& si) {
   const int loops = EXACT ? MAXL : loops_rt;
-  const int cnt_all = *count;
-  const int total = min(cnt_all, capacity);
-  if (count_copy && bx == 0 && threadIdx.x == 0) *count_copy = cnt_all;
   const long long m = (long long)(n / (uint32_t)B);
   const int lm = 63 - __clzll(m);   // m = n / B, both powers of two
   const long long nn = n;
   const int med = (loops - 1) / 2;
-  for (int h0 = bx * EST_NT; h0 < total; h0 += nb * EST_NT) {
+  long long bidx[MAXL], widx[MAXL];
+#pragma unroll
+  for (int l = 0; l < MAXL; ++l) {
+    const int lc = (EXACT || l < loops) ? l : 0;   // a valid address past the loop count
+    const long long p = (long long)(((uint64_t)(uint32_t)ai_dev[lc] * I) & (uint64_t)(n - 1));
+    long long hashed = p >> lm;
+    long long dist = p & (m - 1);
+    if (dist > m / 2) {
+      hashed = (hashed + 1) & (B - 1);
+      dist -= m;
+    }
+    dist = (nn - dist) & (nn - 1);
+    widx[l] = (dist + m / 2) & (nn - 1);
+    bidx[l] = (long long)lc * B + hashed;
+  }
+  double2 F[MAXL], bb[MAXL];
+#pragma unroll
+  for (int l = 0; l < MAXL; ++l) {
+    F[l] = win[widx[l]];
+    bb[l] = to_d2(bins[bidx[l]]);
+  }
+  double vr[MAXL], vi[MAXL];
+#pragma unroll
+  for (int l = 0; l < MAXL; ++l) {
+    // innerLoop.cu:848-852: products rounded, then combined
+    const double abs2 = F[l].x * F[l].x + F[l].y * F[l].y;
+    const double mr = bb[l].x * F[l].x + bb[l].y * F[l].y;
+    const double mi = bb[l].y * F[l].x - bb[l].x * F[l].y;
+    vr[l] = mr / abs2;
+    vi[l] = mi / abs2;
+  }
+  // stable rank selection: position of j in an insertion sort = #(v_i < v_j) + #(i<j, v_i==v_j)
+  rr = ri = 0.0;
+  sr = si = 0;
+#pragma unroll
+  for (int j = 0; j < MAXL; ++j) {
+    if (j < loops) {
+      int pr = 0, pi = 0;
+#pragma unroll
+      for (int i = 0; i < MAXL; ++i) {
+        if (i < loops) {
+          pr += (vr[i] < vr[j]) || (i < j && vr[i] == vr[j]);
+          pi += (vi[i] < vi[j]) || (i < j && vi[i] == vi[j]);
+        }
+      }
+      if (pr == med) {
+        rr = vr[j];
+        sr = j;
+      }
+      if (pi == med) {
+        ri = vi[j];
+        si = j;
+      }
+    }
+  }
+}
+
+// `count` nodes staged in LDS stored as consecutive 8-byte words (coalesced, also when out is
+// pinned host memory written over the bus)
+constexpr int EST_NT = 256;
+static_assert(sizeof(Node) == 24, "Node: key, 4 bytes of padding, two doubles");
+__device__ __forceinline__ void stage_node(unsigned long long* stage, uint32_t I, double rr,
+                                           double ri) {
+  stage[3 * threadIdx.x] = (unsigned long long)I;   // key, then 4 zero bytes of padding
+  stage[3 * threadIdx.x + 1] = (unsigned long long)__double_as_longlong(rr);
+  stage[3 * threadIdx.x + 2] = (unsigned long long)__double_as_longlong(ri);
+}
+__device__ __forceinline__ void store_nodes(const unsigned long long* stage, int count,
+                                            Node* __restrict__ out) {
+  unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
+  for (int j = threadIdx.x; j < 3 * count; j += EST_NT) o[j] = stage[j];
+}
+
+// One thread per hit of a list (the reference's estimation entry point).
+constexpr int EST_GRID = 512;   // blocks of the estimation launch (grid-stride over the hits)
+template <typename Real, int MAXL, bool EXACT>
+__global__ __launch_bounds__(EST_NT) void estimate_kernel(EstArgs j) {
+  __shared__ unsigned long long stage[EST_NT * 3];
+  const int total = min(*j.count, j.capacity);
+  for (int h0 = blockIdx.x * EST_NT; h0 < total; h0 += gridDim.x * EST_NT) {
     const int h = h0 + (int)threadIdx.x;
-    const bool valid = h < total;
-    const uint32_t I = (uint32_t)hits[valid ? h : h0];
-    long long bidx[MAXL], widx[MAXL];
-#pragma unroll
-    for (int l = 0; l < MAXL; ++l) {
-      const int lc = (EXACT || l < loops) ? l : 0;   // a valid address past the loop count
-      const long long p = (long long)(((uint64_t)(uint32_t)ai_dev[lc] * I) & (uint64_t)(n - 1));
-      long long hashed = p >> lm;
-      long long dist = p & (m - 1);
-      if (dist > m / 2) {
-        hashed = (hashed + 1) & (B - 1);
-        dist -= m;
-      }
-      dist = (nn - dist) & (nn - 1);
-      widx[l] = (dist + m / 2) & (nn - 1);
-      bidx[l] = (long long)lc * B + hashed;
-    }
-    double2 F[MAXL], bb[MAXL];
-#pragma unroll
-    for (int l = 0; l < MAXL; ++l) {
-      F[l] = win[widx[l]];
-      bb[l] = to_d2(bins[bidx[l]]);
-    }
-    double vr[MAXL], vi[MAXL];
-#pragma unroll
-    for (int l = 0; l < MAXL; ++l) {
-      // innerLoop.cu:848-852: products rounded, then combined
-      const double abs2 = F[l].x * F[l].x + F[l].y * F[l].y;
-      const double mr = bb[l].x * F[l].x + bb[l].y * F[l].y;
-      const double mi = bb[l].y * F[l].x - bb[l].x * F[l].y;
-      vr[l] = mr / abs2;
-      vi[l] = mi / abs2;
-    }
-    // stable rank selection: position of j in an insertion sort = #(v_i < v_j) + #(i<j, v_i==v_j)
-    double rr = 0.0, ri = 0.0;
-    int sr = 0, si = 0;
-#pragma unroll
-    for (int j = 0; j < MAXL; ++j) {
-      if (j < loops) {
-        int pr = 0, pi = 0;
-#pragma unroll
-        for (int i = 0; i < MAXL; ++i) {
-          if (i < loops) {
-            pr += (vr[i] < vr[j]) || (i < j && vr[i] == vr[j]);
-            pi += (vi[i] < vi[j]) || (i < j && vi[i] == vi[j]);
-          }
-        }
-        if (pr == med) {
-          rr = vr[j];
-          sr = j;
-        }
-        if (pi == med) {
-          ri = vi[j];
-          si = j;
-        }
-      }
-    }
-    stage[3 * threadIdx.x] = (unsigned long long)I;   // key, then 4 zero bytes of padding
-    stage[3 * threadIdx.x + 1] = (unsigned long long)__double_as_longlong(rr);
-    stage[3 * threadIdx.x + 2] = (unsigned long long)__double_as_longlong(ri);
-    if (sel && valid) {
-      sel[2 * h] = (uint8_t)sr;
-      sel[2 * h + 1] = (uint8_t)si;
-    }
+    const uint32_t I = (uint32_t)j.hits[h < total ? h : h0];
+    double rr, ri;
+    int sr, si;
+    estimate_one<Real, MAXL, EXACT>(I, (const typename CT<Real>::T2*)j.bins, j.loops,
+                                    (uint32_t)j.n, j.ai, j.B, j.win, rr, ri, sr, si);
+    stage_node(stage, I, rr, ri);
     __syncthreads();
-    const int words = 3 * min(EST_NT, total - h0);
-    unsigned long long* o = reinterpret_cast<unsigned long long*>(out + h0);
-    for (int j = threadIdx.x; j < words; j += EST_NT) o[j] = stage[j];
-    if (copy) {
-      unsigned long long* c = reinterpret_cast<unsigned long long*>(copy + h0);
-      for (int j = threadIdx.x; j < words; j += EST_NT) c[j] = stage[j];
-    }
+    store_nodes(stage, min(EST_NT, total - h0), j.out + h0);
     __syncthreads();
   }
 }
 
+// The hits of a block's slices, from the count pass's hit masks (no second walk), and their
+// values: the block lists its hits in LDS in window order and estimates one per thread, so the
+// hits are consecutive threads' work however the windows hold them and need no launch of their
+// own between the walk and the estimation (n = 2^27, k = 16000: a transform FP64 829 -> 823 us, FP32
+// 480 -> 472; n = 2^20, k = 1000, FP64 98 -> 94).  Each block first sums
+// the hit totals of the blocks before it (a few KB, read by every block in parallel: no separate
+// scan launch); the last one stores the total hit count.
+constexpr int ND_LIST = 1024;   // hits listed at a time
 template <typename Real, int MAXL, bool EXACT>
-__global__ __launch_bounds__(EST_NT) void estimate_kernel(EstJob j) {
-  estimate_body<Real, MAXL, EXACT>(j.hits, j.count, j.capacity,
-                                   (const typename CT<Real>::T2*)j.bins, j.loops, (uint32_t)j.n,
-                                   j.ai, j.B, j.win, j.out, j.copy, j.sel, j.count_copy, blockIdx.x,
-                                   gridDim.x);
-}
-template <typename Real, int MAXL, bool EXACT>
-__global__ __launch_bounds__(EST_NT) void estimate_jobs_kernel(JobsDev t) {
-  const EstJob* p = job_here<EstJob>(t);
-  if (!p) return;
-  const EstJob j = *p;
-  estimate_body<Real, MAXL, EXACT>(j.hits, j.count, j.capacity,
-                                   (const typename CT<Real>::T2*)j.bins, j.loops, (uint32_t)j.n,
-                                   j.ai, j.B, j.win, j.out, j.copy, j.sel, j.count_copy,
-                                   (int)blockIdx.x - j.block0, j.blocks);
+__device__ __forceinline__ void nodes_body(const NodeJob& j, int bx, int nb) {
+  static_assert(HASH_NT == EST_NT, "a hit per thread of the walk's block");
+  __shared__ unsigned long long stage[EST_NT * 3];
+  __shared__ int list[ND_LIST];
+  __shared__ int sh[16];
+  const HashArgs& h = j.h;
+  const int tid = threadIdx.x;
+  int pre = 0;
+  for (int b = tid; b < bx; b += HASH_NT) pre += h.blocksum[b];
+  const int boff = block_sum(pre, sh);
+  const int tot = h.blocksum[bx];
+  if (bx == nb - 1 && tid == 0) {
+    *h.count = boff + tot;
+    if (j.count_copy) *j.count_copy = boff + tot;
+  }
+  if (tot == 0) return;
+  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
+  const int words = hash_slice_words(h.loops_loc, h.K, (long long)h.n / h.B);
+  const long long gid = (long long)bx * HASH_NT + tid;
+  const unsigned* __restrict__ mk = h.hmask + gid * words;
+  int c = 0;
+  if (s.valid)
+    for (int w = 0; w < words; ++w) c += __popc(mk[w]);
+  // exclusive scan over the bucket's lanes (in window order)
+  const int lane = tid & 63;
+  int x = c;
+  for (int o = 1; o < s.lpj; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if ((lane & (s.lpj - 1)) >= o) x += y;
+  }
+  const long long n = h.n;
+  const long long m = n / h.B;
+  int first = 0;
+  long long start = 0;
+  uint64_t a = 0;
+  if (c) {
+    first = h.hitoff[s.jidx] + (x - c);   // within the block
+    const long long J = h.J[(long long)s.l * h.K + s.i];
+    start = ((J * m - (m >> 1)) + n + s.d0) & (n - 1);   // low + d0
+    a = (uint64_t)(uint32_t)h.a_dev[s.l];
+  }
+  for (int r0 = 0; r0 < tot; r0 += ND_LIST) {
+    if (c) {
+      int pos = first - r0;
+      for (int w = 0; w < words; ++w) {
+        unsigned word = mk[w];
+        while (word) {
+          const int rel = w * 32 + __ffs(word) - 1;
+          word &= word - 1u;
+          const uint64_t p = (uint64_t)((start + rel) & (n - 1));
+          if (pos >= 0 && pos < ND_LIST) list[pos] = (int)((p * a) & ((uint64_t)n - 1));
+          ++pos;
+        }
+      }
+    }
+    __syncthreads();
+    const int o0 = boff + r0;   // (hits past the capacity are counted only)
+    const int lim = min(min(ND_LIST, tot - r0), h.capacity - o0);
+    for (int h0 = 0; h0 < lim; h0 += EST_NT) {
+      const int i = h0 + tid;
+      if (h0 + (tid & ~63) < lim) {   // (waves without a hit leave)
+        const uint32_t I = (uint32_t)list[i < lim ? i : h0];
+        double rr, ri;
+        int sr, si;
+        estimate_one<Real, MAXL, EXACT>(I, (const typename CT<Real>::T2*)j.bins, j.loops,
+                                        (uint32_t)h.n, h.ai_dev, h.B, j.win, rr, ri, sr, si);
+        stage_node(stage, I, rr, ri);
+        if (i < lim) {
+          h.hits[o0 + i] = (int)I;
+          if (j.sel) {
+            j.sel[2 * (size_t)(o0 + i)] = (uint8_t)sr;
+            j.sel[2 * (size_t)(o0 + i) + 1] = (uint8_t)si;
+          }
+        }
+      }
+      __syncthreads();
+      const int k = min(EST_NT, lim - h0);
+      store_nodes(stage, k, j.out + o0 + h0);
+      if (j.copy) store_nodes(stage, k, j.copy + o0 + h0);
+      __syncthreads();
+    }
+    __syncthreads();   // (lim <= 0: the list is read no more before it is written again)
+  }
 }
 
-// f(kernel of one estimation, kernel of many) for the loop count
-template <typename Real, typename F>
+template <typename Real, int MAXL, bool EXACT>
+__global__ __launch_bounds__(EST_NT) void nodes_kernel(NodeJob j) {
+  nodes_body<Real, MAXL, EXACT>(j, blockIdx.x, gridDim.x);
+}
+template <typename Real, int MAXL, bool EXACT>
+__global__ __launch_bounds__(EST_NT) void nodes_jobs_kernel(JobsDev t) {
+  const NodeJob* p = job_here<NodeJob>(t);
+  if (!p) return;
+  const NodeJob j = *p;
+  nodes_body<Real, MAXL, EXACT>(j, (int)blockIdx.x - j.block0, j.blocks);
+}
+
+// f(the loop count as a template constant, whether it is exact)
+template <int V>
+struct IntC {
+  static constexpr int v = V;
+};
+template <typename F>
 static hipError_t with_loops(int loops, F&& f) {
 #define SFFT_EST(L) \
   case L:           \
-    return f(estimate_kernel<Real, L, true>, estimate_jobs_kernel<Real, L, true>);
+    return f(IntC<L>(), IntC<1>());
   switch (loops) {
     SFFT_EST(1) SFFT_EST(2) SFFT_EST(3) SFFT_EST(4) SFFT_EST(5) SFFT_EST(6) SFFT_EST(7)
     SFFT_EST(8) SFFT_EST(9) SFFT_EST(10) SFFT_EST(11) SFFT_EST(12) SFFT_EST(13) SFFT_EST(14)
     SFFT_EST(15) SFFT_EST(16)
     default:
-      return f(estimate_kernel<Real, 32, false>, estimate_jobs_kernel<Real, 32, false>);
+      return f(IntC<32>(), IntC<0>());
   }
 #undef SFFT_EST
 }
 
-hipError_t estimate_launch(int is_fp32, const int* hits, const int* count, int capacity,
-                           const void* bins_f, int loops, int n, const int* ai_dev, int B,
-                           const double2* filter_win, Node* out, uint8_t* sel,
-                           hipStream_t st, int* count_copy) {
-  EstJob j{hits,       count, capacity, bins_f, loops,      n, ai_dev, B,
-           filter_win, out,   nullptr,  sel,    count_copy, 0, 0};
-  auto go = [&](auto one, auto) {
-    hipLaunchKernelGGL(one, dim3(EST_GRID), dim3(EST_NT), 0, st, j);
+hipError_t estimate_launch(const EstArgs& a, hipStream_t st) {
+  return with_loops(a.loops, [&](auto L, auto E) {
+    hipLaunchKernelGGL((estimate_kernel<double, decltype(L)::v, decltype(E)::v != 0>),
+                       dim3(EST_GRID), dim3(EST_NT), 0, st, a);
     return hipGetLastError();
-  };
-  return is_fp32 ? with_loops<float>(loops, go) : with_loops<double>(loops, go);
+  });
 }
 
-void estimate_jobs_add(std::vector<EstGroup>& g, int is_fp32, EstJob j) {
+hipError_t nodes_launch(int is_fp32, const NodeJob& j, hipStream_t st) {
+  const dim3 grid(hash_hit_blocks(j.h)), nt(EST_NT);
+  return with_loops(j.loops, [&](auto L, auto E) {
+    constexpr int l = decltype(L)::v;
+    constexpr bool e = decltype(E)::v != 0;
+    if (is_fp32)
+      hipLaunchKernelGGL((nodes_kernel<float, l, e>), grid, nt, 0, st, j);
+    else
+      hipLaunchKernelGGL((nodes_kernel<double, l, e>), grid, nt, 0, st, j);
+    return hipGetLastError();
+  });
+}
+
+void nodes_jobs_add(std::vector<NodeGroup>& g, int is_fp32, NodeJob j) {
   const int key = j.loops <= 16 ? j.loops : 32;   // one kernel takes every count above 16
-  auto it = std::find_if(g.begin(), g.end(), [&](const EstGroup& x) { return x.loops == key; });
+  auto it = std::find_if(g.begin(), g.end(), [&](const NodeGroup& x) { return x.loops == key; });
   if (it == g.end()) {
     g.emplace_back();
     it = g.end() - 1;
     it->loops = key;
     it->fp32 = is_fp32;
   }
-  // the hits are known on the device only: a few blocks per signal, each taking every
-  // blocks-th group of EST_NT hits
-  j.blocks = std::min(EST_GRID / 16, (j.capacity + EST_NT - 1) / EST_NT);
+  j.blocks = hash_hit_blocks(j.h);
   it->t.add(j, j.blocks);
 }
 
-hipError_t estimate_jobs_launch(const std::vector<EstGroup>& groups, hipStream_t st) {
-  for (const EstGroup& g : groups) {
-    auto go = [&](auto, auto many) {
-      hipLaunchKernelGGL(many, dim3(g.t.dev.blocks), dim3(EST_NT), 0, st, g.t.dev);
+hipError_t nodes_jobs_launch(const std::vector<NodeGroup>& groups, hipStream_t st) {
+  for (const NodeGroup& g : groups) {
+    const hipError_t r = with_loops(g.loops, [&](auto L, auto E) {
+      constexpr int l = decltype(L)::v;
+      constexpr bool e = decltype(E)::v != 0;
+      if (g.fp32)
+        hipLaunchKernelGGL((nodes_jobs_kernel<float, l, e>), dim3(g.t.dev.blocks), dim3(EST_NT),
+                           0, st, g.t.dev);
+      else
+        hipLaunchKernelGGL((nodes_jobs_kernel<double, l, e>), dim3(g.t.dev.blocks), dim3(EST_NT),
+                           0, st, g.t.dev);
       return hipGetLastError();
-    };
-    const hipError_t e =
-        g.fp32 ? with_loops<float>(g.loops, go) : with_loops<double>(g.loops, go);
-    if (e != hipSuccess) return e;
+    });
+    if (r != hipSuccess) return r;
   }
   return hipSuccess;
 }

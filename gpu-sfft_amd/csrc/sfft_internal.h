@@ -255,20 +255,41 @@ struct HashArgs {
 };
 hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st);
 hipError_t hash_bitmap_launch(const HashArgs& h, hipStream_t st);
-hipError_t hash_hits_launch(const HashArgs& h, hipStream_t st);
+hipError_t hash_count_launch(const HashArgs& h, hipStream_t st);   // hit masks and counts
 // blocks that walk `loops` of the location loops (m = n / B)
 int hash_blocks(int loops, int loops_loc, int K, long long m);
 size_t hash_mask_bytes(int loops_loc, int K, long long m);   // hit masks of the slices
 
 // ---- estimation ---------------------------------------------------------------------------
-// sel (optional, 2 bytes per hit): the loops whose values the real / imaginary lower medians
-// returned (stable-rank order).  out may be device memory or the device view of pinned host
-// memory (stored in coalesced 8-byte words either way); count_copy (optional, the same
-// kinds of memory) receives *count.
-hipError_t estimate_launch(int is_fp32, const int* hits, const int* count, int capacity,
-                           const void* bins_f, int loops, int n, const int* ai_dev, int B,
-                           const double2* filter_win, Node* out, uint8_t* sel,
-                           hipStream_t st, int* count_copy = nullptr);
+// The value of every hit of a list (FP64 buckets).
+struct EstArgs {
+  const int* hits;
+  const int* count;      // device; at most `capacity` are estimated
+  int capacity;
+  const void* bins;
+  int loops, n;
+  const int* ai;
+  int B;
+  const double2* win;
+  Node* out;
+};
+hipError_t estimate_launch(const EstArgs& a, hipStream_t st);
+// The hits of the count pass in order, and their nodes.  out may be device memory or the device
+// view of pinned host memory (stored in coalesced 8-byte words either way); count_copy (optional,
+// the same kinds of memory) receives the hit count.
+struct NodeJob {
+  HashArgs h;
+  const void* bins;
+  int loops;
+  const double2* win;
+  Node* out;
+  Node* copy;            // the nodes a second time (device memory), or nullptr
+  uint8_t* sel;          // optional, 2 bytes per hit: the loops whose values the real / imaginary
+                         // lower medians returned (stable-rank order)
+  int* count_copy;
+  int blocks, block0;    // as a job of a batch
+};
+hipError_t nodes_launch(int is_fp32, const NodeJob& j, hipStream_t st);
 
 // ---- value map and its adjoint (FP64) -----------------------------------------------------
 // values[h] = Re v_{sel[2h]}(hits[h]) + i Im v_{sel[2h+1]}(hits[h]) from the bucket spectra

@@ -200,31 +200,16 @@ struct HashJob {
 };
 void hash_jobs_clear(JobTable<HashJob>& t, const HashArgs& h);
 void hash_jobs_bitmap(JobTable<HashJob>& t, const HashArgs& h);
-void hash_jobs_hits(JobTable<HashJob>& t, const HashArgs& h);
+void hash_jobs_count(JobTable<HashJob>& t, const HashArgs& h);
 hipError_t hash_clear_jobs(const JobTable<HashJob>& t, hipStream_t st);
 hipError_t hash_bitmap_jobs(const JobTable<HashJob>& t, hipStream_t st);
-hipError_t hash_hits_jobs(const JobTable<HashJob>& t, hipStream_t st);
+hipError_t hash_count_jobs(const JobTable<HashJob>& t, hipStream_t st);
 
-struct EstJob {
-  const int* hits;
-  const int* count;
-  int capacity;
-  const void* bins;
-  int loops, n;
-  const int* ai;
-  int B;
-  const double2* win;
-  Node* out;
-  Node* copy;   // the nodes a second time (device memory), or nullptr
-  uint8_t* sel;
-  int* count_copy;
-  int blocks, block0;
-};
-struct EstGroup {
+struct NodeGroup {
   int loops = 0, fp32 = 0;
-  JobTable<EstJob> t;
+  JobTable<NodeJob> t;
 };
-void estimate_jobs_add(std::vector<EstGroup>& g, int is_fp32, EstJob j);
-hipError_t estimate_jobs_launch(const std::vector<EstGroup>& g, hipStream_t st);
+void nodes_jobs_add(std::vector<NodeGroup>& g, int is_fp32, NodeJob j);
+hipError_t nodes_jobs_launch(const std::vector<NodeGroup>& g, hipStream_t st);
 
 }  // namespace sfft

@@ -613,11 +613,17 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
 // locate: reverse hash (needs the comb bitmaps and the bucket cutoffs) + estimation
 sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
                        bool marks) {
-  const sfft_params& p = P->p;
-  HIPCK(hash_hits_launch(h, st));
+  HIPCK(hash_count_launch(h, st));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[6], st));
-  HIPCK(estimate_launch(P->fp32, P->hits, h.count, P->cap, P->bins_f, p.loops, p.n, P->d_ai,
-                        p.B, P->win, d_nodes ? d_nodes : P->nodes, P->sel, st, P->cnt_copy));
+  NodeJob j = {};
+  j.h = h;
+  j.bins = P->bins_f;
+  j.loops = P->p.loops;
+  j.win = P->win;
+  j.out = d_nodes ? d_nodes : P->nodes;
+  j.sel = P->sel;
+  j.count_copy = P->cnt_copy;
+  HIPCK(nodes_launch(P->fp32, j, st));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[7], st));
   return SFFT_OK;
 }
