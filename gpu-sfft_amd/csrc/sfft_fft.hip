@@ -1412,9 +1412,10 @@ struct SlabFetch {            // filter-row loads per thread per slab (all in fl
   static constexpr int fb = sizeof(Real) == 8 ? 8 : 16;
 };
 
-// (workgroup bx of the G that share the signal's slabs)
-template <typename Real, int PMAX, int NT>
-__device__ __forceinline__ void fold_slab_body(const SlabArgs& A, uint32_t bx, uint32_t G) {
+// (workgroup bx of the G that share the signal's slabs; DV: the draws are dv's, else in memory)
+template <typename Real, int PMAX, int NT, bool DV>
+__device__ __forceinline__ void fold_slab_body(const SlabArgs& A, const DrawVals& dv, uint32_t bx,
+                                               uint32_t G) {
   using T2 = typename CT<Real>::T2;
   using V2 = typename NV<Real>::type;
   using AC = typename AccOf<Real>::A;
@@ -1538,10 +1539,11 @@ __device__ __forceinline__ void fold_slab_body(const SlabArgs& A, uint32_t bx, u
   if (bx == 0 && tid < clr.nmax) clr.maxf[tid] = 0xFFFFFFFFu;
   int av = 0, aiv = 0, ov = 0;
   if (tid < loops) {
-    av = A.a_dev[tid];
-    aiv = A.ai_dev[tid];
+    av = DV && dv.count ? dv.v[tid] : A.a_dev[tid];
+    aiv = DV && dv.count ? dv.v[loops + tid] : A.ai_dev[tid];
   }
-  if (tid < Rl) ov = A.offs[tid];
+  if (tid < Rl) ov = DV && dv.count ? dv.v[2 * loops + tid] : A.offs[tid];
+  if (DV && bx == 0 && tid < dv.count) dv.out[tid] = dv.v[tid];
   load(xa, 0);
   if (tid < loops) {
     atab[tid] = av;
@@ -1654,8 +1656,8 @@ __device__ __forceinline__ void fold_slab_body(const SlabArgs& A, uint32_t bx, u
 }
 
 template <typename Real, int PMAX, int NT>
-__global__ __launch_bounds__(NT, 4) void fold_slab_kernel(SlabArgs A) {
-  fold_slab_body<Real, PMAX, NT>(A, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(NT, 4) void fold_slab_kernel(SlabArgs A, DrawVals dv) {
+  fold_slab_body<Real, PMAX, NT, true>(A, dv, blockIdx.x, gridDim.x);
 }
 
 // the slabs of many signals: a signal's workgroups stream its slabs, as in a launch of their own
@@ -1664,7 +1666,8 @@ __global__ __launch_bounds__(NT, 4) void fold_slab_jobs_kernel(JobsDev t) {
   const SlabJob* j = job_here<SlabJob>(t);
   if (!j) return;
   const SlabArgs A = j->a;
-  fold_slab_body<Real, PMAX, NT>(A, blockIdx.x - (uint32_t)j->block0, (uint32_t)j->groups);
+  fold_slab_body<Real, PMAX, NT, false>(A, DrawVals(), blockIdx.x - (uint32_t)j->block0,
+                                        (uint32_t)j->groups);
 }
 
 int fold_rows_pitch(int B, int w) { return w / B + 1; }
@@ -1731,13 +1734,13 @@ static size_t slab_lds(int is_fp32, const SlabArgs& A) {
 
 // one workgroup per resident slot (each streams nslabs / grid slabs); any grid is correct
 template <typename Real>
-static hipError_t slab_launch(const SlabArgs& A, hipStream_t st) {
+static hipError_t slab_launch(const SlabArgs& A, const DrawVals& dv, hipStream_t st) {
   const unsigned nslabs = 1u << (A.log2B - A.log2sc);
   const size_t lds = slab_lds(sizeof(Real) == 4, A);
   return with_pmax<Real>(slab_pmax(A.P), [&](auto one, auto) {
     const int res = slab_resident(reinterpret_cast<const void*>(one), SL_NT, lds);
     const unsigned blocks = res > 0 ? std::min(nslabs, (unsigned)res) : nslabs;
-    hipLaunchKernelGGL(one, dim3(blocks), dim3(SL_NT), lds, st, A);
+    hipLaunchKernelGGL(one, dim3(blocks), dim3(SL_NT), lds, st, A, dv);
     return hipGetLastError();
   });
 }
@@ -1877,13 +1880,13 @@ hipError_t fold_columns_launch(int is_fp32, const void* x, const void* fT, void*
                                const int* a_dev, const int* ai_dev, int n, int B, int w,
                                int loops, int tiled, int by_column, int remap, void* yc,
                                const int* offs, int Rl, int W, const FoldClear& clr,
-                               hipStream_t st) {
+                               const DrawVals& dv, hipStream_t st) {
   SlabArgs A;
   const bool slab = slab_args(A, is_fp32, x, fT, bins, a_dev, ai_dev, n, B, w, loops, tiled, yc,
                               offs, Rl, W, clr);
   if (by_column) {
-    if (!slab) return hipErrorInvalidValue;
-    return is_fp32 ? slab_launch<float>(A, st) : slab_launch<double>(A, st);
+    if (!slab || (dv.count && dv.count != 2 * loops + A.Rl)) return hipErrorInvalidValue;
+    return is_fp32 ? slab_launch<float>(A, dv, st) : slab_launch<double>(A, dv, st);
   }
   const int log2B = A.log2B, log2m = A.log2m, log2sigma = A.log2sigma, T = A.T, P = A.P;
   const uint32_t mask = A.mask;

@@ -83,11 +83,12 @@ hipError_t fill_u32(void* p, uint32_t v, size_t words, hipStream_t st) {
 // residue of each location loop to -1 (the bucket selection bitmaps are rewritten whole by the
 // cutoff)
 __global__ void hash_clear_kernel(uint32_t* __restrict__ bm, size_t nbm,
-                                  uint32_t* __restrict__ maxfirst, int nmax) {
+                                  uint32_t* __restrict__ maxfirst, int nmax, DrawVals dv) {
   const size_t s = (size_t)gridDim.x * blockDim.x;
   const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   for (size_t i = i0; i < nbm; i += s) bm[i] = 0u;
   if (i0 < (size_t)nmax) maxfirst[i0] = 0xFFFFFFFFu;
+  if (i0 < (size_t)dv.count) dv.out[i0] = dv.v[i0];   // (block 0: 256 threads, 128 draws at most)
 }
 
 static int clear_blocks(const HashArgs& h) {
@@ -115,9 +116,9 @@ hipError_t hash_clear_jobs(const JobTable<HashJob>& t, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st) {
+hipError_t hash_clear_launch(const HashArgs& h, const DrawVals& dv, hipStream_t st) {
   hipLaunchKernelGGL(hash_clear_kernel, dim3(clear_blocks(h)), dim3(256), 0, st,
-                     (uint32_t*)h.bitmap, h.clear_words, (uint32_t*)h.maxfirst, h.loops_loc);
+                     (uint32_t*)h.bitmap, h.clear_words, (uint32_t*)h.maxfirst, h.loops_loc, dv);
   return hipGetLastError();
 }
 

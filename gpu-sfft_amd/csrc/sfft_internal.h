@@ -141,11 +141,22 @@ hipError_t perm_filter_launch(int is_fp32, const void* x, const void* f, void* b
 // offsets offs[] are copied too, column-major: yc[r*W + lo*m + row] =
 // x[off_r + (row*(B/sigma) + lo)*sigma] (m = n/B, sigma = n/W; needs sigma <= B).  clr: the
 // slab fold (by_column = 1) clears it first; the per-thread fold takes only an empty one.
+// dv: the draws (by_column = 1 reads them here; the per-thread fold from a_dev, ai_dev, offs).
 int fold_rows_pitch(int B, int w);
 // whether the LDS-staged slab fold takes this shape (at most 64 comb loops)
 int fold_slab_applies(int is_fp32, int n, int B, int w, int loops);
 hipError_t filter_rows_launch(int is_fp32, const void* f, void* fT, int B, int w, int tiled,
                               hipStream_t st);
+// A transform's draws as a kernel argument: v = a[loops] | ai[loops] | offsets[RLFC_loops], the
+// layout of the plan's device draws.  The transform's first kernel takes them (no upload command
+// and no wait for one in front of it) and stores them at `out` for the later ones.  count 0: they
+// are in device memory already.
+constexpr int kMaxDraws = 2 * 32 + 64;   // 32 loops, 64 comb loops
+struct DrawVals {
+  int count = 0;
+  int* out = nullptr;
+  int v[kMaxDraws];
+};
 // A clear the slab fold does before its first loads: bm[0, nbm) = 0 and maxf[0, nmax) = all
 // ones (a transform's approved-residue bitmaps and largest approved residues, which the comb
 // cutoff's bitmap kernel fills later on the same stream).  Empty: nothing is cleared.
@@ -159,7 +170,7 @@ hipError_t fold_columns_launch(int is_fp32, const void* x, const void* fT, void*
                                const int* a_dev, const int* ai_dev, int n, int B, int w,
                                int loops, int tiled, int by_column, int remap, void* yc,
                                const int* offs, int Rl, int W, const FoldClear& clr,
-                               hipStream_t st);
+                               const DrawVals& dv, hipStream_t st);
 // same fold, reading the tap values from the staging array T[l*w + i] of the streaming pass
 // batch: one persistent launch over the permute+filter of several signals
 struct PfJob {
@@ -253,7 +264,7 @@ struct HashArgs {
   int capacity;
   int* count;            // device: total hits (may exceed capacity)
 };
-hipError_t hash_clear_launch(const HashArgs& h, hipStream_t st);
+hipError_t hash_clear_launch(const HashArgs& h, const DrawVals& dv, hipStream_t st);
 hipError_t hash_bitmap_launch(const HashArgs& h, hipStream_t st);
 hipError_t hash_count_launch(const HashArgs& h, hipStream_t st);   // hit masks and counts
 // blocks that walk `loops` of the location loops (m = n / B)

@@ -377,6 +377,8 @@ extern "C" void sfft_plan_destroy(sfft_plan* P) {
   if (P->ev_join) (void)hipEventDestroy(P->ev_join);
   for (auto& e : P->ev)
     if (e) (void)hipEventDestroy(e);
+  for (auto& e : P->g_ev)
+    if (e) (void)hipEventDestroy(e);
   if (P->up_ev) (void)hipEventDestroy(P->up_ev);
   if (P->h_draws) (void)hipHostFree(P->h_draws);
   if (P->h_count) (void)hipHostFree(P->h_count);
@@ -454,31 +456,6 @@ HashArgs hash_args(const sfft_plan* P, int* d_count) {
   return h;
 }
 
-// The transform in three stage groups, each enqueued on an explicit stream (the plan's own
-// for a single transform; a batch spreads its signals over several streams and runs the
-// permute+filter of all signals as one launch).  The stage-boundary events of the profiling
-// mode are recorded by the front and back groups when `marks` is set.
-// front: bitmap clear, streaming pass (option), comb FFT (run_comb), then the comb
-// cutoff and the approved bitmaps (run_cut)
-static sfft_status run_comb(sfft_plan* P, const void* d_x, const HashArgs& h, hipStream_t st,
-                            bool marks) {
-  const sfft_params& p = P->p;
-  const int L = p.loops, Rl = p.RLFC_loops;
-  auto mark = [&](int i) -> hipError_t {
-    return (marks && P->profile) ? hipEventRecord(P->ev[i], st) : hipSuccess;
-  };
-  HIPCK(mark(0));
-  HIPCK(hash_clear_launch(h, st));
-  HIPCK(mark(1));
-  // streaming front end: one pass over x fills the tap staging array and the comb samples
-  if (P->stream)
-    HIPCK(stream_scatter_launch(P->fp32, d_x, P->taps, P->comb_y, P->d_a, P->d_offs, p.n, p.w,
-                                L, Rl, p.W_RLFC, st));
-  HIPCK(mark(2));
-  HIPCK(fft_run(comb_fft(P, d_x), st));
-  return SFFT_OK;
-}
-
 // RLFC: comb samples (gathered in pass 0, or from the streaming pass) + W-point FFT, keys of
 // |Y|^2 out of the last pass in its tile order (whole-line stores; the comb cutoff maps the
 // storage positions back to the bins)
@@ -547,24 +524,13 @@ static sfft_status run_cut(sfft_plan* P, const HashArgs& h, hipStream_t st, bool
   return SFFT_OK;
 }
 
-sfft_status run_front(sfft_plan* P, const void* d_x, const HashArgs& h, hipStream_t st,
-                      bool marks) {
-  sfft_status v = run_comb(P, d_x, h, st, marks);
-  return v != SFFT_OK ? v : run_cut(P, h, st, marks);
-}
-
 // fold: permutation + filtering of every loop into bins_t
-sfft_status run_fold(sfft_plan* P, const void* d_x, hipStream_t st, const FoldClear* clr) {
+static sfft_status run_fold(sfft_plan* P, const void* d_x, hipStream_t st) {
   const sfft_params& p = P->p;
-  if (clr && !P->columns) return SFFT_ERR_INVALID;   // only the slab fold clears
   const int tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
   if (P->stream)
     HIPCK(fold_taps_launch(P->fp32, P->taps, P->d_ft, P->bins_t, P->d_ai, p.n, p.B, p.w, p.loops,
                            tiled, st));
-  else if (P->columns)
-    HIPCK(fold_columns_launch(P->fp32, d_x, P->frows, P->bins_t, P->d_a, P->d_ai, p.n, p.B, p.w,
-                              p.loops, tiled, P->bins_perm, 1, P->comb_y, P->d_offs,
-                              p.RLFC_loops, p.W_RLFC, clr ? *clr : FoldClear(), st));
   else
     HIPCK(perm_filter_launch(P->fp32, d_x, P->d_ft, P->bins_t, P->d_ai, p.n, p.B, p.w, p.loops,
                              tiled, st));
@@ -599,7 +565,7 @@ FftLaunch bucket_fft(const sfft_plan* P) {
 }
 
 // bucket: bucket FFT + cutoff (after the fold)
-sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
+static sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
   const sfft_params& p = P->p;
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[4], st));
   HIPCK(fft_run(bucket_fft(P), st));
@@ -611,8 +577,8 @@ sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
 }
 
 // locate: reverse hash (needs the comb bitmaps and the bucket cutoffs) + estimation
-sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
-                       bool marks) {
+static sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
+                              bool marks) {
   HIPCK(hash_count_launch(h, st));
   if (marks && P->profile) HIPCK(hipEventRecord(P->ev[6], st));
   NodeJob j = {};
@@ -628,70 +594,66 @@ sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream
   return SFFT_OK;
 }
 
-sfft_status run_back(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
-                     bool marks) {
-  sfft_status v = run_bucket(P, st, marks);
-  return v != SFFT_OK ? v : run_locate(P, h, d_nodes, st, marks);
+// One transform: its first kernel (run_head), then everything after it (run_rest).  The first
+// kernel takes the draws as an argument and leaves them in device memory for the rest: no upload
+// and no gap after one in front of it (n = 2^14, k = 20, replayed: 73 -> 67 us; n = 2^20, k = 1000, FP64
+// 91 -> 85).  Column front end: the head is the slab fold, which also clears and copies the comb
+// samples.  Else it is the clear.
+static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
+                            const DrawVals& dv) {
+  const sfft_params& p = P->p;
+  auto mark = [&](int i) -> hipError_t {
+    return P->profile ? hipEventRecord(P->ev[i], P->st) : hipSuccess;
+  };
+  HIPCK(mark(0));
+  if (P->columns) {
+    FoldClear clr;
+    clr.bm = h.bitmap;
+    clr.nbm = h.clear_words;
+    clr.maxf = (uint32_t*)h.maxfirst;
+    clr.nmax = h.loops_loc;
+    const int tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
+    HIPCK(mark(1));
+    HIPCK(fold_columns_launch(P->fp32, d_x, P->frows, P->bins_t, P->d_a, P->d_ai, p.n, p.B, p.w,
+                              p.loops, tiled, P->bins_perm, 1, P->comb_y, P->d_offs,
+                              p.RLFC_loops, p.W_RLFC, clr, dv, P->st));
+    HIPCK(mark(2));
+  } else {
+    HIPCK(hash_clear_launch(h, dv, P->st));
+    HIPCK(mark(1));
+  }
+  return SFFT_OK;
 }
 
-// Column front end: the fold also copies the comb samples, so it runs first (and does the
-// transform's clear of the approved-residue bitmaps on its way: no clear launch); then the
-// comb chain (comb FFT from the copied samples, cutoff, bitmaps) on the plan stream and the
-// bucket chain (bucket FFT, cutoff) on the second stream, joined before the reverse hash.  The
-// comb FFT is enqueued before the bucket chain: in a captured graph it is then the fold's
-// first dependent, which the graph replay keeps on the fold's queue, so the longer chain
-// crosses no queue.  Profiling runs everything serially; its "clear" interval is then empty,
-// its "streaming pass" interval is the fold (with the comb copy) and its "fold" interval is
-// empty.
-static sfft_status run_all_columns(sfft_plan* P, const void* d_x, const HashArgs& h,
-                                   Node* d_nodes) {
+// After the head two concurrent chains, joined before the reverse hash: the comb chain (comb FFT,
+// cutoff, bitmaps) on the plan stream and the bucket chain (permute+filter unless the head was
+// the slab fold, bucket FFT, cutoff) on a second stream, so that the latency-bound kernels of
+// one chain fill the gaps of the other's.  Column front end: the comb FFT is enqueued before the
+// bucket chain, so that a captured graph's first root, which the replay keeps on the launching
+// queue, starts the longer chain.  The gathering front end forks after its comb FFT (beside which
+// its permute+filter's gathers lose).  Profiling (and the streaming front end, whose pass feeds
+// the fold) runs everything serially on the plan stream; with the columns the profile's
+// "clear" interval is empty, its "streaming pass" interval is the fold (with the comb copy) and
+// its "fold" interval is empty.
+static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes) {
+  const sfft_params& p = P->p;
   sfft_status v;
-  const bool prof = P->profile != 0;
-  auto mark = [&](int i) -> hipError_t {
-    return prof ? hipEventRecord(P->ev[i], P->st) : hipSuccess;
-  };
-  FoldClear clr;
-  clr.bm = h.bitmap;
-  clr.nbm = h.clear_words;
-  clr.maxf = (uint32_t*)h.maxfirst;
-  clr.nmax = h.loops_loc;
-  HIPCK(mark(0));
-  HIPCK(mark(1));
-  if ((v = run_fold(P, d_x, P->st, &clr)) != SFFT_OK) return v;
-  HIPCK(mark(2));
-  if (prof) {
+  if (P->stream)   // one pass over x fills the tap staging array and the comb samples
+    HIPCK(stream_scatter_launch(P->fp32, d_x, P->taps, P->comb_y, P->d_a, P->d_offs, p.n, p.w,
+                                p.loops, p.RLFC_loops, p.W_RLFC, P->st));
+  if (P->profile && !P->columns) HIPCK(hipEventRecord(P->ev[2], P->st));
+  if (P->profile || P->stream) {
     HIPCK(fft_run(comb_fft(P, d_x), P->st));
     if ((v = run_cut(P, h, P->st, true)) != SFFT_OK) return v;
+    if (!P->columns && (v = run_fold(P, d_x, P->st)) != SFFT_OK) return v;
     if ((v = run_bucket(P, P->st, true)) != SFFT_OK) return v;
     return run_locate(P, h, d_nodes, P->st, true);
   }
-  HIPCK(hipEventRecord(P->ev_fork, P->st));
+  if (P->columns) HIPCK(hipEventRecord(P->ev_fork, P->st));
   HIPCK(fft_run(comb_fft(P, d_x), P->st));
+  if (!P->columns) HIPCK(hipEventRecord(P->ev_fork, P->st));
   HIPCK(hipStreamWaitEvent(P->st2, P->ev_fork, 0));
-  if ((v = run_bucket(P, P->st2, false)) != SFFT_OK) return v;
-  HIPCK(hipEventRecord(P->ev_join, P->st2));
-  if ((v = run_cut(P, h, P->st, false)) != SFFT_OK) return v;
-  HIPCK(hipStreamWaitEvent(P->st, P->ev_join, 0));
-  return run_locate(P, h, d_nodes, P->st, false);
-}
-
-// One transform as two concurrent chains joined before the reverse hash: the comb chain
-// (clear, comb FFT, cutoff, bitmaps) on the plan stream and the bucket chain (permute+filter,
-// bucket FFT, cutoff) on a second stream, so the latency-bound kernels of one chain fill the
-// gaps of the other's gathers.  Profiling (and the streaming front end, whose pass feeds the
-// fold) runs everything serially on the plan stream.
-static sfft_status run_all(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes) {
-  sfft_status v;
-  if (P->columns) return run_all_columns(P, d_x, h, d_nodes);
-  if (P->profile || P->stream) {   // (the streaming pass feeds the fold: one chain)
-    if ((v = run_front(P, d_x, h, P->st, true)) != SFFT_OK) return v;
-    if ((v = run_fold(P, d_x, P->st)) != SFFT_OK) return v;
-    return run_back(P, h, d_nodes, P->st, true);
-  }
-  if ((v = run_comb(P, d_x, h, P->st, false)) != SFFT_OK) return v;
-  HIPCK(hipEventRecord(P->ev_fork, P->st));
-  HIPCK(hipStreamWaitEvent(P->st2, P->ev_fork, 0));
-  if ((v = run_fold(P, d_x, P->st2)) != SFFT_OK) return v;
+  if (!P->columns && (v = run_fold(P, d_x, P->st2)) != SFFT_OK) return v;
   if ((v = run_bucket(P, P->st2, false)) != SFFT_OK) return v;
   HIPCK(hipEventRecord(P->ev_join, P->st2));
   if ((v = run_cut(P, h, P->st, false)) != SFFT_OK) return v;
@@ -700,57 +662,111 @@ static sfft_status run_all(sfft_plan* P, const void* d_x, const HashArgs& h, Nod
 }
 
 static void drop_plan_graph(sfft_plan* P) {
-  if (P->gexec) (void)hipGraphExecDestroy(P->gexec);
+  for (int k = 0; k < 2; ++k) {
+    if (P->gexec[k]) (void)hipGraphExecDestroy(P->gexec[k]);
+    P->gexec[k] = nullptr;
+  }
   if (P->graph) (void)hipGraphDestroy(P->graph);
-  P->gexec = nullptr;
   P->graph = nullptr;
+}
+
+// Graph mode launches the kernels one by one where the head is a slab fold of 64 MB and more: it
+// runs long enough for the launches behind it to be enqueued meanwhile, and the chains then
+// start with less between them than a replay's nodes (n = 2^27, k = 16000, replayed -> launched:
+// FP64 814 -> 790 us, FP32 466 -> 457; n = 2^24 FP32 134 either way; n = 2^20 FP64 85 replayed,
+// 92 launched).
+static bool graph_as_eager(const sfft_plan* P) {
+  return P->columns && (size_t)P->p.n * (P->fp32 ? 8 : 16) >= ((size_t)64 << 20);
+}
+
+static sfft_status capture(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes,
+                           const DrawVals& dv) {
+  HIPCK(hipStreamBeginCapture(P->st, hipStreamCaptureModeThreadLocal));
+  sfft_status v = run_head(P, d_x, h, dv);
+  if (v == SFFT_OK) v = run_rest(P, d_x, h, d_nodes);
+  hipGraph_t g = nullptr;
+  const hipError_t e = hipStreamEndCapture(P->st, &g);
+  P->graph = g;
+  if (v != SFFT_OK) return v;
+  size_t roots = 1;   // the head is the only kernel nothing precedes
+  if (e != hipSuccess || hipGraphGetRootNodes(g, &P->g_head, &roots) != hipSuccess ||
+      roots != 1 || hipGraphKernelNodeGetParams(P->g_head, &P->g_head_params) != hipSuccess)
+    return SFFT_ERR_HIP;
+  return SFFT_OK;
+}
+
+// Replays the captured transform with these draws.  An asynchronous caller may have launched it
+// before and not waited: its two executables take turns, and one is written only when its last
+// launch is done.
+static sfft_status replay(sfft_plan* P, DrawVals& dv, bool async) {
+  const int k = async ? P->g_next : 0;
+  if (async) P->g_next ^= 1;
+  if (P->g_pending[k]) HIPCK(hipEventSynchronize(P->g_ev[k]));
+  P->g_pending[k] = 0;
+  if (!P->gexec[k])
+    HIPCK(hipGraphInstantiate(&P->gexec[k], P->graph, nullptr, nullptr, 0));
+  // the draws are the head's last argument (fold_slab_kernel's second, hash_clear_kernel's fifth)
+  void* args[5];
+  const int n = P->columns ? 2 : 5;
+  for (int i = 0; i < n - 1; ++i) args[i] = P->g_head_params.kernelParams[i];
+  args[n - 1] = &dv;
+  hipKernelNodeParams kp = P->g_head_params;
+  kp.kernelParams = args;
+  HIPCK(hipGraphExecKernelNodeSetParams(P->gexec[k], P->g_head, &kp));
+  HIPCK(hipGraphLaunch(P->gexec[k], P->st));
+  if (async) {
+    if (!P->g_ev[k]) HIPCK(hipEventCreateWithFlags(&P->g_ev[k], hipEventDisableTiming));
+    HIPCK(hipEventRecord(P->g_ev[k], P->st));
+    P->g_pending[k] = 1;
+  }
+  return SFFT_OK;
 }
 
 // One transform enqueued on the plan stream: nodes to d_nodes (device memory, or the device
 // view of pinned host memory; nullptr: the plan's buffer), the count to d_count (nullptr: the
 // plan's) and, when cnt_copy is set, also to *cnt_copy.
 static sfft_status enqueue(sfft_plan* P, const void* d_x, const sfft_draws* dr, Node* d_nodes,
-                           int* d_count, int* cnt_copy) {
+                           int* d_count, int* cnt_copy, bool async) {
   if (!P || !d_x) return SFFT_ERR_INVALID;
   if (!P->has_filter) return SFFT_ERR_NO_FILTER;
-  sfft_status v = upload_draws(P, dr);
+  sfft_status v = draws_check(P, dr);
   if (v != SFFT_OK) return v;
   const HashArgs h = hash_args(P, d_count);
+  const int L = P->p.loops, Rl = P->p.RLFC_loops;
+  DrawVals dv;
+  dv.count = 2 * L + Rl;
+  dv.out = P->d_a;
+  memcpy(dv.v, dr->a, (size_t)L * 4);
+  memcpy(dv.v + L, dr->ai, (size_t)L * 4);
+  memcpy(dv.v + 2 * L, dr->offsets, (size_t)Rl * 4);
   P->cnt_copy = cnt_copy;   // read by run_locate while this transform is enqueued / captured
   struct Reset {
     sfft_plan* P;
     ~Reset() { P->cnt_copy = nullptr; }
   } reset{P};
-  if (!P->use_graph || P->profile) return run_all(P, d_x, h, d_nodes);   // eager
-  if (P->gexec && (P->g_x != d_x || P->g_nodes != d_nodes || P->g_count != d_count ||
+  if (!P->use_graph || P->profile || graph_as_eager(P)) {   // eager
+    v = run_head(P, d_x, h, dv);
+    return v != SFFT_OK ? v : run_rest(P, d_x, h, d_nodes);
+  }
+  if (P->graph && (P->g_x != d_x || P->g_nodes != d_nodes || P->g_count != d_count ||
                    P->g_cnt_copy != cnt_copy))
     drop_plan_graph(P);
-  if (!P->gexec) {
-    HIPCK(hipStreamBeginCapture(P->st, hipStreamCaptureModeThreadLocal));
-    v = run_all(P, d_x, h, d_nodes);
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(P->st, &g);
-    if (v != SFFT_OK || e != hipSuccess) {
-      if (g) (void)hipGraphDestroy(g);
-      return v != SFFT_OK ? v : SFFT_ERR_HIP;
-    }
-    P->graph = g;
-    if (hipGraphInstantiate(&P->gexec, g, nullptr, nullptr, 0) != hipSuccess) {
+  if (!P->graph) {
+    if ((v = capture(P, d_x, h, d_nodes, dv)) != SFFT_OK) {
       drop_plan_graph(P);
-      return SFFT_ERR_HIP;
+      return v;
     }
     P->g_x = d_x;
     P->g_nodes = d_nodes;
     P->g_count = d_count;
     P->g_cnt_copy = cnt_copy;
   }
-  HIPCK(hipGraphLaunch(P->gexec, P->st));
-  return SFFT_OK;
+  return replay(P, dv, async);
 }
 
 extern "C" sfft_status sfft_execute_async(sfft_plan* P, const void* d_x, const sfft_draws* dr,
                                           Node* d_nodes, int* d_count) {
-  return enqueue(P, d_x, dr, d_nodes, d_count, nullptr);
+  return enqueue(P, d_x, dr, d_nodes, d_count, nullptr, true);
 }
 
 // The device view of h when h is pinned host memory with room for `bytes` from h on, else
@@ -783,8 +799,8 @@ void* PinnedRange::view(void* h, size_t bytes) {
   return size - off >= bytes ? dev + off : nullptr;
 }
 
-// Graph mode: the transform's launch sequence is captured once and replayed (the draws are
-// uploaded before each replay, outside the graph).  A plan created without a stream gets a
+// Graph mode: the transform's launch sequence is captured once and replayed (each replay's draws
+// are set in its first kernel's arguments).  A plan created without a stream gets a
 // stream of its own for this (the legacy default stream cannot be captured).
 extern "C" sfft_status sfft_plan_set_graph(sfft_plan* P, int on) {
   if (!P) return SFFT_ERR_INVALID;
@@ -929,7 +945,7 @@ extern "C" sfft_status sfft_execute(sfft_plan* P, const void* d_x, const sfft_dr
   Node* zc =
       h_nodes ? (Node*)PinnedRange().view(h_nodes, (size_t)P->cap * sizeof(Node)) : nullptr;
   if (zc) {
-    sfft_status s = enqueue(P, d_x, dr, zc, P->count, P->h_count_dev);
+    sfft_status s = enqueue(P, d_x, dr, zc, P->count, P->h_count_dev, false);
     if (s != SFFT_OK) return s;
     HIPCK(hipStreamSynchronize(P->st));
     const int cnt = *(volatile int*)P->h_count;
@@ -937,7 +953,7 @@ extern "C" sfft_status sfft_execute(sfft_plan* P, const void* d_x, const sfft_dr
     if (h_count) *h_count = cnt;
     return cnt > P->cap ? SFFT_ERR_HIT_OVERFLOW : SFFT_OK;
   }
-  sfft_status s = enqueue(P, d_x, dr, P->nodes, P->count, nullptr);
+  sfft_status s = enqueue(P, d_x, dr, P->nodes, P->count, nullptr, false);
   if (s != SFFT_OK) return s;
   // the count and, speculatively, as many nodes as the previous transform had plus 1/32 go
   // back in one round trip; the rest (if the count grew past that) in a second one

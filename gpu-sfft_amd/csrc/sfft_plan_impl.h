@@ -79,7 +79,13 @@ struct sfft_plan {
   int use_graph = 0;
   int own_st = 0;
   hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  // two executables of it: a replay's draws are set in one while the other may still run
+  hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  hipEvent_t g_ev[2] = {nullptr, nullptr};  // after the last asynchronous launch of each
+  int g_pending[2] = {0, 0};
+  int g_next = 0;
+  hipGraphNode_t g_head = nullptr;          // the first kernel, which takes the draws
+  hipKernelNodeParams g_head_params = {};
   const void* g_x = nullptr;
   Node* g_nodes = nullptr;
   int* g_count = nullptr;
@@ -109,14 +115,3 @@ struct PinnedRange {
   size_t size = 0;
   void* view(void* h, size_t bytes);
 };
-// the transform in three stage groups on an explicit stream (marks: record the plan's
-// profiling events)
-sfft_status run_front(sfft_plan* P, const void* d_x, const HashArgs& h, hipStream_t st,
-                      bool marks);
-// clr: cleared by the slab fold first (column front end only; nullptr: nothing)
-sfft_status run_fold(sfft_plan* P, const void* d_x, hipStream_t st,
-                     const FoldClear* clr = nullptr);
-sfft_status run_back(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st, bool marks);
-sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks);
-sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
-                       bool marks);
