@@ -449,8 +449,9 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
       for (int grid : grids) {
         float ms = 0;
         v = time_ms(b, reps, [&]() -> sfft_status {
-          HIPCK(perm_filter_batch_launch(b->fp32, b->d_jobs, b->count, b->total_items, b->lpt,
-                                         b->nt, grid, b->st));
+          // (only the gathering signals have a job)
+          HIPCK(perm_filter_batch_launch(b->fp32, b->d_jobs, (int)b->jobs.size(),
+                                         b->total_items, b->lpt, b->nt, grid, b->st));
           return SFFT_OK;
         }, &ms);
         if (v != SFFT_OK) return v;

@@ -337,13 +337,14 @@ def batch_workload(count, seed, q_range=(18, 24), k_range=(50, 4000), Bcst=1.0, 
 
 
 class Batch:
-    """Several signals of uneven n and k transformed together (sfft_batch_*): one persistent
-    permute+filter launch for all signals, the other stages on worker streams, optional
-    hipGraph capture and an autotuner over bit-equivalent launch shapes."""
+    """Several signals of uneven n and k transformed together (sfft_batch_*): every stage of all
+    signals in one launch, optional hipGraph capture and an autotuner over bit-equivalent launch
+    shapes."""
 
     def __init__(self, params_list, precision="fp32", fold_mode=FOLD_REFERENCE,
                  front_end="gather"):
-        """front_end: "gather" or "auto" (the batch always gathers); others are refused."""
+        """front_end: "gather" (every signal), or "auto" (the column fold where it applies, else
+        gathers); others are refused."""
         self.params = [dict(p) for p in params_list]
         self.count = len(self.params)
         self.fp32 = precision == "fp32"

@@ -112,3 +112,30 @@ def test_batch_device_nodes_beside_pinned_ones(S):
         host = pinned.numpy().view(NODE)[i * 524288:i * 524288 + counts[i]]
         assert dev.tobytes() == host.tobytes()
     b.close()
+
+
+def test_tune_of_a_batch_that_gathers_and_folds(S):
+    """the tuner times the gathering signals' launch, whose table holds only them"""
+    import torch
+    prms = [params(CONFIGS[0]), dict(params(CONFIGS[0]), B=64, w=64 * 40 + 7, B_thresh=20),
+            params(CONFIGS[3])]
+    rng = np.random.default_rng(9)
+    xs, taps, dr, b = [], [], [], S.Batch(prms, "fp32", front_end="auto")
+    fronts = [S.lib.sfft_plan_front_end(S.lib.sfft_batch_plan(b._h, i)) for i in range(3)]
+    assert fronts.count(1) == 1 and fronts.count(3) == 2
+    want = []
+    for i, p in enumerate(prms):
+        x, _, _ = sparse_signal(p["n"], p["k"], 80 + i, snr_db=30.0)
+        ft = rng.standard_normal(p["w"]) + 1j * rng.standard_normal(p["w"])
+        win = 1.0 + rng.random(p["n"] // p["B"]) + 0j
+        xs.append(torch.from_numpy(x.astype(np.complex64)).cuda())
+        taps.append(torch.from_numpy(ft.astype(np.complex64)).cuda())
+        dr.append(draws(p["n"], p["loops"], p["RLFC_loops"], p["W_RLFC"], 90 + i))
+        b.set_filter(i, taps[i], win)
+        plan = S.Plan(p, "fp32")
+        plan.set_filter(taps[i], win)
+        want.append(plan.execute(xs[i], *dr[i]))
+    b.tune(xs, dr, reps=1)
+    for (nodes, cnt), (wn, wc) in zip(b.execute(xs, dr), want):
+        assert cnt == wc and nodes.tobytes() == wn.tobytes()
+    b.close()
