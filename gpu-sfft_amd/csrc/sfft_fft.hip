@@ -981,6 +981,110 @@ hipError_t fft_run(const FftLaunch& L, hipStream_t st) {
   });
 }
 
+// ---- the comb FFT and the bucket FFTs of a short transform, pass by pass in one launch --------
+// Where both FFTs run quarter tiles a pass is a few workgroups and some 5 us, most of it the
+// launch: side by side on two streams they cost two launches per pass and the events that fork
+// and join the streams.
+struct OnePass {
+  PassArgs a;
+  int load, store, tw, tiles, batch;
+  int blocks() const { return tiles * batch; }
+};
+
+// (half the waves of a pass alone: both bodies' tiles are in the workgroup's LDS)
+template <typename Real, int LA, int SA, int LB, int SB, int TW>
+__global__ __launch_bounds__((Tile<Real, LA>::nt), (Tile<Real, LA>::waves / 2)) void
+fft_pair_kernel(PassArgs A, PassArgs B, int tiles_a, int blocks_a, int tiles_b) {
+  static_assert(Tile<Real, LA>::nt == Tile<Real, LB>::nt, "one block size");
+  const int i = blockIdx.x;
+  if (i < blocks_a) {
+    fft_pass_body<Real, LA, SA, TW>(A, i % tiles_a, tiles_a, i / tiles_a);
+  } else {
+    const int k = i - blocks_a;
+    fft_pass_body<Real, LB, SB, TW>(B, k % tiles_b, tiles_b, k / tiles_b);
+  }
+}
+
+template <typename Real, int LA, int SA, int LB, int SB, int TW>
+static hipError_t pair_go(const OnePass& a, const OnePass& b, hipStream_t st) {
+  hipLaunchKernelGGL((fft_pair_kernel<Real, LA | kSmallTile, SA, LB | kSmallTile, SB, TW>),
+                     dim3(a.blocks() + b.blocks()), dim3(Tile<Real, LA | kSmallTile>::nt), 0, st,
+                     a.a, b.a, a.tiles, a.blocks(), b.tiles);
+  return hipGetLastError();
+}
+
+// first passes: the last ones too (keys out) or not
+template <typename Real, int LA>
+static hipError_t pair_first(const OnePass& a, const OnePass& b, hipStream_t st) {
+  const bool ka = a.store == kStoreKeys, kb = b.store == kStoreBoth;
+  if (ka && kb) return pair_go<Real, LA, kStoreKeys, kLoadPerm, kStoreBoth, kTwNone>(a, b, st);
+  if (ka) return pair_go<Real, LA, kStoreKeys, kLoadPerm, kStoreCplx, kTwNone>(a, b, st);
+  if (kb) return pair_go<Real, LA, kStoreCplx, kLoadPerm, kStoreBoth, kTwNone>(a, b, st);
+  return pair_go<Real, LA, kStoreCplx, kLoadPerm, kStoreCplx, kTwNone>(a, b, st);
+}
+
+template <typename Real>
+static hipError_t pair_pass(const OnePass& a, const OnePass& b, hipStream_t st) {
+  if (a.load == kLoadCombRows) return pair_first<Real, kLoadCombRows>(a, b, st);
+  if (a.load == kLoadCombRowsG) return pair_first<Real, kLoadCombRowsG>(a, b, st);
+  if (a.tw == kTwSplit)
+    return pair_go<Real, kLoadPlain, kStoreKeys, kLoadPlain, kStoreBoth, kTwSplit>(a, b, st);
+  return pair_go<Real, kLoadPlain, kStoreKeys, kLoadPlain, kStoreBoth, kTwDirect>(a, b, st);
+}
+
+// the passes of L (two at most), or fewer than L has where one of them has no quarter tile
+static int short_passes(const FftLaunch& L, OnePass* out) {
+  int n = 0;
+  if (L.tab->npass > 2) return -1;
+  const hipError_t e = each_pass(L, [&](int, const PassArgs& A, int load, int store, int tw,
+                                        int tiles) {
+    if (!A.small_tile) return hipErrorNotSupported;
+    out[n++] = OnePass{A, load, store, tw, tiles, L.batch};
+    return hipSuccess;
+  });
+  return e == hipSuccess ? n : -1;
+}
+
+// a comb FFT of the copied comb rows (keys out) and the bucket FFTs of column-ordered sums
+// (spectra and keys out), every pass of both in quarter tiles
+static bool pair_passes(const FftLaunch& comb, const FftLaunch& bucket, OnePass (&a)[2],
+                        OnePass (&b)[2], int& na, int& nb) {
+  if (comb.load != kLoadCombRows || comb.store != kStoreKeys || bucket.load != kLoadPerm ||
+      bucket.store != kStoreBoth || comb.tab->is_fp32 != bucket.tab->is_fp32)
+    return false;
+  na = short_passes(comb, a);
+  nb = short_passes(bucket, b);
+  return na > 0 && nb > 0;
+}
+
+bool fft_pair_applies(const FftLaunch& comb, const FftLaunch& bucket) {
+  OnePass a[2], b[2];
+  int na, nb;
+  return pair_passes(comb, bucket, a, b, na, nb);
+}
+
+hipError_t fft_run_pair(const FftLaunch& comb, const FftLaunch& bucket, hipStream_t st) {
+  OnePass a[2], b[2];
+  int na, nb;
+  if (!pair_passes(comb, bucket, a, b, na, nb)) return hipErrorInvalidValue;
+  const int fp32 = comb.tab->is_fp32;
+  auto one = [&](const OnePass& p) {
+    return fp32 ? dispatch_pass<float>(p.a, p.load, p.store, p.tw, p.tiles, p.batch, st)
+                : dispatch_pass<double>(p.a, p.load, p.store, p.tw, p.tiles, p.batch, st);
+  };
+  for (int p = 0; p < 2; ++p) {
+    hipError_t e = hipSuccess;
+    if (p < na && p < nb && a[p].tw == b[p].tw) {
+      e = fp32 ? pair_pass<float>(a[p], b[p], st) : pair_pass<double>(a[p], b[p], st);
+    } else {
+      if (p < na) e = one(a[p]);
+      if (e == hipSuccess && p < nb) e = one(b[p]);
+    }
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t fft_jobs_add(std::vector<FftGroup>& g, const FftLaunch& L) {
   const int fp32 = L.tab->is_fp32;
   return each_pass(L, [&](int p, const PassArgs& A, int load, int store, int tw, int tiles) {

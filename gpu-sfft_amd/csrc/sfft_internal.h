@@ -109,6 +109,10 @@ struct FftLaunch {
   double scale = 1.0;            // kStoreHead
 };
 hipError_t fft_run(const FftLaunch& L, hipStream_t st);
+// the comb FFT (kLoadCombRows, keys) and the bucket FFTs (kLoadPerm, both) of a short transform,
+// their passes in the same launches; only where fft_pair_applies
+bool fft_pair_applies(const FftLaunch& comb, const FftLaunch& bucket);
+hipError_t fft_run_pair(const FftLaunch& comb, const FftLaunch& bucket, hipStream_t st);
 
 // Where the keys of an FFT run with keys_tiled land: the last pass of a multi-pass FFT stores
 // its tile's keys contiguously (whole-line stores), so storage position s holds the key of
@@ -241,6 +245,23 @@ hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int 
                        unsigned* bits = nullptr, const KeyMap* map = nullptr,
                        const uint16_t* digits = nullptr, const SelMark* mark = nullptr,
                        const unsigned* hist = nullptr);
+
+// two selects of segments that one workgroup does (the arguments of select_topk, in order; the
+// first as the comb cutoff: unordered, marking; the second as the bucket cutoff: ordered), one
+// launch
+struct SelectArgs {
+  const void* keys;
+  long long seg_stride;
+  int N, K, segs;
+  int* out;
+  const SelectWork* w;
+  unsigned* bits;
+  const KeyMap* map;
+  const uint16_t* digits;
+  const SelMark* mark;
+};
+hipError_t select_pair(int is_fp32, const SelectArgs& comb, const SelectArgs& bucket,
+                       hipStream_t st);
 
 // ---- reverse hash (bitmap of approved residues, deterministic hit list) -----------------
 struct HashArgs {

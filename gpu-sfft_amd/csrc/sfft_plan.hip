@@ -576,6 +576,28 @@ static sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
   return SFFT_OK;
 }
 
+// Whether a short transform's comb and bucket stages share their launches: the column front end,
+// FFTs in quarter tiles, and both cutoffs of segments that one workgroup does.
+static bool paired(const sfft_plan* P) {
+  return P->bins_perm && select_in_block(P->p.W_RLFC) && select_in_block(P->p.B) &&
+         fft_pair_applies(comb_fft(P, nullptr), bucket_fft(P));
+}
+
+// both FFTs, then both cutoffs (with the approved-residue bitmaps)
+static sfft_status run_pair(sfft_plan* P, const HashArgs& h, hipStream_t st) {
+  const sfft_params& p = P->p;
+  const FftLaunch cf = comb_fft(P, nullptr);
+  HIPCK(fft_run_pair(cf, bucket_fft(P), st));
+  const KeyMap km = fft_keys_map(cf);
+  const SelMark mk = comb_mark(h);
+  const SelectArgs comb = {P->comb_keys, p.W_RLFC, p.W_RLFC, p.B_thresh, p.RLFC_loops, P->J2,
+                           &P->selW, nullptr, &km, P->comb_digits, &mk};
+  const SelectArgs bucket = {P->bkeys, p.B, p.B, p.B_thresh, p.loops_loc, P->J, &P->selB,
+                             P->jsel, nullptr, P->bucket_digits, nullptr};
+  HIPCK(select_pair(P->fp32, comb, bucket, st));
+  return SFFT_OK;
+}
+
 // locate: reverse hash (needs the comb bitmaps and the bucket cutoffs) + estimation
 static sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
                               bool marks) {
@@ -648,6 +670,10 @@ static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, No
     if (!P->columns && (v = run_fold(P, d_x, P->st)) != SFFT_OK) return v;
     if ((v = run_bucket(P, P->st, true)) != SFFT_OK) return v;
     return run_locate(P, h, d_nodes, P->st, true);
+  }
+  if (paired(P)) {
+    if ((v = run_pair(P, h, P->st)) != SFFT_OK) return v;
+    return run_locate(P, h, d_nodes, P->st, false);
   }
   if (P->columns) HIPCK(hipEventRecord(P->ev_fork, P->st));
   HIPCK(fft_run(comb_fft(P, d_x), P->st));

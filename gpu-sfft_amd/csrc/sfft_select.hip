@@ -732,23 +732,39 @@ __device__ __forceinline__ void sb_pick(const unsigned* h, int nb, int r, int* s
   __syncthreads();
 }
 
+// a workgroup's LDS
+template <typename K>
+struct SelBlockLds {
+  using CT = typename CompOf<K>::type;
+  unsigned h[SEL_BINS];
+  K lkey[SB_CAP];
+  int lpos[SB_CAP];
+  unsigned picked[SEL_NT];   // candidates selected, as their owners' bits
+  CT rkey[SB_RANK];
+  int rpos[SB_RANK];
+  int sh[16];
+  int s_pick[3];
+  int s_nc;
+};
+
 template <typename K, int PER>
 __device__ __forceinline__ void sel_block_body(const K* __restrict__ keys, long long seg_stride,
                                                int N, int Ksel, int* __restrict__ out,
                                                unsigned* __restrict__ bits, KeyMap km,
                                                const uint16_t* __restrict__ digits, int vec,
-                                               const SelMark& mark, int seg) {
+                                               const SelMark& mark, int seg,
+                                               SelBlockLds<K>& lds) {
   using CT = typename CompOf<K>::type;
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  __shared__ unsigned h[SEL_BINS];
-  __shared__ K lkey[SB_CAP];
-  __shared__ int lpos[SB_CAP];
-  __shared__ unsigned picked[SEL_NT];   // candidates selected, as their owners' bits
-  __shared__ CT rkey[SB_RANK];
-  __shared__ int rpos[SB_RANK];
-  __shared__ int sh[16];
-  __shared__ int s_pick[3];
-  __shared__ int s_nc;
+  auto& h = lds.h;
+  auto& lkey = lds.lkey;
+  auto& lpos = lds.lpos;
+  auto& picked = lds.picked;
+  auto& rkey = lds.rkey;
+  auto& rpos = lds.rpos;
+  auto& sh = lds.sh;
+  auto& s_pick = lds.s_pick;
+  int& s_nc = lds.s_nc;
   const int tid = threadIdx.x;
   const int IB = index_bits(N), TB = KeyBits<K>::KB + IB;
   const K* kp = keys + (long long)seg * seg_stride;
@@ -1032,8 +1048,37 @@ __global__ __launch_bounds__(SEL_NT) void sel_block_kernel(From f) {
   SelJob j;
   int bx, seg;
   if (!f.get(j, bx, seg, 1)) return;
+  __shared__ SelBlockLds<K> lds;
   sel_block_body<K, PER>((const K*)j.keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits,
-                         j.vec, j.mark, seg);
+                         j.vec, j.mark, seg, lds);
+}
+
+// elements per thread of the one-workgroup select, as an index into 8, 16, 32
+__host__ __device__ __forceinline__ int block_variant(int N) {
+  return N <= 8 * SEL_NT ? 0 : N <= 16 * SEL_NT ? 1 : 2;
+}
+
+// two selects, a workgroup per segment of either
+template <typename K>
+__global__ __launch_bounds__(SEL_NT) void sel_pair_kernel(SelJob a, SelJob b) {
+  __shared__ SelBlockLds<K> lds;
+  const bool first = (int)blockIdx.x < a.segs;
+  const SelJob& j = first ? a : b;
+  const int seg = first ? (int)blockIdx.x : (int)blockIdx.x - a.segs;
+  const K* keys = (const K*)j.keys;
+  switch (block_variant(j.N)) {
+    case 0:
+      sel_block_body<K, 8>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
+                           j.mark, seg, lds);
+      break;
+    case 1:
+      sel_block_body<K, 16>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
+                            j.mark, seg, lds);
+      break;
+    default:
+      sel_block_body<K, 32>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
+                            j.mark, seg, lds);
+  }
 }
 
 // Up to 32768 keys one workgroup beats the chain of launches, in both precisions; at 65536 its
@@ -1089,9 +1134,6 @@ static hipError_t select_job(SelJob& j, const void* keys, long long seg_stride, 
   return hipSuccess;
 }
 
-// elements per thread of the one-workgroup select, as an index into 8, 16, 32
-static int block_variant(int N) { return N <= 8 * SEL_NT ? 0 : N <= 16 * SEL_NT ? 1 : 2; }
-
 template <typename K, typename From>
 static void block_go(int variant, const From& f, dim3 grid, hipStream_t st) {
   if (variant == 0)
@@ -1134,6 +1176,26 @@ hipError_t select_topk(int is_fp32, const void* keys, long long seg_stride, int 
                                   map, digits, mark, hist);
   if (e != hipSuccess) return e;
   return is_fp32 ? select_one<unsigned int>(j, st) : select_one<unsigned long long>(j, st);
+}
+
+hipError_t select_pair(int is_fp32, const SelectArgs& comb, const SelectArgs& bucket,
+                       hipStream_t st) {
+  SelJob j[2];
+  const SelectArgs* args[2] = {&comb, &bucket};
+  for (int i = 0; i < 2; ++i) {
+    const SelectArgs& s = *args[i];
+    if (!select_in_block(s.N)) return hipErrorInvalidValue;
+    const hipError_t e = select_job(j[i], s.keys, s.seg_stride, s.N, s.K, s.segs, s.out, i,
+                                    *s.w, s.bits, s.map, s.digits, s.mark, nullptr);
+    if (e != hipSuccess) return e;
+  }
+  const dim3 grid(comb.segs + bucket.segs);
+  if (is_fp32)
+    hipLaunchKernelGGL((sel_pair_kernel<unsigned int>), grid, dim3(SEL_NT), 0, st, j[0], j[1]);
+  else
+    hipLaunchKernelGGL((sel_pair_kernel<unsigned long long>), grid, dim3(SEL_NT), 0, st, j[0],
+                       j[1]);
+  return hipGetLastError();
 }
 
 hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long seg_stride, int N,
