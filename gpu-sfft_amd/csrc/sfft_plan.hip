@@ -577,7 +577,10 @@ static sfft_status run_bucket(sfft_plan* P, hipStream_t st, bool marks) {
 }
 
 // Whether a short transform's comb and bucket stages share their launches: the column front end,
-// FFTs in quarter tiles, and both cutoffs of segments that one workgroup does.
+// FFTs in quarter tiles, and both cutoffs of segments that one workgroup does.  Each stage is then
+// a few workgroups and some 5 us, so that the second stream's launches and the events around them
+// cost more than they overlap (apart -> shared, eager: n = 2^14, k = 20, FP64 94 -> 58 us;
+// n = 2^20, k = 1000, FP32 77 -> 61).
 static bool paired(const sfft_plan* P) {
   return P->bins_perm && select_in_block(P->p.W_RLFC) && select_in_block(P->p.B) &&
          fft_pair_applies(comb_fft(P, nullptr), bucket_fft(P));
@@ -696,12 +699,15 @@ static void drop_plan_graph(sfft_plan* P) {
   P->graph = nullptr;
 }
 
-// Graph mode launches the kernels one by one where the head is a slab fold of 64 MB and more: it
-// runs long enough for the launches behind it to be enqueued meanwhile, and the chains then
-// start with less between them than a replay's nodes (n = 2^27, k = 16000, replayed -> launched:
-// FP64 814 -> 790 us, FP32 466 -> 457; n = 2^24 FP32 134 either way; n = 2^20 FP64 85 replayed,
-// 92 launched).
+// Graph mode launches the kernels one by one where that is faster than a replay: where the comb
+// and bucket stages share their launches (five or six on one stream, each enqueued while the one
+// before it runs; n = 2^20, k = 1000, FP64 85 us replayed, 76 launched), and where the head is a
+// slab fold of 64 MB and more: it runs long enough for the launches behind it to be enqueued
+// meanwhile, and the chains then start with less between them than a replay's nodes (n = 2^27,
+// k = 16000, replayed -> launched: FP64 814 -> 790 us, FP32 466 -> 457; n = 2^24 FP32 134 either
+// way).
 static bool graph_as_eager(const sfft_plan* P) {
+  if (paired(P)) return true;
   return P->columns && (size_t)P->p.n * (P->fp32 ? 8 : 16) >= ((size_t)64 << 20);
 }
 
