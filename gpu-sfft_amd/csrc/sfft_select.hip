@@ -745,6 +745,7 @@ struct SelBlockLds {
   int sh[16];
   int s_pick[3];
   int s_nc;
+  int ai[32], top[32];       // per location loop marked: its factor, its largest residue
 };
 
 template <typename K, int PER>
@@ -818,6 +819,10 @@ __device__ __forceinline__ void sel_block_body(const K* __restrict__ keys, long 
   for (int i = tid; i < SEL_BINS; i += SEL_NT) h[i] = 0u;
   picked[tid] = 0u;
   if (tid == 0) s_nc = 0;
+  if (tid < mark.loops) {
+    lds.ai[tid] = mark.ai[tid];
+    lds.top[tid] = -1;
+  }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -938,31 +943,25 @@ __device__ __forceinline__ void sel_block_body(const K* __restrict__ keys, long 
   }
   int pos = block_excl_scan_s(__popc(sel), sh);
   int* o = out + (long long)seg * Ksel;
-  for (unsigned m = sel; m; m &= m - 1) {
-    const unsigned nat = (unsigned)key_natural(km, i0 + __ffs(m) - 1);
-    o[pos++] = (int)nat;
-    for (int l = 0; l < mark.loops; ++l) {
-      const unsigned f = (nat * (unsigned)mark.ai[l]) & mark.wmask;
-      atomicOr(&mark.bitmap[(size_t)l * mark.bm_words + (f >> 5)], 1u << (f & 31));
-    }
-  }
-  // the largest approved residue of each location loop
+  for (unsigned m = sel; m; m &= m - 1) o[pos++] = (int)key_natural(km, i0 + __ffs(m) - 1);
+  // the approved residues of each location loop and the largest one (the loops' factors from LDS:
+  // a load of theirs per selected index waited for the atomics before it, n = 2^20, k = 1000: the
+  // two cutoffs' launch 18.2 -> 15.1 us)
   for (int l = 0; l < mark.loops; ++l) {
-    const unsigned a = (unsigned)mark.ai[l];
+    const unsigned a = (unsigned)lds.ai[l];
+    unsigned* bm = mark.bitmap + (size_t)l * mark.bm_words;
     int v = -1;
-    for (unsigned m = sel; m; m &= m - 1)
-      v = max(v, (int)(((unsigned)key_natural(km, i0 + __ffs(m) - 1) * a) &
-                       mark.wmask));
+    for (unsigned m = sel; m; m &= m - 1) {
+      const unsigned f = ((unsigned)key_natural(km, i0 + __ffs(m) - 1) * a) & mark.wmask;
+      atomicOr(&bm[f >> 5], 1u << (f & 31));
+      v = max(v, (int)f);
+    }
 #pragma unroll
     for (int q = 32; q > 0; q >>= 1) v = max(v, __shfl_xor(v, q, 64));
-    __syncthreads();
-    if ((tid & 63) == 0) sh[tid >> 6] = v;
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < SEL_NT / 64; ++w) v = max(v, sh[w]);
-      if (v >= 0) atomicMax(&mark.maxfirst[l], v);
-    }
+    if ((tid & 63) == 0) atomicMax(&lds.top[l], v);
   }
+  __syncthreads();
+  if (tid < mark.loops && lds.top[tid] >= 0) atomicMax(&mark.maxfirst[tid], lds.top[tid]);
 }
 
 // ---- kernels: every workgroup of a launch belongs to a job (sfft_jobs.h); one select is a
