@@ -55,6 +55,8 @@ struct KeyBits<unsigned int> {
 __device__ __forceinline__ int index_bits(int N) { return N > 1 ? 32 - __clz(N - 1) : 0; }
 
 
+constexpr int SPLIT_ROUND = 8 * SEL_NT;   // keys whose loads the split keeps in flight together
+
 // elements per block: about 256 blocks per segment for large N, at least 2048
 static int sel_chunk(int N) {
   int c = 2048;
@@ -295,8 +297,8 @@ __device__ __forceinline__ void sel_split_body(const K* __restrict__ keys, long 
   // the candidates' key loads, so that the loop waits twice per SU elements, not twice per
   // element (the order of a block's candidates and winners is set by the wave appends either
   // way; every later pass is independent of it)
-  constexpr int SU = 8;
-  for (int base = begin; base < end; base += SEL_NT * SU) {
+  constexpr int SU = SPLIT_ROUND / SEL_NT;
+  for (int base = begin; base < end; base += SPLIT_ROUND) {
     unsigned d[SU];
     K k[SU];
 #pragma unroll
@@ -1205,6 +1207,13 @@ hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long
   const hipError_t e = select_job(j, keys, seg_stride, N, K, segs, out, ordered, w, bits,
                                   map, digits, mark, hist);
   if (e != hipSuccess) return e;
+  // a whole round of the split's loads per workgroup: many segments fill the chip by themselves,
+  // and each workgroup first reads the segment's histograms (64 KB), which shorter chunks do not
+  // pay for (64 signals' comb cutoffs of 2^16..2^18 keys: split 117 -> 43 us)
+  if (j.chunk < SPLIT_ROUND) {
+    j.chunk = SPLIT_ROUND;
+    j.nchunks = (N + j.chunk - 1) / j.chunk;
+  }
   g.fp32 = is_fp32;
   if (select_in_block(N)) {
     g.block[block_variant(N)].add(j, segs);
