@@ -172,16 +172,16 @@ struct SelJob {
 };
 struct SelGroup {
   int fp32 = 0;
-  JobTable<SelJob> block[3];   // one workgroup per segment: 8, 16, 32 elements per thread
+  JobTable<SelJob> block;      // one workgroup does a segment
   JobTable<SelJob> wide;       // nchunks x segs workgroups: split, compact / write
   JobTable<SelJob> refine;     // one workgroup per segment
   void pack(JobPack& p) {
-    for (auto& b : block) b.pack(p);
+    block.pack(p);
     wide.pack(p);
     refine.pack(p);
   }
   void bind(const char* base) {
-    for (auto& b : block) b.bind(base);
+    block.bind(base);
     wide.bind(base);
     refine.bind(base);
   }

@@ -1044,42 +1044,32 @@ __global__ __launch_bounds__(SEL_NT) void sel_write_kernel(From f) {
   sel_write_body<K>((const K*)j.keys, j.seg_stride, j.N, j.chunk, j.nchunks, j.K,
                     (const SelState*)j.state, j.cnt, j.out, j.bits, bx, seg);
 }
-template <typename K, int PER, typename From>
+// a segment that one workgroup does: 8, 16 or 32 elements per thread
+template <typename K>
+__device__ __forceinline__ void sel_block_any(const SelJob& j, int seg) {
+  __shared__ SelBlockLds<K> lds;
+  const K* keys = (const K*)j.keys;
+  if (j.N <= 8 * SEL_NT)
+    sel_block_body<K, 8>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
+                         j.mark, seg, lds);
+  else if (j.N <= 16 * SEL_NT)
+    sel_block_body<K, 16>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
+                          j.mark, seg, lds);
+  else
+    sel_block_body<K, 32>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
+                          j.mark, seg, lds);
+}
+template <typename K, typename From>
 __global__ __launch_bounds__(SEL_NT) void sel_block_kernel(From f) {
   SelJob j;
   int bx, seg;
-  if (!f.get(j, bx, seg, 1)) return;
-  __shared__ SelBlockLds<K> lds;
-  sel_block_body<K, PER>((const K*)j.keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits,
-                         j.vec, j.mark, seg, lds);
+  if (f.get(j, bx, seg, 1)) sel_block_any<K>(j, seg);
 }
-
-// elements per thread of the one-workgroup select, as an index into 8, 16, 32
-__host__ __device__ __forceinline__ int block_variant(int N) {
-  return N <= 8 * SEL_NT ? 0 : N <= 16 * SEL_NT ? 1 : 2;
-}
-
 // two selects, a workgroup per segment of either
 template <typename K>
 __global__ __launch_bounds__(SEL_NT) void sel_pair_kernel(SelJob a, SelJob b) {
-  __shared__ SelBlockLds<K> lds;
   const bool first = (int)blockIdx.x < a.segs;
-  const SelJob& j = first ? a : b;
-  const int seg = first ? (int)blockIdx.x : (int)blockIdx.x - a.segs;
-  const K* keys = (const K*)j.keys;
-  switch (block_variant(j.N)) {
-    case 0:
-      sel_block_body<K, 8>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
-                           j.mark, seg, lds);
-      break;
-    case 1:
-      sel_block_body<K, 16>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
-                            j.mark, seg, lds);
-      break;
-    default:
-      sel_block_body<K, 32>(keys, j.seg_stride, j.N, j.K, j.out, j.bits, j.map, j.digits, j.vec,
-                            j.mark, seg, lds);
-  }
+  sel_block_any<K>(first ? a : b, first ? (int)blockIdx.x : (int)blockIdx.x - a.segs);
 }
 
 // Up to 32768 keys one workgroup beats the chain of launches, in both precisions; at 65536 its
@@ -1135,22 +1125,12 @@ static hipError_t select_job(SelJob& j, const void* keys, long long seg_stride, 
   return hipSuccess;
 }
 
-template <typename K, typename From>
-static void block_go(int variant, const From& f, dim3 grid, hipStream_t st) {
-  if (variant == 0)
-    hipLaunchKernelGGL((sel_block_kernel<K, 8, From>), grid, dim3(SEL_NT), 0, st, f);
-  else if (variant == 1)
-    hipLaunchKernelGGL((sel_block_kernel<K, 16, From>), grid, dim3(SEL_NT), 0, st, f);
-  else
-    hipLaunchKernelGGL((sel_block_kernel<K, 32, From>), grid, dim3(SEL_NT), 0, st, f);
-}
-
 template <typename K>
 static hipError_t select_one(const SelJob& j, hipStream_t st) {
   const SelOne f{j};
   const dim3 wide(j.nchunks, j.segs);
   if (select_in_block(j.N)) {
-    block_go<K>(block_variant(j.N), f, dim3(1, j.segs), st);
+    hipLaunchKernelGGL((sel_block_kernel<K, SelOne>), dim3(1, j.segs), dim3(SEL_NT), 0, st, f);
     return hipGetLastError();
   }
   if (j.nsum == 1) {   // no histograms at hand
@@ -1216,7 +1196,7 @@ hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long
   }
   g.fp32 = is_fp32;
   if (select_in_block(N)) {
-    g.block[block_variant(N)].add(j, segs);
+    g.block.add(j, segs);
   } else {
     g.wide.add(j, j.nchunks * segs);
     g.refine.add(j, segs);
@@ -1227,9 +1207,9 @@ hipError_t select_jobs_add(SelGroup& g, int is_fp32, const void* keys, long long
 // every select of the group is ordered, or none is (a batch's bucket cutoffs, or its combs')
 template <typename K>
 static hipError_t select_many(const SelGroup& g, hipStream_t st) {
-  for (int v = 0; v < 3; ++v)
-    if (g.block[v].dev.blocks)
-      block_go<K>(v, SelMany{g.block[v].dev}, dim3(g.block[v].dev.blocks), st);
+  if (g.block.dev.blocks)
+    hipLaunchKernelGGL((sel_block_kernel<K, SelMany>), dim3(g.block.dev.blocks), dim3(SEL_NT), 0,
+                       st, SelMany{g.block.dev});
   if (g.wide.dev.blocks) {
     const SelMany wide{g.wide.dev}, refine{g.refine.dev};
     const dim3 nw(wide.t.blocks);
