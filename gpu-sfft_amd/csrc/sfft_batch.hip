@@ -44,7 +44,7 @@ struct sfft_batch {
   int lpt = 3, nt = 256, grid = 2048;
   std::vector<FftGroup> comb, comb_slab, bucket;   // combs gathered, combs the slab fold copied
   SelGroup sel_comb, sel_bucket;
-  JobTable<HashJob> clear, bitmap, hits;
+  JobTable<HashJob> clear, bitmap;
   std::vector<NodeGroup> est;
   char* d_tab = nullptr;
   size_t tab_bytes = 0;
@@ -182,7 +182,7 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   b->est.clear();
   b->sel_comb = SelGroup();
   b->sel_bucket = SelGroup();
-  b->clear = b->bitmap = b->hits = JobTable<HashJob>();
+  b->clear = b->bitmap = JobTable<HashJob>();
   int item = 0;
   for (int i = 0; i < b->count; ++i) {
     const sfft_plan* P = b->plans[i];
@@ -227,7 +227,6 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
                           P->J, 1, P->selB, P->jsel, nullptr, P->bucket_digits, nullptr,
                           P->hist_B));
     if (!marks) hash_jobs_bitmap(b->bitmap, h);
-    hash_jobs_count(b->hits, h);
     NodeJob e = {};
     e.h = h;
     e.bins = P->bins_f;
@@ -252,7 +251,6 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   b->sel_bucket.pack(pack);
   b->clear.pack(pack);
   b->bitmap.pack(pack);
-  b->hits.pack(pack);
   if (pack.bytes.size() > b->tab_bytes) {
     HIPCK(hipStreamSynchronize(b->st));   // an earlier batch may still read the old tables
     if (b->d_tab) (void)hipFree(b->d_tab);
@@ -274,7 +272,6 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   b->sel_bucket.bind(b->d_tab);
   b->clear.bind(b->d_tab);
   b->bitmap.bind(b->d_tab);
-  b->hits.bind(b->d_tab);
   b->tab_x.assign(d_x, d_x + b->count);
   b->tab_nodes.assign(nodes, nodes + b->count);
   return SFFT_OK;
@@ -298,7 +295,6 @@ static sfft_status enqueue(sfft_batch* b) {
   HIPCK(fft_jobs_launch(b->bucket, b->st));
   HIPCK(select_jobs_launch(b->sel_bucket, b->st));
   HIPCK(hipStreamWaitEvent(b->st, b->ev_join, 0));
-  HIPCK(hash_count_jobs(b->hits, b->st));
   HIPCK(nodes_jobs_launch(b->est, b->st));
   return SFFT_OK;
 }

@@ -1,9 +1,9 @@
 // sfft_hash.hip -- hand-written CDNA4 (gfx950) kernels of the sparse-FFT hot path, part 2.
 //
-//  * hash_*_kernel        reverse hash: approved-residue bitmaps, deterministic hit list
-//                         (loop, bucket, walk order); the votes of earlier loops are tested
-//                         directly from their bucket selections (no vote table)
-//  * estimate_kernel      per-location FP64 filter division and stable lower median
+//  * hash_*_kernel        reverse hash: approved-residue bitmaps, hit masks; the votes of earlier
+//                         loops are tested directly from their bucket selections (no vote table)
+//  * nodes_kernel         deterministic hit list (loop, bucket, walk order) and per-location FP64
+//                         filter division and stable lower median
 //
 // Floating-point operations that must match the CPU oracle bit for bit are written out
 // explicitly (fma where fused); the library is built with -ffp-contract=off.
@@ -333,43 +333,6 @@ __device__ __forceinline__ int hash_count_slice(const HashArgs& h, const HashSlo
   return c;
 }
 
-// (block bx of the nb blocks of one signal's walk)
-__device__ __forceinline__ void hash_count_body(const HashArgs& h, int bx) {
-  __shared__ int sh[16];
-  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
-  const int words = hash_slice_words(h.loops_loc, h.K, (long long)h.n / h.B);
-  const long long gid = (long long)bx * HASH_NT + threadIdx.x;
-  const int c = hash_count_slice(h, s, h.hmask + gid * words, words);
-  int tot = c;   // total of the bucket's lanes (aligned groups of lpj lanes)
-  for (int o = 1; o < s.lpj; o <<= 1) tot += __shfl_xor(tot, o, 64);
-  const int v = (s.valid && s.sub == 0) ? tot : 0;
-  const int ex = block_excl_scan(v, sh);
-  if (s.valid && s.sub == 0) h.hitoff[s.jidx] = ex;
-  if (threadIdx.x == HASH_NT - 1) h.blocksum[bx] = ex + v;
-}
-
-__global__ __launch_bounds__(HASH_NT) void hash_count_kernel(HashArgs h) {
-  hash_count_body(h, blockIdx.x);
-}
-__global__ __launch_bounds__(HASH_NT) void hash_count_jobs_kernel(JobsDev t) {
-  const HashJob* j = job_here<HashJob>(t);
-  if (j) hash_count_body(j->h, (int)blockIdx.x - j->block0);
-}
-void hash_jobs_count(JobTable<HashJob>& t, const HashArgs& h) {
-  HashJob j{h, hash_hit_blocks(h), 0};
-  t.add(j, j.blocks);
-}
-hipError_t hash_count_jobs(const JobTable<HashJob>& t, hipStream_t st) {
-  if (!t.dev.blocks) return hipSuccess;
-  hipLaunchKernelGGL(hash_count_jobs_kernel, dim3(t.dev.blocks), dim3(HASH_NT), 0, st, t.dev);
-  return hipGetLastError();
-}
-
-hipError_t hash_count_launch(const HashArgs& h, hipStream_t st) {
-  hipLaunchKernelGGL(hash_count_kernel, dim3(hash_hit_blocks(h)), dim3(HASH_NT), 0, st, h);
-  return hipGetLastError();
-}
-
 // ============================================================================================
 // estimation
 // ============================================================================================
@@ -487,52 +450,120 @@ __global__ __launch_bounds__(EST_NT) void estimate_kernel(EstArgs j) {
   }
 }
 
-// The hits of a block's slices, from the count pass's hit masks (no second walk), and their
-// values: the block lists its hits in LDS in window order and estimates one per thread, so the
-// hits are consecutive threads' work however the windows hold them and need no launch of their
-// own between the walk and the estimation (n = 2^27, k = 16000: a transform FP64 829 -> 823 us, FP32
-// 480 -> 472; n = 2^20, k = 1000, FP64 98 -> 94).  Each block first sums
-// the hit totals of the blocks before it (a few KB, read by every block in parallel: no separate
-// scan launch); the last one stores the total hit count.
+// The hits of the places before bx, one wave: publishes this place's total, adds up the totals of
+// the 64 places before it at a time until it meets one whose sum with all before it is published,
+// and publishes its own such sum.  A place is taken by a running block, which publishes its total
+// before it waits for anything but its own threads, so every wait ends whatever the order or
+// number of resident blocks.
+constexpr unsigned long long PLACE_TOTAL = 1ull << 32, PLACE_SUM = 2ull << 32;   // | hits; 0: neither
+__device__ __forceinline__ int walk_prefix(unsigned long long* place, int bx, int tot) {
+  const int lane = threadIdx.x & 63;
+  auto publish = [&](unsigned long long v) __attribute__((always_inline)) {
+    if (lane == 0)
+      __hip_atomic_store(&place[bx], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (bx > 0) publish(PLACE_TOTAL | (unsigned)tot);
+  int before = 0;
+  bool summed = bx == 0;
+  for (int b0 = bx - 1; !summed; b0 -= 64) {   // (place 0 always holds a sum)
+    const int b = b0 - lane;
+    unsigned long long v, none, sums;
+    int last;   // the nearest place with a sum, or 63
+    for (;;) {
+      v = b >= 0 ? __hip_atomic_load(&place[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                 : PLACE_SUM;
+      none = __ballot(v == 0ull);
+      sums = __ballot((v & PLACE_SUM) != 0ull);
+      last = sums ? __ffsll((long long)sums) - 1 : 63;
+      if (!none || __ffsll((long long)none) - 1 > last) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    int x = lane <= last ? (int)(unsigned)v : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    before += x;
+    summed = sums != 0ull;
+  }
+  publish(PLACE_SUM | (unsigned)(before + tot));
+  return before;
+}
+
+// A walk's hit masks, and each block's hit total into its place, as a launch before nodes_kernel.
+__global__ __launch_bounds__(HASH_NT) void hash_count_kernel(HashArgs h) {
+  __shared__ int sh[16];
+  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), blockIdx.x);
+  const int words = hash_slice_words(h.loops_loc, h.K, (long long)h.n / h.B);
+  const long long gid = (long long)blockIdx.x * HASH_NT + threadIdx.x;
+  const int tot = block_sum(hash_count_slice(h, s, h.hmask + gid * words, words), sh);
+  if (threadIdx.x == 0) h.place[blockIdx.x] = PLACE_TOTAL | (unsigned)tot;
+}
+
+// Walks of up to this many blocks run in the nodes' launch (WALK).  Walk and nodes as two
+// launches -> one: n = 2^14, k = 20 (3 blocks) 58 -> 52 us, n = 2^20, k = 1000 (125) FP32
+// 61 -> 57, FP64 76 -> 69, 64 signals (places of their own) 1804 -> 1750; but n = 2^24, k = 2503
+// (313) 137 -> 143, n = 2^27, k = 16000 (1000) FP32 470 -> 477, k = 40000 (2500) 1078 -> 1089:
+// the blocks' turns at one ticket cost more than the launch.
+constexpr int WALK_BLOCKS = 256;
+
+// The located indices of one signal in (loop, bucket, walk) order and their values.  A block
+// lists the hits of its slices in LDS in window order and estimates one per thread, so the hits
+// are consecutive threads' work however the windows hold them.  WALK: it takes the next place in
+// the walk and walks its slices itself; else hash_count_kernel has, and the totals of the blocks
+// before it are summed (a few KB, read by every block in parallel: no scan launch).
 constexpr int ND_LIST = 1024;   // hits listed at a time
-template <typename Real, int MAXL, bool EXACT>
-__device__ __forceinline__ void nodes_body(const NodeJob& j, int bx, int nb) {
+template <typename Real, int MAXL, bool EXACT, bool WALK>
+__device__ __forceinline__ void nodes_body(const NodeJob& j, int nb) {
   static_assert(HASH_NT == EST_NT, "a hit per thread of the walk's block");
   __shared__ unsigned long long stage[EST_NT * 3];
   __shared__ int list[ND_LIST];
   __shared__ int sh[16];
+  __shared__ int s_bx, s_tot, s_pre;
   const HashArgs& h = j.h;
   const int tid = threadIdx.x;
-  int pre = 0;
-  for (int b = tid; b < bx; b += HASH_NT) pre += h.blocksum[b];
-  const int boff = block_sum(pre, sh);
-  const int tot = h.blocksum[bx];
+  int bx = blockIdx.x;
+  if (WALK) {
+    if (tid == 0) s_bx = (int)atomicAdd(h.ticket, 1u);
+    __syncthreads();
+    bx = s_bx;
+  }
+  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
+  const int words = hash_slice_words(h.loops_loc, h.K, (long long)h.n / h.B);
+  const long long gid = (long long)bx * HASH_NT + tid;
+  unsigned* mk = h.hmask + gid * words;
+  int c = 0;
+  if (WALK) {
+    c = hash_count_slice(h, s, mk, words);
+  } else if (s.valid) {
+    for (int w = 0; w < words; ++w) c += __popc(mk[w]);
+  }
+  // the threads of a block are its slices in walk order
+  const int first = block_excl_scan(c, sh);
+  if (tid == HASH_NT - 1) s_tot = first + c;
+  __syncthreads();
+  const int tot = s_tot;
+  int boff;
+  if (WALK) {
+    if (tid < 64) {
+      const int before = walk_prefix(h.place, bx, tot);
+      if (tid == 0) s_pre = before;
+    }
+    __syncthreads();
+    boff = s_pre;
+  } else {
+    int pre = 0;
+    for (int b = tid; b < bx; b += HASH_NT) pre += (int)(unsigned)h.place[b];
+    boff = block_sum(pre, sh);
+  }
   if (bx == nb - 1 && tid == 0) {
     *h.count = boff + tot;
     if (j.count_copy) *j.count_copy = boff + tot;
   }
   if (tot == 0) return;
-  const HashSlot s = hash_slot(h, hash_hit_first_d(h), hash_hit_count_d(h), bx);
-  const int words = hash_slice_words(h.loops_loc, h.K, (long long)h.n / h.B);
-  const long long gid = (long long)bx * HASH_NT + tid;
-  const unsigned* __restrict__ mk = h.hmask + gid * words;
-  int c = 0;
-  if (s.valid)
-    for (int w = 0; w < words; ++w) c += __popc(mk[w]);
-  // exclusive scan over the bucket's lanes (in window order)
-  const int lane = tid & 63;
-  int x = c;
-  for (int o = 1; o < s.lpj; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if ((lane & (s.lpj - 1)) >= o) x += y;
-  }
   const long long n = h.n;
   const long long m = n / h.B;
-  int first = 0;
   long long start = 0;
   uint64_t a = 0;
   if (c) {
-    first = h.hitoff[s.jidx] + (x - c);   // within the block
     const long long J = h.J[(long long)s.l * h.K + s.i];
     start = ((J * m - (m >> 1)) + n + s.d0) & (n - 1);   // low + d0
     a = (uint64_t)(uint32_t)h.a_dev[s.l];
@@ -581,16 +612,16 @@ __device__ __forceinline__ void nodes_body(const NodeJob& j, int bx, int nb) {
   }
 }
 
-template <typename Real, int MAXL, bool EXACT>
+template <typename Real, int MAXL, bool EXACT, bool WALK>
 __global__ __launch_bounds__(EST_NT) void nodes_kernel(NodeJob j) {
-  nodes_body<Real, MAXL, EXACT>(j, blockIdx.x, gridDim.x);
+  nodes_body<Real, MAXL, EXACT, WALK>(j, (int)gridDim.x);
 }
 template <typename Real, int MAXL, bool EXACT>
 __global__ __launch_bounds__(EST_NT) void nodes_jobs_kernel(JobsDev t) {
   const NodeJob* p = job_here<NodeJob>(t);
   if (!p) return;
   const NodeJob j = *p;
-  nodes_body<Real, MAXL, EXACT>(j, (int)blockIdx.x - j.block0, j.blocks);
+  nodes_body<Real, MAXL, EXACT, true>(j, j.blocks);
 }
 
 // f(the loop count as a template constant, whether it is exact)
@@ -621,17 +652,27 @@ hipError_t estimate_launch(const EstArgs& a, hipStream_t st) {
   });
 }
 
-hipError_t nodes_launch(int is_fp32, const NodeJob& j, hipStream_t st) {
-  const dim3 grid(hash_hit_blocks(j.h)), nt(EST_NT);
+template <typename Real>
+static hipError_t nodes_go(const NodeJob& j, hipEvent_t between, hipStream_t st) {
+  const int blocks = hash_hit_blocks(j.h);
+  const bool walk = blocks <= WALK_BLOCKS && !between;
+  if (!walk) hipLaunchKernelGGL(hash_count_kernel, dim3(blocks), dim3(HASH_NT), 0, st, j.h);
+  if (between) {
+    const hipError_t e = hipEventRecord(between, st);
+    if (e != hipSuccess) return e;
+  }
   return with_loops(j.loops, [&](auto L, auto E) {
     constexpr int l = decltype(L)::v;
     constexpr bool e = decltype(E)::v != 0;
-    if (is_fp32)
-      hipLaunchKernelGGL((nodes_kernel<float, l, e>), grid, nt, 0, st, j);
+    if (walk)
+      hipLaunchKernelGGL((nodes_kernel<Real, l, e, true>), dim3(blocks), dim3(EST_NT), 0, st, j);
     else
-      hipLaunchKernelGGL((nodes_kernel<double, l, e>), grid, nt, 0, st, j);
+      hipLaunchKernelGGL((nodes_kernel<Real, l, e, false>), dim3(blocks), dim3(EST_NT), 0, st, j);
     return hipGetLastError();
   });
+}
+hipError_t nodes_launch(int is_fp32, const NodeJob& j, hipEvent_t between, hipStream_t st) {
+  return is_fp32 ? nodes_go<float>(j, between, st) : nodes_go<double>(j, between, st);
 }
 
 void nodes_jobs_add(std::vector<NodeGroup>& g, int is_fp32, NodeJob j) {

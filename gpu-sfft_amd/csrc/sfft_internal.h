@@ -273,13 +273,13 @@ struct HashArgs {
   const int* ai_dev;
   unsigned* bitmap;      // loops_loc x words
   int bm_words;
-  size_t clear_words;    // from bitmap on: what a transform clears (the bitmaps, the cutoffs'
-                         // histograms behind them)
+  size_t clear_words;    // from bitmap on: what a transform clears (the bitmaps, and behind them
+                         // the cutoffs' histograms and the walk's ticket and places)
   int* maxfirst;         // loops_loc
   unsigned* jsel;        // loops_loc x jsel_words: the buckets each location loop selected
   int jsel_words;
-  int* hitoff;           // loops_loc x K (local prefix within block)
-  int* blocksum;         // hit total of each count/write block
+  unsigned* ticket;      // the walk's next place (starts at 0)
+  unsigned long long* place;   // what each place has published (starts at 0; PLACE_*)
   unsigned* hmask;       // hash_mask_bytes(): one hit mask per walk slice
   int* hits;             // capacity
   int capacity;
@@ -287,7 +287,6 @@ struct HashArgs {
 };
 hipError_t hash_clear_launch(const HashArgs& h, const DrawVals& dv, hipStream_t st);
 hipError_t hash_bitmap_launch(const HashArgs& h, hipStream_t st);
-hipError_t hash_count_launch(const HashArgs& h, hipStream_t st);   // hit masks and counts
 // blocks that walk `loops` of the location loops (m = n / B)
 int hash_blocks(int loops, int loops_loc, int K, long long m);
 size_t hash_mask_bytes(int loops_loc, int K, long long m);   // hit masks of the slices
@@ -306,7 +305,7 @@ struct EstArgs {
   Node* out;
 };
 hipError_t estimate_launch(const EstArgs& a, hipStream_t st);
-// The hits of the count pass in order, and their nodes.  out may be device memory or the device
+// The reverse hash's hits in order, and their nodes.  out may be device memory or the device
 // view of pinned host memory (stored in coalesced 8-byte words either way); count_copy (optional,
 // the same kinds of memory) receives the hit count.
 struct NodeJob {
@@ -321,7 +320,8 @@ struct NodeJob {
   int* count_copy;
   int blocks, block0;    // as a job of a batch
 };
-hipError_t nodes_launch(int is_fp32, const NodeJob& j, hipStream_t st);
+// (between: recorded between the walk and the estimation, which are then launches of their own)
+hipError_t nodes_launch(int is_fp32, const NodeJob& j, hipEvent_t between, hipStream_t st);
 
 // ---- value map and its adjoint (FP64) -----------------------------------------------------
 // values[h] = Re v_{sel[2h]}(hits[h]) + i Im v_{sel[2h+1]}(hits[h]) from the bucket spectra

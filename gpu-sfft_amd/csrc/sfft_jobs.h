@@ -200,10 +200,8 @@ struct HashJob {
 };
 void hash_jobs_clear(JobTable<HashJob>& t, const HashArgs& h);
 void hash_jobs_bitmap(JobTable<HashJob>& t, const HashArgs& h);
-void hash_jobs_count(JobTable<HashJob>& t, const HashArgs& h);
 hipError_t hash_clear_jobs(const JobTable<HashJob>& t, hipStream_t st);
 hipError_t hash_bitmap_jobs(const JobTable<HashJob>& t, hipStream_t st);
-hipError_t hash_count_jobs(const JobTable<HashJob>& t, hipStream_t st);
 
 struct NodeGroup {
   int loops = 0, fp32 = 0;

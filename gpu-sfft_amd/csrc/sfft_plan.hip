@@ -303,16 +303,15 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   void* selB_base = nullptr;
   items.push_back({&selW_base, select_work_bytes(Rl, (int)W)});
   items.push_back({&selB_base, select_work_bytes(Ll, (int)B)});
-  // the bitmaps, and behind them the histograms of the chained cutoffs, cleared together
+  // the bitmaps, and behind them the histograms of the chained cutoffs and the walk's ticket and
+  // places, cleared together
   const size_t bmw = ((size_t)Ll * P->bm_words + 63) / 64 * 64;
   const size_t histW = select_in_block((int)W) ? 0 : (size_t)Rl * kSelCopies * kSelBins;
   const size_t histB = select_in_block((int)B) ? 0 : (size_t)Ll * kSelCopies * kSelBins;
-  P->clear_words = bmw + histW + histB;
+  P->clear_words = bmw + histW + histB + 2 + 2 * (size_t)nhb;
   items.push_back({(void**)&P->bitmap, P->clear_words * 4});
   items.push_back({(void**)&P->maxfirst, (size_t)Ll * 4});
   items.push_back({(void**)&P->jsel, (size_t)Ll * ((B + 31) / 32) * 4});
-  items.push_back({(void**)&P->hitoff, (size_t)Ll * K * 4});
-  items.push_back({(void**)&P->blocksum, (size_t)nhb * 4});
   items.push_back({(void**)&P->hmask, hash_mask_bytes(Ll, K, (long long)prm->n / prm->B)});
   items.push_back({(void**)&P->hits, (size_t)P->cap * 4});
   items.push_back({(void**)&P->count, 16});
@@ -342,6 +341,7 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   P->d_offs = P->d_a + 2 * L;
   P->hist_W = histW ? P->bitmap + bmw : nullptr;
   P->hist_B = histB ? P->bitmap + bmw + histW : nullptr;
+  P->ticket = P->bitmap + bmw + histW + histB;
   select_work_bind(&P->selW, selW_base, Rl, (int)W);
   select_work_bind(&P->selB, selB_base, Ll, (int)B);
   // select state must start at zero (hist/done are reset by the kernels themselves)
@@ -447,8 +447,8 @@ HashArgs hash_args(const sfft_plan* P, int* d_count) {
   h.maxfirst = P->maxfirst;
   h.jsel = P->jsel;
   h.jsel_words = (p.B + 31) / 32;
-  h.hitoff = P->hitoff;
-  h.blocksum = P->blocksum;
+  h.ticket = P->ticket;
+  h.place = (unsigned long long*)(P->ticket + 2);   // (the words before are an even number)
   h.hmask = P->hmask;
   h.hits = P->hits;
   h.capacity = P->cap;
@@ -604,8 +604,6 @@ static sfft_status run_pair(sfft_plan* P, const HashArgs& h, hipStream_t st) {
 // locate: reverse hash (needs the comb bitmaps and the bucket cutoffs) + estimation
 static sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hipStream_t st,
                               bool marks) {
-  HIPCK(hash_count_launch(h, st));
-  if (marks && P->profile) HIPCK(hipEventRecord(P->ev[6], st));
   NodeJob j = {};
   j.h = h;
   j.bins = P->bins_f;
@@ -614,8 +612,9 @@ static sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hi
   j.out = d_nodes ? d_nodes : P->nodes;
   j.sel = P->sel;
   j.count_copy = P->cnt_copy;
-  HIPCK(nodes_launch(P->fp32, j, st));
-  if (marks && P->profile) HIPCK(hipEventRecord(P->ev[7], st));
+  const bool prof = marks && P->profile;
+  HIPCK(nodes_launch(P->fp32, j, prof ? P->ev[6] : nullptr, st));
+  if (prof) HIPCK(hipEventRecord(P->ev[7], st));
   return SFFT_OK;
 }
 

@@ -45,8 +45,7 @@ struct sfft_plan {
   unsigned* hist_B = nullptr;   // passes count them; nullptr: one workgroup per segment)
   int* maxfirst = nullptr;
   unsigned* jsel = nullptr;     // buckets selected per location loop (bitmaps)
-  int* hitoff = nullptr;
-  int* blocksum = nullptr;
+  unsigned* ticket = nullptr;      // and behind it the walk's places
   unsigned* hmask = nullptr;
   int* hits = nullptr;
   int* count = nullptr;
