@@ -219,7 +219,8 @@ sfft_status sfft_execute(sfft_plan *plan, const void *d_x, const sfft_draws *dra
 
 /* Graph mode (off by default): the transform's kernel sequence is captured into a hipGraph
  * on first use and replayed by later sfft_execute[_async] calls while the signal and result
- * pointers stay the same (re-captured when they change); the draws go with each replay.  A plan
+ * pointers stay the same (re-captured when they change); the draws go with each replay.
+ * Transforms that are faster launched kernel by kernel are launched that way all the same.  A plan
  * created with stream NULL gets a stream of its own for this.  Profiling
  * (sfft_plan_set_profiling) runs the transform eagerly. */
 sfft_status sfft_plan_set_graph(sfft_plan *plan, int on);
