@@ -699,8 +699,8 @@ static void drop_plan_graph(sfft_plan* P) {
 }
 
 // Graph mode launches the kernels one by one where that is faster than a replay: where the comb
-// and bucket stages share their launches (five or six on one stream, each enqueued while the one
-// before it runs; n = 2^20, k = 1000, FP64 85 us replayed, 76 launched), and where the head is a
+// and bucket stages share their launches (four or five on one stream, each enqueued while the one
+// before it runs; n = 2^20, k = 1000, FP64, with one more: 85 us replayed, 76 launched), and where the head is a
 // slab fold of 64 MB and more: it runs long enough for the launches behind it to be enqueued
 // meanwhile, and the chains then start with less between them than a replay's nodes (n = 2^27,
 // k = 16000, replayed -> launched: FP64 814 -> 790 us, FP32 466 -> 457; n = 2^24 FP32 134 either
