@@ -3,7 +3,7 @@
 // Each signal keeps its own plan (parameters, workspace).  One batch execution runs every stage
 // of ALL its signals as one launch (sfft_jobs.h: a table of the signals' arguments, and each
 // workgroup's signal), so
-// small and large signals share the chip and a batch of any size takes about thirty launches.
+// small and large signals share the chip and a batch of any size takes about twenty launches.
 // (One launch per signal and stage took 16-25 launches of a few us per signal: 64 complex64
 // signals of 2^18..2^24, 6.3 ms on four streams, 2.6 ms as one launch per stage.)
 // Signals whose plan takes the column front end (AUTO, where the slab applies) are folded by one

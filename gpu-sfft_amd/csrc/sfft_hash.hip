@@ -247,7 +247,7 @@ size_t hash_mask_bytes(int loops_loc, int K, long long m) {
 // loc's position p = loc * ai_l' mod n lies in the window of a bucket J that l' selected,
 // J = ((p + m/2) mod n) / m, that window is not cut off by the largest approved residue (the
 // walk's early exit), and p's residue p mod W is approved: three table reads instead of a
-// vote pass over every window and a vote table.  The count and write passes cover the loops
+// vote pass over every window and a vote table.  The walk covers the loops
 // [thresh-1, loops_loc) (loops_thresh >= 1 is checked when the plan is made).
 static int hash_hit_blocks(const HashArgs& h) {
   return hash_blocks(h.loops_loc - (h.loops_thresh - 1), h.loops_loc, h.K, (long long)h.n / h.B);
