@@ -2004,7 +2004,8 @@ hipError_t fold_columns_launch(int is_fp32, const void* x, const void* fT, void*
   const int log2B = A.log2B, log2m = A.log2m, log2sigma = A.log2sigma, T = A.T, P = A.P;
   const uint32_t mask = A.mask;
   Rl = A.Rl;
-  if (clr.nbm || clr.nmax) return hipErrorInvalidValue;   // only the slab fold clears
+  // only the slab fold clears and takes the draws
+  if (clr.nbm || clr.nmax || dv.count) return hipErrorInvalidValue;
   // columns per block: one 128-byte line of x (8 complex128 / 16 complex64), fewer if B is
   // smaller
   int log2lw = is_fp32 ? 4 : 3;

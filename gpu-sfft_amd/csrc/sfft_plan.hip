@@ -621,8 +621,8 @@ static sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hi
 // One transform: its first kernel (run_head), then everything after it (run_rest).  The first
 // kernel takes the draws as an argument and leaves them in device memory for the rest: no upload
 // and no gap after one in front of it (n = 2^14, k = 20, replayed: 73 -> 67 us; n = 2^20, k = 1000, FP64
-// 91 -> 85).  Column front end: the head is the slab fold, which also clears and copies the comb
-// samples.  Else it is the clear.
+// 91 -> 85).  Slab fold: the head is the fold, which also clears and copies the comb samples.
+// Else it is the clear.
 static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
                             const DrawVals& dv) {
   const sfft_params& p = P->p;
@@ -630,7 +630,7 @@ static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
     return P->profile ? hipEventRecord(P->ev[i], P->st) : hipSuccess;
   };
   HIPCK(mark(0));
-  if (P->columns) {
+  if (P->bins_perm) {
     FoldClear clr;
     clr.bm = h.bitmap;
     clr.nbm = h.clear_words;
@@ -639,8 +639,8 @@ static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
     const int tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
     HIPCK(mark(1));
     HIPCK(fold_columns_launch(P->fp32, d_x, P->frows, P->bins_t, P->d_a, P->d_ai, p.n, p.B, p.w,
-                              p.loops, tiled, P->bins_perm, 1, P->comb_y, P->d_offs,
-                              p.RLFC_loops, p.W_RLFC, clr, dv, P->st));
+                              p.loops, tiled, 1, 1, P->comb_y, P->d_offs, p.RLFC_loops,
+                              p.W_RLFC, clr, dv, P->st));
     HIPCK(mark(2));
   } else {
     HIPCK(hash_clear_launch(h, dv, P->st));
@@ -649,23 +649,30 @@ static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
   return SFFT_OK;
 }
 
-// After the head two concurrent chains, joined before the reverse hash: the comb chain (comb FFT,
-// cutoff, bitmaps) on the plan stream and the bucket chain (permute+filter unless the head was
-// the slab fold, bucket FFT, cutoff) on a second stream, so that the latency-bound kernels of
+// After the head (and the column fold of a shape that the slab does not take, which copies the
+// comb samples too) two concurrent chains, joined before the reverse hash: the comb chain (comb
+// FFT, cutoff, bitmaps) on the plan stream and the bucket chain (permute+filter of the gathers,
+// bucket FFT, cutoff) on a second stream, so that the latency-bound kernels of
 // one chain fill the gaps of the other's.  Column front end: the comb FFT is enqueued before the
 // bucket chain, so that a captured graph's first root, which the replay keeps on the launching
 // queue, starts the longer chain.  The gathering front end forks after its comb FFT (beside which
 // its permute+filter's gathers lose).  Profiling (and the streaming front end, whose pass feeds
 // the fold) runs everything serially on the plan stream; with the columns the profile's
-// "clear" interval is empty, its "streaming pass" interval is the fold (with the comb copy) and
-// its "fold" interval is empty.
+// "streaming pass" interval is the fold (with the comb copy) and its "fold" interval is empty, and
+// with the slab fold its "clear" interval too.
 static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes) {
   const sfft_params& p = P->p;
   sfft_status v;
   if (P->stream)   // one pass over x fills the tap staging array and the comb samples
     HIPCK(stream_scatter_launch(P->fp32, d_x, P->taps, P->comb_y, P->d_a, P->d_offs, p.n, p.w,
                                 p.loops, p.RLFC_loops, p.W_RLFC, P->st));
-  if (P->profile && !P->columns) HIPCK(hipEventRecord(P->ev[2], P->st));
+  if (P->columns && !P->bins_perm) {
+    const int tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
+    HIPCK(fold_columns_launch(P->fp32, d_x, P->frows, P->bins_t, P->d_a, P->d_ai, p.n, p.B, p.w,
+                              p.loops, tiled, 0, 1, P->comb_y, P->d_offs, p.RLFC_loops,
+                              p.W_RLFC, FoldClear(), DrawVals(), P->st));
+  }
+  if (P->profile && !P->bins_perm) HIPCK(hipEventRecord(P->ev[2], P->st));
   if (P->profile || P->stream) {
     HIPCK(fft_run(comb_fft(P, d_x), P->st));
     if ((v = run_cut(P, h, P->st, true)) != SFFT_OK) return v;
@@ -707,7 +714,7 @@ static void drop_plan_graph(sfft_plan* P) {
 // way).
 static bool graph_as_eager(const sfft_plan* P) {
   if (paired(P)) return true;
-  return P->columns && (size_t)P->p.n * (P->fp32 ? 8 : 16) >= ((size_t)64 << 20);
+  return P->bins_perm && (size_t)P->p.n * (P->fp32 ? 8 : 16) >= ((size_t)64 << 20);
 }
 
 static sfft_status capture(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes,
@@ -738,7 +745,7 @@ static sfft_status replay(sfft_plan* P, DrawVals& dv, bool async) {
     HIPCK(hipGraphInstantiate(&P->gexec[k], P->graph, nullptr, nullptr, 0));
   // the draws are the head's last argument (fold_slab_kernel's second, hash_clear_kernel's fifth)
   void* args[5];
-  const int n = P->columns ? 2 : 5;
+  const int n = P->bins_perm ? 2 : 5;
   for (int i = 0; i < n - 1; ++i) args[i] = P->g_head_params.kernelParams[i];
   args[n - 1] = &dv;
   hipKernelNodeParams kp = P->g_head_params;
