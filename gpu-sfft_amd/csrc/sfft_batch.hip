@@ -14,9 +14,10 @@
 // cutoff, approved bitmaps) on a second stream, and bucket FFT and bucket cutoff (after the
 // permute+filter) on the batch stream; joined there, the reverse hash and the estimation follow.
 // The draws of all signals go up in one copy.  With graphs the two chains are captured once as
-// one graph and replayed (buffers are cleared by kernels, so it holds no memset nodes); the
-// tables and the graph are rebuilt when the signal or node pointers, the filters or the tuned
-// shapes change.
+// one graph and replayed (buffers are cleared by kernels, so it holds no memset nodes).  New
+// signal or node pointers change the tables' contents alone: they are built again in pinned memory
+// and uploaded in stream order, without a wait and under the same graph; new filters or tuned
+// shapes drop the graph as well.
 //
 // Autotuner: times, on the batch itself, only launch shapes that compute the same bits --
 // the permute+filter loops per thread, block size and persistent grid (every shape runs the
@@ -47,8 +48,12 @@ struct sfft_batch {
   JobTable<HashJob> clear, bitmap;
   std::vector<NodeGroup> est;
   char* d_tab = nullptr;
-  size_t tab_bytes = 0;
+  char* h_tab = nullptr;             // pinned
+  size_t tab_bytes = 0;              // of either
+  hipEvent_t tab_ev = nullptr;       // last upload out of h_tab
+  int tab_pending = 0;
   const PfJob* d_jobs = nullptr;
+  bool tab_shape = false;            // the tables are those of the current filters and shapes
   std::vector<const void*> tab_x;    // the pointers the tables hold: signals, nodes
   std::vector<Node*> tab_nodes;
   // the draws of all signals: signal i's (a, ai, offsets) at draw_at[i]
@@ -74,6 +79,13 @@ static void drop_graph(sfft_batch* b) {
   b->graph = nullptr;
 }
 
+// filters or launch shapes change: tables of another layout, and other launches
+static void drop_tables(sfft_batch* b) {
+  drop_graph(b);
+  b->tab_x.clear();
+  b->tab_shape = false;
+}
+
 extern "C" void sfft_batch_destroy(sfft_batch* b) {
   if (!b) return;
   (void)hipStreamSynchronize(b->st);
@@ -85,7 +97,9 @@ extern "C" void sfft_batch_destroy(sfft_batch* b) {
   if (b->ev_join) (void)hipEventDestroy(b->ev_join);
   if (b->up_ev) (void)hipEventDestroy(b->up_ev);
   if (b->own_st && b->st) (void)hipStreamDestroy(b->st);
+  if (b->tab_ev) (void)hipEventDestroy(b->tab_ev);
   if (b->d_tab) (void)hipFree(b->d_tab);
+  if (b->h_tab) (void)hipHostFree(b->h_tab);
   if (b->d_draws) (void)hipFree(b->d_draws);
   if (b->h_draws) (void)hipHostFree(b->h_draws);
   if (b->d_counts) (void)hipFree(b->d_counts);
@@ -134,6 +148,7 @@ extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
       hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) == hipSuccess &&
       hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming) == hipSuccess &&
       hipEventCreateWithFlags(&b->up_ev, hipEventDisableTiming) == hipSuccess &&
+      hipEventCreateWithFlags(&b->tab_ev, hipEventDisableTiming) == hipSuccess &&
       hipMalloc((void**)&b->d_draws, sizeof(int) * b->draw_ints) == hipSuccess &&
       hipHostMalloc((void**)&b->h_draws, sizeof(int) * b->draw_ints, hipHostMallocDefault) ==
           hipSuccess &&
@@ -163,16 +178,18 @@ extern "C" sfft_plan* sfft_batch_plan(sfft_batch* b, int i) {
 extern "C" sfft_status sfft_batch_set_filter(sfft_batch* b, int i, const void* d_filter_time,
                                              const complex_t* h_filter_win) {
   if (!b || i < 0 || i >= b->count) return SFFT_ERR_INVALID;
-  drop_graph(b);
-  b->tab_x.clear();   // the tables hold the taps pointer
+  drop_tables(b);   // (they hold the taps pointer)
   return sfft_plan_set_filter(b->plans[i], d_filter_time, h_filter_win);
 }
 
 // (re)builds every stage's job table for the current shapes and pointers: signal i reads d_x[i]
 // and its nodes go to nodes[i] (the device view of pinned host memory, with a copy in the plan's
-// buffer; nullptr: the plan's buffer alone)
+// buffer; nullptr: the plan's buffer alone).  Where only pointers differ from the tables before,
+// every table keeps its size and place, so a captured graph of the launches stays valid.
 static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes) {
-  drop_graph(b);
+  const bool same_shape = b->tab_shape;
+  if (!same_shape) drop_graph(b);
+  b->tab_shape = false;
   b->tab_x.clear();
   b->jobs.clear();
   b->slab.clear();
@@ -251,17 +268,25 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   b->sel_bucket.pack(pack);
   b->clear.pack(pack);
   b->bitmap.pack(pack);
-  if (pack.bytes.size() > b->tab_bytes) {
+  const size_t bytes = pack.bytes.size();
+  if (b->tab_pending) HIPCK(hipEventSynchronize(b->tab_ev));
+  b->tab_pending = 0;
+  if (bytes > b->tab_bytes) {
+    drop_graph(b);
     HIPCK(hipStreamSynchronize(b->st));   // an earlier batch may still read the old tables
     if (b->d_tab) (void)hipFree(b->d_tab);
-    b->d_tab = nullptr;
+    if (b->h_tab) (void)hipHostFree(b->h_tab);
+    b->d_tab = b->h_tab = nullptr;
     b->tab_bytes = 0;
-    if (hipMalloc((void**)&b->d_tab, pack.bytes.size()) != hipSuccess) return SFFT_ERR_ALLOC;
-    b->tab_bytes = pack.bytes.size();
+    if (hipMalloc((void**)&b->d_tab, bytes) != hipSuccess ||
+        hipHostMalloc((void**)&b->h_tab, bytes, hipHostMallocDefault) != hipSuccess)
+      return SFFT_ERR_ALLOC;
+    b->tab_bytes = bytes;
   }
-  HIPCK(hipMemcpyAsync(b->d_tab, pack.bytes.data(), pack.bytes.size(), hipMemcpyHostToDevice,
-                       b->st));
-  HIPCK(hipStreamSynchronize(b->st));   // the packed bytes go out of scope
+  memcpy(b->h_tab, pack.bytes.data(), bytes);
+  HIPCK(hipMemcpyAsync(b->d_tab, b->h_tab, bytes, hipMemcpyHostToDevice, b->st));
+  HIPCK(hipEventRecord(b->tab_ev, b->st));
+  b->tab_pending = 1;
   b->d_jobs = (const PfJob*)(b->d_tab + at_jobs);
   for (auto& g : b->slab) g.t.bind(b->d_tab);
   for (auto& g : b->comb) g.t.bind(b->d_tab);
@@ -274,6 +299,7 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   b->bitmap.bind(b->d_tab);
   b->tab_x.assign(d_x, d_x + b->count);
   b->tab_nodes.assign(nodes, nodes + b->count);
+  b->tab_shape = true;
   return SFFT_OK;
 }
 
@@ -441,6 +467,7 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
       b->lpt = lpt;
       b->nt = nt;
       if (b->jobs.empty()) continue;   // every signal takes the column front end
+      drop_tables(b);
       if ((v = build_tables(b, d_x, none.data())) != SFFT_OK) return v;
       for (int grid : grids) {
         float ms = 0;
@@ -469,6 +496,7 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
     float bq = 1e30f;
     for (int q : qs) {
       for (auto P : b->plans) (which == 0 ? P->qmax_B : P->qmax_W) = q;
+      drop_tables(b);
       if ((v = build_tables(b, d_x, none.data())) != SFFT_OK) return v;
       float ms = 0;
       v = time_ms(b, reps, [&]() -> sfft_status {
@@ -487,8 +515,7 @@ extern "C" sfft_status sfft_batch_tune(sfft_batch* b, const void* const* d_x,
     P->qmax_B = best_q[0];
     P->qmax_W = best_q[1];
   }
-  b->tab_x.clear();   // built again for the chosen shapes
-  drop_graph(b);
+  drop_tables(b);   // built again for the chosen shapes
   if (choice4) {
     choice4[0] = b->lpt;
     choice4[1] = b->nt;
@@ -505,8 +532,7 @@ extern "C" sfft_status sfft_batch_set_shape(sfft_batch* b, int lpt, int nt, int 
   if (!b || lpt < 1 || lpt > 9 || (nt != 128 && nt != 256) || grid < 1 || qmax_bucket < 0 ||
       qmax_bucket > 32 || qmax_comb < 0 || qmax_comb > 32)
     return SFFT_ERR_INVALID;
-  drop_graph(b);
-  b->tab_x.clear();
+  drop_tables(b);
   b->lpt = lpt;
   b->nt = nt;
   b->grid = grid;

@@ -279,8 +279,8 @@ sfft_status sfft_value_adjoint(sfft_plan *plan, const complex_t *d_grad, const s
  * Every stage of all signals runs as one launch (params[i].front_end must be SFFT_FRONT_AUTO,
  * which takes the columns where a single plan does, or SFFT_FRONT_GATHER); with
  * sfft_batch_set_graph(b, 1) the launch sequence is captured into a hipGraph once and replayed
- * (re-captured when the signal or node pointers, filters or shapes change).  Each signal's
- * results are bit-identical to sfft_execute of the same signal with the same plan parameters
+ * (re-captured when filters or launch shapes change; signal and node pointers may change from
+ * call to call, queued calls included).  Each signal's results are bit-identical to sfft_execute of the same signal with the same plan parameters
  * and draws.  stream NULL: the batch makes its own. */
 typedef struct sfft_batch sfft_batch;
 sfft_status sfft_batch_create(const sfft_params *params, int count, sfft_precision prec,
