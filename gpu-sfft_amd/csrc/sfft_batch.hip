@@ -73,7 +73,10 @@ struct sfft_batch {
 };
 
 static void drop_graph(sfft_batch* b) {
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
+  if (b->exec) {
+    (void)hipStreamSynchronize(b->st);   // (it may still run)
+    (void)hipGraphExecDestroy(b->exec);
+  }
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;
   b->graph = nullptr;

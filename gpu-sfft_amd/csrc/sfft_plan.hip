@@ -696,11 +696,27 @@ static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, No
   return run_locate(P, h, d_nodes, P->st, false);
 }
 
+// whether the last asynchronous launch of executable k still runs
+static bool replay_running(sfft_plan* P, int k) {
+  if (!P->g_pending[k]) return false;
+  if (hipEventQuery(P->g_ev[k]) != hipSuccess) {
+    (void)hipGetLastError();   // (not an error of a launch to come)
+    return true;
+  }
+  P->g_pending[k] = 0;
+  return false;
+}
+
+// Destroys the captured graph once its launches are done: nothing says that an executable may be
+// destroyed while it runs, and programs that did ended in a segmentation fault.
 static void drop_plan_graph(sfft_plan* P) {
+  if (P->gexec[0] || P->gexec[1]) (void)hipStreamSynchronize(P->st);
   for (int k = 0; k < 2; ++k) {
     if (P->gexec[k]) (void)hipGraphExecDestroy(P->gexec[k]);
     P->gexec[k] = nullptr;
+    P->g_pending[k] = 0;
   }
+  P->g_last = 0;
   if (P->graph) (void)hipGraphDestroy(P->graph);
   P->graph = nullptr;
 }
@@ -733,24 +749,28 @@ static sfft_status capture(sfft_plan* P, const void* d_x, const HashArgs& h, Nod
   return SFFT_OK;
 }
 
-// Replays the captured transform with these draws.  An asynchronous caller may have launched it
-// before and not waited: its two executables take turns, and one is written only when its last
-// launch is done.
-static sfft_status replay(sfft_plan* P, DrawVals& dv, bool async) {
-  const int k = async ? P->g_next : 0;
-  if (async) P->g_next ^= 1;
-  if (P->g_pending[k]) HIPCK(hipEventSynchronize(P->g_ev[k]));
+// Replays the captured transform with these draws (fresh: it was captured with them).  An
+// asynchronous caller may have launched it before and not waited: an executable is written only
+// when its last launch is done, so a launch behind one that still runs takes a second executable,
+// instantiated when that first happens, and the two take turns.
+static sfft_status replay(sfft_plan* P, DrawVals& dv, bool async, bool fresh) {
+  int k = P->g_last;
+  if (replay_running(P, k)) k ^= 1;
+  if (replay_running(P, k)) HIPCK(hipEventSynchronize(P->g_ev[k]));
   P->g_pending[k] = 0;
+  P->g_last = k;
   if (!P->gexec[k])
     HIPCK(hipGraphInstantiate(&P->gexec[k], P->graph, nullptr, nullptr, 0));
-  // the draws are the head's last argument (fold_slab_kernel's second, hash_clear_kernel's fifth)
-  void* args[5];
-  const int n = P->bins_perm ? 2 : 5;
-  for (int i = 0; i < n - 1; ++i) args[i] = P->g_head_params.kernelParams[i];
-  args[n - 1] = &dv;
-  hipKernelNodeParams kp = P->g_head_params;
-  kp.kernelParams = args;
-  HIPCK(hipGraphExecKernelNodeSetParams(P->gexec[k], P->g_head, &kp));
+  if (!fresh) {
+    // the draws are the head's last argument (fold_slab_kernel's second, hash_clear_kernel's fifth)
+    void* args[5];
+    const int n = P->bins_perm ? 2 : 5;
+    for (int i = 0; i < n - 1; ++i) args[i] = P->g_head_params.kernelParams[i];
+    args[n - 1] = &dv;
+    hipKernelNodeParams kp = P->g_head_params;
+    kp.kernelParams = args;
+    HIPCK(hipGraphExecKernelNodeSetParams(P->gexec[k], P->g_head, &kp));
+  }
   HIPCK(hipGraphLaunch(P->gexec[k], P->st));
   if (async) {
     if (!P->g_ev[k]) HIPCK(hipEventCreateWithFlags(&P->g_ev[k], hipEventDisableTiming));
@@ -786,20 +806,28 @@ static sfft_status enqueue(sfft_plan* P, const void* d_x, const sfft_draws* dr, 
     v = run_head(P, d_x, h, dv);
     return v != SFFT_OK ? v : run_rest(P, d_x, h, d_nodes);
   }
-  if (P->graph && (P->g_x != d_x || P->g_nodes != d_nodes || P->g_count != d_count ||
-                   P->g_cnt_copy != cnt_copy))
+  // Buffers that were not those of the call before are launched kernel by kernel (a capture and an
+  // instantiation take several launched transforms' time, which a caller that rotates its buffers
+  // would pay on every call); the same ones again are captured, once.  The graph of other buffers
+  // is kept until then.
+  const sfft_plan::GraphKey key = {d_x, d_nodes, d_count, cnt_copy};
+  const bool again = key == P->g_before;
+  P->g_before = key;
+  bool fresh = false;
+  if (!P->graph || !(key == P->g_key)) {
+    if (!again) {
+      v = run_head(P, d_x, h, dv);
+      return v != SFFT_OK ? v : run_rest(P, d_x, h, d_nodes);
+    }
     drop_plan_graph(P);
-  if (!P->graph) {
     if ((v = capture(P, d_x, h, d_nodes, dv)) != SFFT_OK) {
       drop_plan_graph(P);
       return v;
     }
-    P->g_x = d_x;
-    P->g_nodes = d_nodes;
-    P->g_count = d_count;
-    P->g_cnt_copy = cnt_copy;
+    P->g_key = key;
+    fresh = true;
   }
-  return replay(P, dv, async);
+  return replay(P, dv, async, fresh);
 }
 
 extern "C" sfft_status sfft_execute_async(sfft_plan* P, const void* d_x, const sfft_draws* dr,
@@ -837,8 +865,8 @@ void* PinnedRange::view(void* h, size_t bytes) {
   return size - off >= bytes ? dev + off : nullptr;
 }
 
-// Graph mode: the transform's launch sequence is captured once and replayed (each replay's draws
-// are set in its first kernel's arguments).  A plan created without a stream gets a
+// Graph mode: the transform's launch sequence is captured when its buffers are those of the call
+// before, and replayed (each replay's draws are set in its first kernel's arguments).  A plan created without a stream gets a
 // stream of its own for this (the legacy default stream cannot be captured).
 extern "C" sfft_status sfft_plan_set_graph(sfft_plan* P, int on) {
   if (!P) return SFFT_ERR_INVALID;
@@ -849,6 +877,7 @@ extern "C" sfft_status sfft_plan_set_graph(sfft_plan* P, int on) {
     HIPCK(hipStreamCreateWithFlags(&P->st, hipStreamNonBlocking));
     P->own_st = 1;
   }
+  P->g_before = sfft_plan::GraphKey();
   P->use_graph = on ? 1 : 0;
   return SFFT_OK;
 }

@@ -82,13 +82,19 @@ struct sfft_plan {
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   hipEvent_t g_ev[2] = {nullptr, nullptr};  // after the last asynchronous launch of each
   int g_pending[2] = {0, 0};
-  int g_next = 0;
+  int g_last = 0;                           // the one launched last
   hipGraphNode_t g_head = nullptr;          // the first kernel, which takes the draws
   hipKernelNodeParams g_head_params = {};
-  const void* g_x = nullptr;
-  Node* g_nodes = nullptr;
-  int* g_count = nullptr;
-  int* g_cnt_copy = nullptr;
+  struct GraphKey {                         // a transform's buffers
+    const void* x = nullptr;
+    Node* nodes = nullptr;
+    int* count = nullptr;
+    int* cnt_copy = nullptr;
+    bool operator==(const GraphKey& o) const {
+      return x == o.x && nodes == o.nodes && count == o.count && cnt_copy == o.cnt_copy;
+    }
+  };
+  GraphKey g_key, g_before;                 // the captured ones, those of the last call
   hipEvent_t ev[9] = {nullptr, nullptr, nullptr, nullptr, nullptr,
                       nullptr, nullptr, nullptr, nullptr};
 };

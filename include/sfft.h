@@ -218,8 +218,10 @@ sfft_status sfft_execute(sfft_plan *plan, const void *d_x, const sfft_draws *dra
                          Node *h_nodes, int *h_count);
 
 /* Graph mode (off by default): the transform's kernel sequence is captured into a hipGraph
- * on first use and replayed by later sfft_execute[_async] calls while the signal and result
- * pointers stay the same (re-captured when they change); the draws go with each replay.
+ * by the second sfft_execute[_async] call in a row on the same signal and result pointers and
+ * replayed by later calls on them; calls on other pointers are launched kernel by kernel until
+ * those come twice in a row (then that graph replaces this one, once its launches are done).
+ * The draws go with each replay.
  * Transforms that are faster launched kernel by kernel are launched that way all the same.  A plan
  * created with stream NULL gets a stream of its own for this.  Profiling
  * (sfft_plan_set_profiling) runs the transform eagerly. */
