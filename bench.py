@@ -80,8 +80,8 @@ def parse():
                     help="filter design mode (setup, outside the timed region): the "
                          "reference's rounding, or the device design without recurrences")
     ap.add_argument("--launch", default="graph", choices=["graph", "eager"],
-                    help="replay each transform from a hipGraph captured once (the default), "
-                         "or enqueue its kernels eagerly")
+                    help="graph: switch the plan's graph mode on, which gives it a stream of its "
+                         "own (either way the kernels are enqueued one by one)")
     ap.add_argument("--copy-probe-mib", type=int, default=0,
                     help="run one plain device copy of this many MiB before the transforms "
                          "(a known-size kernel that calibrates HBM byte counters)")
@@ -413,7 +413,7 @@ def main():
         "vs_baseline": round(R["ms"] / PUBLISHED_MS, 6)
         if args.config == "n27_k16000" and main_prec == "fp64" else None,
         "dtype": "f32" if main_prec == "fp32" else "f64", "data": "synthetic",
-        "front_end": R["front"], "launch": "hipGraph" if args.launch == "graph" else "eager",
+        "front_end": R["front"], "launch": "eager",
         "config": {"workload": f"{args.config}: sfft n=2^{q} k={k} Bcst={Bcst} "
                                f"loops={ll}+{le} thresh={lt} RLFC={rc}x{rl} "
                                f"{'noise ' + str(snr) + 'dB' if snr else 'noiseless'}, "

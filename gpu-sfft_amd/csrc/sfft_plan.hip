@@ -363,21 +363,16 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   return SFFT_OK;
 }
 
-static void drop_plan_graph(sfft_plan* P);
-
 extern "C" void sfft_plan_destroy(sfft_plan* P) {
   if (!P) return;
   if (P->st) (void)hipStreamSynchronize(P->st);
   else (void)hipDeviceSynchronize();
   if (P->st2) (void)hipStreamSynchronize(P->st2);
-  drop_plan_graph(P);
   if (P->own_st) (void)hipStreamDestroy(P->st);
   if (P->st2) (void)hipStreamDestroy(P->st2);
   if (P->ev_fork) (void)hipEventDestroy(P->ev_fork);
   if (P->ev_join) (void)hipEventDestroy(P->ev_join);
   for (auto& e : P->ev)
-    if (e) (void)hipEventDestroy(e);
-  for (auto& e : P->g_ev)
     if (e) (void)hipEventDestroy(e);
   if (P->up_ev) (void)hipEventDestroy(P->up_ev);
   if (P->h_draws) (void)hipHostFree(P->h_draws);
@@ -394,13 +389,10 @@ extern "C" sfft_status sfft_plan_set_filter(sfft_plan* P, const void* d_filter_t
                                             const complex_t* h_filter_win) {
   if (!P || !d_filter_time || !h_filter_win) return SFFT_ERR_INVALID;
   // A transform still running on the plan's streams reads the old taps and window: let it
-  // finish before the window is rewritten (and before the caller may free the old taps).  A
-  // captured graph holds the old taps pointer as a kernel argument: drop it, so the next
-  // graph-mode execute captures the new one.
+  // finish before the window is rewritten (and before the caller may free the old taps).
   if (P->st) HIPCK(hipStreamSynchronize(P->st));
   else HIPCK(hipDeviceSynchronize());
   if (P->st2) HIPCK(hipStreamSynchronize(P->st2));
-  drop_plan_graph(P);
   if (hipMemcpy(P->win, h_filter_win, (size_t)P->m * 16, hipMemcpyHostToDevice) != hipSuccess)
     return SFFT_ERR_HIP;
   if (P->columns) {   // the column fold's bucket-major copy of the taps
@@ -620,8 +612,7 @@ static sfft_status run_locate(sfft_plan* P, const HashArgs& h, Node* d_nodes, hi
 
 // One transform: its first kernel (run_head), then everything after it (run_rest).  The first
 // kernel takes the draws as an argument and leaves them in device memory for the rest: no upload
-// and no gap after one in front of it (n = 2^14, k = 20, replayed: 73 -> 67 us; n = 2^20, k = 1000, FP64
-// 91 -> 85).  Slab fold: the head is the fold, which also clears and copies the comb samples.
+// and no gap after one in front of it (n = 2^20, k = 1000, FP64: 93 -> 86 us).  Slab fold: the head is the fold, which also clears and copies the comb samples.
 // Else it is the clear.
 static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
                             const DrawVals& dv) {
@@ -653,9 +644,8 @@ static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
 // comb samples too) two concurrent chains, joined before the reverse hash: the comb chain (comb
 // FFT, cutoff, bitmaps) on the plan stream and the bucket chain (permute+filter of the gathers,
 // bucket FFT, cutoff) on a second stream, so that the latency-bound kernels of
-// one chain fill the gaps of the other's.  Column front end: the comb FFT is enqueued before the
-// bucket chain, so that a captured graph's first root, which the replay keeps on the launching
-// queue, starts the longer chain.  The gathering front end forks after its comb FFT (beside which
+// one chain fill the gaps of the other's.  Column front end: the comb FFT, which starts the longer
+// chain, is enqueued before the bucket chain.  The gathering front end forks after its comb FFT (beside which
 // its permute+filter's gathers lose).  Profiling (and the streaming front end, whose pass feeds
 // the fold) runs everything serially on the plan stream; with the columns the profile's
 // "streaming pass" interval is the fold (with the comb copy) and its "fold" interval is empty, and
@@ -696,95 +686,11 @@ static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, No
   return run_locate(P, h, d_nodes, P->st, false);
 }
 
-// whether the last asynchronous launch of executable k still runs
-static bool replay_running(sfft_plan* P, int k) {
-  if (!P->g_pending[k]) return false;
-  if (hipEventQuery(P->g_ev[k]) != hipSuccess) {
-    (void)hipGetLastError();   // (not an error of a launch to come)
-    return true;
-  }
-  P->g_pending[k] = 0;
-  return false;
-}
-
-// Destroys the captured graph once its launches are done: nothing says that an executable may be
-// destroyed while it runs, and programs that did ended in a segmentation fault.
-static void drop_plan_graph(sfft_plan* P) {
-  if (P->gexec[0] || P->gexec[1]) (void)hipStreamSynchronize(P->st);
-  for (int k = 0; k < 2; ++k) {
-    if (P->gexec[k]) (void)hipGraphExecDestroy(P->gexec[k]);
-    P->gexec[k] = nullptr;
-    P->g_pending[k] = 0;
-  }
-  P->g_last = 0;
-  if (P->graph) (void)hipGraphDestroy(P->graph);
-  P->graph = nullptr;
-}
-
-// Graph mode launches the kernels one by one where that is faster than a replay: where the comb
-// and bucket stages share their launches (four or five on one stream, each enqueued while the one
-// before it runs; n = 2^20, k = 1000, FP64, with one more: 85 us replayed, 76 launched), and where the head is a
-// slab fold of 64 MB and more: it runs long enough for the launches behind it to be enqueued
-// meanwhile, and the chains then start with less between them than a replay's nodes (n = 2^27,
-// k = 16000, replayed -> launched: FP64 814 -> 790 us, FP32 466 -> 457; n = 2^24 FP32 134 either
-// way).
-static bool graph_as_eager(const sfft_plan* P) {
-  if (paired(P)) return true;
-  return P->bins_perm && (size_t)P->p.n * (P->fp32 ? 8 : 16) >= ((size_t)64 << 20);
-}
-
-static sfft_status capture(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes,
-                           const DrawVals& dv) {
-  HIPCK(hipStreamBeginCapture(P->st, hipStreamCaptureModeThreadLocal));
-  sfft_status v = run_head(P, d_x, h, dv);
-  if (v == SFFT_OK) v = run_rest(P, d_x, h, d_nodes);
-  hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(P->st, &g);
-  P->graph = g;
-  if (v != SFFT_OK) return v;
-  size_t roots = 1;   // the head is the only kernel nothing precedes
-  if (e != hipSuccess || hipGraphGetRootNodes(g, &P->g_head, &roots) != hipSuccess ||
-      roots != 1 || hipGraphKernelNodeGetParams(P->g_head, &P->g_head_params) != hipSuccess)
-    return SFFT_ERR_HIP;
-  return SFFT_OK;
-}
-
-// Replays the captured transform with these draws (fresh: it was captured with them).  An
-// asynchronous caller may have launched it before and not waited: an executable is written only
-// when its last launch is done, so a launch behind one that still runs takes a second executable,
-// instantiated when that first happens, and the two take turns.
-static sfft_status replay(sfft_plan* P, DrawVals& dv, bool async, bool fresh) {
-  int k = P->g_last;
-  if (replay_running(P, k)) k ^= 1;
-  if (replay_running(P, k)) HIPCK(hipEventSynchronize(P->g_ev[k]));
-  P->g_pending[k] = 0;
-  P->g_last = k;
-  if (!P->gexec[k])
-    HIPCK(hipGraphInstantiate(&P->gexec[k], P->graph, nullptr, nullptr, 0));
-  if (!fresh) {
-    // the draws are the head's last argument (fold_slab_kernel's second, hash_clear_kernel's fifth)
-    void* args[5];
-    const int n = P->bins_perm ? 2 : 5;
-    for (int i = 0; i < n - 1; ++i) args[i] = P->g_head_params.kernelParams[i];
-    args[n - 1] = &dv;
-    hipKernelNodeParams kp = P->g_head_params;
-    kp.kernelParams = args;
-    HIPCK(hipGraphExecKernelNodeSetParams(P->gexec[k], P->g_head, &kp));
-  }
-  HIPCK(hipGraphLaunch(P->gexec[k], P->st));
-  if (async) {
-    if (!P->g_ev[k]) HIPCK(hipEventCreateWithFlags(&P->g_ev[k], hipEventDisableTiming));
-    HIPCK(hipEventRecord(P->g_ev[k], P->st));
-    P->g_pending[k] = 1;
-  }
-  return SFFT_OK;
-}
-
 // One transform enqueued on the plan stream: nodes to d_nodes (device memory, or the device
 // view of pinned host memory; nullptr: the plan's buffer), the count to d_count (nullptr: the
 // plan's) and, when cnt_copy is set, also to *cnt_copy.
 static sfft_status enqueue(sfft_plan* P, const void* d_x, const sfft_draws* dr, Node* d_nodes,
-                           int* d_count, int* cnt_copy, bool async) {
+                           int* d_count, int* cnt_copy) {
   if (!P || !d_x) return SFFT_ERR_INVALID;
   if (!P->has_filter) return SFFT_ERR_NO_FILTER;
   sfft_status v = draws_check(P, dr);
@@ -797,42 +703,18 @@ static sfft_status enqueue(sfft_plan* P, const void* d_x, const sfft_draws* dr, 
   memcpy(dv.v, dr->a, (size_t)L * 4);
   memcpy(dv.v + L, dr->ai, (size_t)L * 4);
   memcpy(dv.v + 2 * L, dr->offsets, (size_t)Rl * 4);
-  P->cnt_copy = cnt_copy;   // read by run_locate while this transform is enqueued / captured
+  P->cnt_copy = cnt_copy;   // read by run_locate while this transform is enqueued
   struct Reset {
     sfft_plan* P;
     ~Reset() { P->cnt_copy = nullptr; }
   } reset{P};
-  if (!P->use_graph || P->profile || graph_as_eager(P)) {   // eager
-    v = run_head(P, d_x, h, dv);
-    return v != SFFT_OK ? v : run_rest(P, d_x, h, d_nodes);
-  }
-  // Buffers that were not those of the call before are launched kernel by kernel (a capture and an
-  // instantiation take several launched transforms' time, which a caller that rotates its buffers
-  // would pay on every call); the same ones again are captured, once.  The graph of other buffers
-  // is kept until then.
-  const sfft_plan::GraphKey key = {d_x, d_nodes, d_count, cnt_copy};
-  const bool again = key == P->g_before;
-  P->g_before = key;
-  bool fresh = false;
-  if (!P->graph || !(key == P->g_key)) {
-    if (!again) {
-      v = run_head(P, d_x, h, dv);
-      return v != SFFT_OK ? v : run_rest(P, d_x, h, d_nodes);
-    }
-    drop_plan_graph(P);
-    if ((v = capture(P, d_x, h, d_nodes, dv)) != SFFT_OK) {
-      drop_plan_graph(P);
-      return v;
-    }
-    P->g_key = key;
-    fresh = true;
-  }
-  return replay(P, dv, async, fresh);
+  v = run_head(P, d_x, h, dv);
+  return v != SFFT_OK ? v : run_rest(P, d_x, h, d_nodes);
 }
 
 extern "C" sfft_status sfft_execute_async(sfft_plan* P, const void* d_x, const sfft_draws* dr,
                                           Node* d_nodes, int* d_count) {
-  return enqueue(P, d_x, dr, d_nodes, d_count, nullptr, true);
+  return enqueue(P, d_x, dr, d_nodes, d_count, nullptr);
 }
 
 // The device view of h when h is pinned host memory with room for `bytes` from h on, else
@@ -865,20 +747,20 @@ void* PinnedRange::view(void* h, size_t bytes) {
   return size - off >= bytes ? dev + off : nullptr;
 }
 
-// Graph mode: the transform's launch sequence is captured when its buffers are those of the call
-// before, and replayed (each replay's draws are set in its first kernel's arguments).  A plan created without a stream gets a
-// stream of its own for this (the legacy default stream cannot be captured).
+// Graph mode launches the kernels, as every transform does.  Replaying a captured transform saved
+// 0-12 us of host time where it was not slower anyway (n = 2^14 gathered FP64 72 -> 65 us,
+// n = 2^22, k = 1000, FP32 110 -> 105, FP64 105 either way; n = 2^20 FP64 68 -> 74), and programs
+// that replayed the graphs of several plans or of changing buffers ended now and then in a
+// segmentation fault inside sfft_execute, for which no cause was found.  A plan created without a
+// stream still gets a stream of its own.
 extern "C" sfft_status sfft_plan_set_graph(sfft_plan* P, int on) {
   if (!P) return SFFT_ERR_INVALID;
-  drop_plan_graph(P);
   if (on && !P->st) {
     HIPCK(hipStreamSynchronize(nullptr));
     if (P->up_pending) HIPCK(hipEventSynchronize(P->up_ev));
     HIPCK(hipStreamCreateWithFlags(&P->st, hipStreamNonBlocking));
     P->own_st = 1;
   }
-  P->g_before = sfft_plan::GraphKey();
-  P->use_graph = on ? 1 : 0;
   return SFFT_OK;
 }
 
@@ -1012,7 +894,7 @@ extern "C" sfft_status sfft_execute(sfft_plan* P, const void* d_x, const sfft_dr
   Node* zc =
       h_nodes ? (Node*)PinnedRange().view(h_nodes, (size_t)P->cap * sizeof(Node)) : nullptr;
   if (zc) {
-    sfft_status s = enqueue(P, d_x, dr, zc, P->count, P->h_count_dev, false);
+    sfft_status s = enqueue(P, d_x, dr, zc, P->count, P->h_count_dev);
     if (s != SFFT_OK) return s;
     HIPCK(hipStreamSynchronize(P->st));
     const int cnt = *(volatile int*)P->h_count;
@@ -1020,7 +902,7 @@ extern "C" sfft_status sfft_execute(sfft_plan* P, const void* d_x, const sfft_dr
     if (h_count) *h_count = cnt;
     return cnt > P->cap ? SFFT_ERR_HIT_OVERFLOW : SFFT_OK;
   }
-  sfft_status s = enqueue(P, d_x, dr, P->nodes, P->count, nullptr, false);
+  sfft_status s = enqueue(P, d_x, dr, P->nodes, P->count, nullptr);
   if (s != SFFT_OK) return s;
   // the count and, speculatively, as many nodes as the previous transform had plus 1/32 go
   // back in one round trip; the rest (if the count grew past that) in a second one

@@ -66,35 +66,13 @@ struct sfft_plan {
   int* h_draws = nullptr;
   int* h_count = nullptr;
   int* h_count_dev = nullptr;   // device view of h_count
-  // where the estimation kernel also stores the hit count (nullptr: nowhere); part of the
-  // captured graph, like the node and count pointers
+  // where the estimation kernel also stores the hit count (nullptr: nowhere)
   int* cnt_copy = nullptr;
   hipEvent_t up_ev = nullptr;   // last upload out of h_draws
   int up_pending = 0;
   // optional stage timing (hipEvents at the reference's stage boundaries)
   int profile = 0;
-  // optional hipGraph of the whole transform (front, fold, back), replayed while the signal
-  // and output pointers stay the same; own_st: a stream made for it when the plan had none
-  int use_graph = 0;
-  int own_st = 0;
-  hipGraph_t graph = nullptr;
-  // two executables of it: a replay's draws are set in one while the other may still run
-  hipGraphExec_t gexec[2] = {nullptr, nullptr};
-  hipEvent_t g_ev[2] = {nullptr, nullptr};  // after the last asynchronous launch of each
-  int g_pending[2] = {0, 0};
-  int g_last = 0;                           // the one launched last
-  hipGraphNode_t g_head = nullptr;          // the first kernel, which takes the draws
-  hipKernelNodeParams g_head_params = {};
-  struct GraphKey {                         // a transform's buffers
-    const void* x = nullptr;
-    Node* nodes = nullptr;
-    int* count = nullptr;
-    int* cnt_copy = nullptr;
-    bool operator==(const GraphKey& o) const {
-      return x == o.x && nodes == o.nodes && count == o.count && cnt_copy == o.cnt_copy;
-    }
-  };
-  GraphKey g_key, g_before;                 // the captured ones, those of the last call
+  int own_st = 0;               // st was made by sfft_plan_set_graph: the plan had none
   hipEvent_t ev[9] = {nullptr, nullptr, nullptr, nullptr, nullptr,
                       nullptr, nullptr, nullptr, nullptr};
 };

@@ -166,7 +166,7 @@ class Plan:
         _check(lib.sfft_plan_set_profiling(self._h, int(on)), "sfft_plan_set_profiling")
 
     def set_graph(self, on=True):
-        """Capture the transform into a hipGraph on first use and replay it afterwards."""
+        """Accepted; every transform is launched kernel by kernel (see sfft_plan_set_graph)."""
         _check(lib.sfft_plan_set_graph(self._h, int(on)), "sfft_plan_set_graph")
 
     def stage_times(self):

@@ -217,14 +217,11 @@ sfft_status sfft_execute_async(sfft_plan *plan, const void *d_x, const sfft_draw
 sfft_status sfft_execute(sfft_plan *plan, const void *d_x, const sfft_draws *draws,
                          Node *h_nodes, int *h_count);
 
-/* Graph mode (off by default): the transform's kernel sequence is captured into a hipGraph
- * by the second sfft_execute[_async] call in a row on the same signal and result pointers and
- * replayed by later calls on them; calls on other pointers are launched kernel by kernel until
- * those come twice in a row (then that graph replaces this one, once its launches are done).
- * The draws go with each replay.
- * Transforms that are faster launched kernel by kernel are launched that way all the same.  A plan
- * created with stream NULL gets a stream of its own for this.  Profiling
- * (sfft_plan_set_profiling) runs the transform eagerly. */
+/* Graph mode (off by default).  Every transform is launched kernel by kernel, in graph mode
+ * too: replays of captured transforms gained little and were not safe with several plans or
+ * changing buffers in one program.  A plan created with stream NULL gets a stream of its own
+ * when this is switched on.  (A caller may capture sfft_execute_async on the plan's stream into
+ * a graph of its own; the draws of the captured call are then part of it.) */
 sfft_status sfft_plan_set_graph(sfft_plan *plan, int on);
 
 /* Stage timing with hipEvents on the plan stream (off by default).  After a completed

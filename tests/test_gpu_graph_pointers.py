@@ -1,6 +1,6 @@
-"""Graph mode with signal and result buffers that change from call to call: queued transforms give
-the launched ones' results, and a call on new buffers does not wait for the transforms queued before
-it."""
+"""Transforms whose signal and result buffers change from call to call, in graph mode: queued ones
+give the waited-for ones' results, and a call on new buffers does not wait for the transforms queued
+before it."""
 import numpy as np
 import pytest
 
@@ -9,8 +9,8 @@ from helpers import SMALL_CONFIGS, draws, oracle_filter, params, sparse_signal
 
 pytestmark = pytest.mark.gpu
 
-# configurations and front ends whose transforms graph mode replays
-REPLAYED = [(SMALL_CONFIGS[1], "gather", "fp64"), ((22, 300, 0.99, 2, 2, 3, 256, 2), "columns", "fp32")]
+# transforms whose comb and bucket stages run on two streams
+CONFIGS = [(SMALL_CONFIGS[1], "gather", "fp64"), ((22, 300, 0.99, 2, 2, 3, 256, 2), "columns", "fp32")]
 IDS = ["q14_gather_fp64", "q22_columns_fp32"]
 
 
@@ -39,7 +39,7 @@ def _setup(cfg, front_end, precision, sets):
     return plan, stream, xs, ds, want, bufs
 
 
-@pytest.mark.parametrize("cfg,front_end,precision", REPLAYED, ids=IDS)
+@pytest.mark.parametrize("cfg,front_end,precision", CONFIGS, ids=IDS)
 def test_queued_on_changing_buffers(cfg, front_end, precision):
     import torch
     plan, stream, xs, ds, want, bufs = _setup(cfg, front_end, precision, 3)
@@ -66,7 +66,7 @@ def test_queued_on_changing_buffers(cfg, front_end, precision):
     plan.close()
 
 
-@pytest.mark.parametrize("cfg,front_end,precision", REPLAYED, ids=IDS)
+@pytest.mark.parametrize("cfg,front_end,precision", CONFIGS, ids=IDS)
 def test_new_buffers_do_not_wait(cfg, front_end, precision):
     import torch
     plan, stream, xs, ds, want, bufs = _setup(cfg, front_end, precision, 3)
@@ -79,7 +79,7 @@ def test_new_buffers_do_not_wait(cfg, front_end, precision):
             torch.mm(a, a, out=out)
         busy.record(stream)
     waited = []
-    for s in (0, 1, 2, 2, 2, 0):                 # (the third set: launched, captured, replayed)
+    for s in (0, 1, 2, 2, 2, 0):
         plan.execute_async(xs[s], *ds[s], d_nodes=bufs[s][0], d_count=bufs[s][1])
         waited.append(busy.query())
     torch.cuda.synchronize()
