@@ -110,6 +110,10 @@ extern "C" void sfft_batch_destroy(sfft_batch* b) {
   delete b;
 }
 
+static sfft_status pack_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes,
+                               JobPack& pack, size_t* at_jobs);
+static sfft_status reserve_tables(sfft_batch* b, size_t bytes);
+
 extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
                                          sfft_precision prec, void* stream, sfft_batch** out) {
   if (!params || count <= 0 || !out) return SFFT_ERR_INVALID;
@@ -170,6 +174,16 @@ extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
     P->d_ai = P->d_a + P->p.loops;
     P->d_offs = P->d_a + 2 * P->p.loops;
   }
+  // the tables' memory: their size is known from the shapes
+  const std::vector<const void*> no_x(count, nullptr);
+  const std::vector<Node*> no_nodes(count, nullptr);
+  JobPack pack;
+  size_t at_jobs = 0;
+  if (pack_tables(b, no_x.data(), no_nodes.data(), pack, &at_jobs) == SFFT_OK &&
+      reserve_tables(b, pack.bytes.size()) != SFFT_OK) {
+    sfft_batch_destroy(b);
+    return SFFT_ERR_ALLOC;
+  }
   *out = b;
   return SFFT_OK;
 }
@@ -189,11 +203,8 @@ extern "C" sfft_status sfft_batch_set_filter(sfft_batch* b, int i, const void* d
 // and its nodes go to nodes[i] (the device view of pinned host memory, with a copy in the plan's
 // buffer; nullptr: the plan's buffer alone).  Where only pointers differ from the tables before,
 // every table keeps its size and place, so a captured graph of the launches stays valid.
-static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes) {
-  const bool same_shape = b->tab_shape;
-  if (!same_shape) drop_graph(b);
-  b->tab_shape = false;
-  b->tab_x.clear();
+static sfft_status pack_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes,
+                               JobPack& pack, size_t* at_jobs) {
   b->jobs.clear();
   b->slab.clear();
   b->comb.clear();
@@ -260,8 +271,7 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   }
   b->total_items = item;
   slab_jobs_share(b->slab);
-  JobPack pack;
-  const size_t at_jobs = pack.put(b->jobs.data(), sizeof(PfJob) * b->jobs.size());
+  *at_jobs = pack.put(b->jobs.data(), sizeof(PfJob) * b->jobs.size());
   for (auto& g : b->slab) g.t.pack(pack);
   for (auto& g : b->comb) g.t.pack(pack);
   for (auto& g : b->comb_slab) g.t.pack(pack);
@@ -271,20 +281,37 @@ static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* con
   b->sel_bucket.pack(pack);
   b->clear.pack(pack);
   b->bitmap.pack(pack);
+  return SFFT_OK;
+}
+
+// room for tables of `bytes` (no graph of the old ones, none in use)
+static sfft_status reserve_tables(sfft_batch* b, size_t bytes) {
+  if (b->d_tab) (void)hipFree(b->d_tab);
+  if (b->h_tab) (void)hipHostFree(b->h_tab);
+  b->d_tab = b->h_tab = nullptr;
+  b->tab_bytes = 0;
+  if (hipMalloc((void**)&b->d_tab, bytes) != hipSuccess ||
+      hipHostMalloc((void**)&b->h_tab, bytes, hipHostMallocDefault) != hipSuccess)
+    return SFFT_ERR_ALLOC;
+  b->tab_bytes = bytes;
+  return SFFT_OK;
+}
+
+static sfft_status build_tables(sfft_batch* b, const void* const* d_x, Node* const* nodes) {
+  if (!b->tab_shape) drop_graph(b);
+  b->tab_shape = false;
+  b->tab_x.clear();
+  JobPack pack;
+  size_t at_jobs = 0;
+  sfft_status v = pack_tables(b, d_x, nodes, pack, &at_jobs);
+  if (v != SFFT_OK) return v;
   const size_t bytes = pack.bytes.size();
   if (b->tab_pending) HIPCK(hipEventSynchronize(b->tab_ev));
   b->tab_pending = 0;
   if (bytes > b->tab_bytes) {
     drop_graph(b);
     HIPCK(hipStreamSynchronize(b->st));   // an earlier batch may still read the old tables
-    if (b->d_tab) (void)hipFree(b->d_tab);
-    if (b->h_tab) (void)hipHostFree(b->h_tab);
-    b->d_tab = b->h_tab = nullptr;
-    b->tab_bytes = 0;
-    if (hipMalloc((void**)&b->d_tab, bytes) != hipSuccess ||
-        hipHostMalloc((void**)&b->h_tab, bytes, hipHostMallocDefault) != hipSuccess)
-      return SFFT_ERR_ALLOC;
-    b->tab_bytes = bytes;
+    if ((v = reserve_tables(b, bytes)) != SFFT_OK) return v;
   }
   memcpy(b->h_tab, pack.bytes.data(), bytes);
   HIPCK(hipMemcpyAsync(b->d_tab, b->h_tab, bytes, hipMemcpyHostToDevice, b->st));

@@ -18,7 +18,7 @@ CAP = 524288
 
 
 class _Setup:
-    """two sets of signals and draws of one batch on a torch stream, and their results"""
+    """two sets of signals and draws of one batch on a stream of the caller's, and their results"""
 
     def __init__(self, precision, graph):
         import torch
@@ -29,7 +29,9 @@ class _Setup:
         prms.append(dict(prms[0], B=64, w=64 * 40 + 7, B_thresh=20))   # the slab does not take it
         self.count = len(prms)
         arr = (S._lib.Params * self.count)(*[S.core._cparams(p, 0, 0, "auto") for p in prms])
-        self.stream = torch.cuda.Stream()
+        handle = C.c_void_p()
+        assert C.CDLL("libamdhip64.so").hipStreamCreateWithFlags(C.byref(handle), 1) == 0
+        self.stream = torch.cuda.ExternalStream(handle.value)
         self.b = C.c_void_p()
         assert S.lib.sfft_batch_create(arr, self.count, 1 if precision == "fp32" else 0,
                                        C.c_void_p(self.stream.cuda_stream), C.byref(self.b)) == 0
