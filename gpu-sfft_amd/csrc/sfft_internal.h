@@ -334,8 +334,9 @@ hipError_t adjoint_seed_launch(const int* hits, int nh, const uint8_t* sel, cons
                                int n, const int* ai_dev, int B, int loops, const double2* win,
                                int* head, int* next, double2* u, hipStream_t st);
 // gx[(i ai_l) mod n] = sum of conj(f[i]) gb[l][bucket(i)], loop by loop, every entry written
-hipError_t adjoint_taps_launch(const double2* f, const double2* gb, const int* a_dev, int n,
-                               int B, int w, int loops, int tiled, double2* gx, hipStream_t st);
+hipError_t adjoint_taps_launch(const double2* f, const double2* gb, const int* a_dev,
+                               const int* ai_dev, int n, int B, int w, int loops, int tiled,
+                               double2* gx, hipStream_t st);
 
 // ---- small utilities ---------------------------------------------------------------------
 // scratch memory kept between calls (sfft_pool.hip): allocated and freed in stream order, from

@@ -841,8 +841,8 @@ extern "C" sfft_status sfft_value_adjoint(sfft_plan* P, const complex_t* d_grad,
   f.store = kStoreCplx;
   HIPCK(fft_run(f, P->st));
   const int tiled = (p.fold_mode == SFFT_FOLD_REFERENCE) && (p.n < (1 << 27));
-  HIPCK(adjoint_taps_launch((const double2*)P->d_ft, (const double2*)P->bins_f, P->d_a, p.n,
-                            p.B, p.w, p.loops, tiled, (double2*)d_grad_x, P->st));
+  HIPCK(adjoint_taps_launch((const double2*)P->d_ft, (const double2*)P->bins_f, P->d_a,
+                            P->d_ai, p.n, p.B, p.w, p.loops, tiled, (double2*)d_grad_x, P->st));
   return SFFT_OK;
 }
 
