@@ -156,10 +156,10 @@ extern "C" sfft_status sfft_batch_create(const sfft_params* params, int count,
       hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming) == hipSuccess &&
       hipEventCreateWithFlags(&b->up_ev, hipEventDisableTiming) == hipSuccess &&
       hipEventCreateWithFlags(&b->tab_ev, hipEventDisableTiming) == hipSuccess &&
-      hipMalloc((void**)&b->d_draws, sizeof(int) * b->draw_ints) == hipSuccess &&
+      dev_alloc((void**)&b->d_draws, sizeof(int) * b->draw_ints) == hipSuccess &&
       hipHostMalloc((void**)&b->h_draws, sizeof(int) * b->draw_ints, hipHostMallocDefault) ==
           hipSuccess &&
-      hipMalloc((void**)&b->d_counts, sizeof(int) * (size_t)count) == hipSuccess &&
+      dev_alloc((void**)&b->d_counts, sizeof(int) * (size_t)count) == hipSuccess &&
       hipHostMalloc((void**)&b->h_counts, sizeof(int) * (size_t)count, hipHostMallocDefault) ==
           hipSuccess &&
       hipHostGetDevicePointer((void**)&b->h_counts_dev, b->h_counts, 0) == hipSuccess;
@@ -290,7 +290,7 @@ static sfft_status reserve_tables(sfft_batch* b, size_t bytes) {
   if (b->h_tab) (void)hipHostFree(b->h_tab);
   b->d_tab = b->h_tab = nullptr;
   b->tab_bytes = 0;
-  if (hipMalloc((void**)&b->d_tab, bytes) != hipSuccess ||
+  if (dev_alloc((void**)&b->d_tab, bytes) != hipSuccess ||
       hipHostMalloc((void**)&b->h_tab, bytes, hipHostMallocDefault) != hipSuccess)
     return SFFT_ERR_ALLOC;
   b->tab_bytes = bytes;

@@ -236,7 +236,7 @@ extern "C" Node* outer_loop(complex_t* d_x, int n, complex_t* d_filter_time,
 // ---------------------------------------------------------------------------------------------
 static int cutoff_device(int fp32, const void* d_keys, int N, int K, int* d_out, hipStream_t st) {
   void* w = nullptr;
-  if (hipMalloc(&w, select_work_bytes(1, N)) != hipSuccess) return -1;
+  if (dev_alloc((void**)&w, select_work_bytes(1, N)) != hipSuccess) return -1;
   (void)hipMemsetAsync(w, 0, select_work_bytes(1, N), st);
   SelectWork sw;
   select_work_bind(&sw, w, 1, N);
@@ -259,7 +259,7 @@ extern "C" int samples_indices(complex_t* d_samp, int B, int samp_size, int* d_o
   const double t0 = wall_now();
   if (B < 1 || B >= samp_size) return -1;   // cutoff asserts samp_size >= B + 1
   unsigned long long* keys = nullptr;
-  if (hipMalloc(&keys, (size_t)samp_size * 8) != hipSuccess) return -1;
+  if (dev_alloc((void**)&keys, (size_t)samp_size * 8) != hipSuccess) return -1;
   hipLaunchKernelGGL(keys_c128_kernel, dim3((samp_size + 255) / 256), dim3(256), 0, nullptr,
                      (const double2*)d_samp, keys, samp_size);
   const int rc = cutoff_device(0, keys, samp_size, B, d_output, nullptr);
@@ -335,10 +335,10 @@ extern "C" int restr_loc_freq_coeff(complex_t* d_x, int n, int B_thresh, int W_R
   void *b0 = nullptr, *b1 = nullptr, *keys = nullptr;
   int* doff = nullptr;
   int rc = -1;
-  if (hipMalloc(&b0, (size_t)W_RLFC * 16) == hipSuccess &&
-      hipMalloc(&b1, (size_t)W_RLFC * 16) == hipSuccess &&
-      hipMalloc(&keys, (size_t)W_RLFC * 8) == hipSuccess &&
-      hipMalloc(&doff, 4) == hipSuccess &&
+  if (dev_alloc((void**)&b0, (size_t)W_RLFC * 16) == hipSuccess &&
+      dev_alloc((void**)&b1, (size_t)W_RLFC * 16) == hipSuccess &&
+      dev_alloc((void**)&keys, (size_t)W_RLFC * 8) == hipSuccess &&
+      dev_alloc((void**)&doff, 4) == hipSuccess &&
       hipMemcpy(doff, &offset, 4, hipMemcpyHostToDevice) == hipSuccess) {
     FftLaunch c;
     c.tab = &tab;
@@ -383,9 +383,9 @@ extern "C" int perm_filter_cutoff(complex_t* d_x, int n, complex_t* d_filter_tim
   int rc = -1;
   FftTables tab;
   if (fft_tables_create(lB, 0, 0, &tab) != hipSuccess) return -1;
-  if (hipMalloc(&bins_t, (size_t)B * 16) == hipSuccess &&
-      hipMalloc(&scr, (size_t)B * 16) == hipSuccess &&
-      hipMalloc(&keys, (size_t)B * 8) == hipSuccess && hipMalloc(&dai, 4) == hipSuccess &&
+  if (dev_alloc((void**)&bins_t, (size_t)B * 16) == hipSuccess &&
+      dev_alloc((void**)&scr, (size_t)B * 16) == hipSuccess &&
+      dev_alloc((void**)&keys, (size_t)B * 8) == hipSuccess && dev_alloc((void**)&dai, 4) == hipSuccess &&
       hipMemcpy(dai, &ai, 4, hipMemcpyHostToDevice) == hipSuccess &&
       perm_filter_launch(0, d_x, d_filter_time, bins_t, dai, n, B, d_filter_size, 1, tiled,
                          nullptr) == hipSuccess) {
@@ -426,8 +426,8 @@ extern "C" int reverse_hash(int* d_J, int n, int B_thresh, int B, int a, int ai,
   int *maxfirst = nullptr, *cnt = nullptr, *j2 = nullptr;
   const size_t words = ((size_t)W_RLFC + 31) / 32;
   int rc = -1;
-  if (hipMalloc(&bm, words * 4) == hipSuccess && hipMalloc(&maxfirst, 4) == hipSuccess &&
-      hipMalloc(&cnt, 4) == hipSuccess && hipMalloc(&j2, (size_t)num_RLFC * 4) == hipSuccess &&
+  if (dev_alloc((void**)&bm, words * 4) == hipSuccess && dev_alloc((void**)&maxfirst, 4) == hipSuccess &&
+      dev_alloc((void**)&cnt, 4) == hipSuccess && dev_alloc((void**)&j2, (size_t)num_RLFC * 4) == hipSuccess &&
       hipMemcpy(j2, d_J2, (size_t)num_RLFC * 4, hipMemcpyDefault) == hipSuccess &&
       hipMemcpy(cnt, I_F, 4, hipMemcpyHostToDevice) == hipSuccess &&
       fill_u32(bm, 0u, words, nullptr) == hipSuccess &&
@@ -461,10 +461,10 @@ extern "C" Node* estimate_values(int* d_I, int* I_F, complex_t* d_bins_f, int lo
   Node* h = (Node*)malloc(sizeof(Node) * (size_t)(cnt > 0 ? cnt : 1));
   void *dwin = nullptr, *dnodes = nullptr;
   int *dperm = nullptr, *dcnt = nullptr;
-  bool ok = hipMalloc(&dwin, (size_t)m * 16) == hipSuccess &&
-            hipMalloc(&dnodes, sizeof(Node) * (size_t)(cnt > 0 ? cnt : 1)) == hipSuccess &&
-            hipMalloc(&dperm, (size_t)loops * 4) == hipSuccess &&
-            hipMalloc(&dcnt, 4) == hipSuccess &&
+  bool ok = dev_alloc((void**)&dwin, (size_t)m * 16) == hipSuccess &&
+            dev_alloc((void**)&dnodes, sizeof(Node) * (size_t)(cnt > 0 ? cnt : 1)) == hipSuccess &&
+            dev_alloc((void**)&dperm, (size_t)loops * 4) == hipSuccess &&
+            dev_alloc((void**)&dcnt, 4) == hipSuccess &&
             hipMemcpy(dwin, win.data(), (size_t)m * 16, hipMemcpyHostToDevice) == hipSuccess &&
             hipMemcpy(dperm, permute, (size_t)loops * 4, hipMemcpyHostToDevice) == hipSuccess &&
             hipMemcpy(dcnt, &cnt, 4, hipMemcpyHostToDevice) == hipSuccess &&
@@ -494,7 +494,7 @@ extern "C" int sfft_filter_taps(double lobefrac, double tolerance, double* t0_ou
 extern "C" void cuShift(complex_t* d_x, int n, int r) {   // cuExperiment.cu:507-522
   r = (n + r) % n;
   complex_t* tmp = nullptr;
-  if (hipMalloc(&tmp, (size_t)n * sizeof(complex_t)) != hipSuccess) return;
+  if (dev_alloc((void**)&tmp, (size_t)n * sizeof(complex_t)) != hipSuccess) return;
   (void)hipMemcpy(tmp, d_x + (n - r), (size_t)r * sizeof(complex_t), hipMemcpyDeviceToDevice);
   (void)hipMemcpy(tmp + r, d_x, (size_t)(n - r) * sizeof(complex_t), hipMemcpyDeviceToDevice);
   (void)hipMemcpy(d_x, tmp, (size_t)n * sizeof(complex_t), hipMemcpyDeviceToDevice);
@@ -561,8 +561,8 @@ extern "C" void run_experiment(complex_t* d_x, int n, complex_t* d_filter_time,
 static void fft_results(complex_t* d_x, int n) {   // cudafft_results + print_timing
   void *out = nullptr, *scr = nullptr;
   const int ln = ilog2_(n);
-  if (ln < 1 || hipMalloc(&out, (size_t)n * 16) != hipSuccess ||
-      hipMalloc(&scr, (size_t)n * 16) != hipSuccess) {
+  if (ln < 1 || dev_alloc((void**)&out, (size_t)n * 16) != hipSuccess ||
+      dev_alloc((void**)&scr, (size_t)n * 16) != hipSuccess) {
     if (out) (void)hipFree(out);
     return;
   }
@@ -595,7 +595,7 @@ extern "C" void make_multiple_t(double lobefrac, double tolerance, int n, int b_
     return;
   }
   complex_t* d_ft = nullptr;
-  if (hipMalloc(&d_ft, (size_t)w * sizeof(complex_t)) != hipSuccess) return;
+  if (dev_alloc((void**)&d_ft, (size_t)w * sizeof(complex_t)) != hipSuccess) return;
   std::vector<complex_t> ff((size_t)n);
   const sfft_status s = sfft_make_filter(lobefrac, tolerance, n, b_f, w, d_ft, ff.data(), nullptr);
   if (s != SFFT_OK) {
@@ -630,8 +630,8 @@ extern "C" int cudafft_experiment(int n, double lobefrac, double tolerance, int 
     x_f[LARGE_FREQ[i]].y = 0.0;
   }
   void *a = nullptr, *b = nullptr, *scr = nullptr;
-  if (hipMalloc(&a, (size_t)n * 16) != hipSuccess || hipMalloc(&b, (size_t)n * 16) != hipSuccess ||
-      hipMalloc(&scr, (size_t)n * 16) != hipSuccess)
+  if (dev_alloc((void**)&a, (size_t)n * 16) != hipSuccess || dev_alloc((void**)&b, (size_t)n * 16) != hipSuccess ||
+      dev_alloc((void**)&scr, (size_t)n * 16) != hipSuccess)
     return -1;
   // inverse FFT -> time signal (cuExperiment.cu:91-93)
   (void)hipMemcpy(a, x_f.data(), (size_t)n * 16, hipMemcpyHostToDevice);

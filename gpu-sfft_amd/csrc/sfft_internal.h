@@ -340,10 +340,11 @@ hipError_t adjoint_taps_launch(const double2* f, const double2* gb, const int* a
 
 // ---- small utilities ---------------------------------------------------------------------
 // scratch memory kept between calls (sfft_pool.hip): allocated and freed in stream order, from
-// a pool of the library's own that keeps a bounded amount; work_trim gives the idle rest back
+// a pool of the library's own that keeps a bounded amount
 hipError_t work_alloc(void** p, size_t bytes, hipStream_t st);
 void work_free(void* p, hipStream_t st);
-void work_trim();
+// hipMalloc, once more after giving the idle scratch back (it may be what is missing)
+hipError_t dev_alloc(void** p, size_t bytes);
 hipError_t fill_u32(void* p, uint32_t v, size_t words, hipStream_t st);
 
 }  // namespace sfft

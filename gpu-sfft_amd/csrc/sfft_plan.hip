@@ -140,7 +140,7 @@ hipError_t fft_tables_create(int log2n, int inverse, int is_fp32, FftTables* t) 
     log2Lprev = log2Lcur;
   }
   void* d = nullptr;
-  hipError_t err = hipMalloc(&d, t->bytes ? t->bytes : 16);
+  hipError_t err = dev_alloc(&d, t->bytes ? t->bytes : 16);
   if (err != hipSuccess) return err;
   if (t->bytes) {
     err = hipMemcpy(d, host.data(), t->bytes, hipMemcpyHostToDevice);
@@ -322,13 +322,9 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   items.push_back({(void**)&P->adj_next, (size_t)P->cap * 2 * 4});
   size_t total = 0;
   for (auto& it : items) total = align_up(total, 256) + align_up(it.bytes, 256);
-  if (hipMalloc(&P->ws, total) != hipSuccess) {
-    (void)hipGetLastError();
-    work_trim();   // the scratch kept between calls may be what is missing
-    if (hipMalloc(&P->ws, total) != hipSuccess) {
-      delete P;
-      return SFFT_ERR_ALLOC;
-    }
+  if (dev_alloc(&P->ws, total) != hipSuccess) {
+    delete P;
+    return SFFT_ERR_ALLOC;
   }
   P->ws_bytes = total;
   size_t off = 0;

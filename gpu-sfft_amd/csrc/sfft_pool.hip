@@ -9,7 +9,9 @@
 // user recorded when it returned the block, and the next user's stream waits for that event on
 // the device, whichever stream and thread it is.  At most kKeepBytes stay idle on a device;
 // blocks beyond that, and blocks that kKeepUses allocations in a row had no use for, go back to
-// the runtime, and all idle blocks do when a plan's workspace cannot be allocated.
+// the runtime, and all idle blocks do when device memory cannot be allocated (dev_alloc) and when
+// the caller asks for it (sfft_release_scratch).
+#include <algorithm>
 #include <cstdint>
 #include <map>
 #include <mutex>
@@ -134,16 +136,36 @@ void work_free(void* p, hipStream_t st) {
   }
 }
 
-void work_trim() {
+// the bytes given back; on a stream of its own (the default one may not be used while another
+// thread captures)
+static size_t work_trim() {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
   std::lock_guard<std::mutex> lock(g_mu);
+  const bool any = std::any_of(g_idle.begin(), g_idle.end(),
+                               [&](const Block& b) { return b.dev == dev; });
+  hipStream_t st = nullptr;
+  if (!any || hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return 0;
+  size_t bytes = 0;
   for (size_t i = g_idle.size(); i-- > 0;)
     if (g_idle[i].dev == dev) {
-      give_back(g_idle[i], nullptr);
+      bytes += g_idle[i].bytes;
+      give_back(g_idle[i], st);
       g_idle.erase(g_idle.begin() + i);
     }
-  (void)hipStreamSynchronize(nullptr);
+  (void)hipStreamSynchronize(st);   // (the runtime gives its pool's memory back here)
+  (void)hipStreamDestroy(st);
+  return bytes;
+}
+
+hipError_t dev_alloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  if (work_trim()) e = hipMalloc(p, bytes);
+  (void)hipGetLastError();   // (reported by the status alone)
+  return e;
 }
 
 }  // namespace sfft
+
+extern "C" size_t sfft_release_scratch(void) { return sfft::work_trim(); }

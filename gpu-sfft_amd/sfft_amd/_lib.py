@@ -79,7 +79,7 @@ EXPORTED_FUNCTIONS = [
     "sfft_batch_set_graph", "sfft_batch_execute_async", "sfft_batch_execute",
     "sfft_batch_counts_device", "sfft_batch_tune", "sfft_batch_set_shape",
     "sfft_fft_device", "sfft_twiddle", "sfft_fft_plan_passes", "sfft_version",
-    "sfft_device_count", "sfft_filter_taps", "sfft_make_filter", "sfft_make_filter_ex",
+    "sfft_device_count", "sfft_release_scratch", "sfft_filter_taps", "sfft_make_filter", "sfft_make_filter_ex",
     "sfft_filter_window", "sfft_filter_window_device",
     "sfft_dft_any_device", "sfft_convert_c128_to_c64", "sfft_convert_c64_to_c128",
     "sfft_signal_spectrum", "sfft_signal_synthesize", "sfft_truth_spectrum", "sfft_metric",
@@ -168,6 +168,8 @@ def _declare(L):
     L.sfft_fft_plan_passes.restype = _i
     L.sfft_version.restype = C.c_char_p
     L.sfft_device_count.restype = _i
+    L.sfft_release_scratch.argtypes = []
+    L.sfft_release_scratch.restype = C.c_size_t
     L.sfft_filter_taps.argtypes = [_d, _d, C.POINTER(_d)]
     L.sfft_filter_taps.restype = _i
     L.sfft_make_filter.argtypes = [_d, _d, _i, _i, _i, _p, _p, _p]

@@ -579,6 +579,12 @@ def fft(x, inverse=False, out=None):
     return out
 
 
+def release_scratch():
+    """Gives the current device's idle scratch memory (kept between dense FFTs, truth spectra,
+    filter designs, syntheses and metrics; at most 1 GiB) back; returns its bytes."""
+    return lib.sfft_release_scratch()
+
+
 def dft_any(x, inverse=False):
     """In-place arbitrary-length FP64 DFT (Bluestein) of a device complex128 vector."""
     _check(lib.sfft_dft_any_device(_ptr(x), x.numel(), int(inverse), _stream_handle()),

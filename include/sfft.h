@@ -375,6 +375,10 @@ sfft_status sfft_metric(const Node *nodes, int I_F, int k, const int *locs, comp
 /* ---- library-wide ------------------------------------------------------------------------ */
 const char *sfft_version(void);
 int sfft_device_count(void);
+/* The dense FFT, the truth spectrum, the filter design, the synthesis and the metric keep their
+ * scratch memory between calls (at most 1 GiB idle per device).  Gives the current device's idle
+ * scratch back to the runtime, after the work that used it, and returns its bytes.  Any thread. */
+size_t sfft_release_scratch(void);
 
 #ifdef __cplusplus
 }
