@@ -38,7 +38,8 @@ hipError_t aux_vote_counts(const int* J, int nJ, long long n, int B, int W, int 
 hipError_t aux_bitmap_from_list(const int* J2, int nJ2, int ai, int W, unsigned* bm,
                                 int* maxfirst, hipStream_t st);
 
-// canonical device FFT with caller-provided scratch (in != out for multi-pass sizes)
+// canonical device FFT with caller-provided scratch (in == out for one pass or an even number of
+// passes only)
 hipError_t fft_plain(const void* in, void* out, void* scratch, int log2n, int count, int inverse,
                      int is_fp32, hipStream_t st);
 // the same with L's special load or store (kLoadWiden, kLoadTaps, kStoreHead)

@@ -129,13 +129,6 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return (nb & 7) ? b : (b & 7) * (nb >> 3) + (b >> 3);
 }
 
-template <typename T2>
-__device__ __forceinline__ T2 outer_tw(const PassArgs& A, uint32_t e, int log2Lcur) {
-  if (log2Lcur <= kMaxPassLog) return ((const T2*)A.tdir)[e];
-  const uint32_t lo = e & ((1u << A.s) - 1u), hi = e >> A.s;
-  return cmul(((const T2*)A.thi)[hi], ((const T2*)A.tlo)[lo]);
-}
-
 // LDS layout of a tile: column c at lds[c * RP + LPAD(v)] with one padding slot after every 16
 // elements and a one-slot skew between columns, so the radix-4 stage's stride-4 and stride-16
 // stores and the column-interleaved loads spread over the LDS banks.
@@ -372,8 +365,8 @@ __device__ __forceinline__ void fft_stage2(T2* lds, int RP, int r, int log2ncol,
 }
 
 // TW: the pass's outer twiddles, known at compile time so that the load phase is straight-line
-// code: 0 none (the first pass), 1 direct table entries, 2 products of a high and a low entry
-enum PassTw { kTwNone = 0, kTwDirect = 1, kTwSplit = 2 };
+// code: none (the first pass) or products of a high and a low table entry
+enum PassTw { kTwNone = 0, kTwSplit = 1 };
 
 // (bx, by) of nbx: the workgroup's tile and batch (comb gathers: tile and batch in bx alone)
 template <typename Real, int LOADX, int STORE, int TW>
@@ -473,7 +466,6 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
   // threads) or 16 bytes x 2 (FP64, 1024 threads: within 64 registers); the comb-gathering
   // pass issues all of its loads together
   constexpr int LB = (LOAD == kLoadComb) ? EPT : (sizeof(Real) == 8 ? 2 : 4);
-  constexpr bool split = (TW == kTwSplit);   // log2Lcur > kMaxPassLog
   const T2* __restrict__ twR = (const T2*)A.twR;
   const T2* __restrict__ tw4 = (const T2*)A.tw4;
   // batch kb: loads elements e = tid + (kb + k)*NT (k < LB), with the outer twiddle applied
@@ -518,39 +510,29 @@ __device__ __forceinline__ void fft_pass_body(const PassArgs& A, int bx, int nbx
       val[k].y = vv[k].y;
     }
     if constexpr (!first) {
-      // outer twiddles W_Lcur^((t0+c)*v): a direct table entry, or the product of a high and
-      // a low table entry (every table load of the batch issued first, as for the data)
+      // outer twiddles W_Lcur^((t0+c)*v): the product of a high and a low table entry (every
+      // table load of the batch issued first, as for the data)
       V2 tw[LB], tl[LB];
-      if constexpr (split) {
-        const V2* __restrict__ thi = (const V2*)A.thi;
-        const V2* __restrict__ tlo = (const V2*)A.tlo;
-        const uint32_t lmask = (1u << A.s) - 1u;
+      const V2* __restrict__ thi = (const V2*)A.thi;
+      const V2* __restrict__ tlo = (const V2*)A.tlo;
+      const uint32_t lmask = (1u << A.s) - 1u;
 #pragma unroll
-        for (int k = 0; k < LB; ++k) {
-          const int e = min(tid + (kb + k) * NT, TE - 1);
-          const uint32_t ex = (uint32_t)((t0 + (e & (ncol - 1))) * (e >> log2ncol));
-          tw[k] = thi[ex >> A.s];
-          tl[k] = tlo[ex & lmask];
-        }
+      for (int k = 0; k < LB; ++k) {
+        const int e = min(tid + (kb + k) * NT, TE - 1);
+        const uint32_t ex = (uint32_t)((t0 + (e & (ncol - 1))) * (e >> log2ncol));
+        tw[k] = thi[ex >> A.s];
+        tl[k] = tlo[ex & lmask];
+      }
 #pragma unroll
-        for (int k = 0; k < LB; ++k) {
-          T2 hi, lo;
-          hi.x = tw[k].x;
-          hi.y = tw[k].y;
-          lo.x = tl[k].x;
-          lo.y = tl[k].y;
-          const T2 w = cmul(hi, lo);
-          tw[k].x = w.x;
-          tw[k].y = w.y;
-        }
-      } else {
-        const V2* __restrict__ tdir = (const V2*)A.tdir;
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-          const int e = min(tid + (kb + k) * NT, TE - 1);
-          const uint32_t ex = (uint32_t)((t0 + (e & (ncol - 1))) * (e >> log2ncol));
-          tw[k] = tdir[ex];
-        }
+      for (int k = 0; k < LB; ++k) {
+        T2 hi, lo;
+        hi.x = tw[k].x;
+        hi.y = tw[k].y;
+        lo.x = tl[k].x;
+        lo.y = tl[k].y;
+        const T2 w = cmul(hi, lo);
+        tw[k].x = w.x;
+        tw[k].y = w.y;
       }
 #pragma unroll
       for (int k = 0; k < LB; ++k) {
@@ -773,12 +755,25 @@ static hipError_t launch_pass(const PassArgs& A, int tiles, int batch, hipStream
   return launch_tile<Real, LOAD, STORE, TW>(A, tiles, batch, st);
 }
 
+// the stores that a special load occurs with: combs give keys alone, buckets spectra and keys
+static constexpr bool occurs(int load, int store) {
+  if (load == kLoadPerm) return store != kStoreKeys;
+  if (load == kLoadComb || load == kLoadCombRows || load == kLoadCombRowsG)
+    return store != kStoreBoth;
+  return true;
+}
+
 template <typename Real, int LOAD, int TW>
 static hipError_t dispatch_store(const PassArgs& A, int store, int tiles, int batch,
                                  hipStream_t st) {
   if (store == kStoreCplx) return launch_pass<Real, LOAD, kStoreCplx, TW>(A, tiles, batch, st);
-  if (store == kStoreKeys) return launch_pass<Real, LOAD, kStoreKeys, TW>(A, tiles, batch, st);
-  return launch_pass<Real, LOAD, kStoreBoth, TW>(A, tiles, batch, st);
+  if constexpr (occurs(LOAD, kStoreKeys)) {
+    if (store == kStoreKeys) return launch_pass<Real, LOAD, kStoreKeys, TW>(A, tiles, batch, st);
+  }
+  if constexpr (occurs(LOAD, kStoreBoth)) {
+    if (store == kStoreBoth) return launch_pass<Real, LOAD, kStoreBoth, TW>(A, tiles, batch, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 // the FP64-only loads and stores (truth spectra, filter design)
@@ -798,8 +793,6 @@ static hipError_t dispatch_fp64(const PassArgs& A, int load, int store, int tw, 
   if (load != kLoadPlain) return hipErrorInvalidValue;
   if (tw == kTwSplit)
     return launch_pass<double, kLoadPlain, kStoreHead, kTwSplit>(A, tiles, batch, st);
-  if (tw == kTwDirect)
-    return launch_pass<double, kLoadPlain, kStoreHead, kTwDirect>(A, tiles, batch, st);
   return launch_pass<double, kLoadPlain, kStoreHead, kTwNone>(A, tiles, batch, st);
 }
 
@@ -819,8 +812,6 @@ static hipError_t dispatch_pass(const PassArgs& A, int load, int store, int tw, 
     return launch_pass<Real, kLoadRows, kStoreCplx, kTwNone>(A, tiles, 1, st);
   if (tw == kTwSplit)
     return dispatch_store<Real, kLoadPlain, kTwSplit>(A, store, tiles, batch, st);
-  if (tw == kTwDirect)
-    return dispatch_store<Real, kLoadPlain, kTwDirect>(A, store, tiles, batch, st);
   return dispatch_store<Real, kLoadPlain, kTwNone>(A, store, tiles, batch, st);
 }
 
@@ -949,7 +940,6 @@ static hipError_t each_pass(const FftLaunch& L, F&& fn) {
     A.inverse = T.inverse;
     A.twR = T.twR[p];
     A.tw4 = T.tw4[p];
-    A.tdir = T.tdir[p];
     A.thi = T.thi[p];
     A.tlo = T.tlo[p];
     A.s = T.s[p];
@@ -969,7 +959,7 @@ static hipError_t each_pass(const FftLaunch& L, F&& fn) {
     A.digits = last ? L.digits : nullptr;
     A.hist = last ? L.hist : nullptr;
     const int store = last ? L.store : kStoreCplx;
-    const int tw = (p == 0) ? kTwNone : (log2Lcur > kMaxPassLog ? kTwSplit : kTwDirect);
+    const int tw = (p == 0) ? kTwNone : kTwSplit;
     if (load != kLoadPlain && tw != kTwNone) return hipErrorInvalidValue;
     const hipError_t e = fn(p, A, load, store, tw, tiles);
     if (e != hipSuccess) return e;
@@ -1036,9 +1026,7 @@ template <typename Real>
 static hipError_t pair_pass(const OnePass& a, const OnePass& b, hipStream_t st) {
   if (a.load == kLoadCombRows) return pair_first<Real, kLoadCombRows>(a, b, st);
   if (a.load == kLoadCombRowsG) return pair_first<Real, kLoadCombRowsG>(a, b, st);
-  if (a.tw == kTwSplit)
-    return pair_go<Real, kLoadPlain, kStoreKeys, kLoadPlain, kStoreBoth, kTwSplit>(a, b, st);
-  return pair_go<Real, kLoadPlain, kStoreKeys, kLoadPlain, kStoreBoth, kTwDirect>(a, b, st);
+  return pair_go<Real, kLoadPlain, kStoreKeys, kLoadPlain, kStoreBoth, kTwSplit>(a, b, st);
 }
 
 // the passes of L (two at most), or fewer than L has where one of them has no quarter tile
@@ -1142,9 +1130,16 @@ static hipError_t launch_jobs(const FftGroup& g, hipStream_t st) {
 
 template <typename Real, int LOAD, int TW>
 static hipError_t jobs_store(const FftGroup& g, hipStream_t st) {
+  // (a batch's combs never start with a plain load)
+  constexpr bool keys = occurs(LOAD, kStoreKeys) && !(LOAD == kLoadPlain && TW == kTwNone);
   if (g.store == kStoreCplx) return launch_jobs<Real, LOAD, kStoreCplx, TW>(g, st);
-  if (g.store == kStoreKeys) return launch_jobs<Real, LOAD, kStoreKeys, TW>(g, st);
-  return launch_jobs<Real, LOAD, kStoreBoth, TW>(g, st);
+  if constexpr (keys) {
+    if (g.store == kStoreKeys) return launch_jobs<Real, LOAD, kStoreKeys, TW>(g, st);
+  }
+  if constexpr (occurs(LOAD, kStoreBoth)) {
+    if (g.store == kStoreBoth) return launch_jobs<Real, LOAD, kStoreBoth, TW>(g, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 template <typename Real>
@@ -1155,7 +1150,6 @@ static hipError_t jobs_pass(const FftGroup& g, hipStream_t st) {
   if (g.load == kLoadPerm) return jobs_store<Real, kLoadPerm, kTwNone>(g, st);
   if (g.load != kLoadPlain) return hipErrorInvalidValue;
   if (g.tw == kTwSplit) return jobs_store<Real, kLoadPlain, kTwSplit>(g, st);
-  if (g.tw == kTwDirect) return jobs_store<Real, kLoadPlain, kTwDirect>(g, st);
   return jobs_store<Real, kLoadPlain, kTwNone>(g, st);
 }
 

@@ -450,7 +450,8 @@ __global__ __launch_bounds__(EST_NT) void estimate_kernel(EstArgs j) {
   }
 }
 
-// The hits of the places before bx, one wave: publishes this place's total, adds up the totals of
+// The hits of the places before bx, one wave (the decoupled look-back of Merrill and Garland's
+// single-pass prefix scan): publishes this place's total, adds up the totals of
 // the 64 places before it at a time until it meets one whose sum with all before it is published,
 // and publishes its own such sum.  A place is taken by a running block, which publishes its total
 // before it waits for anything but its own threads, so every wait ends whatever the order or

@@ -28,7 +28,6 @@ struct FftTables {
   int npass = 0;
   int logs[kMaxPasses] = {0, 0, 0, 0};
   const void* twR[kMaxPasses] = {nullptr, nullptr, nullptr, nullptr};   // R entries
-  const void* tdir[kMaxPasses] = {nullptr, nullptr, nullptr, nullptr};  // Lcur entries
   const void* thi[kMaxPasses] = {nullptr, nullptr, nullptr, nullptr};   // Lcur >> s
   const void* tlo[kMaxPasses] = {nullptr, nullptr, nullptr, nullptr};   // 1 << s
   const void* tw4[kMaxPasses] = {nullptr, nullptr, nullptr, nullptr};   // radix-4 quads
@@ -70,8 +69,9 @@ enum FftLoad { kLoadPlain = 0, kLoadComb = 1, kLoadCombRows = 2, kLoadPerm = 3, 
 enum FftStore { kStoreCplx = 0, kStoreKeys = 1, kStoreBoth = 2, kStoreHead = 3 };
 
 // One canonical FFT of `batch` transforms.  Passes ping-pong between out and scratch so that
-// the last pass lands in `out` (keys for kStoreKeys/kStoreBoth).  in may equal out only for
-// single-pass sizes.  The comb loader reads element j of batch b from
+// the last pass lands in `out` (keys for kStoreKeys/kStoreBoth).  in may equal out where the
+// first pass does not write out while others read in: for one pass, and for an even number of
+// passes (the first writes the scratch).  The comb loader reads element j of batch b from
 // x[offs[b] + j * sigma] (pass 0); in is then ignored.
 struct FftLaunch {
   const FftTables* tab = nullptr;
@@ -203,8 +203,8 @@ hipError_t stream_scatter_launch(int is_fp32, const void* x, void* T, void* y, c
 // ---- top-K select over `segs` key segments of N keys (stride seg_stride) ----------------
 struct SelectWork {
   void* state = nullptr;      // per segment: threshold, top digit, counters
-  unsigned* hist = nullptr;   // segs * 4096 column sums, then segs * nchunks * 4096 rows
-  unsigned* done = nullptr;   // segs (zero between calls)
+  unsigned* hist = nullptr;   // segs * 4096 column sums, then segs * nchunks * 4096 rows (nullptr:
+                              // counted, every select takes the FFT's histograms)
   int* cnt = nullptr;         // segs * nchunks: selected before each block (ordered mode)
   void* cand_key = nullptr;   // segs * N keys
   int* cand_idx = nullptr;    // segs * N
@@ -218,8 +218,8 @@ struct SelectWork {
 };
 // any N >= 2 (the composite key's index field takes ceil(log2 N) bits); the workspace must
 // start zeroed
-size_t select_work_bytes(int segs, int N);
-void select_work_bind(SelectWork* w, void* base, int segs, int N);
+size_t select_work_bytes(int segs, int N, bool counted = false);
+void select_work_bind(SelectWork* w, void* base, int segs, int N, bool counted = false);
 // out[s*K + j]: the K largest keys of segment s (ties by lower index); ascending indices when
 // `ordered`, otherwise the same set in arbitrary order.  bits (optional, ordered mode): the
 // selection as a bitmap, ceil(N/32) words per segment, every word written.  map (optional,

@@ -79,7 +79,6 @@ struct PassArgs {
   int inverse;
   const void* twR;
   const void* tw4;      // radix-4 stage twiddle quads (see fft_tables_create)
-  const void* tdir;
   const void* thi;
   const void* tlo;
   int s;

@@ -68,11 +68,11 @@ hipError_t fft_tables_create(int log2n, int inverse, int is_fp32, FftTables* t) 
   t->is_fp32 = is_fp32;
   t->npass = fft_plan_passes(log2n, t->logs);
   const size_t esz = is_fp32 ? 8 : 16;
-  // layout: per pass [twR (R)] [tdir (Lcur) | thi (Lcur>>s) tlo (1<<s)] [tw4]; tw4: for
+  // layout: per pass [twR (R)] [thi (Lcur>>s) tlo (1<<s), after the first pass] [tw4]; tw4: for
   // each radix-4 stage with ns = 4^k > 1 (k = 1, 2, ... while 2k <= r - 2), ns quads
   // {twR[jm*t], twR[2*jm*t], twR[3*jm*t], 0} (t = R / (4*ns), jm < ns), stage k at quad
   // (4^k - 4) / 3: a stage's three twiddles of neighbouring butterflies are neighbours
-  size_t cnt[kMaxPasses][5] = {};
+  size_t cnt[kMaxPasses][4] = {};
   size_t total = 0;
   int log2Lprev = 0;
   for (int p = 0; p < t->npass; ++p) {
@@ -80,17 +80,13 @@ hipError_t fft_tables_create(int log2n, int inverse, int is_fp32, FftTables* t) 
     const int log2Lcur = log2Lprev + r;
     cnt[p][0] = (size_t)1 << r;
     if (p > 0) {
-      if (log2Lcur <= kMaxPassLog) {
-        cnt[p][1] = (size_t)1 << log2Lcur;
-      } else {
-        // low table of at most 256 entries: read at scattered indices, it stays in L1
-        t->s[p] = (log2Lcur + 1) / 2 < 8 ? (log2Lcur + 1) / 2 : 8;
-        cnt[p][2] = ((size_t)1 << log2Lcur) >> t->s[p];
-        cnt[p][3] = (size_t)1 << t->s[p];
-      }
+      // low table of at most 256 entries: read at scattered indices, it stays in L1
+      t->s[p] = (log2Lcur + 1) / 2 < 8 ? (log2Lcur + 1) / 2 : 8;
+      cnt[p][1] = ((size_t)1 << log2Lcur) >> t->s[p];
+      cnt[p][2] = (size_t)1 << t->s[p];
     }
-    for (int k = 1; 2 * k <= r - 2; ++k) cnt[p][4] += (size_t)4 << (2 * k);
-    for (int j = 0; j < 5; ++j) total += cnt[p][j];
+    for (int k = 1; 2 * k <= r - 2; ++k) cnt[p][3] += (size_t)4 << (2 * k);
+    for (int j = 0; j < 4; ++j) total += cnt[p][j];
     log2Lprev = log2Lcur;
   }
   t->bytes = total * esz;
@@ -114,7 +110,7 @@ hipError_t fft_tables_create(int log2n, int inverse, int is_fp32, FftTables* t) 
     off += esz;
   };
   log2Lprev = 0;
-  size_t start[kMaxPasses][5] = {};
+  size_t start[kMaxPasses][4] = {};
   for (int p = 0; p < t->npass; ++p) {
     const int r = t->logs[p];
     const int log2Lcur = log2Lprev + r;
@@ -122,12 +118,10 @@ hipError_t fft_tables_create(int log2n, int inverse, int is_fp32, FftTables* t) 
     start[p][0] = off;
     for (uint64_t e = 0; e < R; ++e) put(e, R);
     start[p][1] = off;
-    for (size_t e = 0; e < cnt[p][1]; ++e) put(e, Lcur);
+    for (size_t e = 0; e < cnt[p][1]; ++e) put((uint64_t)e << t->s[p], Lcur);
     start[p][2] = off;
-    for (size_t e = 0; e < cnt[p][2]; ++e) put((uint64_t)e << t->s[p], Lcur);
+    for (size_t e = 0; e < cnt[p][2]; ++e) put(e, Lcur);
     start[p][3] = off;
-    for (size_t e = 0; e < cnt[p][3]; ++e) put(e, Lcur);
-    start[p][4] = off;
     for (int k = 1; 2 * k <= r - 2; ++k) {
       const uint64_t ns = 1ull << (2 * k), ts = R / (4 * ns);
       for (uint64_t jm = 0; jm < ns; ++jm) {
@@ -153,10 +147,9 @@ hipError_t fft_tables_create(int log2n, int inverse, int is_fp32, FftTables* t) 
   for (int p = 0; p < t->npass; ++p) {
     unsigned char* base = (unsigned char*)d;
     t->twR[p] = base + start[p][0];
-    t->tdir[p] = cnt[p][1] ? base + start[p][1] : nullptr;
-    t->thi[p] = cnt[p][2] ? base + start[p][2] : nullptr;
-    t->tlo[p] = cnt[p][3] ? base + start[p][3] : nullptr;
-    t->tw4[p] = cnt[p][4] ? base + start[p][4] : nullptr;
+    t->thi[p] = cnt[p][1] ? base + start[p][1] : nullptr;
+    t->tlo[p] = cnt[p][2] ? base + start[p][2] : nullptr;
+    t->tw4[p] = cnt[p][3] ? base + start[p][3] : nullptr;
   }
   return hipSuccess;
 }
@@ -301,8 +294,8 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   items.push_back({(void**)&P->J2, (size_t)Rl * K * 4});
   void* selW_base = nullptr;
   void* selB_base = nullptr;
-  items.push_back({&selW_base, select_work_bytes(Rl, (int)W)});
-  items.push_back({&selB_base, select_work_bytes(Ll, (int)B)});
+  items.push_back({&selW_base, select_work_bytes(Rl, (int)W, true)});
+  items.push_back({&selB_base, select_work_bytes(Ll, (int)B, true)});
   // the bitmaps, and behind them the histograms of the chained cutoffs and the walk's ticket and
   // places, cleared together
   const size_t bmw = ((size_t)Ll * P->bm_words + 63) / 64 * 64;
@@ -338,9 +331,9 @@ extern "C" sfft_status sfft_plan_create(const sfft_params* prm, sfft_precision p
   P->hist_W = histW ? P->bitmap + bmw : nullptr;
   P->hist_B = histB ? P->bitmap + bmw + histW : nullptr;
   P->ticket = P->bitmap + bmw + histW + histB;
-  select_work_bind(&P->selW, selW_base, Rl, (int)W);
-  select_work_bind(&P->selB, selB_base, Ll, (int)B);
-  // select state must start at zero (hist/done are reset by the kernels themselves)
+  select_work_bind(&P->selW, selW_base, Rl, (int)W, true);
+  select_work_bind(&P->selB, selB_base, Ll, (int)B, true);
+  // select state must start at zero
   if (hipMemset(P->ws, 0, total) != hipSuccess ||
       fft_tables_create(P->log2B, 0, P->fp32, &P->tabB) != hipSuccess ||
       fft_tables_create(P->log2W, 0, P->fp32, &P->tabW) != hipSuccess ||

@@ -64,14 +64,17 @@ static int sel_chunk(int N) {
   return c;
 }
 
-size_t select_work_bytes(int segs, int N) {
-  const int nch = (N + sel_chunk(N) - 1) / sel_chunk(N);
-  return (size_t)segs * sizeof(SelState) + (size_t)segs * (nch + 1) * SEL_BINS * 4 +
-         (size_t)segs * 4 + (size_t)segs * nch * 4 * 3 + (size_t)segs * N * 8 * 2 +
-         (size_t)segs * N * 4 * 3 + 4096;
+static size_t hist_words(int segs, int nch, bool counted) {
+  return counted ? 0 : (size_t)segs * (nch + 1) * SEL_BINS;
 }
 
-void select_work_bind(SelectWork* w, void* base, int segs, int N) {
+size_t select_work_bytes(int segs, int N, bool counted) {
+  const int nch = (N + sel_chunk(N) - 1) / sel_chunk(N);
+  return (size_t)segs * sizeof(SelState) + hist_words(segs, nch, counted) * 4 +
+         (size_t)segs * nch * 4 * 3 + (size_t)segs * N * 8 * 2 + (size_t)segs * N * 4 * 3 + 4096;
+}
+
+void select_work_bind(SelectWork* w, void* base, int segs, int N, bool counted) {
   const int nch = (N + sel_chunk(N) - 1) / sel_chunk(N);
   char* p = (char*)base;
   auto take = [&](size_t bytes) {
@@ -80,8 +83,7 @@ void select_work_bind(SelectWork* w, void* base, int segs, int N) {
     return r;
   };
   w->state = take((size_t)segs * sizeof(SelState));
-  w->hist = (unsigned*)take((size_t)segs * (nch + 1) * SEL_BINS * 4);
-  w->done = (unsigned*)take((size_t)segs * 4);
+  w->hist = counted ? nullptr : (unsigned*)take(hist_words(segs, nch, false) * 4);
   w->cnt = (int*)take((size_t)segs * nch * 4);
   w->cand_key = take((size_t)segs * N * 8);
   w->cand_idx = (int*)take((size_t)segs * N * 4);
@@ -250,8 +252,8 @@ __device__ __forceinline__ void sel_split_body(const K* __restrict__ keys, long 
     s_d0 = 0;
   }
   // the top digit d0 holding the K-th largest key, from the column sums: every block finds
-  // the same one (16 KB of sums, no separate pick launch); block 0 records it and the count
-  // still needed inside it for the refine
+  // the same one (16 KB of sums, or the FFT's kSelCopies histograms of 16 KB each: no separate
+  // pick launch); block 0 records it and the count still needed inside it for the refine
   {
     const unsigned* gh = ghist + (size_t)seg * nsum * SEL_BINS;
     unsigned v[4];
@@ -1088,6 +1090,7 @@ static hipError_t select_job(SelJob& j, const void* keys, long long seg_stride, 
   if (ordered && digits && !select_in_block(N)) return hipErrorInvalidValue;
   if (mark && !select_in_block(N)) return hipErrorInvalidValue;   // the one-workgroup select marks
   if (N < 2 || K < 1 || K > N || segs < 1) return hipErrorInvalidValue;
+  if (!hist && !w.hist && !select_in_block(N)) return hipErrorInvalidValue;
   j = SelJob();
   j.chunk = sel_chunk(N);
   j.nchunks = (N + j.chunk - 1) / j.chunk;
@@ -1108,7 +1111,7 @@ static hipError_t select_job(SelJob& j, const void* keys, long long seg_stride, 
   // work layout: column sums, then the per-block histogram rows
   j.sums = hist ? hist : w.hist;
   j.nsum = hist ? kSelCopies : 1;
-  j.rows = w.hist + (size_t)segs * SEL_BINS;
+  j.rows = w.hist ? w.hist + (size_t)segs * SEL_BINS : nullptr;
   j.state = w.state;
   j.blk_key = w.blk_key;
   j.blk_idx = w.blk_idx;
