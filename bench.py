@@ -201,7 +201,7 @@ def run_precision(args, S, prm, prec, seeds_draws, snr, log):
     nodes, cnt = plan.execute(x, *seeds_draws[0], copy=True)
     acc = S.metric(nodes, k, locs, X)
     log(f"[bench] {prec}: {args.steps} steps {ms:.3f} ms/step over {D} draw sets (per-set "
-        f"medians {min(per_draw):.3f}..{max(per_draw):.3f}, {args.launch}); stages(ms) "
+        f"medians {min(per_draw):.3f}..{max(per_draw):.3f}); stages(ms) "
         + " ".join(f"{kk}={v:.3f}" for kk, v in stages_ms.items()))
     log(f"[bench] {prec}: I_F={cnt} missed={acc['missed_est']},{acc['missed_res']} "
         f"MSE*k={acc['mse_k']:.4e} MSE={acc['mse']:.4e}")

@@ -14,7 +14,7 @@ NAME_PART filters the kernel names (substring match, any of them).
     python3 gpu-sfft_amd/sfft_amd/rocpd_summary.py timeline RUN_results.db [LAST]
 
 `timeline`: per transform of a `--kernel-trace` run (from its first kernel, `hash_clear_kernel`
-or, with the column front end, `fold_slab_kernel`, to the next `estimate_kernel`, its last),
+or, with the slab fold, `fold_slab_kernel`, to the next `nodes_kernel`, its last),
 the span, the union of kernel busy time and the idle rest; then the last LAST transforms of
 each precision (default 1) kernel by kernel: start, duration, grid, workgroup, LDS bytes and
 VGPRs per dispatch.
@@ -99,12 +99,12 @@ def counters(path, parts):
 
 def _transforms(rows):
     """(first, last) row indices of each transform: from its first kernel (hash_clear_kernel,
-    or fold_slab_kernel where the slab fold does the clear) to its estimate_kernel."""
+    or fold_slab_kernel where the slab fold does the clear) to its nodes_kernel."""
     out, i = [], 0
     while i < len(rows):
         if "hash_clear_kernel" in rows[i]["name"] or "fold_slab_kernel" in rows[i]["name"]:
             j = i
-            while j < len(rows) and "estimate_kernel" not in rows[j]["name"]:
+            while j < len(rows) and "nodes_kernel" not in rows[j]["name"]:
                 j += 1
             if j < len(rows):
                 out.append((i, j))
@@ -135,7 +135,7 @@ def timeline(path, last):
             else:
                 busy, cs, ce = busy + ce - cs, s, e
         busy += ce - cs
-        prec = "fp32" if any("<float" in d["name"] or "unsigned int>" in d["name"]
+        prec = "fp32" if any("<float" in d["name"] or "<unsigned int" in d["name"]
                              for d in rows[i:j + 1]) else "fp64"
         spans.setdefault(prec, []).append((i, j))
         print(f"{prec:9s} {(e0 - s0) / 1e3:8.1f} {busy / 1e3:8.1f} {(e0 - s0 - busy) / 1e3:8.1f} "
