@@ -631,14 +631,17 @@ static sfft_status run_head(sfft_plan* P, const void* d_x, const HashArgs& h,
 
 // After the head (and the column fold of a shape that the slab does not take, which copies the
 // comb samples too) two concurrent chains, joined before the reverse hash: the comb chain (comb
-// FFT, cutoff, bitmaps) on the plan stream and the bucket chain (permute+filter of the gathers,
-// bucket FFT, cutoff) on a second stream, so that the latency-bound kernels of
-// one chain fill the gaps of the other's.  Column front end: the comb FFT, which starts the longer
-// chain, is enqueued before the bucket chain.  The gathering front end forks after its comb FFT (beside which
-// its permute+filter's gathers lose).  Profiling (and the streaming front end, whose pass feeds
-// the fold) runs everything serially on the plan stream; with the columns the profile's
-// "streaming pass" interval is the fold (with the comb copy) and its "fold" interval is empty, and
-// with the slab fold its "clear" interval too.
+// FFT, cutoff, bitmaps) and the bucket chain (permute+filter of the gathers, bucket FFT, cutoff),
+// so that the latency-bound kernels of one chain fill the gaps of the other's.  Column front end:
+// the comb chain, the longer one, on the plan stream, its FFT enqueued first, and the bucket chain
+// on a second stream.  The gathering front end forks after its comb FFT (beside which its
+// permute+filter's gathers lose); the permute+filter follows on the plan stream and the comb
+// cutoff waits for the second one, so that the gathers' workgroups are spread over the chip before
+// the cutoff's take their places (the other way round the cutoff's first kernel came first and
+// crowded them: n = 2^27, k = 16000 FP64 1080 -> 942 us, FP32 828 -> 816, n = 2^20 FP64 122 -> 109).
+// Profiling (and the streaming front end, whose pass feeds the fold) runs everything serially on
+// the plan stream; with the columns the profile's "streaming pass" interval is the fold (with the
+// comb copy) and its "fold" interval is empty, and with the slab fold its "clear" interval too.
 static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, Node* d_nodes) {
   const sfft_params& p = P->p;
   sfft_status v;
@@ -663,14 +666,22 @@ static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, No
     if ((v = run_pair(P, h, P->st)) != SFFT_OK) return v;
     return run_locate(P, h, d_nodes, P->st, false);
   }
-  if (P->columns) HIPCK(hipEventRecord(P->ev_fork, P->st));
-  HIPCK(fft_run(comb_fft(P, d_x), P->st));
-  if (!P->columns) HIPCK(hipEventRecord(P->ev_fork, P->st));
-  HIPCK(hipStreamWaitEvent(P->st2, P->ev_fork, 0));
-  if (!P->columns && (v = run_fold(P, d_x, P->st2)) != SFFT_OK) return v;
-  if ((v = run_bucket(P, P->st2, false)) != SFFT_OK) return v;
-  HIPCK(hipEventRecord(P->ev_join, P->st2));
-  if ((v = run_cut(P, h, P->st, false)) != SFFT_OK) return v;
+  if (P->columns) {
+    HIPCK(hipEventRecord(P->ev_fork, P->st));
+    HIPCK(fft_run(comb_fft(P, d_x), P->st));
+    HIPCK(hipStreamWaitEvent(P->st2, P->ev_fork, 0));
+    if ((v = run_bucket(P, P->st2, false)) != SFFT_OK) return v;
+    HIPCK(hipEventRecord(P->ev_join, P->st2));
+    if ((v = run_cut(P, h, P->st, false)) != SFFT_OK) return v;
+  } else {
+    HIPCK(fft_run(comb_fft(P, d_x), P->st));
+    HIPCK(hipEventRecord(P->ev_fork, P->st));
+    if ((v = run_fold(P, d_x, P->st)) != SFFT_OK) return v;
+    HIPCK(hipStreamWaitEvent(P->st2, P->ev_fork, 0));
+    if ((v = run_cut(P, h, P->st2, false)) != SFFT_OK) return v;
+    HIPCK(hipEventRecord(P->ev_join, P->st2));
+    if ((v = run_bucket(P, P->st, false)) != SFFT_OK) return v;
+  }
   HIPCK(hipStreamWaitEvent(P->st, P->ev_join, 0));
   return run_locate(P, h, d_nodes, P->st, false);
 }
