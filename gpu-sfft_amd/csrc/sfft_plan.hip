@@ -567,6 +567,15 @@ static bool paired(const sfft_plan* P) {
          fft_pair_applies(comb_fft(P, nullptr), bucket_fft(P));
 }
 
+// Whether the two chains of a column transform run one behind the other on the plan stream: signals
+// of up to 16 MB, whose kernels end before the host has enqueued the next ones, so that the events
+// around a second stream (four calls of some 14) cost more than the overlap gains (two streams ->
+// one, waited for: 4 MB 95 -> 70 us, 8 MB 105 -> 99, 16 MB 108 -> 105 FP32 and 105 -> 91 FP64; 32 MB
+// 107 -> 101 FP64 but 111 -> 120 FP32; 64 MB 112 -> 116).
+static bool one_stream(const sfft_plan* P) {
+  return P->columns && (size_t)P->p.n * (P->fp32 ? 8 : 16) <= ((size_t)16 << 20);
+}
+
 // both FFTs, then both cutoffs (with the approved-residue bitmaps)
 static sfft_status run_pair(sfft_plan* P, const HashArgs& h, hipStream_t st) {
   const sfft_params& p = P->p;
@@ -664,6 +673,12 @@ static sfft_status run_rest(sfft_plan* P, const void* d_x, const HashArgs& h, No
   }
   if (paired(P)) {
     if ((v = run_pair(P, h, P->st)) != SFFT_OK) return v;
+    return run_locate(P, h, d_nodes, P->st, false);
+  }
+  if (one_stream(P)) {
+    HIPCK(fft_run(comb_fft(P, d_x), P->st));
+    if ((v = run_cut(P, h, P->st, false)) != SFFT_OK) return v;
+    if ((v = run_bucket(P, P->st, false)) != SFFT_OK) return v;
     return run_locate(P, h, d_nodes, P->st, false);
   }
   if (P->columns) {
