@@ -820,8 +820,10 @@ static hipError_t dispatch_pass(const PassArgs& A, int load, int store, int tw, 
 // quarter still holds whole lines of 128 bytes per row (complex64 sub-FFTs of up to 128 points,
 // complex128 of up to 64; 2^24 points as transforms of 2^12, complex64 256 -> 101 us,
 // complex128 274 -> 208; of 2^13 and 2^14, complex64 211 -> 111 and 145 -> 111; a complex128 tile
-// that 128-point sub-FFTs fill stays full: 215 against 223 at 2^14); and, with half lines, where
-// the launch would be fewer than 128 full tiles, half the CUs.
+// that 128-point sub-FFTs fill stays full: 215 against 223 at 2^14), unless the pass counts its keys'
+// histogram, whose 4096 bins are cleared and added up once per tile (two combs of 2^23 complex64
+// points: 167 us in quarter tiles, 119 in full ones); and, with half lines, where the launch
+// would be fewer than 128 full tiles, half the CUs.
 struct PassShape {
   int log2q, small_tile;
 };
@@ -843,7 +845,8 @@ static PassShape pass_shape(const FftTables& T, const FftLaunch& L, int p, int r
   const int line = T.is_fp32 ? 4 : 3;
   const long long tiles = ((long long)L.batch << T.log2n) >> (nf + r);
   const bool fits = ((1 << nf) << r) <= cap / 4;
-  const bool lines = ((1 << nf) << r) < cap && nq >= (line < nf ? line : nf);
+  const bool counts = p == T.npass - 1 && L.hist;
+  const bool lines = !counts && ((1 << nf) << r) < cap && nq >= (line < nf ? line : nf);
   const bool idle = tiles < 128 && nq >= (line - 1 < nf ? line - 1 : nf);
   if (fits || lines || idle) return {quarter, 1};
   return {full, 0};
